@@ -4,6 +4,14 @@
 namespace {
 using namespace dt;
 
+// The general kernel writes scale bytes one by one and no padding: the blocked buffer starts out as zeros
+int zero_blocked_padding(uint8_t* scale, int64_t SR, int64_t SC, hipStream_t s) {
+  if (SR % 128 == 0 && SC % 4 == 0) return DT_OK;  // the cast writes every byte
+  const int64_t n = dt_blocked_scale_bytes(SR, SC);
+  fill_bytes_kernel<<<(unsigned)std::min<int64_t>(ceil_div(n, 256), 4096), 256, 0, s>>>(scale, n, 0);
+  return launch_status();
+}
+
 struct MxArgs {
   const void* x;
   int64_t rows, cols;
@@ -104,6 +112,9 @@ int launch_mx(const MxArgs& a) {
   }
   const int64_t total = outer * inner_blocks;
   if (ceil_div(total, kBlock) > 0x7FFFFFFFll) return DT_ERR_INVALID_SHAPE;
+  if constexpr (LAYOUT == DT_SCALE_BLOCKED) {
+    if (int st = zero_blocked_padding(a.scale, outer, inner_blocks, a.stream)) return st;
+  }
   mx_any_kernel<IN, OUT, LAYOUT><<<(unsigned)ceil_div(total, kBlock), kBlock, 0, a.stream>>>(
       a.x, outer, inner_blocks, xos, xes, dos, des, s_rows, s_cols, s_t, a.data, a.scale);
   return launch_status();
@@ -148,12 +159,6 @@ int launch_dual_in(const DualArgs& a, int out_dtype, int layout) {
   return layout == DT_SCALE_BLOCKED ? launch_dual<IN, DT_E5M2, DT_SCALE_BLOCKED>(a) : launch_dual<IN, DT_E5M2, DT_SCALE_PLAIN>(a);
 }
 
-int zero_blocked_padding(uint8_t* scale, int64_t SR, int64_t SC, hipStream_t s) {
-  if (SR % 128 == 0 && SC % 4 == 0) return DT_OK;  // the cast writes every byte
-  const int64_t n = dt_blocked_scale_bytes(SR, SC);
-  dt::fill_bytes_kernel<<<(unsigned)std::min<int64_t>(dt::ceil_div(n, 256), 4096), 256, 0, s>>>(scale, n, 0);
-  return dt::launch_status();
-}
 }  // namespace
 
 extern "C" int64_t dt_blocked_scale_bytes(int64_t R, int64_t C) {
@@ -175,9 +180,6 @@ extern "C" int dt_mx_fp8_quantize(const void* x, int in_dtype, int64_t rows, int
   if (!x || !data || !scale) return DT_ERR_NULL_POINTER;
   if (!dt::aligned(x, in_dtype == DT_F32 ? 4 : 2)) return DT_ERR_MISALIGNED;
   hipStream_t s = dt::as_hip(stream);
-  if (scale_layout == DT_SCALE_BLOCKED) {  // zero the padding the cast itself never writes
-    if (int st = zero_blocked_padding(scale, axis == 1 ? rows : cols, (axis == 1 ? cols : rows) / 32, s)) return st;
-  }
   MxArgs a{x, rows, cols, axis, transpose, static_cast<uint8_t*>(data), scale, s};
   switch (in_dtype) {
     case DT_F32: return launch_mx_in<DT_F32>(a, out_dtype, scale_layout);
@@ -200,10 +202,6 @@ extern "C" int dt_mx_fp8_quantize_dual(const void* x, int in_dtype, int64_t rows
   DualArgs a{x, rows, cols, static_cast<uint8_t*>(data_rows), scale_rows, static_cast<uint8_t*>(data_cols_t), scale_cols_t, s};
   const bool fast_ok = dt::tuning("mx.dual") != 0;
   if (fast_ok) {
-    if (scale_layout == DT_SCALE_BLOCKED) {
-      if (int st = zero_blocked_padding(scale_rows, rows, cols / 32, s)) return st;
-      if (int st = zero_blocked_padding(scale_cols_t, cols, rows / 32, s)) return st;
-    }
     int st;
     switch (in_dtype) {
       case DT_F32: st = launch_dual_in<DT_F32>(a, out_dtype, scale_layout); break;
@@ -279,9 +277,6 @@ extern "C" int dt_mx_fp4_quantize(const void* x, int in_dtype, int64_t rows, int
     if (cols % 4 != 0 || rows >= (1ll << 31) || cols >= (1ll << 31)) return DT_ERR_INVALID_SHAPE;
     if (!dt::aligned(x, 4 * kB) || (cols * kB) % (4 * kB) != 0 || !dt::aligned(data, 16) || !dt::aligned(scale, 4))
       return DT_ERR_MISALIGNED;
-    if (blocked) {
-      if (int st = zero_blocked_padding(scale, cols, rows / 32, s)) return st;
-    }
     MxArgs a{x, rows, cols, 0, 1, static_cast<uint8_t*>(data), scale, s};
     switch (in_dtype) {
       case DT_F32: return blocked ? launch_mx_fp4_cols<DT_F32, DT_SCALE_BLOCKED>(a) : launch_mx_fp4_cols<DT_F32, DT_SCALE_PLAIN>(a);
@@ -291,9 +286,6 @@ extern "C" int dt_mx_fp4_quantize(const void* x, int in_dtype, int64_t rows, int
   }
   if (rows * cols / 32 >= (1ll << 28)) return DT_ERR_INVALID_SHAPE;  // block indices are 32 bits wide in the kernel
   if (!dt::aligned(x, 16) || !dt::aligned(data, 4)) return DT_ERR_MISALIGNED;
-  if (blocked) {
-    if (int st = zero_blocked_padding(scale, rows, cols / 32, s)) return st;
-  }
   MxArgs a{x, rows, cols, 1, 0, static_cast<uint8_t*>(data), scale, s};
   switch (in_dtype) {
     case DT_F32: return blocked ? launch_mx_fp4<DT_F32, DT_SCALE_BLOCKED>(a) : launch_mx_fp4<DT_F32, DT_SCALE_PLAIN>(a);
@@ -337,10 +329,6 @@ extern "C" int dt_mx_fp4_quantize_dual(const void* x, int in_dtype, int64_t rows
   hipStream_t s = dt::as_hip(stream);
   DualArgs a{x, rows, cols, static_cast<uint8_t*>(data_rows), scale_rows, static_cast<uint8_t*>(data_cols_t), scale_cols_t, s};
   if (dt::tuning("mx.dual") != 0) {
-    if (scale_layout == DT_SCALE_BLOCKED) {
-      if (int st = zero_blocked_padding(scale_rows, rows, cols / 32, s)) return st;
-      if (int st = zero_blocked_padding(scale_cols_t, cols, rows / 32, s)) return st;
-    }
     int st;
     switch (in_dtype) {
       case DT_F32: st = launch_dual_fp4_in<DT_F32>(a, scale_layout); break;
@@ -359,12 +347,10 @@ extern "C" int dt_to_blocked(const uint8_t* scale, int64_t R, int64_t C, uint8_t
   if (R == 0 || C == 0) return DT_OK;
   if (!scale || !out) return DT_ERR_NULL_POINTER;
   hipStream_t s = dt::as_hip(stream);
-  if (R % 128 != 0 || C % 4 != 0) {
-    const int64_t n = dt_blocked_scale_bytes(R, C);
-    dt::fill_bytes_kernel<<<(unsigned)std::min<int64_t>(dt::ceil_div(n, 256), 4096), 256, 0, s>>>(out, n, 0);
-    if (int st = dt::launch_status()) return st;
-  }
+  const int64_t groups = dt_blocked_scale_bytes(R, C) / 16;
   if (dt::ceil_div(R * C, 256) > 0x7FFFFFFFll) return DT_ERR_INVALID_SHAPE;
-  dt::to_blocked_kernel<<<(unsigned)dt::ceil_div(R * C, 256), 256, 0, s>>>(scale, R, C, out);
+  const unsigned grid = (unsigned)std::min<int64_t>(dt::ceil_div(groups, (int64_t)dt::kBlock), (int64_t)dt::device_facts().cu_count * 16);
+  if (C % 4 == 0 && dt::aligned(scale, 4)) dt::to_blocked_kernel<true><<<grid, dt::kBlock, 0, s>>>(scale, R, C, groups, out);
+  else dt::to_blocked_kernel<false><<<grid, dt::kBlock, 0, s>>>(scale, R, C, groups, out);
   return dt::launch_status();
 }

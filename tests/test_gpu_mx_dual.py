@@ -184,3 +184,50 @@ def test_transposed_column_cast_both_kernels(d, cabi, shape, in_dtype):
             assert torch.equal(util.codes(data), cd) and torch.equal(util.codes(scale), cs.flatten())
             data, scale = d.mx_fp8_quantize_blocked(g, 0, out_dtype)
             assert torch.equal(util.codes(data), cd) and torch.equal(util.codes(scale), co.to_blocked(cs))
+
+
+@pytest.mark.parametrize("shape", [(1, 32), (33, 96), (127, 160), (129, 64), (32, 32), (96, 416), (160, 288), (384, 512)],
+                         ids=lambda s: f"{s[0]}x{s[1]}")
+@pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
+def test_blocked_casts_write_their_padding_and_nothing_else(cabi, gpu_device, shape, in_dtype):
+    """Every cast with blocked scales into a buffer full of 0xAB: the padding rows and columns come out as
+    zeros, the bytes around the buffer stay (both whole words and a buffer one byte off, where it may be)."""
+    R, C = shape
+    x = _wide_range(shape, 77, in_dtype).to(gpu_device)
+
+    def blocked(off, R_, C_):
+        n = cabi.lib().dt_blocked_scale_bytes(R_, C_)
+        whole = torch.full((n + 64,), 0xAB, dtype=torch.uint8, device=gpu_device)
+        return whole, whole[16 + off:16 + off + n]
+
+    def check(whole, part, plain, R_, C_):
+        want = co.to_blocked(plain.view(torch.uint8).view(R_, C_).cpu())
+        assert torch.equal(part.cpu(), want)
+        off = part.storage_offset()
+        assert (whole[:off] == 0xAB).all() and (whole[off + part.numel():] == 0xAB).all()
+
+    for off in (0, 1):
+        w, s = blocked(off, R, C // 32)
+        cabi.mx_fp8_quantize(x, layout=cabi.SCALE_BLOCKED, scale=s)
+        check(w, s, cabi.mx_fp8_quantize(x)[1], R, C // 32)
+        w, s = blocked(off, R, C // 32)
+        cabi.mx_fp4_quantize(x, layout=cabi.SCALE_BLOCKED, scale=s)
+        check(w, s, cabi.mx_fp4_quantize(x)[1], R, C // 32)
+    plain = cabi.mx_fp8_quantize(x)[1].view(torch.uint8).view(R, C // 32)
+    for src in (plain, torch.cat([plain.flatten().new_zeros(1), plain.flatten()])[1:].view(R, C // 32)):
+        assert torch.equal(cabi.to_blocked(src).cpu(), co.to_blocked(plain.cpu()))
+    if R % 32:
+        return
+    w, s = blocked(0, C, R // 32)
+    cabi.mx_fp8_quantize(x, axis=0, transpose=True, layout=cabi.SCALE_BLOCKED, scale=s)
+    check(w, s, cabi.mx_fp8_quantize(x, axis=0, transpose=True)[1], C, R // 32)
+    w, s = blocked(0, C, R // 32)
+    cabi.mx_fp4_quantize(x, layout=cabi.SCALE_BLOCKED, scale=s, axis=0)
+    check(w, s, cabi.mx_fp4_quantize(x, axis=0)[1], C, R // 32)
+    for both, one in ((cabi.mx_fp8_quantize_dual, lambda a: cabi.mx_fp8_quantize(x, axis=a, transpose=a == 0)),
+                      (cabi.mx_fp4_quantize_dual, lambda a: cabi.mx_fp4_quantize(x, axis=a))):
+        (wr, sr), (wc, sc) = blocked(0, R, C // 32), blocked(0, C, R // 32)
+        dr, dc = torch.empty_like(one(1)[0]), torch.empty_like(one(0)[0])
+        both(x, layout=cabi.SCALE_BLOCKED, outs=(dr, sr, dc, sc))
+        check(wr, sr, one(1)[1], R, C // 32)
+        check(wc, sc, one(0)[1], C, R // 32)
