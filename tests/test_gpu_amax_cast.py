@@ -299,6 +299,33 @@ def test_rowwise_shapes(d, in_dtype, fp8_dtype, shape):
 
 
 @pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vecs", [1, 2, 64, 65, 256, 257, 1024, 1025])
+def test_rowwise_rows_between_vectors(d, cabi, in_dtype, vecs):
+    """Widths one element short of, past, and in the middle of a whole number of vectors, so that rows start
+    at every place inside a vector: maxima and NaN in the first and last element of a row, which single lanes
+    take, and nothing written outside the output."""
+    kv = 8 if in_dtype == torch.bfloat16 else 4
+    for extra in (1, kv // 2, kv - 1):
+        cols, rows = vecs * kv + extra, 2 * kv + 3
+        a = util.rows_log_uniform_sigma((rows, cols), 91 + cols, in_dtype)
+        a[0::4, 0], a[1::4, cols - 1], a[5, 0], a[6, cols - 1] = 3.0e4, -3.0e4, float("nan"), float("inf")
+        x = a.cuda()
+        for fp8_dtype in FP8:
+            ref, ramax, rscale = co.dynamic_scaled_quant_rowwise(a, fp8_dtype)
+            whole = torch.full((rows * cols + 64,), 0xAB, dtype=torch.uint8, device="cuda")
+            out = whole[32:32 + rows * cols].view(rows, cols)
+            amax, scale = torch.empty(rows, 1, device="cuda"), torch.empty(rows, 1, device="cuda")
+            st = cabi.lib().dt_dynamic_scaled_quant_rowwise(x.data_ptr(), cabi.IN_DTYPE[in_dtype], rows, cols, cabi.OUT_DTYPE[fp8_dtype],
+                                                            out.data_ptr(), amax.data_ptr(), scale.data_ptr(),
+                                                            torch.cuda.current_stream().cuda_stream)
+            assert st == 0
+            assert torch.equal(amax.cpu().view(torch.int32), ramax.view(torch.int32))
+            assert torch.equal(scale.cpu().view(torch.int32), rscale.view(torch.int32))
+            assert torch.equal(util.codes(out), ref)
+            assert (whole[:32] == 0xAB).all() and (whole[-32:] == 0xAB).all()
+
+
+@pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("extra", [0, 3])
 @pytest.mark.parametrize("vecs", [1, 40, 257, 300, 512, 513, 1024, 1030, 2048, 2500, 4096, 4100, 8192, 8193, 9000, 16384, 16385])
 def test_rowwise_long_rows(d, in_dtype, vecs, extra):
