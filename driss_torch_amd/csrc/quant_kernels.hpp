@@ -188,9 +188,19 @@ inline int reduction_grid(int64_t nvec, int unroll, const char* knob) {
   return want < 1 ? 1 : (int)want;
 }
 
-// Enqueue the amax reduction.  nscales: 0 = amax only, 1 = scale for fmax0, 2 = both.  With
-// scales a cast pass over the same tensor follows, so the loads are left cacheable unless
-// the "amax.stream_before_cast" knob says otherwise.
+// Enqueue the amax reduction.  nscales: 0 = amax only, 1 = scale for fmax0, 2 = both.
+//
+// Streaming or cacheable loads: a cast of the same tensor follows nearly every reduction (always when
+// scales are asked for), and its workgroups walk the tensor in the reduction's order, so that a run of
+// vectors is read by the same XCD both times and comes out of that XCD's L2 if the first read left it
+// there (or out of the memory-side cache, which streaming loads pass by).  The eight L2s hold 32 MiB.
+// Up to that size cacheable loads cost the reduction nothing (us, rotated buffers, streaming -> cacheable,
+// alone: bf16 16 MiB 8.1 -> 8.0, 32 MiB 10.3 -> 9.8; fp32 32 MiB 10.1 -> 9.8) and the cast behind it gains
+// (both: bf16 8 MiB 10.9 -> 9.4, 16 MiB 13.5 -> 11.6, 32 MiB 19.6 -> 15.0; fp32 32 MiB 18.1 -> 13.3); above it
+// a reduction alone is 3 to 10 % faster with streaming loads (48 MiB 12.2 -> 12.6, 128 MiB 22.1 -> 23.3,
+// 428 MiB 64.7 -> 71.4).  With scales they are cacheable at any size: the sum of both kernels is never
+// longer (128 MiB 54.5 -> 51.5, 428 MiB 169.5 -> 169.8); the knob "amax.stream_before_cast" says otherwise.
+constexpr int64_t kAmaxCacheableBytes = (int64_t)32 << 20;
 template <int IN>
 inline int launch_amax(const void* x, int64_t numel, void* ws, float* amax_out, float* scale_out, int nscales,
                        float fmax0, float fmax1, hipStream_t stream) {
@@ -198,10 +208,10 @@ inline int launch_amax(const void* x, int64_t numel, void* ws, float* amax_out, 
   Split sp = split_for_vectors<IN>(x, numel);
   int grid = reduction_grid(sp.nvec, kUnroll, "amax.blocks_per_cu");
   uint8_t* w = static_cast<uint8_t*>(ws);
-  const bool nt = nscales == 0 || tuning("amax.stream_before_cast");
+  const bool nt = nscales == 0 ? numel * InTraits<IN>::kBytes > kAmaxCacheableBytes : tuning("amax.stream_before_cast") != 0;
   uint64_t* const log = phase_log((size_t)grid * 32);
 #define DT_AMAX(NS, NT) amax_kernel<IN, kUnroll, NS, NT><<<grid, kBlock, 0, stream>>>(x, sp, w, amax_out, scale_out, fmax0, fmax1, log)
-  if (nscales == 0) DT_AMAX(0, true);
+  if (nscales == 0) { if (nt) DT_AMAX(0, true); else DT_AMAX(0, false); }
   else if (nscales == 1) { if (nt) DT_AMAX(1, true); else DT_AMAX(1, false); }
   else { if (nt) DT_AMAX(2, true); else DT_AMAX(2, false); }
 #undef DT_AMAX
