@@ -34,7 +34,7 @@ struct Knob {
 //   mx.colt_pipe: the transposed column cast as a grid of this many workgroups per CU that walk the tiles
 //                 with the next tile's loads in flight (0 = one workgroup per tile)
 //   mx.row_band4: 1 = row-wise MX cast with blocked scales walks 4 rows x 512 elements per wave pass
-//   gemm.variant: 0 = pick the tile by problem size, 1 = 128x128 tiles, 2 = 256x256 tiles,
+//   gemm.variant: 0 = pick the tile by problem size, 1 = 128x128 tiles, 2 = 256x256 tiles, 5 = 256x192 tiles,
 //                 7 = 256x256 tiles without the L2 prefetch loads, 9 = the kernel for at most 64 rows
 //                 whatever the other dimensions
 //   gemm.few_rows_tiles: 16-column tiles per wave of that kernel: 0 = by the number of columns, 1, 2

@@ -24,12 +24,19 @@
 
 #include <atomic>
 #include <type_traits>
+#include <utility>
 
 #include "dt_device.hpp"
 #include "dt_host.hpp"
 #include "mx_few_rows.hpp"
 
 namespace dt {
+
+// f(0), f(1), ... f(N - 1) with the index as a compile-time constant
+template <typename F, int... I>
+__device__ __forceinline__ void unrolled_for(F& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -95,6 +102,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;  // wave tile
   constexpr int TM = WM / 16, TN = WN / 16;            // MFMA tiles per wave
   constexpr int KC = FP4 ? 2 : 1;                      // 128-element MFMAs (and blocked scale chunks) per K-step
+  constexpr bool HELD = TOUCH && MODE == kPlain;  // the main loop's schedule, see there
 
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   constexpr int kGroupsA = BM / kGroupRows, kGroupsB = BN / kGroupRows;
@@ -105,7 +113,9 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   constexpr int kWaves = WAVES_M * WAVES_N;
   constexpr int kLoadsA = kGroupsA / kWaves, kLoadsB = kGroupsB / kWaves;  // DMA loads per wave and step
   static_assert(kLoadsA * kWaves == kGroupsA && kLoadsB * kWaves == kGroupsB, "tile/waves mismatch");
-  static_assert(BM % 128 == 0 && BN % 128 == 0 && BM <= 256 && BN <= 256, "scale chunks are 128 rows");
+  static_assert(BM % 128 == 0 && BM <= 256 && BN <= 256, "scale chunks are 128 rows");
+  // A 192-column tile starts on a chunk of 128 scale rows or in the middle of one: it spans two either way
+  static_assert(BN % 128 == 0 || BN == 192, "a tile's scales are two chunks at most");
 
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -274,22 +284,22 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   // the XCD that asks for it.  So each workgroup also "touches" lines of a K-step further ahead
   // with one 4-byte LDS-DMA load per wave (no register destination; the bytes land in a dump
   // area nobody reads).  The 4 tile columns that share an A panel inside an XCD (and the 8 tile
-  // rows that share a B panel) split the panel's lines between them: 64 lines of A and 32 of B
-  // per workgroup and step, 96 / waves per wave.  A line nobody touched is merely slower.
+  // rows that share a B panel) split the panel's lines between them: 64 lines of A and BN / 8 of B
+  // per workgroup and step, an equal share per wave.  A line nobody touched is merely slower.
   constexpr int kTouch = TOUCH ? 1 : 0;       // touch loads per wave and step
   constexpr int kTouchAhead = 2;              // K-steps ahead of the stage refill
   constexpr int kVmPerStep = kLoadsPerStep + kTouch;
   const uint8_t* touch_ptr = A;
   if constexpr (TOUCH) {
-    static_assert(BM == 256 && BN == 256 && 96 % kWaves == 0, "touch shares are laid out for the 256 x 256 tile");
-    constexpr int kTouchLines = 96 / kWaves;  // per wave
-    const int idx = wave * kTouchLines + (lane < kTouchLines ? lane : kTouchLines - 1);  // 0..95: 64 lines of A, then 32 of B
+    static_assert(BM == 256 && (64 + BN / 8) % kWaves == 0, "touch shares are laid out for tiles of 256 rows");
+    constexpr int kTouchLines = (64 + BN / 8) / kWaves;  // per wave
+    const int idx = wave * kTouchLines + (lane < kTouchLines ? lane : kTouchLines - 1);  // 64 lines of A, then BN / 8 of B
     if (idx < 64) {
       int r = m0 + (tile_n & 3) * 64 + idx;
       r = r < M ? r : M - 1;
       touch_ptr = A + (int64_t)r * lda;
     } else {
-      int r = n0 + (tile_m & 7) * 32 + (idx - 64);
+      int r = n0 + (tile_m & 7) * (BN / 8) + (idx - 64);
       r = r < N ? r : N - 1;
       touch_ptr = B + (int64_t)r * ldb;
     }
@@ -355,6 +365,15 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   struct HalfWords {
     uint32_t w[KC][4];  // [chunk of the step][tile of the half]
   };
+  // 192-column tiles: where the words of the wave's tile t start in the slot (the same for the whole wave)
+  uint32_t sc_tile_b[6] = {};
+  if constexpr (TN == 6) {
+#pragma unroll
+    for (int t = 0; t < 6; ++t) {
+      const int T = ((n0 & 127) >> 4) + wn * 6 + t;
+      sc_tile_b[t] = (uint32_t)((T >> 3) * 512 + (T & 1) * 256 + ((T & 7) >> 1) * 4);
+    }
+  }
   // BYTES (e4m3, and only for scales that are used in the basic block that loads them, i.e. in the step
   // they belong to): each lane reads the one byte it needs, the K-block lane / 16 of its row's word, and
   // nothing has to be shifted.  Across the loop's back edge the compiler would move the byte's zero
@@ -366,7 +385,14 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
     HalfWords r;
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
-      if constexpr (BYTES) {
+      if constexpr (H == 3) {  // tiles of any parity: a read each
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+          const uint32_t at = o + c * 1024 + sc_tile_b[half * 3 + t];
+          if constexpr (BYTES) r.w[c][t] = lds[at];
+          else r.w[c][t] = *reinterpret_cast<const uint32_t*>(lds + at);
+        }
+      } else if constexpr (BYTES) {
         if constexpr (H == 4) {
           r.w[c][0] = lds[o + c * 1024 + half * 8];       r.w[c][1] = lds[o + c * 1024 + 256 + half * 8];
           r.w[c][2] = lds[o + c * 1024 + half * 8 + 4];   r.w[c][3] = lds[o + c * 1024 + 256 + half * 8 + 4];
@@ -398,7 +424,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   // their shifts over there, between the last MFMA of one step and the first of the next.  An empty
   // statement that reads the value keeps the shift (and the wait for the word) in the slot it is written in.
   auto pin_here = [](int v) { asm volatile("" : : "v"(v)); };
-  static_assert((TM == 8 || TM == 4) && (TN == 8 || TN == 4), "wave tile is 128 or 64 rows/columns");
+  static_assert((TM == 8 || TM == 4) && (TN == 8 || TN == 6 || TN == 4), "wave tile is 128 or 64 rows, 128, 96 or 64 columns");
 
   // Software pipeline.  Ring slot s holds K-step ks with ks % NST == s.  The TM x TN grid of MFMAs
   // of a step is cut into four quadrants over the fragment halves lo = [0, H) and hi = [H, 2H),
@@ -427,6 +453,218 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   // kScaleLast (not the quadrant's last: what follows a step's last MFMA runs with the MFMA pipe idle),
   // from words or bytes requested in slot kScaleRead (words: slot 0).
   constexpr int kScaleLast = S >= 8 ? S - 2 : S - 1, kScaleRead = S >= 8 ? 1 : 0;
+  uint64_t t_loop = 0;
+  const int a_row0 = wm * WM, b_row0 = wn * WN;
+  // only the wave's first row differs between waves: fold it into the per-lane bases
+  const uint32_t lane_lo_a = frag_lo + (a_row0 >> 3) * kGroupStride, lane_hi_a = frag_hi + (a_row0 >> 3) * kGroupStride;
+  const uint32_t lane_lo_b = frag_lo + (b_row0 >> 3) * kGroupStride, lane_hi_b = frag_hi + (b_row0 >> 3) * kGroupStride;
+  // with 4 tiles per wave the wave sits in the lower or upper 8 bytes of the 16-byte scale groups
+  const uint32_t sc_lane_a = ((a_row0 & ~127) >> 7) * 512 + l16 * 16 + kOffSA + ((TM == 4 && (wm & 1)) ? 8 : 0);
+  const uint32_t sc_lane_b = (TN == 6 ? 0 : ((b_row0 & ~127) >> 7) * 512) + l16 * 16 + kOffSB + ((TN == 4 && (wn & 1)) ? 8 : 0);
+  if constexpr (HELD) {
+    // ---- The held schedule: every B fragment of a step meets all TM fragments of A before the next one is
+    // taken up.  On random operands the launch runs at the chip's power limit, so what counts is the energy of
+    // an MFMA, and that depends on what changes between neighbours.  MFMAs alone, 16 x 16 x 128 on N(0,1)-like
+    // operands in registers, PFLOP/s e4m3 / e2m1: first operand the same for 8 of them 4.39 / 7.15, for 4
+    // 4.10 / 6.43, second operand the same for 8 3.99 / 5.97, both changed each time 3.71 / 5.47 (32 x 32 x 64:
+    // 3.71; operands of ones 4.87 whatever the order).  The quadrants below hold the first operand for 4.
+    // In a launch (us, before -> this schedule, e4m3): 8192^3 366.0 -> 359.3, 8192 x 4096 x 14336 308.1 ->
+    // 303.1, 4096 x 8192 x 4096 101.9 -> 99.2, 5120^3 108.3 -> 105.1, 2000 x 5120 x 5120 51.3 -> 49.2;
+    // e2m1: 8192^3 235.5 -> 229.7, 5120^3 70.7 -> 66.2, 2048 x 5120 x 5120 34.5 -> 30.9; with a partly filled
+    // last step 8192 x 8192 x 8160 425.4 -> 406.5 and 274.7 -> 261.0.
+    //
+    // All of A's fragments of a step are in registers, two sets of them that alternate; B's come through a
+    // ring of four.  Per step: b[0..2] were read before it began, b[3 + j] is requested when b[j] is taken
+    // up; with b[TN - 1] requested nobody needs the slot in LDS any more and the barrier follows.  Behind it
+    // come the next step's A, its b[0..2], and the refill of the slot, whose last loads go out at the start
+    // of the next step (they are waited for at its barrier, half a step later): so the LDS serves few reads
+    // while the refill lands and most reads after that.  Two steps per turn of the loop, so that the slot, the
+    // register set and every LDS address are constants.
+    constexpr int kRing = 4;                   // B fragments in registers: the one in use and three to come
+    constexpr int kBar = 8 * (TN - 4) + 5;     // time slot of the step's barrier: b[TN - 1] was requested five slots before
+    constexpr int kSlots = 8 * TN;             // time slots of a step: one e4m3 MFMA or two e2m1 MFMAs each
+    constexpr int kPostLoads = kLoadsA + kLoadsB - kLoadsB % kRun - (kLoadsB % kRun ? 0 : kRun);  // whole runs: sent before the step ends
+    static_assert(TM == 8 && NST == 2 && !SPLIT && !PARTS && TOUCH, "the held schedule");
+    Frag fa[2][TM], fb[kRing];
+    int sa[2][KC][TM], sb[KC][kRing];
+    // slot 0 and slot 1 of the LDS ring: a step's slot is known at compile time, its addresses are constants
+    const uint32_t loa[2] = {lane_lo_a, lane_lo_a + kStageBytes}, hia[2] = {lane_hi_a, lane_hi_a + kStageBytes};
+    const uint32_t lob[2] = {lane_lo_b, lane_lo_b + kStageBytes}, hib[2] = {lane_hi_b, lane_hi_b + kStageBytes};
+    const uint32_t scb_a[2] = {sc_lane_a + kq, sc_lane_a + kq + kStageBytes}, scb_b[2] = {sc_lane_b + kq, sc_lane_b + kq + kStageBytes};
+    auto read_a = [&](auto p_tag, int i) {
+      constexpr int P = decltype(p_tag)::value;
+      fa[P][i] = load_frag(loa[P], hia[P], 0, i * 16);
+    };
+    auto read_sa = [&](auto p_tag, int i) {
+      constexpr int P = decltype(p_tag)::value;
+#pragma unroll
+      for (int c = 0; c < KC; ++c) sa[P][c][i] = lds[scb_a[P] + c * 1024 + (i & 1) * 256 + (i >> 1) * 4];
+    };
+    // tile j of the step in slot P (r: its place in the ring of registers)
+    auto read_b = [&](auto p_tag, int j, int r) {
+      constexpr int P = decltype(p_tag)::value;
+      fb[r] = load_frag(lob[P], hib[P], kOffB, j * 16);
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        if constexpr (TN == 6) sb[c][r] = lds[scb_b[P] + c * 1024 + sc_tile_b[j]];
+        else sb[c][r] = lds[scb_b[P] + c * 1024 + (j & 1) * 256 + (j >> 1) * 4];
+      }
+    };
+    auto pin = [](int& v) { asm volatile("" : "+v"(v)); };
+    // KTAIL: the scale bytes of K-blocks past the end of K become 0 on both sides (see k_bytes above), here
+    // with an AND per byte once it has arrived: no branch in the loop, and no pass over the staged chunk
+    // behind a barrier of its own.  scale_mask[P]: for the step in slot P, per chunk.
+    int lane_mask[KC], scale_mask[2][KC];
+#pragma unroll
+    for (int c = 0; c < KC; ++c) lane_mask[c] = kq < K / 32 - (tail_step * KC + c) * 4 ? 0xFF : 0;
+    auto set_mask = [&](auto p_tag, int step) __attribute__((always_inline)) {
+      constexpr int P = decltype(p_tag)::value;
+      if constexpr (KTAIL) {
+#pragma unroll
+        for (int c = 0; c < KC; ++c) scale_mask[P][c] = step == tail_step ? lane_mask[c] : 0xFF;
+      }
+    };
+    auto mask_b = [&](auto p_tag, int r) __attribute__((always_inline)) {
+      constexpr int P = decltype(p_tag)::value;
+      if constexpr (KTAIL) {
+#pragma unroll
+        for (int c = 0; c < KC; ++c) sb[c][r] &= scale_mask[P][c];
+      }
+    };
+    auto settle_sa = [&](auto p_tag) __attribute__((always_inline)) {
+      constexpr int P = decltype(p_tag)::value;
+#pragma unroll
+      for (int t = 0; t < TM; ++t)
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+          if constexpr (KTAIL) sa[P][c][t] &= scale_mask[P][c];
+          pin(sa[P][c][t]);
+        }
+    };
+    auto bases_of = [&](StepBases& at, int ks) __attribute__((always_inline)) {
+      const int kn = ks < k_steps ? ks : k_steps - 1;
+      at.a = base_a(kn);
+      at.b = base_b(kn);
+#pragma unroll
+      for (int c = 0; c < KC; ++c) at.s[c] = base_s(kn, c);
+    };
+    int ks = 0;
+    auto step = [&](auto p_tag) __attribute__((always_inline)) {
+      constexpr int P = decltype(p_tag)::value;
+      constexpr std::integral_constant<int, P> kThis{};
+      constexpr std::integral_constant<int, 1 - P> kNext{};
+      constexpr uint32_t kSlotThis = P * kStageBytes, kSlotNext = (1 - P) * kStageBytes;
+      StepBases head, post;
+      uint32_t tail_now = 0;
+      (void)tail_now;
+      __builtin_amdgcn_sched_barrier(0);
+      auto slot = [&](auto m_tag) __attribute__((always_inline)) {
+        constexpr int m = decltype(m_tag)::value;
+        constexpr int j = m / (8 * KC), c = (m / 8) % KC, i = m % 8, r = (P * TN + j) % kRing;
+        if constexpr (!FP4) {
+          const v8i vb = __builtin_shufflevector(fb[r].lo, fb[r].hi, 0, 1, 2, 3, 4, 5, 6, 7);
+          const v8i va = __builtin_shufflevector(fa[P][i].lo, fa[P][i].hi, 0, 1, 2, 3, 4, 5, 6, 7);
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(vb, va, acc[i][j], 0, 0, 0, sb[0][r], 0, sa[P][0][i]);
+        } else {
+          const v4i pb = c == 0 ? fb[r].lo : fb[r].hi, pa = c == 0 ? fa[P][i].lo : fa[P][i].hi;
+          asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0] cbsz:4 blgp:4"
+                       : "+a"(acc[i][j])
+                       : "v"(pb), "v"(pa), "v"(sb[c][r]), "v"(sa[P][c][i]));
+        }
+        if constexpr (m % KC != KC - 1) {
+          __builtin_amdgcn_sched_barrier(0);
+          return;
+        }
+        constexpr int z = m / KC;  // the time slot that ends here
+        // B: three fragments ahead of the one in use, of this step and then of the next
+        if constexpr (z % 8 == 0) {
+          constexpr int jn = z / 8 + 3;
+          if constexpr (jn < TN) read_b(kThis, jn, (P * TN + jn) % kRing);
+          else read_b(kNext, jn - TN, (P * TN + jn) % kRing);
+        }
+        // the rest of the refill of the other slot (step ks + 1), begun behind the last barrier
+        if constexpr (z == 0) { bases_of(head, ks + 1); asm volatile("" : : "s"(head.b), "s"(head.s[0])); }
+        if constexpr (z % 2 == 1) {
+          constexpr int n = kPostLoads + z / 2;
+          if constexpr (n < kLoadsPerStep) fetch_one(n, head, kSlotNext, 0u);
+          else if constexpr (n == kLoadsPerStep) touch(ks + 1 + kTouchAhead);
+        }
+        if constexpr (z == kBar - 8) {
+          bases_of(post, ks + 2);
+          asm volatile("" : : "s"(post.a), "s"(post.b));
+          if constexpr (KTAIL) tail_now = ks + 2 == tail_step ? tail_adj : 0u;
+        }
+        if constexpr (KTAIL && z > kBar - 8 && z <= kBar) {  // the next refill is the partly filled step, and so are all after it
+          constexpr int i = z - (kBar - 7);
+          offA[i] -= tail_now;
+          if constexpr (i < kLoadsB) offB[i] -= tail_now;
+        }
+        if constexpr (z % 8 == 7) {  // the B fragment of the next eight slots
+          if constexpr (z / 8 + 1 < TN) mask_b(kThis, (P * TN + z / 8 + 1) % kRing);
+          else mask_b(kNext, (P * TN + TN) % kRing);
+        }
+        if constexpr (z == kBar - 4) set_mask(kNext, ks + 1);
+        if constexpr (z == kBar) {
+          // every fragment of this step has been requested; once they are in, its slot is free, and the wait
+          // for step ks + 1 to have landed (all but the touch, the youngest) sits here too
+          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_waitcnt vmcnt(%0)" ::"n"(kTouch) : "memory");
+          __syncthreads();
+        }
+        if constexpr (z > kBar) {
+          constexpr int y = z - kBar - 1;  // 0 .. 25
+          // A of the next step: fragments at y = 0, 2, 5, 7, 10, 12, 15, 17, two scales each at 1, 3, 6, 8 (the
+          // last one is a quarter of a step old when the loop turns and waits for all of them)
+          if constexpr (y % 5 == 0 && y / 5 * 2 < TM) read_a(kNext, y / 5 * 2);
+          if constexpr (y % 5 == 2 && y / 5 * 2 + 1 < TM) read_a(kNext, y / 5 * 2 + 1);
+          if constexpr (y < 10 && (y % 5 == 1 || y % 5 == 3)) {
+            read_sa(kNext, y / 5 * 4 + (y % 5 - 1));
+            read_sa(kNext, y / 5 * 4 + (y % 5 - 1) + 1);
+          }
+          if constexpr (y % 2 == 0 && y / 2 < kPostLoads) fetch_one(y / 2, post, kSlotThis, 0u);
+          if constexpr (y == 25) settle_sa(kNext);  // (pinned: left alone the compiler moves their widening behind the loop's turn)
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      unrolled_for(slot, std::make_integer_sequence<int, kSlots * KC>{});
+      ++ks;
+    };
+    constexpr std::integral_constant<int, 0> kP0{};
+    constexpr std::integral_constant<int, 1> kP1{};
+    const bool odd = (k_steps & 1) != 0;  // then the first step runs alone, in slot 1, and the pairs start in slot 0
+    const uint32_t first = odd ? (uint32_t)kStageBytes : 0u;
+    fetch(0, first);
+    StepBases second;
+    bases_of(second, 1);
+#pragma unroll
+    for (int n = 0; n < kPostLoads; ++n) fetch_one(n, second, (uint32_t)kStageBytes - first, KTAIL && k_steps <= 2 ? tail_adj : 0u);
+    touch(2);
+    if constexpr (KTAIL) {
+      if (k_steps <= 2) tail_in_place();  // the rest of that refill, and all others
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPostLoads + 1) : "memory");
+    __syncthreads();
+    auto first_fragments = [&](auto p_tag) {
+      constexpr int P = decltype(p_tag)::value;
+#pragma unroll
+      for (int t = 0; t < 3; ++t) read_b(p_tag, t, (P * TN + t) % kRing);
+#pragma unroll
+      for (int t = 0; t < TM; ++t) { read_a(p_tag, t); read_sa(p_tag, t); }
+      set_mask(p_tag, 0);
+      mask_b(p_tag, (P * TN) % kRing);
+      settle_sa(p_tag);
+    };
+    t_loop = clock_reading();
+    if (odd) {
+      first_fragments(kP1);
+      step(kP1);
+    } else {
+      first_fragments(kP0);
+    }
+    while (ks < k_steps) {
+      step(kP0);
+      step(kP1);
+    }
+  } else {
 #pragma unroll
   for (int p = 0; p < NST; ++p) fetch(p < k_steps ? p : k_steps - 1, (uint32_t)(p * kStageBytes));
 #pragma unroll
@@ -439,13 +677,6 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
       __syncthreads();
     }
   }
-  const int a_row0 = wm * WM, b_row0 = wn * WN;
-  // only the wave's first row differs between waves: fold it into the per-lane bases
-  const uint32_t lane_lo_a = frag_lo + (a_row0 >> 3) * kGroupStride, lane_hi_a = frag_hi + (a_row0 >> 3) * kGroupStride;
-  const uint32_t lane_lo_b = frag_lo + (b_row0 >> 3) * kGroupStride, lane_hi_b = frag_hi + (b_row0 >> 3) * kGroupStride;
-  // with 4 tiles per wave the wave sits in the lower or upper 8 bytes of the 16-byte scale groups
-  const uint32_t sc_lane_a = ((a_row0 & ~127) >> 7) * 512 + l16 * 16 + kOffSA + ((TM == 4 && (wm & 1)) ? 8 : 0);
-  const uint32_t sc_lane_b = ((b_row0 & ~127) >> 7) * 512 + l16 * 16 + kOffSB + ((TN == 4 && (wn & 1)) ? 8 : 0);
   Frag fa[TM], fb[TN];
   int sa[KC][TM], sb[KC][TN];
   {
@@ -468,7 +699,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   if constexpr (KTAIL) {
     if (tail_step >= 0 && tail_step < NST) tail_in_place();
   }
-  const uint64_t t_loop = clock_reading();
+  t_loop = clock_reading();
   // What a step needs of its ring slot `cur` and of the next step's `nxt`: the slots' offsets and the
   // per-lane fragment and scale addresses in them.  They are carried from step to step (this step's
   // `nxt` set is the next step's `cur` set) and the new `nxt` set is worked out in the middle of the
@@ -629,6 +860,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
     cur = nxt; nxt = nxt2;
     cla = nla; cha = nha; clb = nlb; chb = nhb; csa = nsa; csb = nsb;
   } while (++ks < k_steps);
+  }
   // the clamped refills of the last steps may still be landing: the epilogue reuses the LDS
   // (the no-ops cover the distance an assembly-written MFMA needs before its result is read)
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_waitcnt vmcnt(0)" ::: "memory");
@@ -705,6 +937,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   // in its own LDS region (row pitch WN*2 + 16 bytes: conflict-free 8-byte writes) and reads
   // it back as 16 bytes per lane, 16 lanes per row, so a store instruction writes whole
   // 256-byte row segments.  The loop's last barrier has already retired every panel read.
+  // (the lane number is counted anew: kept from the top of the kernel it would be spilled around the loop)
+  const int elane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), e16 = elane & 15, eq = elane >> 4;
   constexpr int kEpiPitch = WN * 2 + 16;
   uint8_t* epi = lds + wave * (WM * kEpiPitch);
   // rows 16 i0 .. 16 i1 of the wave's tile: convert and park
@@ -716,13 +950,16 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
         u32x2 w;
         w.x = pack_bf16x2(acc[i][j].x, acc[i][j].y);
         w.y = pack_bf16x2(acc[i][j].z, acc[i][j].w);
-        *reinterpret_cast<u32x2*>(epi + (i * 16 + l16) * kEpiPitch + (j * 16 + kq * 4) * 2) = w;
+        *reinterpret_cast<u32x2*>(epi + (i * 16 + e16) * kEpiPitch + (j * 16 + eq * 4) * 2) = w;
       }
   };
   constexpr int kChunksPerRow = WN * 2 / 16;             // 16-byte chunks per tile row
-  constexpr int kRowsPerPass = kWave / kChunksPerRow;    // rows one store instruction covers
-  const int erow = lane / kChunksPerRow, echunk = lane % kChunksPerRow;
-  const int n = n0 + wn * WN + echunk * 8;
+  constexpr int kStripPasses = 16 * kChunksPerRow / kWave;  // store instructions per strip of 16 rows
+  static_assert(kStripPasses * kWave == 16 * kChunksPerRow, "whole instructions per strip");
+  // row of the strip and chunk of the row that pass p gives this lane (a 96-column wave tile has 12 chunks
+  // a row, so they change from pass to pass; otherwise the row moves by a constant)
+  auto pass_row = [&](int p) { return (p * kWave + elane) / kChunksPerRow; };
+  auto pass_chunk = [&](int p) { return (p * kWave + elane) % kChunksPerRow; };
   // a tile wholly inside the matrix with an aligned output (the common case): no edge tests, the
   // row pointer moves by a constant
   if (wide_stores && m0 + BM <= M && n0 + BN <= N) {
@@ -731,20 +968,22 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
     // reads behind the writes).  8192^3, us per launch on constant / random operands: all rows parked
     // first 278.3 / 380.6, in halves 276.0 / -, in quarters 274.8 / 377.8, by strips 274.3 / 376.2
     // (without any epilogue the launch takes 259 / 352: 12 of those 19 us are the stores)
-    uint16_t* dst = out + (int64_t)(m0 + wm * WM + erow) * ldo + n;
-    const int64_t pass_stride = (int64_t)kRowsPerPass * ldo;
-    const uint8_t* src = epi + erow * kEpiPitch + echunk * 16;
-    constexpr int kEpiParts = TM;
-    constexpr int kHalfTiles = TM / kEpiParts, kHalfRows = WM / kEpiParts;
-    static_assert(kHalfRows % kRowsPerPass == 0, "a store pass stays inside a part");
+    uint16_t* dst[kStripPasses];
+    const uint8_t* src[kStripPasses];
 #pragma unroll
-    for (int half = 0; half < kEpiParts; ++half) {
-      park_rows(half * kHalfTiles, (half + 1) * kHalfTiles);
+    for (int p = 0; p < kStripPasses; ++p) {
+      dst[p] = out + (int64_t)(m0 + wm * WM + pass_row(p)) * ldo + (n0 + wn * WN + pass_chunk(p) * 8);
+      src[p] = epi + pass_row(p) * kEpiPitch + pass_chunk(p) * 16;
+    }
+    const int64_t strip_stride = 16 * ldo;
+#pragma unroll
+    for (int strip = 0; strip < TM; ++strip) {
+      park_rows(strip, strip + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int r = half * kHalfRows; r < (half + 1) * kHalfRows; r += kRowsPerPass) {
-        *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(src + r * kEpiPitch);
-        dst += pass_stride;
+      for (int p = 0; p < kStripPasses; ++p) {
+        *reinterpret_cast<u32x4*>(dst[p]) = *reinterpret_cast<const u32x4*>(src[p] + strip * 16 * kEpiPitch);
+        dst[p] += strip_stride;
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -761,9 +1000,9 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   }
   park_rows(0, TM);
 #pragma unroll
-  for (int r = 0; r < WM; r += kRowsPerPass) {
-    const int row = r + erow;
-    const int m = m0 + wm * WM + row;
+  for (int p = 0; p < TM * kStripPasses; ++p) {
+    const int row = pass_row(p), echunk = pass_chunk(p);
+    const int m = m0 + wm * WM + row, n = n0 + wn * WN + echunk * 8;
     if (m >= M || n >= N) continue;
     const u32x4 v = *reinterpret_cast<const u32x4*>(epi + row * kEpiPitch + echunk * 16);
     uint16_t* dst = out + (int64_t)m * ldo + n;
@@ -890,13 +1129,26 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
   if ((variant == 9 && few_rows_fits(M, K)) || (variant == 0 && few_rows_pays(FP4, M, N, K, workspace != nullptr)))
     return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
   const int64_t tiles256 = ceil_div(M, 256) * ceil_div(N, 256);
+  // 256 x 192 tiles where they fill the chip's one round better than 256 x 256 tiles do (which leave a
+  // quarter of it idle or more).  At the chip's power limit a round of them takes 0.78 of a round of the
+  // large tiles, not 0.75, so they only pay while both are one round (us, 256 x 256 -> 256 x 192, e4m3 and
+  // e2m1: 2048 x 4352 x 4096, 136 -> 184 tiles, 38.5 -> 34.3 and 26.0 -> 23.6; 2048 x 5120 x 5120, 160 -> 216,
+  // 48.3 -> 45.3 and 30.9 -> 29.3; 2000 x 6144 x 8192, 192 -> 256, 80.0 -> 77.7 and 50.9 -> 49.2; two rounds
+  // against one and a half: 4096 x 5632 x 4096 77.9 and 77.9, 4096 x 9216 x 4096 120.9 -> 123.5).
+  const int64_t tiles192 = ceil_div(M, 256) * ceil_div(N, 192);
+  if (variant == 5 || (variant == 0 && 2 * tiles256 > device_facts().cu_count && tiles192 > tiles256 &&
+                       tiles192 <= device_facts().cu_count))
+    return launch_gemm<256, 192, 2, 2, 2, FP4, true>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
   const bool big = variant == 2 || variant == 7 || (variant == 0 && tiles256 >= device_facts().cu_count / 2);
   // <tile M, tile N, waves M, waves N, LDS ring slots, e2m1 operands>
   if (big && variant == 7) return launch_gemm<256, 256, 2, 2, 2, FP4, false>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
   // Between a quarter and half a round of 256 x 256 tiles: as 256 x 128 halves they fill the chip
   // once (0.8 of a round of tiles), as 128 x 128 tiles they would take two rounds (2 x 0.55)
+  // (rows past M make half of every tile of a matrix of at most 128 rows idle: there the 128 x 128 tiles
+  // are one round as well, 96 x 28672 x 4096 34.6 -> 30.6 us, e2m1 21.4 -> 16.9)
+  const int64_t tiles128 = ceil_div(M, 128) * ceil_div(N, 128);
   if (variant == 0 && tuning("gemm.tail_quads") != 0 && 4 * tiles256 > device_facts().cu_count &&
-      2 * tiles256 <= device_facts().cu_count)
+      2 * tiles256 <= device_facts().cu_count && tiles128 > device_facts().cu_count)
     return launch_gemm<256, 128, 2, 2, 3, FP4, false, kHalves>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, 1, nullptr,
                                                                tiles256, 0);
   if (big) {

@@ -366,6 +366,36 @@ def test_mx_gemm_random_sizes(d, cabi, variant, size):
         cabi.set_tuning("gemm.variant", 0)
 
 
+@pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
+@pytest.mark.parametrize("K", [32, 96, 128, 160, 256, 288, 384, 512, 640, 672, 1024, 1184])
+def test_mx_gemm_schedules_agree(d, cabi, fp4, K):
+    """The schedule that holds a B fragment for all of A (256 x 256 and 256 x 192 tiles) against the quadrant
+    one: every entry is summed in the same order, so the bits are the same.  One step, odd and even numbers of
+    them, partly filled last steps, tiles that start in the middle of a chunk of scales, ragged edges."""
+    M, N = 520, 776  # 192-column tiles at columns 192 (in the middle of a chunk) and 768 (8 columns in it)
+    x, w = _wide_operand((M, K), 3000 + K).cuda(), _wide_operand((N, K), 3001 + K).cuda()
+    if fp4:
+        (a, sa), (b, sb), op = d.mx_fp4_quantize(x, True), d.mx_fp4_quantize(w, True), d.mx_fp4_bf16
+    else:
+        (a, sa), (b, sb), op = d.mx_fp8_quantize_blocked(x), d.mx_fp8_quantize_blocked(w), d.mx_fp8_bf16
+    outs = {}
+    for variant in (7, 2, 5):
+        cabi.set_tuning("gemm.variant", variant)
+        try:
+            outs[variant] = op(a, b.t(), sa, sb)
+        finally:
+            cabi.set_tuning("gemm.variant", 0)
+    assert torch.isfinite(outs[7]).all() and outs[7].abs().max() > 0
+    assert torch.equal(outs[2], outs[7]) and torch.equal(outs[5], outs[7])
+
+
+def _wide_operand(shape, seed):
+    """N(0, 1) rows with scales that differ from block to block, so that a scale of the wrong row or block shows"""
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(shape, generator=g).view(shape[0], -1, 32)
+    return (x * torch.exp2(torch.randint(-6, 7, x.shape[:2] + (1,), generator=g).float())).view(shape).bfloat16()
+
+
 @pytest.mark.parametrize("splits", [0, 2, 3, 5, 16])
 @pytest.mark.parametrize("size", [(16, 2048, 256), (133, 1664, 264), (300, 1024, 136), (1, 640, 8), (64, 8192, 512),
                                   (40, 4192, 136)], ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
