@@ -59,13 +59,13 @@ __device__ __forceinline__ uint32_t fp32_bits_of(const void* x, int64_t i) {
 // folds it into a running maximum in the workspace with one atomic and takes a ticket; the
 // workgroup that draws the last ticket writes amax (and, when NSCALES > 0, the fp8 scales
 // derived from it) and re-arms the workspace for the next launch.
-template <int IN, int UNROLL, int NSCALES, bool NT>
-__global__ __launch_bounds__(kBlock) void amax_kernel(const void* __restrict__ x, Split sp,
+template <int IN, int BLOCK, int UNROLL, int NSCALES, bool NT>
+__global__ __launch_bounds__(BLOCK) void amax_kernel(const void* __restrict__ x, Split sp,
                                                       uint8_t* __restrict__ ws, float* __restrict__ amax_out,
                                                       float* __restrict__ scale_out, float fmax0, float fmax1,
                                                       uint64_t* __restrict__ phase_log) {
   constexpr int kB = InTraits<IN>::kBytes, kV = InTraits<IN>::kVec;
-  __shared__ uint32_t lds[kBlock / kWave];
+  __shared__ uint32_t lds[BLOCK / kWave];
   const int tid = threadIdx.x;
   // phase_log (only in a build with DT_PHASE_LOG, and normally null there): readings of the constant-rate
   // 100 MHz counter per workgroup -- start, share loaded, workgroup's maximum known, atomics done -- for
@@ -93,8 +93,10 @@ __global__ __launch_bounds__(kBlock) void amax_kernel(const void* __restrict__ x
   // system never runs dry between batches.  (Every load of the steady state is unconditional: the wait
   // counts the compiler derives are exact only along straight-line code.)
   constexpr int P = UNROLL / 2;
-  const int64_t stride = (int64_t)gridDim.x * kBlock, step = P * stride;
-  int64_t i = (int64_t)blockIdx.x * kBlock + tid;
+  const int64_t stride = (int64_t)gridDim.x * BLOCK, step = P * stride;
+  // a workgroup's quarters of 256 threads take runs of kBlock vectors a whole grid apart, so that run r is
+  // read by workgroup r % gridDim whatever BLOCK is, and by XCD r % 8 like in the cast that follows
+  int64_t i = ((int64_t)(tid / kBlock) * gridDim.x + blockIdx.x) * kBlock + tid % kBlock;
   auto whole_batch_at = [&](int64_t j) { return j + (P - 1) * stride < sp.nvec; };
   auto load_batch = [&](u32x4 (&w)[P], int64_t j) {
 #pragma unroll
@@ -133,7 +135,7 @@ __global__ __launch_bounds__(kBlock) void amax_kernel(const void* __restrict__ x
     if (tid < sp.head) m = umax(m, absbits_of<IN>(x, tid));
     if (tid < sp.tail) m = umax(m, absbits_of<IN>(x, sp.head + sp.nvec * kV + tid));
   }
-  m = block_umax<kBlock / kWave>(m, lds);
+  m = block_umax<BLOCK / kWave>(m, lds);
   stamp(2);
 
   // Publishing the tensor's maximum: amax, the scales derived from it, into the workspace and to the caller
@@ -180,10 +182,11 @@ __global__ __launch_bounds__(kBlock) void amax_kernel(const void* __restrict__ x
   }
 }
 
-inline int reduction_grid(int64_t nvec, int unroll, const char* knob) {
-  int64_t want = ceil_div(nvec, (int64_t)kBlock * unroll);
+inline int reduction_grid(int64_t nvec, int block, int unroll, const char* knob) {
+  int64_t want = ceil_div(nvec, (int64_t)block * unroll);
   int64_t cap = (int64_t)device_facts().cu_count * tuning(knob);
   if (cap > kMaxPartials) cap = kMaxPartials;
+  if (want > 8) want = ceil_div(want, (int64_t)8) * 8;  // whole rounds of the XCDs, see the cast
   if (want > cap) want = cap;
   return want < 1 ? 1 : (int)want;
 }
@@ -206,11 +209,19 @@ inline int launch_amax(const void* x, int64_t numel, void* ws, float* amax_out, 
                        float fmax0, float fmax1, hipStream_t stream) {
   constexpr int kUnroll = 8;
   Split sp = split_for_vectors<IN>(x, numel);
-  int grid = reduction_grid(sp.nvec, kUnroll, "amax.blocks_per_cu");
+  // Workgroups of 512 or 1024 threads where the tensor then takes few of them: a workgroup ends with two
+  // dependent atomics on one address, which the device performs one after the other, and 256 workgroups
+  // queue there for 2 us.  us with 256 / 512 / 1024 threads: bf16 2 MiB 3.9 / 3.8 / 4.0, 4 MiB 4.7 / 4.2 / 4.5,
+  // 8 MiB 7.0 / 5.2 / 4.9, 16 MiB 8.1 / 8.2 / 6.3, 32 MiB (256 workgroups again) 10.6 / 10.6 / 10.6, 128 MiB
+  // 22.4 / 22.4 / 23.1.
+  const int64_t small_blocks = ceil_div(sp.nvec, (int64_t)kBlock * kUnroll);
+  const int block = small_blocks <= 64 || small_blocks > 512 ? 256 : small_blocks <= 128 ? 512 : 1024;
+  int grid = reduction_grid(sp.nvec, block, kUnroll, "amax.blocks_per_cu");
   uint8_t* w = static_cast<uint8_t*>(ws);
   const bool nt = nscales == 0 ? numel * InTraits<IN>::kBytes > kAmaxCacheableBytes : tuning("amax.stream_before_cast") != 0;
   uint64_t* const log = phase_log((size_t)grid * 32);
-#define DT_AMAX(NS, NT) amax_kernel<IN, kUnroll, NS, NT><<<grid, kBlock, 0, stream>>>(x, sp, w, amax_out, scale_out, fmax0, fmax1, log)
+#define DT_AMAX_B(NS, NT, B) amax_kernel<IN, B, kUnroll, NS, NT><<<grid, B, 0, stream>>>(x, sp, w, amax_out, scale_out, fmax0, fmax1, log)
+#define DT_AMAX(NS, NT) do { if (block == 1024) DT_AMAX_B(NS, NT, 1024); else if (block == 512) DT_AMAX_B(NS, NT, 512); else DT_AMAX_B(NS, NT, 256); } while (0)
   if (nscales == 0) { if (nt) DT_AMAX(0, true); else DT_AMAX(0, false); }
   else if (nscales == 1) { if (nt) DT_AMAX(1, true); else DT_AMAX(1, false); }
   else { if (nt) DT_AMAX(2, true); else DT_AMAX(2, false); }
@@ -407,6 +418,10 @@ inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, vo
     const int per_cu = tuning(knob) > 0 ? tuning(knob) : (small && !PAIR ? 3 : 1);
     int64_t grid = ceil_div(nvec, (int64_t)kBlock * unroll);
     if (grid > (int64_t)device_facts().cu_count * per_cu) grid = (int64_t)device_facts().cu_count * per_cu;
+    // whole rounds of the eight XCDs: run r of kBlock vectors is then read by XCD r % 8, as in the reduction
+    // before it, and comes out of that XCD's L2 (reduction and cast, 1000 x 3000 bf16: 9.7 us
+    // with 46 and 734 workgroups, 7.9 with 48 and 736)
+    if (grid > 8) grid = ceil_div(grid, (int64_t)8) * 8;
     if (grid < 1) grid = 1;
     if (unroll == 2) cast_kernel<IN, OUT, ROUND_BF16, ROUND_SCALE, PAIR, 2><<<(unsigned)grid, kBlock, 0, stream>>>(x, nvec, tail, scale, o, o2);
     else cast_kernel<IN, OUT, ROUND_BF16, ROUND_SCALE, PAIR, 4><<<(unsigned)grid, kBlock, 0, stream>>>(x, nvec, tail, scale, o, o2);

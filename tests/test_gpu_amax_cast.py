@@ -283,6 +283,26 @@ def test_dynamic_quant_config2_full_size(d):
     assert torch.equal(util.codes(single), r4)
 
 
+@pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vecs", [1, 131072, 262144, 524288, 1048576], ids=str)
+def test_amax_between_workgroup_sizes(d, in_dtype, vecs):
+    """Tensors of as many 16-byte vectors as the largest that take workgroups of 256, 512, 1024 threads, and one
+    vector and three elements to either side of that: the maximum wherever a workgroup, a quarter of one or
+    the ragged end of the tensor begins or ends, aligned and one element off."""
+    kv = 8 if in_dtype == torch.bfloat16 else 4
+    g = torch.Generator(device="cuda").manual_seed(vecs)
+    for n in sorted({max(1, vecs * kv + k) for k in (-kv, -3, 0, 3, kv)}):
+        buf = torch.randn(n + 1, generator=g, device="cuda").to(in_dtype)
+        for x in (buf[:n].view(1, n), buf[1:].view(1, n)):
+            for at in {0, 255 * kv, 256 * kv, 1023 * kv + 1, 1024 * kv, n // 2, n // 4 * 3, n - 4, n - 1}:
+                if not 0 <= at < n:
+                    continue
+                old, value = x[0, at].clone(), 100.0 + (at % 7)
+                x[0, at] = -value
+                assert d.amax(x).item() == value, (n, at)
+                x[0, at] = old
+
+
 @pytest.mark.parametrize("fp8_dtype", FP8)
 @pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("shape", [(3, 7), (64, 8), (33, 512), (100, 4096), (5, 4097), (9, 8200), (4, 20000), (2, 131072)])
