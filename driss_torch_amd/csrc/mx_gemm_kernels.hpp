@@ -22,6 +22,7 @@
 // that the stores are whole 256-byte row segments (direct 8-byte stores cost 12% of the run).
 #pragma once
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 #include <utility>
@@ -938,7 +939,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   // it back as 16 bytes per lane, 16 lanes per row, so a store instruction writes whole
   // 256-byte row segments.  The loop's last barrier has already retired every panel read.
   // (the lane number is counted anew: kept from the top of the kernel it would be spilled around the loop)
-  const int elane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), e16 = elane & 15, eq = elane >> 4;
+  const uint32_t elane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) & 63u;
+  const int e16 = (int)(elane & 15u), eq = (int)(elane >> 4);
   constexpr int kEpiPitch = WN * 2 + 16;
   uint8_t* epi = lds + wave * (WM * kEpiPitch);
   // rows 16 i0 .. 16 i1 of the wave's tile: convert and park
@@ -958,8 +960,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   static_assert(kStripPasses * kWave == 16 * kChunksPerRow, "whole instructions per strip");
   // row of the strip and chunk of the row that pass p gives this lane (a 96-column wave tile has 12 chunks
   // a row, so they change from pass to pass; otherwise the row moves by a constant)
-  auto pass_row = [&](int p) { return (p * kWave + elane) / kChunksPerRow; };
-  auto pass_chunk = [&](int p) { return (p * kWave + elane) % kChunksPerRow; };
+  auto pass_row = [&](uint32_t p) { return (int)((p * kWave + elane) / kChunksPerRow); };
+  auto pass_chunk = [&](uint32_t p) { return (int)((p * kWave + elane) % kChunksPerRow); };
   // a tile wholly inside the matrix with an aligned output (the common case): no edge tests, the
   // row pointer moves by a constant
   if (wide_stores && m0 + BM <= M && n0 + BN <= N) {
@@ -1071,17 +1073,22 @@ int launch_gemm(const uint8_t* a, const uint8_t* b, const uint8_t* sfa, const ui
 
 inline size_t split_workspace_bytes() { return kSplitTicketBytes + (size_t)device_facts().cu_count * kSplitTileBytes; }
 
-// Split-K factor for the 128 x 128 tiling.  A grid of a third of a workgroup per CU or less leaves
+// Split-K factor for the 128 x 128 tiling.  A grid of half a workgroup per CU or less leaves
 // most of the chip idle while each workgroup walks the whole K, one K-step per memory latency / 3:
 // share K between as many workgroups per tile as fill the chip once.  What it costs is the last
 // workgroup of a tile reading every share through one CU (about 1 us per share of a full tile),
-// so a share is at least 16 K-steps and two shares are not worth it (measured on MI355X, e4m3,
-// us without -> with: 16 x 8192 x 8192 31 -> 19, 128 x 8192 x 8192 31 -> 24, 1024 x 1024 x 16384
-// 58 -> 34, 512 x 512 x 65536 219 -> 50, 128 x 128 x 16384 56 -> 25; no gain: 256 x 8192 x 8192 with
-// two shares 31.5 -> 32.4, 1024 x 1024 x 4096 with four shares of 8 steps 18.3 -> 19.3).  The knob
+// so a share is at least 16 K-steps, or 10 while there are at most four shares of a K of 5120 elements or
+// more (measured on MI355X, e4m3, B rotated through memory, us without -> with: 16 x 8192 x 8192 31 -> 19,
+// 128 x 8192 x 8192 42 -> 24, 1024 x 1024 x 16384 58 -> 34, 512 x 512 x 65536 219 -> 50, 128 x 128 x 16384
+// 56 -> 25, 128 x 5120 x 5120 with four shares of 10 steps 19.9 -> 17.5, with six 19.4, 256 x 5120 x 5120 with
+// three 22.7 -> 19.9, 256 x 4096 x 4096 with three 15.7 -> 16.4; e2m1 128 x 8192 x 8192 with three 24.5 -> 18.2).
+// Two shares pay where they fill four fifths of the chip or more and save more steps than the 8 us that
+// parking and adding a whole chip's tiles takes: from 56 steps on, or 32 when B comes from memory and each
+// step takes longer (256 x 8192 x 8192 41 -> 33, 512 x 4096 x 14336 69 -> 46, 128 x 14336 x 4096 24.8 -> 22.6;
+// not 1000 x 2048 x 6144 23.0 -> 25.4, 128 x 5120 x 5120 19.9 -> 22.1, nor e2m1 96 x 14336 x 4096 14.7 -> 16.0). The knob
 // gemm.split_k forces a factor (1 = never split); whatever is asked for, every split owns a step
 // and the workspace holds all shares.
-inline int plan_splits(int64_t M, int64_t N, int64_t k_steps, size_t workspace_bytes) {
+inline int plan_splits(bool fp4, int64_t M, int64_t N, int64_t k_steps, size_t workspace_bytes) {
   const int64_t tiles = ceil_div(M, 128) * ceil_div(N, 128);
   if (workspace_bytes <= kSplitTicketBytes || tiles > (int64_t)(kSplitTicketBytes / 4)) return 1;
   const int64_t room = (int64_t)((workspace_bytes - kSplitTicketBytes) / kSplitTileBytes) / tiles;
@@ -1091,11 +1098,12 @@ inline int plan_splits(int64_t M, int64_t N, int64_t k_steps, size_t workspace_b
     want = forced;
   } else {
     const int cus = device_facts().cu_count;
-    if (tiles * 3 > cus) return 1;
+    const int64_t shares = std::max(k_steps * (fp4 ? 2 : 1) >= 40 ? std::min<int64_t>(k_steps / 10, 4) : 0, k_steps / 16);
     want = cus / tiles;
-    if (want > k_steps / 16) want = k_steps / 16;
+    if (want > shares) want = shares;
     if (want > kAutoMaxSplits) want = kAutoMaxSplits;
-    if (want < 3) return 1;
+    const bool two_pay = tiles * 5 >= cus * 2 && (k_steps >= 56 || (k_steps >= 32 && N * k_steps * kBK >= ((int64_t)32 << 20)));
+    if (want < 2 || (want == 2 && !two_pay)) return 1;
   }
   if (want > kMaxSplits) want = kMaxSplits;
   if (want > room) want = room;
@@ -1176,7 +1184,7 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
     }
     return launch_gemm<256, 256, 2, 2, 2, FP4, true>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
   }
-  const int splits = workspace ? plan_splits(M, N, ceil_div(k_bytes, (int64_t)kBK), workspace_bytes) : 1;
+  const int splits = workspace ? plan_splits(FP4, M, N, ceil_div(k_bytes, (int64_t)kBK), workspace_bytes) : 1;
   if (splits > 1)
     return launch_gemm<128, 128, 2, 2, 4, FP4, false, kSplitK>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, splits, workspace);
   return launch_gemm<128, 128, 2, 2, 4, FP4, false>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
