@@ -3,6 +3,8 @@
 // amax.hip, saturated_cast.hip and dynamic_scaled_quant.hip.
 #pragma once
 
+#include <algorithm>
+
 #include "dt_device.hpp"
 #include "dt_host.hpp"
 
@@ -196,27 +198,33 @@ inline int reduction_grid(int64_t nvec, int block, int unroll, const char* knob)
 // Streaming or cacheable loads: a cast of the same tensor follows nearly every reduction (always when
 // scales are asked for), and its workgroups walk the tensor in the reduction's order, so that a run of
 // vectors is read by the same XCD both times and comes out of that XCD's L2 if the first read left it
-// there (or out of the memory-side cache, which streaming loads pass by).  The eight L2s hold 32 MiB.
-// Up to that size cacheable loads cost the reduction nothing (us, rotated buffers, streaming -> cacheable,
-// alone: bf16 16 MiB 8.1 -> 8.0, 32 MiB 10.3 -> 9.8; fp32 32 MiB 10.1 -> 9.8) and the cast behind it gains
-// (both: bf16 8 MiB 10.9 -> 9.4, 16 MiB 13.5 -> 11.6, 32 MiB 19.6 -> 15.0; fp32 32 MiB 18.1 -> 13.3); above it
-// a reduction alone is 3 to 10 % faster with streaming loads (48 MiB 12.2 -> 12.6, 128 MiB 22.1 -> 23.3,
-// 428 MiB 64.7 -> 71.4).  With scales they are cacheable at any size: the sum of both kernels is never
-// longer (128 MiB 54.5 -> 51.5, 428 MiB 169.5 -> 169.8); the knob "amax.stream_before_cast" says otherwise.
-constexpr int64_t kAmaxCacheableBytes = (int64_t)32 << 20;
+// there, or out of the memory-side cache, which streaming loads pass by.  Up to 40 MiB a reduction alone
+// is not slower with cacheable loads than it was with streaming ones from 256 workgroups, and the cast behind
+// it gains (us, rotated buffers, that -> here; alone: 16 MiB 8.1 -> 6.8, 32 MiB 10.3 -> 9.5, 40 MiB 11.35 -> 10.8;
+// both kernels of delayed scaling: bf16 8 MiB 10.9 -> 8.1, 16 MiB 13.6 -> 10.5, 32 MiB 19.6 -> 14.8, 40 MiB
+// 23.0 -> 18.1, fp32 32 MiB 18.3 -> 13.2).  Above it the reduction alone would pay for a cast that may not come
+// (48 MiB 12.3 -> 12.7 alone, 25.7 -> 21.6 with it; 428 MiB 64.7 -> 71.4 and 169 -> 168).  With scales the loads are
+// cacheable at any size: the sum of both kernels is never longer (128 MiB 54.5 -> 51.5, 428 MiB 169.5 ->
+// 169.8); the knob "amax.stream_before_cast" says otherwise.
+constexpr int64_t kAmaxCacheableBytes = (int64_t)40 << 20;
 template <int IN>
 inline int launch_amax(const void* x, int64_t numel, void* ws, float* amax_out, float* scale_out, int nscales,
                        float fmax0, float fmax1, hipStream_t stream) {
   constexpr int kUnroll = 8;
   Split sp = split_for_vectors<IN>(x, numel);
-  // Workgroups of 512 or 1024 threads where the tensor then takes few of them: a workgroup ends with two
-  // dependent atomics on one address, which the device performs one after the other, and 256 workgroups
-  // queue there for 2 us.  us with 256 / 512 / 1024 threads: bf16 2 MiB 3.9 / 3.8 / 4.0, 4 MiB 4.7 / 4.2 / 4.5,
-  // 8 MiB 7.0 / 5.2 / 4.9, 16 MiB 8.1 / 8.2 / 6.3, 32 MiB (256 workgroups again) 10.6 / 10.6 / 10.6, 128 MiB
-  // 22.4 / 22.4 / 23.1.
-  const int64_t small_blocks = ceil_div(sp.nvec, (int64_t)kBlock * kUnroll);
-  const int block = small_blocks <= 64 || small_blocks > 512 ? 256 : small_blocks <= 128 ? 512 : 1024;
+  // Few, large workgroups for all but the smallest and the largest tensors: a workgroup ends with two
+  // dependent atomics on one address, which the device performs one after the other, and 256 workgroups that
+  // arrive together queue there for 2 us.  us with 256 workgroups of 256 threads -> here: bf16 4 MiB 4.7 -> 4.2
+  // (512 threads), 8 MiB 6.8 -> 4.8 and 16 MiB 8.0 -> 6.3 (1024 threads, 8 vectors each, so at most 128
+  // workgroups), 24 MiB 8.9 -> 7.9, 32 MiB 10.5 -> 9.4, 48 MiB 12.3 -> 11.5, 64 MiB 14.3 -> 14.0 (at most five
+  // workgroups per eight CUs; with 96 / 128 / 192 workgroups 32 MiB takes 10.8 / 9.7 / 9.9).  Beyond that a
+  // reduction alone is bound by memory and spread out enough (128 MiB 22.4 -> 23.8); with a cast behind it the
+  // large workgroups stay ahead up to 96 MiB (both kernels, one output: 63 MiB 27.8 -> 26.4, 80 MiB 34.3 -> 32.4,
+  // 95 MiB 40.3 -> 38.9; both outputs 47.8 -> 46.9, at 128 MiB 61.4 -> 61.7).
+  const int64_t small_blocks = ceil_div(sp.nvec, (int64_t)kBlock * kUnroll);  // of 32 KiB
+  const int block = small_blocks <= 64 || small_blocks > (nscales ? 3072 : 2048) ? 256 : small_blocks <= 128 ? 512 : 1024;
   int grid = reduction_grid(sp.nvec, block, kUnroll, "amax.blocks_per_cu");
+  if (block == 1024) grid = std::min(grid, std::max(8, device_facts().cu_count * 5 / 64 * 8));
   uint8_t* w = static_cast<uint8_t*>(ws);
   const bool nt = nscales == 0 ? numel * InTraits<IN>::kBytes > kAmaxCacheableBytes : tuning("amax.stream_before_cast") != 0;
   uint64_t* const log = phase_log((size_t)grid * 32);

@@ -284,9 +284,9 @@ def test_dynamic_quant_config2_full_size(d):
 
 
 @pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("vecs", [1, 131072, 262144, 524288, 1048576], ids=str)
+@pytest.mark.parametrize("vecs", [1, 131072, 262144, 524288, 1048576, 4194304], ids=str)
 def test_amax_between_workgroup_sizes(d, in_dtype, vecs):
-    """Tensors of as many 16-byte vectors as the largest that take workgroups of 256, 512, 1024 threads, and one
+    """Tensors of as many 16-byte vectors as the largest that take workgroups of 256, 512, 1024 threads (and few of them), and one
     vector and three elements to either side of that: the maximum wherever a workgroup, a quarter of one or
     the ragged end of the tensor begins or ends, aligned and one element off."""
     kv = 8 if in_dtype == torch.bfloat16 else 4
