@@ -413,6 +413,30 @@ def test_mx_gemm_split_k(d, cabi, splits, size):
         cabi.set_tuning("gemm.split_k", 0)
 
 
+@pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
+@pytest.mark.parametrize("size", [(256, 8192, 8192), (250, 7200, 8184),  # two shares of a tile, even and not
+                                  (100, 4128, 14336),  # two shares of 16 and 17 steps
+                                  (128, 5120, 5120), (65, 5152, 5000),  # up to four shares of ten steps or more
+                                  (1000, 2048, 2048)],  # too few steps for any
+                         ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
+def test_mx_gemm_few_shares_by_rule(d, cabi, size, fp4):
+    """the sizes around which the library's own rule shares K or does not: integers of at most 4, so that every
+    partial sum (at most 16 K < 2^18) is exact in fp32 whatever the order and the result is one bit pattern"""
+    M, K, N = size
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    a = torch.randint(-4, 5, (M, K), generator=g, device="cuda").float()
+    b = torch.randint(-4, 5, (N, K), generator=g, device="cuda").float()
+    want = (a @ b.t()).bfloat16()
+    if fp4:
+        (qa, sa), (qb, sb) = (d.mx_fp4_quantize(t.bfloat16(), blocked=True) for t in (a, b))
+        product = d.mx_fp4_bf16
+    else:
+        (qa, sa), (qb, sb) = (d.mx_fp8_quantize_blocked(t.bfloat16()) for t in (a, b))
+        product = d.mx_fp8_bf16
+    for _ in range(2):  # the second call finds the tickets as the first one left them
+        assert torch.equal(product(qa, qb.t(), sa, sb), want)
+
+
 @pytest.mark.parametrize("size", [(4352, 256, 4096), (4100, 256, 4360), (4352, 384, 4352), (8200, 128, 4104),
                                   (2304, 128, 2304), (2200, 256, 2312)],  # the last two: 81 and 90 tiles, halves only
                          ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
