@@ -259,8 +259,9 @@ __global__ __launch_bounds__(kBlock) void mx_row_kernel(const void* __restrict__
     if (first) {
       const uint32_t col_tiles = (kblocks + 3u) >> 2;
       uint8_t* const band = scale + (uint64_t)(rows >> 7) * col_tiles * 512u;
-      for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < col_tiles * 128u; i += gridDim.x * kBlock) {
-        const uint32_t j = i & 127u, r = (j & 3u) * 32u + (j >> 2);  // row of word j of a 512-byte tile
+      // (64 bits: a single row may have 2^28 blocks, and its band 2^33 words; once per launch, outside the cast's loop)
+      for (uint64_t i = blockIdx.x * kBlock + threadIdx.x; i < (uint64_t)col_tiles * 128u; i += (uint64_t)gridDim.x * kBlock) {
+        const uint32_t j = (uint32_t)i & 127u, r = (j & 3u) * 32u + (j >> 2);  // row of word j of a 512-byte tile
         if (r >= first) reinterpret_cast<u32_byte*>(band)[i] = 0u;
       }
     }

@@ -184,6 +184,33 @@ def test_mx_casts_past_2_32_elements(d):
     assert torch.equal(o[3].view(torch.uint8).view(C, R // 32)[c0:, -1:].cpu(), ps)
 
 
+@pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
+@pytest.mark.parametrize("cols", [TWO32 - 4096, TWO32])
+def test_row_casts_zero_the_padding_of_a_single_very_long_row(d, fp4, cols):
+    """One row, whose blocked scales are a band of 128 rows with 127 of padding: 2^32 words of it, and a few
+    fewer, so that a count or an index of 32 bits would wrap to nothing or past the end."""
+    from driss_torch_amd import cabi
+
+    base = util.student_t((1, 4096), 2011)
+    x = _periodic(base.view(-1), cols // 4096).view(1, cols)
+    n = cabi.lib().dt_blocked_scale_bytes(1, cols // 32)
+    assert n == cols // 128 * 512
+    scale = torch.full((n,), 0xAB, dtype=torch.uint8, device="cuda")
+    if fp4:
+        data, _ = cabi.mx_fp4_quantize(x, layout=cabi.SCALE_BLOCKED, scale=scale)
+        want, want_scale = co.mx_fp4_quantize(base)
+    else:
+        data, _ = cabi.mx_fp8_quantize(x, layout=cabi.SCALE_BLOCKED, scale=scale)
+        want, want_scale = co.mx_quantize(base)
+    assert _all_rows_equal(data.view(torch.uint8), want.view(torch.uint8).view(-1))
+    tile = torch.zeros((32, 512), dtype=torch.uint8)  # the base row's tiles of four blocks, each in front of its padding
+    tile[:, :4] = want_scale.view(torch.uint8).view(32, 4)
+    del x, data
+    per_chunk = 1 << 30
+    for at in range(0, n, per_chunk):
+        assert _all_rows_equal(scale[at:at + per_chunk], tile.view(-1)), at
+
+
 def _random_mx_operand(rows, K, seed):
     """device uint8 e4m3 codes [rows, K] without NaN, plain scale bytes [rows, K/32] in 120..134"""
     g = torch.Generator(device="cuda").manual_seed(seed)
