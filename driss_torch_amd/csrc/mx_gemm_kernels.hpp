@@ -567,6 +567,9 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
           const v8i va = __builtin_shufflevector(fa[P][i].lo, fa[P][i].hi, 0, 1, 2, 3, 4, 5, 6, 7);
           acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(vb, va, acc[i][j], 0, 0, 0, sb[0][r], 0, sa[P][0][i]);
         } else {
+          // The compiler's hazard pass does not look into this statement.  What a VALU instruction writes (the zeros
+          // of acc, the masked scales; everything else comes out of the LDS) has to be two wait states away from
+          // the MFMA that reads it: it is written before the slot in front of that MFMA's, which holds two MFMAs.
           const v4i pb = c == 0 ? fb[r].lo : fb[r].hi, pa = c == 0 ? fa[P][i].lo : fa[P][i].hi;
           asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0] cbsz:4 blgp:4"
                        : "+a"(acc[i][j])
@@ -600,7 +603,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
           offA[i] -= tail_now;
           if constexpr (i < kLoadsB) offB[i] -= tail_now;
         }
-        if constexpr (z % 8 == 7) {  // the B fragment of the next eight slots
+        if constexpr (z % 8 == 6) {  // the B fragment of the next eight slots but one
           if constexpr (z / 8 + 1 < TN) mask_b(kThis, (P * TN + z / 8 + 1) % kRing);
           else mask_b(kNext, (P * TN + TN) % kRing);
         }
@@ -622,7 +625,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
             read_sa(kNext, y / 5 * 4 + (y % 5 - 1) + 1);
           }
           if constexpr (y % 2 == 0 && y / 2 < kPostLoads) fetch_one(y / 2, post, kSlotThis, 0u);
-          if constexpr (y == 25) settle_sa(kNext);  // (pinned: left alone the compiler moves their widening behind the loop's turn)
+          if constexpr (y == 24) settle_sa(kNext);  // a slot before the step ends (pinned: left alone the compiler moves their widening behind the loop's turn)
         }
         __builtin_amdgcn_sched_barrier(0);
       };
@@ -632,20 +635,31 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
     constexpr std::integral_constant<int, 0> kP0{};
     constexpr std::integral_constant<int, 1> kP1{};
     const bool odd = (k_steps & 1) != 0;  // then the first step runs alone, in slot 1, and the pairs start in slot 0
-    const uint32_t first = odd ? (uint32_t)kStageBytes : 0u;
-    fetch(0, first);
-    StepBases second;
-    bases_of(second, 1);
-#pragma unroll
-    for (int n = 0; n < kPostLoads; ++n) fetch_one(n, second, (uint32_t)kStageBytes - first, KTAIL && k_steps <= 2 ? tail_adj : 0u);
-    touch(2);
-    if constexpr (KTAIL) {
-      if (k_steps <= 2) tail_in_place();  // the rest of that refill, and all others
-    }
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPostLoads + 1) : "memory");
-    __syncthreads();
-    auto first_fragments = [&](auto p_tag) {
+    auto begin = [&](auto p_tag) {
       constexpr int P = decltype(p_tag)::value;
+      constexpr uint32_t kSlotFirst = P * kStageBytes, kSlotSecond = (1 - P) * kStageBytes;
+      fetch(0, kSlotFirst);
+      // acc becomes zero here, while the first loads go out, four registers per instruction (0 x 0 + 0).  Left to
+      // the compiler, its registers were written one by one behind the first step's barrier or, for an odd number
+      // of steps, right in front of each one's first MFMA (us, that -> this: e2m1 8192 x 4096 x 256 21.0 -> 20.2,
+      // 2048 x 5120 x 5120 29.7 -> 29.4, e4m3 4096 x 4096 x 1024 21.0 -> 20.6; long K the same).
+      const uint64_t zero = 0;
+      asm volatile("s_nop 1" : : "v"(zero));
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) asm volatile("v_mfma_f32_4x4x4_16b_f16 %0, %1, %1, 0" : "=a"(acc[i][j]) : "v"(zero));
+      StepBases second;
+      bases_of(second, 1);
+#pragma unroll
+      for (int n = 0; n < kPostLoads; ++n) fetch_one(n, second, kSlotSecond, KTAIL && k_steps <= 2 ? tail_adj : 0u);
+      touch(2);
+      if constexpr (KTAIL) {
+        if (k_steps <= 2) tail_in_place();  // the rest of that refill, and all others
+      }
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPostLoads + 1) : "memory");
+      __syncthreads();
+      t_loop = clock_reading();
 #pragma unroll
       for (int t = 0; t < 3; ++t) read_b(p_tag, t, (P * TN + t) % kRing);
 #pragma unroll
@@ -653,13 +667,14 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
       set_mask(p_tag, 0);
       mask_b(p_tag, (P * TN) % kRing);
       settle_sa(p_tag);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (FP4) asm volatile("s_nop 1");  // the first MFMA reads what was masked last
     };
-    t_loop = clock_reading();
     if (odd) {
-      first_fragments(kP1);
+      begin(kP1);
       step(kP1);
     } else {
-      first_fragments(kP0);
+      begin(kP0);
     }
     while (ks < k_steps) {
       step(kP0);
