@@ -22,7 +22,6 @@
 // that the stores are whole 256-byte row segments (direct 8-byte stores cost 12% of the run).
 #pragma once
 
-#include <algorithm>
 #include <atomic>
 #include <type_traits>
 #include <utility>
@@ -30,6 +29,7 @@
 #include "dt_device.hpp"
 #include "dt_host.hpp"
 #include "mx_few_rows.hpp"
+#include "mx_gemm_plan.hpp"
 
 namespace dt {
 
@@ -43,13 +43,8 @@ typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-constexpr int kBK = 128;             // K bytes per step = one 16x16x128 MFMA
 constexpr int kGroupRows = 8;        // rows filled by one wave-wide LDS-DMA load
 constexpr int kGroupStride = 1024;   // 8 rows of 128 bytes; the chunk swizzle alone makes fragment reads conflict-free (measured)
-constexpr size_t kSplitTicketBytes = 1024;        // head of the split-K workspace: one counter per 128 x 128 tile
-constexpr size_t kSplitTileBytes = 128 * 128 * 4;  // parked fp32 accumulators of one tile and split
-constexpr int kMaxSplits = 16;      // what gemm.split_k may force
-constexpr int kAutoMaxSplits = 12;  // what the library picks by itself
 
 typedef const __attribute__((address_space(1))) void* gptr_t;
 typedef __attribute__((address_space(3))) void* lptr_t;
@@ -1088,46 +1083,6 @@ int launch_gemm(const uint8_t* a, const uint8_t* b, const uint8_t* sfa, const ui
 
 inline size_t split_workspace_bytes() { return kSplitTicketBytes + (size_t)device_facts().cu_count * kSplitTileBytes; }
 
-// Split-K factor for the 128 x 128 tiling.  A grid of half a workgroup per CU or less leaves
-// most of the chip idle while each workgroup walks the whole K, one K-step per memory latency / 3:
-// share K between as many workgroups per tile as fill the chip once.  What it costs is the last
-// workgroup of a tile reading every share through one CU (about 1 us per share of a full tile),
-// so a share is at least 16 K-steps, or 10 while there are at most four shares of a K of 5120 elements or
-// more (measured on MI355X, e4m3, B rotated through memory, us without -> with: 16 x 8192 x 8192 31 -> 19,
-// 128 x 8192 x 8192 42 -> 24, 1024 x 1024 x 16384 58 -> 34, 512 x 512 x 65536 219 -> 50, 128 x 128 x 16384
-// 56 -> 25, 128 x 5120 x 5120 with four shares of 10 steps 19.9 -> 17.5, with six 19.4, 256 x 5120 x 5120 with
-// three 22.7 -> 19.9, 256 x 4096 x 4096 with three 15.7 -> 16.4; e2m1 128 x 8192 x 8192 with three 24.5 -> 18.2).
-// Two shares pay where they fill four fifths of the chip or more and save more steps than the 8 us that
-// parking and adding a whole chip's tiles takes: from 56 steps on, or 32 when B comes from memory and each
-// step takes longer (256 x 8192 x 8192 41 -> 33, 512 x 4096 x 14336 69 -> 46, 128 x 14336 x 4096 24.8 -> 22.6;
-// not 1000 x 2048 x 6144 23.0 -> 25.4, 128 x 5120 x 5120 19.9 -> 22.1, nor e2m1 96 x 14336 x 4096 14.7 -> 16.0). The knob
-// gemm.split_k forces a factor (1 = never split); whatever is asked for, every split owns a step
-// and the workspace holds all shares.
-inline int plan_splits(bool fp4, int64_t M, int64_t N, int64_t k_steps, size_t workspace_bytes) {
-  const int64_t tiles = ceil_div(M, 128) * ceil_div(N, 128);
-  if (workspace_bytes <= kSplitTicketBytes || tiles > (int64_t)(kSplitTicketBytes / 4)) return 1;
-  const int64_t room = (int64_t)((workspace_bytes - kSplitTicketBytes) / kSplitTileBytes) / tiles;
-  const int forced = tuning("gemm.split_k");
-  int64_t want;
-  if (forced > 0) {
-    want = forced;
-  } else {
-    const int cus = device_facts().cu_count;
-    const int64_t shares = std::max(k_steps * (fp4 ? 2 : 1) >= 40 ? std::min<int64_t>(k_steps / 10, 4) : 0, k_steps / 16);
-    want = cus / tiles;
-    if (want > shares) want = shares;
-    if (want > kAutoMaxSplits) want = kAutoMaxSplits;
-    const bool two_pay = tiles * 5 >= cus * 2 && (k_steps >= 56 || (k_steps >= 32 && N * k_steps * kBK >= ((int64_t)32 << 20)));
-    if (want < 2 || (want == 2 && !two_pay)) return 1;
-  }
-  if (want > kMaxSplits) want = kMaxSplits;
-  if (want > room) want = room;
-  if (want > k_steps) want = k_steps;
-  if (want < 2) return 1;
-  const int64_t per = ceil_div(k_steps, want);
-  return (int)ceil_div(k_steps, per);
-}
-
 // Shared argument checks and tile choice.  K counts elements, lda/ldb bytes.
 template <bool FP4>
 int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb, int64_t M, int64_t N, int64_t K,
@@ -1151,57 +1106,36 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
   const int variant = tuning("gemm.variant");
   if ((variant == 9 && few_rows_fits(M, K)) || (variant == 0 && few_rows_pays(FP4, M, N, K, workspace != nullptr)))
     return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
-  const int64_t tiles256 = ceil_div(M, 256) * ceil_div(N, 256);
-  // 256 x 192 tiles where they fill the chip's one round better than 256 x 256 tiles do (which leave a
-  // quarter of it idle or more).  At the chip's power limit a round of them takes 0.78 of a round of the
-  // large tiles, not 0.75, so they only pay while both are one round (us, 256 x 256 -> 256 x 192, e4m3 and
-  // e2m1: 2048 x 4352 x 4096, 136 -> 184 tiles, 38.5 -> 34.3 and 26.0 -> 23.6; 2048 x 5120 x 5120, 160 -> 216,
-  // 48.3 -> 45.3 and 30.9 -> 29.3; 2000 x 6144 x 8192, 192 -> 256, 80.0 -> 77.7 and 50.9 -> 49.2; two rounds
-  // against one and a half: 4096 x 5632 x 4096 77.9 and 77.9, 4096 x 9216 x 4096 120.9 -> 123.5).
-  const int64_t tiles192 = ceil_div(M, 256) * ceil_div(N, 192);
-  if (variant == 5 || (variant == 0 && 2 * tiles256 > device_facts().cu_count && tiles192 > tiles256 &&
-                       tiles192 <= device_facts().cu_count))
-    return launch_gemm<256, 192, 2, 2, 2, FP4, true>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
-  const bool big = variant == 2 || variant == 7 || (variant == 0 && tiles256 >= device_facts().cu_count / 2);
+  const int cus = device_facts().cu_count;
+  const GemmPlan plan = plan_gemm(FP4, M, N, K, workspace ? workspace_bytes : 0, cus, variant, tuning("gemm.tail_quads"), tuning("gemm.split_k"));
+  // tiles of 256 x 256 in whole rounds of the chip, and those behind them
+  const int64_t tiles256 = ceil_div(M, 256) * ceil_div(N, 256), whole = tiles256 / cus * cus, left = tiles256 - whole;
   // <tile M, tile N, waves M, waves N, LDS ring slots, e2m1 operands>
-  if (big && variant == 7) return launch_gemm<256, 256, 2, 2, 2, FP4, false>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
-  // Between a quarter and half a round of 256 x 256 tiles: as 256 x 128 halves they fill the chip
-  // once (0.8 of a round of tiles), as 128 x 128 tiles they would take two rounds (2 x 0.55)
-  // (rows past M make half of every tile of a matrix of at most 128 rows idle: there the 128 x 128 tiles
-  // are one round as well, 96 x 28672 x 4096 34.6 -> 30.6 us, e2m1 21.4 -> 16.9)
-  const int64_t tiles128 = ceil_div(M, 128) * ceil_div(N, 128);
-  if (variant == 0 && tuning("gemm.tail_quads") != 0 && 4 * tiles256 > device_facts().cu_count &&
-      2 * tiles256 <= device_facts().cu_count && tiles128 > device_facts().cu_count)
-    return launch_gemm<256, 128, 2, 2, 3, FP4, false, kHalves>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, 1, nullptr,
-                                                               tiles256, 0);
-  if (big) {
-    // Whole rounds of the chip on 256 x 256 tiles; what is left over would keep the chip for another
-    // full round however few tiles it is.  When its quadrants fit the chip at once it runs as
-    // 128 x 128 quadrants instead: one round of those takes 0.5-0.6 of a round of tiles (measured on
-    // MI355X, e4m3, us: 4096 x 5120 x 4096, 256 + 64 tiles, 97 -> 77; 4352^2 x 4096, 256 + 33, 97 -> 78;
-    // 4096 x 4352 x 8192, 256 + 16, 177 -> 134; 6144^3, 512 + 64, 216 -> 186; 8448 x 8192^2, 1024 + 32,
-    // 473 -> 436), two rounds of quadrants take as long as the round of tiles (4096 x 6144 x 4096,
-    // 256 + 128: 97 -> 96).  Up to half a round of leftover tiles runs as 256 x 128 halves, a round of
-    // which takes 0.8 of a round of tiles (the same shape 97 -> 87.5; 8192 x 5120 x 8192, 512 + 128,
-    // 273 -> 258).  The results are the same bits either way.
-    const int cus = device_facts().cu_count;
-    const int64_t rounds = tiles256 / cus, left = tiles256 % cus;
-    const int tail = tuning("gemm.tail_quads");
-    if (variant == 0 && tail != 0 && rounds >= 1 && left > 0 && cus % 8 == 0 && (tail >= 2 || 2 * left <= cus)) {
-      const int st = launch_gemm<256, 256, 2, 2, 2, FP4, true>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, 1, nullptr,
-                                                                rounds * cus);
+  switch (plan.tiles) {
+    case kTiles256x192:
+      return launch_gemm<256, 192, 2, 2, 2, FP4, true>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
+    case kTiles256:
+      return launch_gemm<256, 256, 2, 2, 2, FP4, true>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
+    case kTiles256ThenQuads:
+    case kTiles256ThenHalves: {
+      const int st = launch_gemm<256, 256, 2, 2, 2, FP4, true>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, 1, nullptr, whole);
       if (st != DT_OK) return st;
-      if (tail == 2 || (tail == 1 && 4 * left <= cus))
+      if (plan.tiles == kTiles256ThenQuads)
         return launch_gemm<128, 128, 2, 2, 4, FP4, false, kQuads>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, 1, nullptr,
-                                                                  left, (int)(rounds * cus));
+                                                                  left, (int)whole);
       return launch_gemm<256, 128, 2, 2, 3, FP4, false, kHalves>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, 1, nullptr,
-                                                                 left, (int)(rounds * cus));
+                                                                 left, (int)whole);
     }
-    return launch_gemm<256, 256, 2, 2, 2, FP4, true>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
+    case kTiles256Halves:
+      return launch_gemm<256, 128, 2, 2, 3, FP4, false, kHalves>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, 1, nullptr,
+                                                                 tiles256, 0);
+    case kTiles256QuadrantSchedule:
+      return launch_gemm<256, 256, 2, 2, 2, FP4, false>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
+    case kTiles128:
+      break;
   }
-  const int splits = workspace ? plan_splits(FP4, M, N, ceil_div(k_bytes, (int64_t)kBK), workspace_bytes) : 1;
-  if (splits > 1)
-    return launch_gemm<128, 128, 2, 2, 4, FP4, false, kSplitK>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, splits, workspace);
+  if (plan.splits > 1)
+    return launch_gemm<128, 128, 2, 2, 4, FP4, false, kSplitK>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, plan.splits, workspace);
   return launch_gemm<128, 128, 2, 2, 4, FP4, false>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
 }
 

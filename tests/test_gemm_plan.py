@@ -1,0 +1,70 @@
+"""The rule that picks the tiles of a block-scaled product and the workgroups that share K, compiled on its own
+for the host: which launch each size takes, at the sizes where the rule turns."""
+import ctypes as C
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+T128, HALVES, T192, T256, THEN_QUADS, THEN_HALVES, QUADRANT_SCHEDULE = range(7)
+CUS = 256
+ALL = 1024 + CUS * 128 * 128 * 4  # a workspace with room for a tile per CU
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    where = tmp_path_factory.mktemp("plan")
+    (where / "plan.cpp").write_text(
+        '#include "mx_gemm_plan.hpp"\n'
+        'extern "C" int plan(int fp4, long M, long N, long K, long ws, int cus, int variant, int tail, int split_k) {\n'
+        "  const dt::GemmPlan p = dt::plan_gemm(fp4 != 0, M, N, K, (size_t)ws, cus, variant, tail, split_k);\n"
+        "  return p.tiles * 100 + p.splits;\n}\n")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-I/opt/rocm/include",
+                    f"-I{ROOT / 'include'}", f"-I{ROOT / 'driss_torch_amd' / 'csrc'}", str(where / "plan.cpp"), "-o",
+                    str(where / "plan.so")], check=True)
+    f = C.CDLL(str(where / "plan.so")).plan
+    f.argtypes = [C.c_int] + [C.c_long] * 4 + [C.c_int] * 4
+
+    def call(fp4, M, N, K, ws=ALL, cus=CUS, variant=0, tail=1, split_k=0):
+        return divmod(f(int(fp4), M, N, K, ws, cus, variant, tail, split_k), 100)
+
+    return call
+
+
+@pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
+@pytest.mark.parametrize("size,tiles", [
+    # a quarter to half a round of 256 x 256 tiles: one round of 128 x 128 tiles where that is enough ...
+    ((65, 16648), T128), ((96, 28672), T128), ((128, 32512), T128), ((300, 10000), T128), ((1152, 3584), T128),
+    # ... also at exactly half a round of the large tiles, with half of each outside the matrix, and mirrored
+    ((65, 32520), T128), ((128, 32768), T128), ((32768, 128), T128), ((32700, 65), T128),
+    # one column more is two rounds of them, but one of 256 x 192 tiles
+    ((128, 32776), T192), ((128, 49152), T192), ((128, 49160), T256),
+    # halves where 128 x 128 tiles do not fit
+    ((129, 16648), HALVES), ((256, 32768), HALVES), ((2048, 4096), HALVES), ((300, 14336), HALVES), ((2048, 2048), T128),
+    ((2304, 2304), HALVES),
+    # more than half a round
+    ((2048, 4352), T192), ((2000, 6144), T192), ((2048, 6400), T256), ((4096, 4096), T256),
+    # whole rounds and what is left over
+    ((4096, 5120), THEN_QUADS), ((4096, 6144), THEN_HALVES), ((4096, 6400), T256), ((8192, 8192), T256)], ids=str)
+def test_tiles_by_size(plan, fp4, size, tiles):
+    assert plan(fp4, *size, 1024)[0] == tiles
+
+
+def test_one_round_of_small_tiles_is_never_given_to_fewer_large_ones(plan):
+    """wherever 128 x 128 tiles are one round, a plan of larger ones has to keep more than half of the chip busy"""
+    for rows in (64, 65, 128, 129, 256, 300, 640, 1152, 2048, 4096, 20000, 32768):
+        for n in range(128, 60000, 248):
+            for m, n_ in ((rows, n), (n, rows)):
+                up = lambda a, b: -(-a // b)  # noqa: E731
+                if up(m, 128) * up(n_, 128) <= CUS:
+                    assert plan(False, m, n_, 1024)[0] == T128, (m, n_)
+
+
+def test_knobs(plan):
+    assert plan(False, 2048, 6144, 1024, variant=1) == (T128, 1)
+    assert plan(False, 16, 64, 1024, variant=2)[0] == T256
+    assert plan(False, 16, 64, 1024, variant=5)[0] == T192
+    assert plan(False, 16, 64, 1024, variant=7)[0] == QUADRANT_SCHEDULE
+    assert plan(False, 4096, 5120, 1024, tail=0)[0] == T256 and plan(False, 2048, 4096, 1024, tail=0)[0] == T256
+    assert plan(False, 4096, 5120, 1024, tail=3)[0] == THEN_HALVES and plan(False, 4096, 6400, 1024, tail=2)[0] == THEN_QUADS

@@ -477,6 +477,27 @@ def test_mx_gemm_strided_operands_and_output(d, cabi, size):
     assert (out_wide[:, :8] == 7.0).all() and (out_wide[:, 8 + N:] == 7.0).all()  # nothing written outside
 
 
+@pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
+@pytest.mark.parametrize("size", [(128, 288, 32512), (65, 288, 32520), (128, 256, 32768), (128, 288, 32776), (32700, 256, 128)],
+                         ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
+def test_mx_gemm_one_band_of_rows(d, cabi, size, fp4):
+    """A band of at most 128 rows (or columns) around the width where its 128 x 128 tiles are one round of the
+    chip and its 256 x 256 tiles half of one: the same bits as on 128 x 128 tiles, whatever is picked."""
+    M, K, N = size
+    x, w = _wide_operand((M, K), 5000 + M).cuda(), _wide_operand((N, K), 5001 + N).cuda()
+    if fp4:
+        (a, sa), (b, sb), op = d.mx_fp4_quantize(x, True), d.mx_fp4_quantize(w, True), d.mx_fp4_bf16
+    else:
+        (a, sa), (b, sb), op = d.mx_fp8_quantize_blocked(x), d.mx_fp8_quantize_blocked(w), d.mx_fp8_bf16
+    got = op(a, b.t(), sa, sb)
+    cabi.set_tuning("gemm.variant", 1)
+    try:
+        assert torch.equal(op(a, b.t(), sa, sb), got)
+    finally:
+        cabi.set_tuning("gemm.variant", 0)
+    assert torch.isfinite(got).all() and got.abs().max() > 0
+
+
 def _random_plan_sizes(seed, n):
     import random
 
