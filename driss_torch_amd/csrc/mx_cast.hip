@@ -350,7 +350,8 @@ extern "C" int dt_to_blocked(const uint8_t* scale, int64_t R, int64_t C, uint8_t
   const int64_t groups = dt_blocked_scale_bytes(R, C) / 16;
   if (dt::ceil_div(R * C, 256) > 0x7FFFFFFFll) return DT_ERR_INVALID_SHAPE;
   const unsigned grid = (unsigned)std::min<int64_t>(dt::ceil_div(groups, (int64_t)dt::kBlock), (int64_t)dt::device_facts().cu_count * 16);
-  if (C % 4 == 0 && dt::aligned(scale, 4)) dt::to_blocked_kernel<true><<<grid, dt::kBlock, 0, s>>>(scale, R, C, groups, out);
-  else dt::to_blocked_kernel<false><<<grid, dt::kBlock, 0, s>>>(scale, R, C, groups, out);
+  if (R * C < 4) dt::to_blocked_kernel<true, uint32_t><<<grid, dt::kBlock, 0, s>>>(scale, R, C, groups, out);
+  else if ((groups >> 5) <= 0xFFFFFFFFll) dt::to_blocked_kernel<false, uint32_t><<<grid, dt::kBlock, 0, s>>>(scale, R, C, groups, out);
+  else dt::to_blocked_kernel<false, uint64_t><<<grid, dt::kBlock, 0, s>>>(scale, R, C, groups, out);
   return dt::launch_status();
 }

@@ -231,3 +231,16 @@ def test_blocked_casts_write_their_padding_and_nothing_else(cabi, gpu_device, sh
         both(x, layout=cabi.SCALE_BLOCKED, outs=(dr, sr, dc, sc))
         check(wr, sr, one(1)[1], R, C // 32)
         check(wc, sc, one(0)[1], C, R // 32)
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (1, 3), (3, 1), (2, 2), (1, 4), (1, 5), (5, 5), (128, 1), (129, 7), (200, 130), (257, 133)],
+                         ids=lambda s: f"{s[0]}x{s[1]}")
+def test_to_blocked_of_any_width_at_any_byte(cabi, gpu_device, shape):
+    """Words of a scale matrix that begin at every byte of a word, its last ones, and matrices smaller than one."""
+    R, C = shape
+    plain = torch.randint(1, 256, (R, C), generator=torch.Generator().manual_seed(R * 1000 + C), dtype=torch.int32).to(torch.uint8)
+    for off in range(4):
+        whole = torch.full((off + R * C + 8,), 0xAB, dtype=torch.uint8, device=gpu_device)
+        part = whole[off:off + R * C].view(R, C)
+        part.copy_(plain)
+        assert torch.equal(cabi.to_blocked(part).cpu(), co.to_blocked(plain)), off
