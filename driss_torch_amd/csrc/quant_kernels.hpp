@@ -50,12 +50,6 @@ __device__ __forceinline__ uint32_t absbits_of(const void* x, int64_t i) {
     return ((uint32_t)static_cast<const uint16_t*>(x)[i] & 0x7FFFu) << 16;  // bf16 -> f32 bits
 }
 
-template <int IN>
-__device__ __forceinline__ uint32_t fp32_bits_of(const void* x, int64_t i) {
-  if constexpr (IN == DT_F32) return static_cast<const uint32_t*>(x)[i];
-  else return (uint32_t)static_cast<const uint16_t*>(x)[i] << 16;
-}
-
 // --------------------------------------------------------------------------- amax ----
 // Every workgroup reduces a grid-strided share of the vectors to one unsigned magnitude,
 // folds it into a running maximum in the workspace with one atomic and takes a ticket; the

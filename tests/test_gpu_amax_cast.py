@@ -346,6 +346,21 @@ def test_rowwise_rows_between_vectors(d, cabi, in_dtype, vecs):
 
 
 @pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape", [(127, 1001), (129, 1001), (2095, 1001), (2096, 1001), (100, 20971), (101, 20971), (62, 33333), (63, 33333)],
+                         ids=lambda s: f"{s[0]}x{s[1]}")
+def test_rowwise_rows_between_vectors_few_or_many(d, in_dtype, shape):
+    """Either side of the number of rows that get a workgroup each, and of the output that is streamed (2 MiB)."""
+    a = util.rows_log_uniform_sigma(shape, 92 + shape[0], in_dtype)
+    a[0, 0], a[-1, -1], a[1, -1] = 3.0e4, -3.0e4, float("nan")
+    for fp8_dtype in FP8:
+        ref, ramax, rscale = co.dynamic_scaled_quant_rowwise(a, fp8_dtype)
+        out, amax, scale = d.dynamic_scaled_quant_rowwise(a.cuda(), fp8_dtype)
+        assert torch.equal(amax.cpu().view(torch.int32), ramax.view(torch.int32))
+        assert torch.equal(scale.cpu().view(torch.int32), rscale.view(torch.int32))
+        assert torch.equal(util.codes(out), ref)
+
+
+@pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("extra", [0, 3])
 @pytest.mark.parametrize("vecs", [1, 40, 257, 300, 512, 513, 1024, 1030, 2048, 2500, 4096, 4100, 8192, 8193, 9000, 16384, 16385])
 def test_rowwise_long_rows(d, in_dtype, vecs, extra):
