@@ -92,32 +92,54 @@ __global__ __launch_bounds__(BLOCK) void amax_kernel(const void* __restrict__ x,
   const int64_t stride = (int64_t)gridDim.x * BLOCK, step = P * stride;
   // a workgroup's quarters of 256 threads take runs of kBlock vectors a whole grid apart, so that run r is
   // read by workgroup r % gridDim whatever BLOCK is, and by XCD r % 8 like in the cast that follows
-  int64_t i = ((int64_t)(tid / kBlock) * gridDim.x + blockIdx.x) * kBlock + tid % kBlock;
-  auto whole_batch_at = [&](int64_t j) { return j + (P - 1) * stride < sp.nvec; };
-  auto load_batch = [&](u32x4 (&w)[P], int64_t j) {
+  const int64_t i = ((int64_t)(tid / kBlock) * gridDim.x + blockIdx.x) * kBlock + tid % kBlock;
+  // First and last of the vectors i of the workgroup: whether a batch is whole is asked for all of its threads at once,
+  // and the loop below has one way out.  (With lanes that leave it by themselves, or two ways out, the compiler waits
+  // for a batch before it requests the next.)
+  const int64_t first = (int64_t)blockIdx.x * kBlock, last = ((int64_t)(BLOCK / kBlock - 1) * gridDim.x + blockIdx.x) * kBlock + kBlock - 1;
+  const uint32_t lane_bytes = (uint32_t)i * 16u;  // a grid's worth of vectors is far below 2^28: scalar bases and 32-bit lane offsets
+  auto whole_batch_at = [&](int64_t k) { return last + k + (P - 1) * stride < sp.nvec; };
+  auto load_batch = [&](u32x4 (&w)[P], int64_t k) {
 #pragma unroll
-    for (int u = 0; u < P; ++u) w[u] = ld_maybe_stream<NT>(v + j + u * stride);
+    for (int u = 0; u < P; ++u)
+      w[u] = ld_maybe_stream<NT>(reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(v + k + u * stride) + lane_bytes));
+  };
+  // What is left behind the last whole batch: all of its loads at once and under way before that batch is looked at
+  // (past the end the last vector again, which changes no maximum).  One at a time behind it, as it was, they cost a
+  // memory latency each, and most sizes leave some (us, bf16: 576 x 2048 5.4 -> 4.3, 700 x 2000 5.4 ->
+  // 4.4, with the cast behind it 14 x 7528 6.9 -> 5.8, 3111 x 2048 10.9 -> 10.1).
+  auto load_rest = [&](u32x4 (&w)[P], int64_t k) {
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+      const int64_t j = i + k + u * stride;
+      w[u] = ld_maybe_stream<NT>(v + (j < sp.nvec ? j : sp.nvec - 1));
+    }
   };
   auto absorb_batch = [&](const u32x4 (&w)[P]) {
 #pragma unroll
     for (int u = 0; u < P; ++u) absorb(w[u]);
   };
-  if (whole_batch_at(i)) {
-    u32x4 wa[P], wb[P];
-    load_batch(wa, i);
-    i += step;
-    for (;;) {
-      if (!whole_batch_at(i)) { absorb_batch(wa); break; }
-      load_batch(wb, i);
-      i += step;
+  u32x4 wa[P], wb[P], wc[P];
+  if (whole_batch_at(0)) {
+    load_batch(wa, 0);
+    int64_t k = step;  // of the next batch
+    for (; whole_batch_at(k + step); k += 2 * step) {
+      load_batch(wb, k);
+      __builtin_amdgcn_sched_barrier(0);  // (or the compiler looks at wa first, and waits for it)
       absorb_batch(wa);
-      if (!whole_batch_at(i)) { absorb_batch(wb); break; }
-      load_batch(wa, i);
-      i += step;
+      load_batch(wa, k + step);
       absorb_batch(wb);
     }
+    const bool second = first + k < sp.nvec, third = first + k + step < sp.nvec;  // a whole batch and a part of one at most
+    if (second) load_rest(wb, k);
+    if (third) load_rest(wc, k + step);
+    absorb_batch(wa);
+    if (second) absorb_batch(wb);
+    if (third) absorb_batch(wc);
+  } else if (first < sp.nvec) {
+    load_rest(wa, 0);
+    absorb_batch(wa);
   }
-  for (; i < sp.nvec; i += stride) absorb(ld_maybe_stream<NT>(v + i));
   stamp(1);
 
   uint32_t m;
@@ -200,7 +222,11 @@ inline int reduction_grid(int64_t nvec, int block, int unroll, const char* knob)
 // (48 MiB 12.3 -> 12.7 alone, 25.7 -> 21.6 with it; 428 MiB 64.7 -> 71.4 and 169 -> 168).  With scales the loads are
 // cacheable at any size: the sum of both kernels is never longer (128 MiB 54.5 -> 51.5, 428 MiB 169.5 ->
 // 169.8); the knob "amax.stream_before_cast" says otherwise.
-constexpr int64_t kAmaxCacheableBytes = (int64_t)40 << 20;
+// Between 1.5 and 4 MiB a reduction alone streams after all: from memory it is 0.3 us faster that way, the cast
+// behind it no slower, and out of the caches both are the same (us, cacheable -> streaming: 1.5 MiB 4.2 -> 3.9 and with
+// the cast 6.3 -> 6.1, 2 MiB 4.4 -> 4.1 and 6.6 -> 6.2, 4 MiB 4.8 -> 4.5 and 7.3 -> 7.0; 5 MiB 5.8 -> 5.5 and 8.4 -> 8.2,
+// but out of the caches 6.2 -> 7.1 with the cast; 1 MiB, which comes out of the caches anyway, 3.6 -> 3.8).
+constexpr int64_t kAmaxCacheableBytes = (int64_t)40 << 20, kAmaxStreamedFrom = (int64_t)3 << 19, kAmaxStreamedTo = (int64_t)4 << 20;
 template <int IN>
 inline int launch_amax(const void* x, int64_t numel, void* ws, float* amax_out, float* scale_out, int nscales,
                        float fmax0, float fmax1, hipStream_t stream) {
@@ -220,7 +246,9 @@ inline int launch_amax(const void* x, int64_t numel, void* ws, float* amax_out, 
   int grid = reduction_grid(sp.nvec, block, kUnroll, "amax.blocks_per_cu");
   if (block == 1024) grid = std::min(grid, std::max(8, device_facts().cu_count * 5 / 64 * 8));
   uint8_t* w = static_cast<uint8_t*>(ws);
-  const bool nt = nscales == 0 ? numel * InTraits<IN>::kBytes > kAmaxCacheableBytes : tuning("amax.stream_before_cast") != 0;
+  const int64_t bytes = numel * InTraits<IN>::kBytes;
+  const bool nt = nscales == 0 ? bytes > kAmaxCacheableBytes || (bytes >= kAmaxStreamedFrom && bytes <= kAmaxStreamedTo)
+                               : tuning("amax.stream_before_cast") != 0;
   uint64_t* const log = phase_log((size_t)grid * 32);
 #define DT_AMAX_B(NS, NT, B) amax_kernel<IN, B, kUnroll, NS, NT><<<grid, B, 0, stream>>>(x, sp, w, amax_out, scale_out, fmax0, fmax1, log)
 #define DT_AMAX(NS, NT) do { if (block == 1024) DT_AMAX_B(NS, NT, 1024); else if (block == 512) DT_AMAX_B(NS, NT, 512); else DT_AMAX_B(NS, NT, 256); } while (0)

@@ -303,6 +303,23 @@ def test_amax_between_workgroup_sizes(d, in_dtype, vecs):
                 x[0, at] = old
 
 
+@pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vecs", [5, 300, 1100, 4095, 13174, 147456, 175000, 281600, 390001, 700003], ids=str)
+def test_amax_of_what_whole_batches_leave(d, in_dtype, vecs):
+    """As many vectors as leave part of a batch, one or two, to some or all of the workgroups: a maximum in any run of
+    256 vectors is found, one run after the other for the small tensors, every 37th and the last ones for the large."""
+    kv = 8 if in_dtype == torch.bfloat16 else 4
+    n = vecs * kv
+    x = torch.zeros((1, n), dtype=in_dtype, device="cuda")
+    runs = -(-vecs // 256)
+    for run in sorted({r for r in range(runs) if r % (1 if runs < 64 else 37) == 0} | {max(0, runs - 1 - k) for k in range(9)}):
+        at = min(n - 1, run * 256 * kv + (run * 977) % (256 * kv))
+        x[0, at] = -2.0 - run % 5
+        assert d.amax(x).item() == 2.0 + run % 5, (run, at)
+        x[0, at] = 0.0
+    assert d.amax(x).item() == 0.0
+
+
 @pytest.mark.parametrize("fp8_dtype", FP8)
 @pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("shape", [(3, 7), (64, 8), (33, 512), (100, 4096), (5, 4097), (9, 8200), (4, 20000), (2, 131072)])
