@@ -25,6 +25,8 @@ struct Knob {
 //                 tensor; sizes in [resident_gap_lo_kib, resident_gap_hi_kib) take the two kernels
 //                 dynamic.resident_overflow: 1 = tensors of up to 4 x the chip's capacity keep what fits
 //                 and read only the rest twice
+//   amax.blocks_per_cu: most workgroups per CU of a reduction in workgroups of 256 or 512 threads (those of 1024 are at
+//                 most five per eight CUs whatever it says)
 //   rowwise.block_from_vecs: rows of at least this many 16-byte vectors get a workgroup each (shorter
 //                 ones a wave each)
 //   mx.dual:      1 = dt_mx_fp8_quantize_dual reads x once (0: two single casts)
@@ -35,8 +37,8 @@ struct Knob {
 //                 with the next tile's loads in flight (0 = one workgroup per tile)
 //   mx.row_band4: 1 = row-wise MX cast with blocked scales walks 4 rows x 512 elements per wave pass
 //   gemm.variant: 0 = pick the tile by problem size, 1 = 128x128 tiles, 2 = 256x256 tiles, 5 = 256x192 tiles,
-//                 7 = 256x256 tiles without the L2 prefetch loads, 9 = the kernel for at most 64 rows
-//                 whatever the other dimensions
+//                 7 = 256x256 tiles on the main loop of the smaller ones (quadrants of the wave tile, no L2 prefetch;
+//                 the same bits), 9 = the kernel for at most 64 rows whatever the other dimensions
 //   gemm.few_rows_tiles: 16-column tiles per wave of that kernel: 0 = by the number of columns, 1, 2
 //   gemm.tail_quads: 1 = tiles left over after whole rounds of 256x256 tiles run as 128x128 quadrants
 //                 or 256x128 halves when those fit the chip at once, 0 = never, 2 = always as

@@ -282,9 +282,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   // area nobody reads).  The 4 tile columns that share an A panel inside an XCD (and the 8 tile
   // rows that share a B panel) split the panel's lines between them: 64 lines of A and BN / 8 of B
   // per workgroup and step, an equal share per wave.  A line nobody touched is merely slower.
-  constexpr int kTouch = TOUCH ? 1 : 0;       // touch loads per wave and step
+  constexpr int kTouch = 1;                   // touch loads per wave and step
   constexpr int kTouchAhead = 2;              // K-steps ahead of the stage refill
-  constexpr int kVmPerStep = kLoadsPerStep + kTouch;
   const uint8_t* touch_ptr = A;
   if constexpr (TOUCH) {
     static_assert(BM == 256 && (64 + BN / 8) % kWaves == 0, "touch shares are laid out for tiles of 256 rows");
@@ -300,19 +299,14 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
       touch_ptr = B + (int64_t)r * ldb;
     }
   }
-  auto touch_address = [&](int step) -> const uint8_t* {
+  auto touch = [&](int step) {
     const int kt = step < k_steps ? step : k_steps - 1;
-    return touch_ptr + (uint32_t)kt * kBK;
+    const uint8_t* const p = touch_ptr + (uint32_t)kt * kBK;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+                 :
+                 : "s"(lds_base + (uint32_t)(NST * kStageBytes)), "v"(p)
+                 : "memory");
   };
-  auto touch_at = [&](const uint8_t* p) {
-    if constexpr (TOUCH) {
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
-                   :
-                   : "s"(lds_base + (uint32_t)(NST * kStageBytes)), "v"(p)
-                   : "memory");
-    }
-  };
-  auto touch = [&](int step) { touch_at(touch_address(step)); };
 
   // The staged scale chunks of the partly filled step, once they have landed in ring slot `stage`: a
   // word holds the four K-block bytes of a row; the bytes of K-blocks past the end of K become 0.  A
@@ -381,14 +375,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
     HalfWords r;
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
-      if constexpr (H == 3) {  // tiles of any parity: a read each
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-          const uint32_t at = o + c * 1024 + sc_tile_b[half * 3 + t];
-          if constexpr (BYTES) r.w[c][t] = lds[at];
-          else r.w[c][t] = *reinterpret_cast<const uint32_t*>(lds + at);
-        }
-      } else if constexpr (BYTES) {
+      if constexpr (BYTES) {
         if constexpr (H == 4) {
           r.w[c][0] = lds[o + c * 1024 + half * 8];       r.w[c][1] = lds[o + c * 1024 + 256 + half * 8];
           r.w[c][2] = lds[o + c * 1024 + half * 8 + 4];   r.w[c][3] = lds[o + c * 1024 + 256 + half * 8 + 4];
@@ -676,11 +663,10 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
       step(kP1);
     }
   } else {
+  static_assert(!TOUCH && (TN == 8 || TN == 4), "the quadrant schedule has no prefetch and takes whole chunks of scales");
 #pragma unroll
   for (int p = 0; p < NST; ++p) fetch(p < k_steps ? p : k_steps - 1, (uint32_t)(p * kStageBytes));
-#pragma unroll
-  for (int p = 0; p < kTouchAhead; ++p) touch(NST + p);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * kLoadsPerStep + kTouchAhead * kTouch) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * kLoadsPerStep) : "memory");
   __syncthreads();
   if constexpr (KTAIL) {
     if (tail_step == 0) {  // a single, partly filled step: its scales are read next
@@ -724,15 +710,12 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
       if (ks + NST == tail_step) tail_in_place();  // from this step's refill on
     }
     uint32_t nla, nha, nlb, nhb, nsa, nsb, nxt2;
-    // the bases of step ks + NST, the refill of `cur` (clamped at the end: ignored), and the address of
-    // the touch: scalar bookkeeping of the step's second half, done in slots of the first quadrant
-    // that have nothing else to do, one item per slot
+    // the bases of step ks + NST, the refill of `cur` (clamped at the end: ignored): scalar bookkeeping of
+    // the step's second half, done in slots of the first quadrant that have nothing else to do, one item per slot
     StepBases at;
-    const uint8_t* touch_p;
     constexpr int kBook = S >= 8 ? 2 : S - 2;  // first of those slots (a short quadrant takes it all in one)
     constexpr int kBookStep = S >= 8 ? 1 : 0;
     int n_dma = 0;
-    bool touched = false;
     HalfWords hw;  // scale words of the half a quadrant brings in
     __builtin_amdgcn_sched_barrier(0);
     // MFMAs over a tiles i0.., b tiles j0.. with the b tile as the outer index (the b half of a
@@ -767,17 +750,14 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
     auto dma = [&]() {
       if (n_dma < kLoadsPerStep) fetch_one(n_dma++, at, cur, 0u);
     };
-    // e4m3: the step's loads (stage refill, then the touch as the youngest) are spread evenly over the 2 S
+    // e4m3: the step's loads (the stage refill) are spread evenly over the 2 S
     // slots behind the bar: a wave gets one such load out per 40-odd cycles, so two of them in neighbouring
     // slots of 32 cycles hold the second one's slot up (issued in runs of two to five they cost 120 cycles a
     // step).  e2m1 keeps them out of the slots that request a fragment instead (measured both ways).
     auto vm_ops_of_slot = [&](int slot) {  // slot: 0 .. 2 S - 1
 #pragma unroll
-      for (int i = 0; i < kVmPerStep; ++i) {
-        if ((i * 2 * S) / kVmPerStep != slot) continue;
-        if (i < kLoadsPerStep) dma();
-        else { touch_at(touch_p); touched = true; }
-      }
+      for (int i = 0; i < kLoadsPerStep; ++i)
+        if ((i * 2 * S) / kLoadsPerStep == slot) dma();
     };
     // ---- before the bar: (lo,hi) pulls b[lo], (lo,lo) pulls a[hi], both from this step's slot
     // (a quadrant has S = HA * HB time slots; the HB fragments of a b half are requested every
@@ -791,7 +771,6 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
 #pragma unroll
       for (int c = 0; c < KC; ++c)
         if (q == kBook + (2 + c) * kBookStep) { at.s[c] = base_s(kn, c); asm volatile("" : : "s"(at.s[c])); }
-      if (TOUCH && q == kBook + (2 + KC) * kBookStep) { touch_p = touch_address(ks + NST + kTouchAhead); asm volatile("" : : "v"(touch_p)); }
       if (q % HA == 0) fb[q / HA] = load_frag(clb, chb, kOffB, (q / HA) * 16);
       if (const int t = q - (kScaleLast - HB + 1); t >= 0 && t < HB) {
 #pragma unroll
@@ -814,10 +793,9 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
       }
     });
     // every fragment of this step has been requested; once they are in, the slot is free
-    // (the queue holds, in issue order, per step in flight its stage loads and then its touch
-    // load: all but the loads of step ks+1 and whatever precedes them may stay outstanding.  The
-    // touch has to stay the youngest: it misses the L2 by design, and loads complete in order)
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_waitcnt vmcnt(%0)" ::"n"((NST - 2) * kVmPerStep + kTouch) : "memory");
+    // (the queue holds, in issue order, the stage loads of the steps in flight: all but those of step
+    // ks+1 and whatever precedes them may stay outstanding)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_waitcnt vmcnt(%0)" ::"n"((NST - 2) * kLoadsPerStep) : "memory");
     __syncthreads();
     if constexpr (KTAIL) {
       if (ks + 1 == tail_step) {  // the partly filled last step has landed: nobody has read its scales yet
@@ -854,9 +832,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
       const bool frag_slot = q % kStepB == 0 && q / kStepB < HB;
       if (frag_slot) fb[HB + q / kStepB] = load_frag(nlb, nhb, kOffB, (HB + q / kStepB) * 16);
       if constexpr (!FP4) vm_ops_of_slot(S + q);
-      else if (frag_slot) {}
-      else if (q == S - 3 && n_dma >= kLoadsPerStep) { touch_at(touch_p); touched = true; }
-      else dma();
+      else if (!frag_slot) dma();
       if (const int t = q - (kScaleLast - HB + 1); t >= 0 && t < HB) {
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
@@ -867,7 +843,6 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
     });
 #pragma unroll
     for (int t = 0; t < kLoadsPerStep; ++t) dma();
-    if (!touched) touch_at(touch_p);
     cur = nxt; nxt = nxt2;
     cla = nla; cha = nha; clb = nlb; chb = nhb; csa = nsa; csb = nsb;
   } while (++ks < k_steps);
