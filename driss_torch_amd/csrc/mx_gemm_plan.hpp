@@ -21,8 +21,9 @@ constexpr int kAutoMaxSplits = 12;  // what the library picks by itself
 // most of the chip idle while each workgroup walks the whole K, one K-step per memory latency / 3:
 // share K between as many workgroups per tile as fill the chip once.  What it costs is the last
 // workgroup of a tile reading every share through one CU (about 1 us per share of a full tile),
-// so a share is at least 16 K-steps, or 10 while there are at most four shares of a K of 5120 elements or
-// more (measured on MI355X, e4m3, B rotated through memory, us without -> with: 16 x 8192 x 8192 31 -> 19,
+// so shares are 16 K-steps on average or more, or 10 while there are at most four shares of a K of 5120 elements
+// or more (the last one is what is left: 41 steps are shared 11 + 11 + 11 + 8;
+// measured on MI355X, e4m3, B rotated through memory, us without -> with: 16 x 8192 x 8192 31 -> 19,
 // 128 x 8192 x 8192 42 -> 24, 1024 x 1024 x 16384 58 -> 34, 512 x 512 x 65536 219 -> 50, 128 x 128 x 16384
 // 56 -> 25, 128 x 5120 x 5120 with four shares of 10 steps 19.9 -> 17.5, with six 19.4, 256 x 5120 x 5120 with
 // three 22.7 -> 19.9, 256 x 4096 x 4096 with three 15.7 -> 16.4; e2m1 128 x 8192 x 8192 with three 24.5 -> 18.2).

@@ -11,6 +11,16 @@ T128, HALVES, T192, T256, THEN_QUADS, THEN_HALVES, QUADRANT_SCHEDULE = range(7)
 CUS = 256
 ALL = 1024 + CUS * 128 * 128 * 4  # a workspace with room for a tile per CU
 
+# (M, K, N): workgroups that share K per 128 x 128 tile, e4m3 and e2m1; the GPU tests compute the same products
+SHARES = {(256, 8192, 8192): (2, 2), (250, 7200, 8184): (2, 1),  # two shares of a tile, even and not
+          (256, 16384, 8192): (2, 2),
+          (100, 4128, 14336): (2, 1),  # 33 steps: shares of 17 and 16
+          (128, 5120, 5120): (4, 1), (65, 5152, 5000): (4, 1),  # 40 steps, and 41 as 11 + 11 + 11 + 8
+          (200, 5120, 5120): (3, 1),
+          (128, 8192, 8192): (4, 3), (120, 8064, 8184): (4, 3), (128, 8096, 8000): (4, 3),  # e2m1: 11 + 11 + 10, last step whole, half, in part
+          (128, 16416, 4096): (8, 4),
+          (256, 4096, 4096): (1, 1), (1000, 2048, 2048): (1, 1)}  # too few steps for any
+
 
 @pytest.fixture(scope="module")
 def plan(tmp_path_factory):
@@ -68,3 +78,24 @@ def test_knobs(plan):
     assert plan(False, 16, 64, 1024, variant=7)[0] == QUADRANT_SCHEDULE
     assert plan(False, 4096, 5120, 1024, tail=0)[0] == T256 and plan(False, 2048, 4096, 1024, tail=0)[0] == T256
     assert plan(False, 4096, 5120, 1024, tail=3)[0] == THEN_HALVES and plan(False, 4096, 6400, 1024, tail=2)[0] == THEN_QUADS
+
+
+@pytest.mark.parametrize("size", SHARES, ids=lambda s: "x".join(map(str, s)))
+def test_shares_of_k(plan, size):
+    M, K, N = size
+    for fp4 in (False, True):
+        assert plan(fp4, M, N, K) == (T128, SHARES[size][fp4])
+        assert plan(fp4, M, N, K, ws=0) == (T128, 1) and plan(fp4, M, N, K, split_k=1) == (T128, 1)
+
+
+def test_shares_own_a_step_and_fit_the_workspace(plan):
+    for fp4 in (False, True):
+        for K in (32, 256, 288, 1024, 5152, 16416, 65536):
+            steps = -(-K // (256 if fp4 else 128))
+            for M, N in ((1, 8), (128, 128), (300, 264), (1024, 1024), (128, 16384)):
+                tiles = -(-M // 128) * -(-N // 128)
+                for split_k in (0, 2, 3, 5, 16, 99):
+                    for room in (1, tiles, 2 * tiles + 1, 256):
+                        n = plan(fp4, M, N, K, ws=1024 + room * 128 * 128 * 4, split_k=split_k)[1]
+                        assert 1 <= n <= 16 and (n == 1 or n * tiles <= room)
+                        assert (n - 1) * -(-steps // n) < steps  # the last share owns a step

@@ -7,6 +7,7 @@ import torch
 from oracle import c_oracle as co
 from oracle import eager
 from tests import util
+from tests.test_gemm_plan import SHARES
 
 pytestmark = pytest.mark.gpu
 
@@ -229,7 +230,7 @@ def test_mx_gemm_both_tile_shapes(d, cabi, variant, size):
         cabi.set_tuning("gemm.variant", 0)
 
 
-@pytest.mark.parametrize("variant", [0, 1, 2, 7])
+@pytest.mark.parametrize("variant", [0, 1, 2, 5, 7])
 @pytest.mark.parametrize("K", [32, 64, 96, 160, 224, 416, 1120])
 def test_mx_gemm_k_of_any_whole_number_of_blocks(d, cabi, variant, K):
     """K a multiple of 32 but not of 128 (the reference's own scale-length check leaves multiples of 128
@@ -264,7 +265,7 @@ def _poisoned_blocked(d, sc):
     return d.to_blocked(full)
 
 
-@pytest.mark.parametrize("variant", [0, 1, 2, 7, 9])
+@pytest.mark.parametrize("variant", [0, 1, 2, 5, 7, 9])
 @pytest.mark.parametrize("size", [(40, 96, 264), (133, 160, 264), (64, 1120, 520), (300, 416, 136), (16, 4128, 2048)],
                          ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
 def test_mx_gemm_ignores_the_padding_of_the_scale_buffers(d, cabi, variant, size):
@@ -354,7 +355,7 @@ def _random_gemm_sizes(seed, n):
     return [(rng.randint(1, 700), 128 * rng.randint(1, 9), 8 * rng.randint(1, 100)) for _ in range(n)]
 
 
-@pytest.mark.parametrize("variant", [0, 2, 7])
+@pytest.mark.parametrize("variant", [0, 2, 5, 7])
 @pytest.mark.parametrize("size", _random_gemm_sizes(7, 8), ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
 def test_mx_gemm_random_sizes(d, cabi, variant, size):
     """(M, K, N) with M arbitrary, N a multiple of 8 (src/mx_fp8_bf16.cu:187), K a multiple of 128: ragged edge
@@ -389,6 +390,43 @@ def test_mx_gemm_schedules_agree(d, cabi, fp4, K):
     assert torch.equal(outs[2], outs[7]) and torch.equal(outs[5], outs[7])
 
 
+@pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
+@pytest.mark.parametrize("K", [96, 160, 256, 384, 672, 768, 1120, 1280, 1312])
+def test_mx_gemm_schedules_agree_on_every_form_of_operand(d, cabi, fp4, K):
+    """The same comparison on what a caller may pass beside library-made contiguous operands: padding of the scales
+    full of NaN codes, row strides above K, an output inside a wider one that begins 8 bytes off a 16-byte boundary,
+    a row count and a column count that are no multiples of 8 -- for every number of steps, odd and even, whole and
+    partly filled last ones."""
+    M, N = 300, 580  # four tiles of 192 columns, the last with 4
+    kb = K // 2 if fp4 else K
+    x, w = _wide_operand((M, K), 4000 + K).cuda(), _wide_operand((N, K), 4001 + K).cuda()
+    quantize = cabi.mx_fp4_quantize if fp4 else cabi.mx_fp8_quantize
+    product = cabi.mx_fp4_bf16 if fp4 else cabi.mx_fp8_bf16
+    (a, sa), (b, sb) = ((q.view(torch.uint8), s.view(torch.uint8).view(-1, K // 32)) for q, s in (quantize(x), quantize(w)))
+    dtype = torch.uint8 if fp4 else E4
+
+    def strided(t, before, after):
+        wide = torch.full((t.shape[0], before + kb + after), 0x7F, dtype=torch.uint8, device="cuda")
+        wide[:, before:before + kb] = t
+        return wide[:, before:before + kb].view(dtype)
+
+    a_view, b_view = strided(a, 16, 48 - kb % 16), strided(b, 64, 16 - kb % 16)
+    outs = {}
+    for variant in (7, 2, 5):
+        cabi.set_tuning("gemm.variant", variant)
+        try:
+            outs[variant] = product(a.view(dtype), b.view(dtype), d.to_blocked(sa), d.to_blocked(sb))
+            for lead, pitch in ((4, N + 24), (8, N + 28)):  # 8 bytes off a boundary; on it, with a pitch of whole vectors
+                out = torch.full((M, pitch), 7.0, dtype=torch.bfloat16, device="cuda")
+                product(a_view, b_view, _poisoned_blocked(d, sa), _poisoned_blocked(d, sb), out[:, lead:lead + N])
+                assert torch.equal(out[:, lead:lead + N], outs[variant]), (variant, lead)
+                assert (out[:, :lead] == 7.0).all() and (out[:, lead + N:] == 7.0).all(), (variant, lead)
+        finally:
+            cabi.set_tuning("gemm.variant", 0)
+    assert torch.isfinite(outs[7]).all() and outs[7].abs().max() > 0
+    assert torch.equal(outs[2], outs[7]) and torch.equal(outs[5], outs[7])
+
+
 def _wide_operand(shape, seed):
     """N(0, 1) rows with scales that differ from block to block, so that a scale of the wrong row or block shows"""
     g = torch.Generator().manual_seed(seed)
@@ -414,18 +452,20 @@ def test_mx_gemm_split_k(d, cabi, splits, size):
 
 
 @pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
-@pytest.mark.parametrize("size", [(256, 8192, 8192), (250, 7200, 8184),  # two shares of a tile, even and not
-                                  (100, 4128, 14336),  # two shares of 16 and 17 steps
-                                  (128, 5120, 5120), (65, 5152, 5000),  # up to four shares of ten steps or more
-                                  (1000, 2048, 2048)],  # too few steps for any
-                         ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
+@pytest.mark.parametrize("size", SHARES, ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
 def test_mx_gemm_few_shares_by_rule(d, cabi, size, fp4):
-    """the sizes around which the library's own rule shares K or does not: integers of at most 4, so that every
-    partial sum (at most 16 K < 2^18) is exact in fp32 whatever the order and the result is one bit pattern"""
+    """The sizes around which the library's own rule shares K or does not (how many shares each has is checked where
+    the rule is): integers of at most 4 times a power of two of each block's own, up to 2^3 in one operand and 2^2 in
+    the other, so that a share that took its scales elsewhere along K would show, and every partial sum
+    (at most 2^9 K < 2^24) is exact in fp32 whatever the order: the result is one bit pattern."""
     M, K, N = size
     g = torch.Generator(device="cuda").manual_seed(M + K)
-    a = torch.randint(-4, 5, (M, K), generator=g, device="cuda").float()
-    b = torch.randint(-4, 5, (N, K), generator=g, device="cuda").float()
+
+    def integers(rows, top):
+        v = torch.randint(-4, 5, (rows, K // 32, 32), generator=g, device="cuda").float()
+        return (v * torch.exp2(torch.randint(0, top + 1, (rows, K // 32, 1), generator=g, device="cuda").float())).view(rows, K)
+
+    a, b = integers(M, 3), integers(N, 2)
     want = (a @ b.t()).bfloat16()
     if fp4:
         (qa, sa), (qb, sb) = (d.mx_fp4_quantize(t.bfloat16(), blocked=True) for t in (a, b))
