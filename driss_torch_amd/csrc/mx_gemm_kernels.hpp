@@ -446,11 +446,15 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   const uint32_t sc_lane_b = (TN == 6 ? 0 : ((b_row0 & ~127) >> 7) * 512) + l16 * 16 + kOffSB + ((TN == 4 && (wn & 1)) ? 8 : 0);
   if constexpr (HELD) {
     // ---- The held schedule: every B fragment of a step meets all TM fragments of A before the next one is
-    // taken up.  On random operands the launch runs at the chip's power limit, so what counts is the energy of
-    // an MFMA, and that depends on what changes between neighbours.  MFMAs alone, 16 x 16 x 128 on N(0,1)-like
-    // operands in registers, PFLOP/s e4m3 / e2m1: first operand the same for 8 of them 4.39 / 7.15, for 4
-    // 4.10 / 6.43, second operand the same for 8 3.99 / 5.97, both changed each time 3.71 / 5.47 (32 x 32 x 64:
-    // 3.71; operands of ones 4.87 whatever the order).  The quadrants below hold the first operand for 4.
+    // taken up.  With one wave per SIMD what stands between the MFMAs is lost, and here that is less: two steps
+    // per turn of the loop make slots, register sets and LDS addresses constants, and scales come as bytes that
+    // need no shift, so that a step of e4m3 has 108 other instructions where the quadrants below have 133 (3 and
+    // 26 of them vector arithmetic), a step of e2m1 144 and 171.  8192^3, shader cycles, quadrants -> here: e4m3
+    // 681 000 -> 658 000 on N(0,1)-derived operands and 682 000 -> 648 000 on ones, e2m1 438 000 -> 428 000.  On
+    // random operands the launch runs at the chip's power limit, where the clock gives back a third of that (1.89
+    // -> 1.87 GHz).  The order by itself saves little power: MFMAs alone on operands in registers, PFLOP/s e4m3 /
+    // e2m1 after a second of them, first operand kept for 8 MFMAs 4.22 / 7.07, for 4 (the quadrants) 4.19 / 7.04,
+    // second operand kept for 8 4.22 / 7.06, both changed each time 4.07 / 6.84; ones 4.81 / 9.24 in any order.
     // In a launch (us, before -> this schedule, e4m3): 8192^3 366.0 -> 359.3, 8192 x 4096 x 14336 308.1 ->
     // 303.1, 4096 x 8192 x 4096 101.9 -> 99.2, 5120^3 108.3 -> 105.1, 2000 x 5120 x 5120 51.3 -> 49.2;
     // e2m1: 8192^3 235.5 -> 229.7, 5120^3 70.7 -> 66.2, 2048 x 5120 x 5120 34.5 -> 30.9; with a partly filled
