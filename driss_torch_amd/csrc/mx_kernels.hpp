@@ -945,8 +945,9 @@ __global__ void fill_bytes_kernel(uint8_t* p, int64_t n, uint8_t value) {
 // matrices, so the four loads are unconditional: whatever the width and the alignment, a word is loaded where it
 // lies (the matrix's last three positions: its last word, shifted), rows past the end re-read the last row, and
 // what is not the row's becomes zero afterwards.  (Byte by byte under a test each, rows of no whole words took one
-// latency after the other: 448 x 137 3.04 -> 1.83 us, 16384 x 511 15.2 -> 9.2; 8192 x 256 3.8 and 3.9.)  TINY: a matrix of fewer than four bytes, read byte by byte.  TileNumber:
-// 32 bits wherever they count the tiles, for the division.
+// latency after the other: 448 x 137 3.04 -> 1.83 us, 16384 x 511 15.2 -> 9.2; 8192 x 256 3.8 and 3.9.)  TINY: a
+// matrix of fewer than four bytes, read byte by byte.  TileNumber: 32 bits wherever they count the tiles, for the
+// division.
 template <bool TINY, typename TileNumber>
 __global__ __launch_bounds__(kBlock) void to_blocked_kernel(const uint8_t* __restrict__ in, int64_t R, int64_t C, int64_t groups,
                                                             uint8_t* __restrict__ out) {

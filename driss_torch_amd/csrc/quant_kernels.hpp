@@ -95,7 +95,8 @@ __global__ __launch_bounds__(BLOCK) void amax_kernel(const void* __restrict__ x,
   const int64_t i = ((int64_t)(tid / kBlock) * gridDim.x + blockIdx.x) * kBlock + tid % kBlock;
   // First and last of the vectors i of the workgroup: whether a batch is whole is asked for all of its threads at once,
   // and the loop below has one way out.  (With lanes that leave it by themselves, or two ways out, the compiler waits
-  // for a batch before it requests the next.)
+  // for a batch before it requests the next: 5000 x 7000 bf16 15.4 -> 14.4 us, 9000 x 9000 27.5 -> 26.4, 16384 x 8000
+  // 41.2 -> 40.4; 2048 x 109760 67.2 and 67.4 in a graph, 64.9 -> 65.7 launched one after the other.)
   const int64_t first = (int64_t)blockIdx.x * kBlock, last = ((int64_t)(BLOCK / kBlock - 1) * gridDim.x + blockIdx.x) * kBlock + kBlock - 1;
   const uint32_t lane_bytes = (uint32_t)i * 16u;  // a grid's worth of vectors is far below 2^28: scalar bases and 32-bit lane offsets
   auto whole_batch_at = [&](int64_t k) { return last + k + (P - 1) * stride < sp.nvec; };
@@ -107,7 +108,8 @@ __global__ __launch_bounds__(BLOCK) void amax_kernel(const void* __restrict__ x,
   // What is left behind the last whole batch: all of its loads at once and under way before that batch is looked at
   // (past the end the last vector again, which changes no maximum).  One at a time behind it, as it was, they cost a
   // memory latency each, and most sizes leave some (us, bf16: 576 x 2048 5.4 -> 4.3, 700 x 2000 5.4 ->
-  // 4.4, with the cast behind it 14 x 7528 6.9 -> 5.8, 3111 x 2048 10.9 -> 10.1).
+  // 4.4, with the cast behind it 14 x 7528 6.9 -> 5.8, 3111 x 2048 10.9 -> 10.1).  (Through a buffer descriptor that ends
+  // with the tensor, as rows are read, 5000 x 7000 takes 14.5 -> 15.0 us, 9000 x 9000 26.5 -> 26.8.)
   auto load_rest = [&](u32x4 (&w)[P], int64_t k) {
 #pragma unroll
     for (int u = 0; u < P; ++u) {
