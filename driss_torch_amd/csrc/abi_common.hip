@@ -36,14 +36,15 @@ struct Knob {
 //   mx.colt_pipe: the transposed column cast as a grid of this many workgroups per CU that walk the tiles
 //                 with the next tile's loads in flight (0 = one workgroup per tile)
 //   mx.row_band4: 1 = row-wise MX cast with blocked scales walks 4 rows x 512 elements per wave pass
-//   gemm.variant: 0 = pick the tile by problem size, 1 = 128x128 tiles, 2 = 256x256 tiles, 5 = 256x192 tiles,
+//   gemm.variant: 0 = pick the tile by problem size, 1 = 128x128 tiles, 2 = 256x256 tiles, 3 = tiles of 64 or 128 rows
+//                 and columns as gemm.tile_m and gemm.tile_n say (0 = by the estimate), 5 = 256x192 tiles,
 //                 7 = 256x256 tiles on the main loop of the smaller ones (quadrants of the wave tile, no L2 prefetch;
 //                 the same bits), 9 = the kernel for at most 64 rows whatever the other dimensions
 //   gemm.few_rows_tiles: 16-column tiles per wave of that kernel: 0 = by the number of columns, 1, 2
 //   gemm.tail_quads: 1 = tiles left over after whole rounds of 256x256 tiles run as 128x128 quadrants
 //                 or 256x128 halves when those fit the chip at once, 0 = never, 2 = always as
 //                 quadrants, 3 = always as halves
-//   gemm.split_k: 0 = share K between workgroups when the 128x128 tiling leaves CUs idle (needs the
+//   gemm.split_k: 0 = share K between workgroups when the small tiles leave CUs idle (needs the
 //                 workspace of the _ws entry points), 1 = never, n = n workgroups per tile
 Knob g_knobs[] = {
     {"gemm.few_rows_tiles", 0},
@@ -64,6 +65,8 @@ Knob g_knobs[] = {
     {"mx.colt_via_dual", 1},
     {"mx.row_band4", 1},
     {"gemm.variant", 0},
+    {"gemm.tile_m", 0},
+    {"gemm.tile_n", 0},
     {"gemm.split_k", 0},
     {"gemm.tail_quads", 1},
     {"dynamic.resident", 0},

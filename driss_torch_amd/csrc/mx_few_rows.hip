@@ -359,10 +359,13 @@ constexpr size_t kLdsLimit = 160 * 1024;
 // Two tiles per group halve the workgroups' reads of A (every group reads all of it) and win wherever they
 // still give every CU a group (8192 x 8192, us, one tile / two: e4m3 1 row 16.2 / 15.6, 8 rows 16.8 / 15.8,
 // 16 rows 18.3 / 16.5, 56 rows 28.9 / 20.9; e2m1 1 row 10.9 / 9.4, 56 rows 16.5 / 12.2).
+int tiles_per_group(int64_t N) {
+  const int tiles = tuning("gemm.few_rows_tiles");
+  return tiles ? (tiles == 2 ? 2 : 1) : (N >= 32 * (int64_t)device_facts().cu_count ? 2 : 1);
+}
 Plan plan_for(bool fp4, int64_t M, int64_t N) {
   Plan p;
-  const int tiles = tuning("gemm.few_rows_tiles");
-  p.nt = tiles ? (tiles == 2 ? 2 : 1) : (N >= 32 * (int64_t)device_facts().cu_count ? 2 : 1);
+  p.nt = tiles_per_group(N);
   const int mt = (int)((M + 15) / 16);
   int up = tuning("gemm.few_rows_steps");
   if (up != 1 && up != 2) up = mt == 1 ? 2 : 1;
@@ -401,25 +404,7 @@ int launch_instance(const uint8_t* a, const uint8_t* b, const uint8_t* sfa, cons
 // What the kernel takes at all: its 32-bit lane offsets into A's blocked scales span 4 K bytes
 bool few_rows_fits(int64_t M, int64_t K) { return M <= 64 && K <= ((int64_t)1 << 29); }
 
-// Where the kernel above beats the 128 x 128 tiles that share K through a workspace (measured on MI355X,
-// us, B rotated through enough buffers that it comes from HBM; few rows / tiles):
-//   8192 x 8192:  e4m3 M = 8 15.7 / 20.7, 16 16.4 / 20.0, 32 18.1 / 20.5, 64 21.7 / 21.8; e2m1 10.1 / 21.8, 10.5 / 21.9, 11.6 / 22.0, 13.0 / 22.3
-//   4096 x 14336 (N x K): e4m3 16.5 / 20.8, 18.5 / 21.3, 22.0 / 21.6, 26.9 / 23.0; e2m1 9.9 / 18.1 ... 14.3 / 19.4
-//   16384 x 4096: e4m3 15.3 / 20.3, 16.0 / 20.3, 18.9 / 20.6, 23.9 / 22.0; e2m1 11.1 / 14.4 ... 14.1 / 14.3
-//   2048 x 8192, 1024 x 8192, 4096 x 4096, 8192 x 2048: 0.25 to 0.7 of the tiles' time for every M
-//   28672 x 4096: e4m3 27.2 / 31.1, 28.7 / 28.9, 33.3 / 29.1, 41.4 / 30.3; e2m1 17.4 / 16.5 ... 24.3 / 16.8
-//   32768 x 1024: 1.1 to 1.9 times the tiles' time
-// A group of columns costs its reduction and two barriers whatever K is, so many groups with a short K
-// lose; and with e4m3 operands and more than 32 rows the workgroups' reads of A (every workgroup reads
-// all of it) weigh as much as B once the problem is large.
-bool few_rows_pays(bool fp4, int64_t M, int64_t N, int64_t K, bool have_workspace) {
-  (void)have_workspace;
-  if (!few_rows_fits(M, K)) return false;
-  if (N < 1024 || K < 2048) return false;
-  if (K < 8192 && N > 16384) return false;
-  if (!fp4 && M > 32 && N * K > ((int64_t)1 << 25)) return false;
-  return true;
-}
+int few_rows_columns(int64_t N) { return 16 * tiles_per_group(N); }
 
 int launch_few_rows(bool fp4, const uint8_t* a, const uint8_t* b, const uint8_t* sfa, const uint8_t* sfb, int64_t M, int64_t N,
                     int64_t K, int64_t lda, int64_t ldb, void* out, int64_t ldo, hipStream_t stream) {

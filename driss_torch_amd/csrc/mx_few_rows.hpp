@@ -9,8 +9,8 @@ namespace dt {
 // Can the kernel for few rows take the problem at all (M <= 64 and a K its 32-bit offsets span)?
 bool few_rows_fits(int64_t M, int64_t K);
 
-// Does the kernel for few rows beat the tiles for this problem?  (fp4: e2m1 operands; K counts elements.)
-bool few_rows_pays(bool fp4, int64_t M, int64_t N, int64_t K, bool have_workspace);
+// Columns of B that a workgroup of it takes at a time, 16 or 32.
+int few_rows_columns(int64_t N);
 
 // M <= 64; operands as for dt_mx_fp8_bf16 / dt_mx_fp4_bf16, already checked.  Returns a dt_status.
 int launch_few_rows(bool fp4, const uint8_t* a, const uint8_t* b, const uint8_t* sfa, const uint8_t* sfb, int64_t M,

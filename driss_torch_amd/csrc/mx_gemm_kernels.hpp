@@ -30,6 +30,7 @@
 #include "dt_host.hpp"
 #include "mx_few_rows.hpp"
 #include "mx_gemm_plan.hpp"
+#include "mx_ring.hpp"
 
 namespace dt {
 
@@ -56,22 +57,11 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 // which are the same two 16-byte reads a lane makes for e4m3.  Everything else (panels, DMA,
 // swizzle, ring, quadrant schedule, epilogue) is shared; a K-step carries twice the scales.
 //
-// SPLIT: the K-steps of a tile are shared between `splits` workgroups (workgroup = tile + split *
-// tiles).  Each parks its fp32 accumulators in `partial`, lane for lane, and takes a ticket of
-// its tile; whoever draws the last ticket adds the parked accumulators in split order (so the sum
-// does not depend on who came last), writes the bf16 tile and puts the ticket counter back to
-// zero.  Nobody waits for anybody.
-// The parked accumulators travel as device-scope relaxed atomics (stores that write through the
-// XCD's L2, loads that miss it): ordinary stores would need a release and an acquire fence around
-// the ticket, i.e. a write-back and an invalidation of the whole L2 that every other workgroup
-// of the XCD is reading its panels through (measured: 1024^3 20.5 us with the fences, 8.8 us
-// without splitting).
-//
 // MODE kQuads: the workgroup computes one 128 x 128 quadrant of a 256 x 256 tile, for the tiles that
 // the 256 x 256 kernel leaves over when its grid is cut to whole rounds of the chip (tiles_m,
 // tiles_n and first_block then describe the 256 x 256 tiling).
 // MODE kHalves: the same with the 256 x 128 halves of a tile.
-enum GemmMode { kPlain = 0, kSplitK = 1, kQuads = 2, kHalves = 3 };
+enum GemmMode { kPlain = 0, kQuads = 2, kHalves = 3 };
 // KTAIL: the last K-step is partly filled (K is not a multiple of 128 bytes of a row).  Everything that
 // deals with it is compiled only then: a branch or two in the K loop cost the kernel for whole steps 3 to
 // 6 % (measured), whatever they guard.
@@ -79,9 +69,7 @@ template <int BM, int BN, int WAVES_M, int WAVES_N, int NST, bool FP4, bool TOUC
 __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, const uint8_t* __restrict__ sfa,
     const uint8_t* __restrict__ sfb, int M, int N, int K, int64_t lda, int64_t ldb, uint16_t* __restrict__ out,
-    int64_t ldo, int tiles_m, int tiles_n, int wide_stores, int splits, v4f* __restrict__ partial,
-    uint32_t* __restrict__ tickets, int first_block, uint64_t* __restrict__ phase_log) {
-  constexpr bool SPLIT = MODE == kSplitK;
+    int64_t ldo, int tiles_m, int tiles_n, int wide_stores, int first_block, uint64_t* __restrict__ phase_log) {
   // phase_log (only in a build with DT_PHASE_LOG, and normally null there; dt_set_phase_log): per workgroup
   // four readings of the 100 MHz constant-rate counter -- start, K loop entered, K loop left, output
   // stored -- and where it ran (XCC_ID, HW_ID), stored at the very end.
@@ -90,7 +78,6 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
     else return 0;
   };
   const uint64_t t_start = clock_reading();
-  static_assert(!(SPLIT && TOUCH), "the prefetch shares assume that a workgroup walks the whole K");
   static_assert(MODE != kQuads || (BM == 128 && BN == 128), "quadrants of a 256 x 256 tile");
   static_assert(MODE != kHalves || (BM == 256 && BN == 128), "halves of a 256 x 256 tile");
   constexpr bool PARTS = MODE == kQuads || MODE == kHalves;
@@ -121,11 +108,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   // ids so that neighbours in the tile grid share an L2, then walk tiles in column groups.
   int bid = blockIdx.x;
   const int nb = tiles_m * tiles_n;
-  int split = 0, quad = 0;
-  if constexpr (SPLIT) {
-    split = bid / nb;
-    bid -= split * nb;
-  }
+  int quad = 0;
   if constexpr (PARTS) {
     // workgroup 8 * (kParts * g + part) + x: part `part` of tile first_block + 8 g + x, so that a tile's
     // parts run on one XCD (x) and first_block (a multiple of 8) continues the big kernel's runs
@@ -158,21 +141,10 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   // 128-element scale chunks; when the last step has no second chunk at all (K % 256 in 1..128) its
   // second MFMA is switched off through the scale operand (see scale_bits).
   const int k_bytes = FP4 ? K / 2 : K;
-  int k_steps = (k_bytes + kBK - 1) / kBK;
+  const int k_steps = (k_bytes + kBK - 1) / kBK;
   const int k_chunks = (K + 127) / 128;                           // blocked scale chunks per 128 rows
-  int tail_step = KTAIL ? k_steps - 1 : -1;                            // index of a partly filled step
-  int half_step = (KTAIL && FP4 && (k_chunks & 1)) ? k_steps - 1 : -1;  // index of a step without a second scale chunk
-  // SPLIT: this workgroup walks steps ks_begin .. ks_begin + k_steps; from here on steps and scale
-  // chunks count from ks_begin (the host makes sure that every split owns a step)
-  int ks_begin = 0, k_chunks_left = k_chunks;
-  if constexpr (SPLIT) {
-    const int per = (k_steps + splits - 1) / splits;
-    ks_begin = split * per;
-    k_steps = k_steps - ks_begin < per ? k_steps - ks_begin : per;
-    half_step -= ks_begin;
-    tail_step -= ks_begin;
-    k_chunks_left -= ks_begin * KC;
-  }
+  const int tail_step = KTAIL ? k_steps - 1 : -1;                            // index of a partly filled step
+  const int half_step = (KTAIL && FP4 && (k_chunks & 1)) ? k_steps - 1 : -1;  // index of a step without a second scale chunk
 
   // ---- global -> LDS.  Wave w owns groups w*kLoads .. of each panel; lane L fills row L/8,
   // chunk position L%8 of the group, i.e. it fetches logical chunk (L%8) ^ (L/8) of that row.
@@ -184,8 +156,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   // three loads are one instruction each.  Load n of a run carries offset n * kGroupStride; its lane
   // offset is lowered by as much, and the scalar bases by kRunBias so that no lane offset goes negative.
   constexpr uint32_t kRun = 4, kRunBias = (kRun - 1) * kGroupStride;
-  const uint8_t* const A_tile = A + (int64_t)m0 * lda + (int64_t)ks_begin * kBK - kRunBias;
-  const uint8_t* const B_tile = B + (int64_t)n0 * ldb + (int64_t)ks_begin * kBK - kRunBias;
+  const uint8_t* const A_tile = A + (int64_t)m0 * lda - kRunBias;
+  const uint8_t* const B_tile = B + (int64_t)n0 * ldb - kRunBias;
   const int lrow = lane >> 3, lchunk = (lane & 7) ^ lrow;
   // in a partly filled step of v valid chunks, chunk c >= v reads chunk c % v again
   const int tail_chunks = (k_bytes % kBK) / 16;
@@ -211,7 +183,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   const int chunk_max = (wave_is_b ? (N + 127) / 128 : (M + 127) / 128) - 1;
   const int chunk0 = (wave_is_b ? n0 : m0) / 128;  // the tile's first chunk row: part of the scalar base
   const int chunk = chunk0 + (lane >> 5) < chunk_max ? chunk0 + (lane >> 5) : chunk_max;
-  const uint8_t* sc_base = (wave_is_b ? sfb : sfa) + ((int64_t)chunk0 * k_chunks + (int64_t)ks_begin * KC) * 512;
+  const uint8_t* sc_base = (wave_is_b ? sfb : sfa) + (int64_t)chunk0 * k_chunks * 512;
   const uint32_t sc_off = (uint32_t)((int64_t)(chunk - chunk0) * k_chunks * 512 + (lane & 31) * 16);
   const int sc_dst = wave_is_b ? kOffSB : kOffSA;
   // load number n of a step: n < kLoadsA -> A group, < kLoadsA+kLoadsB -> B group, else scales
@@ -245,7 +217,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   auto base_b = [&](int ks) { return B_tile + (int64_t)ks * kBK; };
   auto base_s = [&](int ks, int c) {  // chunk c of the step; past the end it re-reads the last one (switched off)
     int kc = ks * KC + c;
-    kc = kc < k_chunks_left ? kc : k_chunks_left - 1;
+    kc = kc < k_chunks ? kc : k_chunks - 1;
     return sc_base + (int64_t)kc * 512;
   };
   auto fetch_one = [&](int n, const StepBases& at, uint32_t buf, uint32_t adj) {
@@ -316,7 +288,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   auto mask_tail_scales = [&](uint32_t stage) {
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
-      const int valid = k_blocks - ((ks_begin + tail_step) * KC + c) * 4;  // K-blocks of this chunk inside K
+      const int valid = k_blocks - (tail_step * KC + c) * 4;  // K-blocks of this chunk inside K
       if (valid >= 4) continue;
       const uint32_t keep = valid <= 0 ? 0u : (1u << (8 * valid)) - 1u;
       uint32_t* const wa = reinterpret_cast<uint32_t*>(lds + stage + kOffSA + c * 1024) + tid;
@@ -471,7 +443,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
     constexpr int kBar = 8 * (TN - 4) + 5;     // time slot of the step's barrier: b[TN - 1] was requested five slots before
     constexpr int kSlots = 8 * TN;             // time slots of a step: one e4m3 MFMA or two e2m1 MFMAs each
     constexpr int kPostLoads = kLoadsA + kLoadsB - kLoadsB % kRun - (kLoadsB % kRun ? 0 : kRun);  // whole runs: sent before the step ends
-    static_assert(TM == 8 && NST == 2 && !SPLIT && !PARTS && TOUCH, "the held schedule");
+    static_assert(TM == 8 && NST == 2 && !PARTS && TOUCH, "the held schedule");
     Frag fa[2][TM], fb[kRing];
     int sa[2][KC][TM], sb[KC][kRing];
     // slot 0 and slot 1 of the LDS ring: a step's slot is known at compile time, its addresses are constants
@@ -857,70 +829,6 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
   __syncthreads();
   const uint64_t t_loop_end = clock_reading();
 
-  if constexpr (SPLIT) {
-    __shared__ uint32_t drawn;
-    const int tile_id = tile_m * tiles_n + tile_n;
-    const size_t per_split = (size_t)nb * (kWaves * TM * TN * kWave);  // accumulators (4 floats each) per split
-    // a wave's 16 x 16 tile is two planes of 64 x 8 bytes (the accumulator's first and second pair
-    // of floats), so that each 8-byte store instruction writes 512 contiguous bytes
-    uint64_t* const mine = reinterpret_cast<uint64_t*>(partial + ((size_t)tile_id * kWaves + wave) * (TM * TN * kWave)) + lane;
-    // 16 x 16 tiles wholly outside the matrix are neither parked nor added (uniform per wave)
-    auto inside = [&](int i, int j) { return m0 + wm * WM + i * 16 < M && n0 + wn * WN + j * 16 < N; };
-    typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
-    auto park = [](uint64_t* q, v4f v) {
-      const u64x2 w = __builtin_bit_cast(u64x2, v);
-      __hip_atomic_store(q, w.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(q + kWave, w.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    auto fetch_parked = [](const uint64_t* q) -> v4f {
-      u64x2 w;
-      w.x = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      w.y = __hip_atomic_load(q + kWave, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return __builtin_bit_cast(v4f, w);
-    };
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        if (inside(i, j)) park(mine + (split * per_split + (i * TN + j) * kWave) * 2, acc[i][j]);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the parked values have arrived before the ticket is drawn
-    __syncthreads();
-    if (tid == 0) drawn = __hip_atomic_fetch_add(tickets + tile_id, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (drawn != (uint32_t)(splits - 1)) return;
-    if (tid == 0) tickets[tile_id] = 0u;  // every split has drawn: ready for the next launch
-    // The loads of kBatch splits first, then the additions in split order: a round trip to memory
-    // per kBatch splits, not one per split and tile.  The workgroup's own share is read back like
-    // the others (the same bits as in its registers), which keeps the loop free of selects; tiles
-    // outside the matrix and splits past the last add zeros.
-    constexpr int kBatch = 4;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (int sp0 = 0; sp0 < splits; sp0 += kBatch) {
-      v4f p[kBatch][TM][TN];
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            p[u][i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-            if (sp0 + u < splits && inside(i, j))
-              p[u][i][j] = fetch_parked(mine + ((sp0 + u) * per_split + (i * TN + j) * kWave) * 2);
-          }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] += p[u][i][j];
-    }
-    __syncthreads();  // `drawn` and the epilogue staging share no bytes, but keep the waves together
-  }
-
   // ---- epilogue: fp32 -> bf16 (v_cvt_pk_bf16_f32, round to nearest even) and out through LDS.
   // A lane holds 4 consecutive columns of one row per tile; written straight to memory that is
   // 32-byte pieces of 16 different rows per store.  Instead every wave parks its WM x WN tile
@@ -1010,8 +918,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* kWave) void mx_gemm_kernel(
 // quadrants of `blocks` 256 x 256 tiles from tile number first_block on)
 template <int BM, int BN, int WAVES_M, int WAVES_N, int NST, bool FP4, bool TOUCH, int MODE, bool KTAIL>
 int launch_gemm_impl(const uint8_t* a, const uint8_t* b, const uint8_t* sfa, const uint8_t* sfb, int64_t M, int64_t N,
-                int64_t K, int64_t lda, int64_t ldb, void* out, int64_t ldo, hipStream_t stream, int splits,
-                void* workspace, int64_t blocks, int first_block) {
+                int64_t K, int64_t lda, int64_t ldb, void* out, int64_t ldo, hipStream_t stream,
+                int64_t blocks, int first_block) {
   constexpr bool kParts = MODE == kQuads || MODE == kHalves;
   constexpr int kTileM = kParts ? 256 : BM, kTileN = kParts ? 256 : BN;
   const int tiles_m = (int)ceil_div(M, kTileM), tiles_n = (int)ceil_div(N, kTileN);
@@ -1023,7 +931,7 @@ int launch_gemm_impl(const uint8_t* a, const uint8_t* b, const uint8_t* sfa, con
   if (lds_bytes < epi_bytes) lds_bytes = epi_bytes;
   // A grid that fits the chip once should land one workgroup per CU: asking for more than half
   // of the LDS keeps the dispatcher from pairing two workgroups on one CU while others idle.
-  if ((int64_t)tiles_m * tiles_n * splits <= device_facts().cu_count && lds_bytes < 82 * 1024) lds_bytes = 82 * 1024;
+  if ((int64_t)tiles_m * tiles_n <= device_facts().cu_count && lds_bytes < 82 * 1024) lds_bytes = 82 * 1024;
   auto kernel = mx_gemm_kernel<BM, BN, WAVES_M, WAVES_N, NST, FP4, TOUCH, MODE, KTAIL>;
   if (lds_bytes > 64 * 1024) {
     // once per instantiation and device, with the largest size asked for so far (a host call per launch otherwise)
@@ -1038,26 +946,24 @@ int launch_gemm_impl(const uint8_t* a, const uint8_t* b, const uint8_t* sfa, con
       if (tracked) allowed[dev].store((int)lds_bytes, std::memory_order_relaxed);
     }
   }
-  uint8_t* const ws = static_cast<uint8_t*>(workspace);  // ticket counters, then the parked accumulators
-  int64_t grid = (int64_t)tiles_m * tiles_n * splits;
+  int64_t grid = (int64_t)tiles_m * tiles_n;
   if (blocks > 0) grid = kParts ? (MODE == kQuads ? 32 : 16) * ceil_div(blocks, (int64_t)8) : blocks;
   kernel<<<(unsigned)grid, WAVES_M * WAVES_N * kWave, lds_bytes, stream>>>(
       a, b, sfa, sfb, (int)M, (int)N, (int)K, lda, ldb, static_cast<uint16_t*>(out), ldo, tiles_m, tiles_n,
-      (ldo % 8 == 0 && aligned(out, 16)) ? 1 : 0, splits, ws ? reinterpret_cast<v4f*>(ws + kSplitTicketBytes) : nullptr,
-      reinterpret_cast<uint32_t*>(ws), first_block, phase_log((size_t)grid * 64));
+      (ldo % 8 == 0 && aligned(out, 16)) ? 1 : 0, first_block, phase_log((size_t)grid * 64));
   return launch_status();
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int NST, bool FP4, bool TOUCH, int MODE = kPlain>
 int launch_gemm(const uint8_t* a, const uint8_t* b, const uint8_t* sfa, const uint8_t* sfb, int64_t M, int64_t N,
-                int64_t K, int64_t lda, int64_t ldb, void* out, int64_t ldo, hipStream_t stream, int splits = 1,
-                void* workspace = nullptr, int64_t blocks = 0, int first_block = 0) {
+                int64_t K, int64_t lda, int64_t ldb, void* out, int64_t ldo, hipStream_t stream, int64_t blocks = 0,
+                int first_block = 0) {
   const int64_t k_bytes = FP4 ? K / 2 : K;
   if (k_bytes % kBK != 0)  // a partly filled last step: the build of the kernel that deals with it
-    return launch_gemm_impl<BM, BN, WAVES_M, WAVES_N, NST, FP4, TOUCH, MODE, true>(a, b, sfa, sfb, M, N, K, lda, ldb, out, ldo, stream,
-                                                                                 splits, workspace, blocks, first_block);
-  return launch_gemm_impl<BM, BN, WAVES_M, WAVES_N, NST, FP4, TOUCH, MODE, false>(a, b, sfa, sfb, M, N, K, lda, ldb, out, ldo, stream,
-                                                                                splits, workspace, blocks, first_block);
+    return launch_gemm_impl<BM, BN, WAVES_M, WAVES_N, NST, FP4, TOUCH, MODE, true>(a, b, sfa, sfb, M, N, K, lda, ldb, out, ldo, stream, blocks,
+                                                                                 first_block);
+  return launch_gemm_impl<BM, BN, WAVES_M, WAVES_N, NST, FP4, TOUCH, MODE, false>(a, b, sfa, sfb, M, N, K, lda, ldb, out, ldo, stream, blocks,
+                                                                                 first_block);
 }
 
 inline size_t split_workspace_bytes() { return kSplitTicketBytes + (size_t)device_facts().cu_count * kSplitTileBytes; }
@@ -1082,11 +988,24 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
   const uint8_t* A = static_cast<const uint8_t*>(a);
   const uint8_t* B = static_cast<const uint8_t*>(b);
   hipStream_t s = as_hip(stream);
-  const int variant = tuning("gemm.variant");
-  if ((variant == 9 && few_rows_fits(M, K)) || (variant == 0 && few_rows_pays(FP4, M, N, K, workspace != nullptr)))
-    return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
-  const int cus = device_facts().cu_count;
-  const GemmPlan plan = plan_gemm(FP4, M, N, K, workspace ? workspace_bytes : 0, cus, variant, tuning("gemm.tail_quads"), tuning("gemm.split_k"));
+  const int variant = tuning("gemm.variant"), split_k = tuning("gemm.split_k"), cus = device_facts().cu_count;
+  const size_t room = workspace ? workspace_bytes : 0;
+  const bool ragged = ring_ragged(k_bytes, A, B, lda, ldb);
+  const auto ring = [&](int tile_m, int tile_n, int splits) {
+    const RingArgs p{A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, workspace, s};
+    return FP4 ? launch_ring_e2m1(p, ragged, tile_m, tile_n, splits) : launch_ring_e4m3(p, ragged, tile_m, tile_n, splits);
+  };
+  const auto by_estimate = [&]() {
+    return plan_ring(FP4, M, N, K, ragged, room, cus, split_k, variant == 3 ? tuning("gemm.tile_m") : 0, variant == 3 ? tuning("gemm.tile_n") : 0);
+  };
+  if (variant == 9 && few_rows_fits(M, K)) return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
+  if (variant == 3 || (variant == 0 && few_rows_fits(M, K))) {
+    const RingPlan r = by_estimate();
+    if (variant == 0 && split_k == 0 && few_rows_beats(r, FP4, M, N, K, ragged, cus, few_rows_columns(N)))
+      return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
+    return ring(r.tile_m, r.tile_n, r.splits);
+  }
+  const GemmPlan plan = plan_gemm(FP4, M, N, K, room, cus, variant, tuning("gemm.tail_quads"), split_k);
   // tiles of 256 x 256 in whole rounds of the chip, and those behind them
   const int64_t tiles256 = ceil_div(M, 256) * ceil_div(N, 256), whole = tiles256 / cus * cus, left = tiles256 - whole;
   // <tile M, tile N, waves M, waves N, LDS ring slots, e2m1 operands>
@@ -1097,25 +1016,24 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
       return launch_gemm<256, 256, 2, 2, 2, FP4, true>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
     case kTiles256ThenQuads:
     case kTiles256ThenHalves: {
-      const int st = launch_gemm<256, 256, 2, 2, 2, FP4, true>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, 1, nullptr, whole);
+      const int st = launch_gemm<256, 256, 2, 2, 2, FP4, true>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, whole);
       if (st != DT_OK) return st;
       if (plan.tiles == kTiles256ThenQuads)
-        return launch_gemm<128, 128, 2, 2, 4, FP4, false, kQuads>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, 1, nullptr,
-                                                                  left, (int)whole);
-      return launch_gemm<256, 128, 2, 2, 3, FP4, false, kHalves>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, 1, nullptr,
-                                                                 left, (int)whole);
+        return launch_gemm<128, 128, 2, 2, 4, FP4, false, kQuads>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, left,
+                                                                  (int)whole);
+      return launch_gemm<256, 128, 2, 2, 3, FP4, false, kHalves>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, left,
+                                                                 (int)whole);
     }
     case kTiles256Halves:
-      return launch_gemm<256, 128, 2, 2, 3, FP4, false, kHalves>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, 1, nullptr,
-                                                                 tiles256, 0);
+      return launch_gemm<256, 128, 2, 2, 3, FP4, false, kHalves>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, tiles256, 0);
     case kTiles256QuadrantSchedule:
       return launch_gemm<256, 256, 2, 2, 2, FP4, false>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
     case kTiles128:
       break;
   }
-  if (plan.splits > 1)
-    return launch_gemm<128, 128, 2, 2, 4, FP4, false, kSplitK>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, plan.splits, workspace);
-  return launch_gemm<128, 128, 2, 2, 4, FP4, false>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
+  if (variant == 1) return ring(128, 128, plan.splits);
+  const RingPlan r = by_estimate();
+  return ring(r.tile_m, r.tile_n, r.splits);
 }
 
 }  // namespace dt

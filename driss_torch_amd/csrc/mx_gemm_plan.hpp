@@ -17,8 +17,8 @@ constexpr size_t kSplitTileBytes = 128 * 128 * 4;  // parked fp32 accumulators o
 constexpr int kMaxSplits = 16;      // what gemm.split_k may force
 constexpr int kAutoMaxSplits = 12;  // what the library picks by itself
 
-// Split-K factor for the 128 x 128 tiling.  A grid of half a workgroup per CU or less leaves
-// most of the chip idle while each workgroup walks the whole K, one K-step per memory latency / 3:
+// Split-K factor for the 128 x 128 tiling on request (gemm.variant 1; plan_ring below is the library's own choice, and the figures
+// here are those of the kernel before that one).  A grid of half a workgroup per CU or less leaves most of the chip idle while each workgroup walks the whole K, one K-step per memory latency / 3:
 // share K between as many workgroups per tile as fill the chip once.  What it costs is the last
 // workgroup of a tile reading every share through one CU (about 1 us per share of a full tile),
 // so shares are 16 K-steps on average or more, or 10 while there are at most four shares of a K of 5120 elements
@@ -57,7 +57,7 @@ inline int plan_splits(bool fp4, int64_t M, int64_t N, int64_t k_steps, size_t w
 }
 
 enum GemmTiles {
-  kTiles128,                 // 128 x 128, with K shared where splits > 1
+  kTiles128,                 // small tiles, see plan_ring; on request 128 x 128 with K shared where splits > 1
   kTiles256Halves,           // 256 x 128 halves of 256 x 256 tiles
   kTiles256x192,
   kTiles256,
@@ -111,6 +111,66 @@ inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, size_t work
     }
   }
   return {kTiles128, plan_splits(fp4, M, N, ceil_div(fp4 ? K / 2 : K, (int64_t)kBK), workspace_bytes, cus, split_k)};
+}
+
+// The kernel for few tiles (mx_ring_kernels.hpp): tiles of 64 or 128 rows and columns, K shared between `splits` workgroups.
+struct RingPlan {
+  int tile_m, tile_n, splits;
+  int64_t ns;  // what the estimate below gives, in nanoseconds
+};
+
+// What a CU can have under way is what this kernel's time is made of, so the tiles and shares that a product takes
+// follow from an estimate: a step costs 2 ns per line of 128 bytes that a workgroup asks for (a CU holds some 512
+// requests, which take a microsecond from memory), or what its fragment reads and MFMAs take, and a workgroup about 3 us around
+// its steps; sharing K costs the parked sums' way through memory.  The constants are a fit to 262 problems
+// of 1 to 3712 rows, both operand types, K on and off a multiple of 128, in each of up to 25 forms, B from memory and from the
+// memory-side cache: the form that the estimate picks takes 0.4 % longer than the best one of each problem on average, 7 % at most
+// (19 % for up to 64 rows).  `ragged`: the rows are not whole lines, a step more is on its way.
+inline RingPlan plan_ring(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, size_t workspace_bytes, int cus, int split_k, int tile_m,
+                          int tile_n) {
+  const int64_t steps = ceil_div(fp4 ? K / 2 : K, (int64_t)kBK);
+  const int64_t parked = workspace_bytes > kSplitTicketBytes ? (int64_t)(workspace_bytes - kSplitTicketBytes) : 0;
+  RingPlan best{0, 0, 1, 0};
+  for (int bm = 64; bm <= 128; bm += 64) {
+    if (tile_m && bm != tile_m) continue;
+    for (int bn = 64; bn <= 128; bn += 64) {
+      if (tile_n && bn != tile_n) continue;
+      const int64_t tiles = ceil_div(M, (int64_t)bm) * ceil_div(N, (int64_t)bn);
+      const int area = bm * bn / 64;  // of 256
+      const int lines = (int)std::min<int64_t>(M, bm) + (int)std::min<int64_t>(N, bn) + 8;
+      const int step = std::max(2 * lines, 120 + 250 * area / 256), whole = 300 + 1400 * (bm + bn) / 256;
+      const auto consider = [&](int shares, int64_t ns) {
+        if (best.tile_m == 0 || ns < best.ns) best = RingPlan{bm, bn, shares, ns};
+      };
+      const int extra = ragged ? 1 : 0;
+      if (split_k <= 1 || tiles > (int64_t)(kSplitTicketBytes / 4))
+        consider(1, whole + ceil_div(tiles, (int64_t)cus) * ((steps + extra) * step + 2900));
+      if (tiles > (int64_t)(kSplitTicketBytes / 4) || split_k == 1) continue;
+      // shares of six steps or more, a CU each; as many as asked for where that is said, if the workspace holds them
+      const int t = (int)tiles, n = (int)steps, room = (int)std::min<int64_t>(parked / ((int64_t)bm * bn * 4 * t), kMaxSplits);
+      const int most = std::min(room, split_k > 0 ? std::min(split_k, n) : std::min(std::min(cus / t, n / 6), kAutoMaxSplits));
+      for (int splits = split_k > 0 ? std::max(most, 1) : 2; splits <= std::max(most, 1); ++splits) {
+        const int per = (n + splits - 1) / splits, shares = (n + per - 1) / per, groups = t * shares;
+        const int rounds = groups <= cus ? 1 : (groups + cus - 1) / cus;
+        int64_t ns = whole + (int64_t)rounds * ((int64_t)(per + extra) * step + 2900);
+        if (shares > 1) ns += 1200 + (550 * shares + 4000 * std::min(groups, cus) / cus) * area / 256;
+        consider(shares, ns);
+      }
+    }
+  }
+  return best;
+}
+
+// Does the kernel for at most 64 rows (mx_few_rows.hip) take a product in less time than `ring`?  Its workgroups walk whole rows of
+// B, 16 or 32 columns each, with all of A beside them: per round of the chip 1.8 us, and per step and column 5 ns (6 off
+// whole lines) and 2.2 ns per row of A.  The other kernel reads B at no more than 4.3 TB/s.  (Fitted to 150 problems of 1 to 64 rows:
+// what the two estimates pick takes 1.2 % longer than the better kernel at its best; what was there before, few rows for K of 2048 and
+// N of 1024 on with exceptions, took 27 % longer.)  columns: of a workgroup.
+inline bool few_rows_beats(const RingPlan& ring, bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, int cus, int columns) {
+  const int64_t k_bytes = fp4 ? K / 2 : K, steps = ceil_div(k_bytes, (int64_t)kBK), rows = ceil_div(M, (int64_t)8) * 8;
+  const int64_t rounds = ceil_div(ceil_div(N, (int64_t)columns), (int64_t)cus);
+  const int64_t few = 1300 + 1800 * rounds + rounds * steps * (10 * columns * (ragged ? 6 : 5) + 22 * rows) / 10 - 7 * rows;
+  return few < std::max(ring.ns, 3000 + N * k_bytes / 4300);
 }
 
 }  // namespace dt

@@ -1,0 +1,11 @@
+// The e4m3 instantiations of the kernel in mx_ring_kernels.hpp.
+#include "mx_ring_kernels.hpp"
+
+namespace dt {
+
+int launch_ring_e4m3(const RingArgs& p, bool ragged, int tile_m, int tile_n, int splits) {
+  if (tile_m == 64) return tile_n == 64 ? ring::launch_tile<2, 2, false>(p, ragged, splits) : ring::launch_tile<2, 4, false>(p, ragged, splits);
+  return tile_n == 64 ? ring::launch_tile<4, 2, false>(p, ragged, splits) : ring::launch_tile<4, 4, false>(p, ragged, splits);
+}
+
+}  // namespace dt
