@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "driss_torch_hip.h"
 
 namespace dt {
@@ -22,7 +24,76 @@ struct DeviceFacts {
 };
 const DeviceFacts& device_facts();  // of the current device, cached per device
 
-int tuning(const char* key);  // current value of a launch knob
+// Launch-shape knobs.  Workgroups per CU for the persistent grids, chosen on MI355X.
+//   dynamic.resident: 1 = per-tensor dynamic quantization of a tensor that fits the chip runs as one
+//                 kernel that keeps it in registers and LDS.  That kernel waits inside for all of its
+//                 workgroups and so assumes that this process has the GPU to itself: 0 unless the caller
+//                 opts in (dt_set_exclusive_gpu, or DRISS_TORCH_RESIDENT=1 in the environment when the
+//                 library is loaded); dynamic.resident_min_kib = smallest such
+//                 tensor; sizes in [resident_gap_lo_kib, resident_gap_hi_kib) take the two kernels
+//                 dynamic.resident_overflow: 1 = tensors of up to 4 x the chip's capacity keep what fits
+//                 and read only the rest twice
+//   amax.blocks_per_cu: most workgroups per CU of a reduction in workgroups of 256 or 512 threads (those of 1024 are at
+//                 most five per eight CUs whatever it says)
+//   rowwise.block_from_vecs: rows of at least this many 16-byte vectors get a workgroup each (shorter
+//                 ones a wave each)
+//   mx.dual:      1 = dt_mx_fp8_quantize_dual reads x once (0: two single casts)
+//   mx.colt_via_dual: 1 = the transposed column cast runs as the one-read kernel without its row half
+//   mx.dual_order: tile order of the one-read kernel: -1 = chosen by shape, 0 = down the rows first, 1 = along
+//                 the columns first, 2 = bands of 8 row tiles
+//   mx.colt_pipe: the transposed column cast as a grid of this many workgroups per CU that walk the tiles
+//                 with the next tile's loads in flight (0 = one workgroup per tile)
+//   mx.row_band4: 1 = row-wise MX cast with blocked scales walks 4 rows x 512 elements per wave pass
+//   gemm.variant: 0 = pick the tile by problem size, 1 = 128x128 tiles, 2 = 256x256 tiles, 3 = tiles of 64 or 128 rows
+//                 and columns as gemm.tile_m and gemm.tile_n say (0 = by the estimate), 5 = 256x192 tiles,
+//                 7 = 256x256 tiles on the main loop of the smaller ones (quadrants of the wave tile, no L2 prefetch;
+//                 the same bits), 9 = the kernel for at most 64 rows whatever the other dimensions
+//   gemm.few_rows_tiles: 16-column tiles per wave of that kernel: 0 = by the number of columns, 1, 2
+//   gemm.tail_quads: 1 = tiles left over after whole rounds of 256x256 tiles run as 128x128 quadrants
+//                 or 256x128 halves when those fit the chip at once, 0 = never, 2 = always as
+//                 quadrants, 3 = always as halves
+//   gemm.split_k: 0 = share K between workgroups when the small tiles leave CUs idle (needs the
+//                 workspace of the _ws entry points), 1 = never, n = n workgroups per tile
+#define DT_KNOBS(X) \
+  X(gemm, few_rows_tiles, 0)               \
+  X(gemm, few_rows_stagger, 1)             \
+  X(gemm, few_rows_steps, 0)               \
+  X(gemm, few_rows_per_cu, 0)              \
+  X(amax, blocks_per_cu, 1)                \
+  X(amax, stream_before_cast, 0)           \
+  X(cast, blocks_per_cu, 0)                \
+  X(cast, unroll, 0)                       \
+  X(cast, pair_blocks_per_cu, 0)           \
+  X(rowwise, block_from_vecs, 257)         \
+  X(mx, blocks_per_cu, 32)                 \
+  X(mx, col_blocks_per_cu, 32)             \
+  X(mx, dual, 1)                           \
+  X(mx, dual_order, -1)                    \
+  X(mx, colt_pipe, 2)                      \
+  X(mx, colt_via_dual, 1)                  \
+  X(mx, row_band4, 1)                      \
+  X(gemm, variant, 0)                      \
+  X(gemm, tile_m, 0)                       \
+  X(gemm, tile_n, 0)                       \
+  X(gemm, split_k, 0)                      \
+  X(gemm, tail_quads, 1)                   \
+  X(dynamic, resident, 0)                  \
+  X(dynamic, resident_min_kib, 32768)      \
+  X(dynamic, resident_gap_lo_kib, 0)       \
+  X(dynamic, resident_gap_hi_kib, 0)       \
+  X(dynamic, resident_overflow, 1)         \
+  X(dynamic, resident_spin_limit, 1 << 19)
+
+enum class Knob : int {
+#define DT_KNOB_ID(group, name, value) group##_##name,
+  DT_KNOBS(DT_KNOB_ID)
+#undef DT_KNOB_ID
+  count
+};
+// Set from any thread while launches on other threads read them.  A launch reads several: by their place in the
+// list (by name, as dt_set_tuning finds them, one cost a launch 50 to 100 ns).
+extern std::atomic<int> g_knob_values[];
+inline int tuning(Knob k) { return g_knob_values[(int)k].load(std::memory_order_relaxed); }
 
 // Per-workgroup clock readings for the benchmark's phase report exist only in a build with
 // -DDT_PHASE_LOG (a second library made for that report); in the product build kPhaseLog is false, the

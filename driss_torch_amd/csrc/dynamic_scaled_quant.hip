@@ -157,7 +157,7 @@ extern "C" int dt_set_exclusive_gpu(int on) {
   return dt_set_tuning("dynamic.resident", on ? 1 : 0);
 }
 
-extern "C" int dt_get_exclusive_gpu(void) { return dt::tuning("dynamic.resident") ? 1 : 0; }
+extern "C" int dt_get_exclusive_gpu(void) { return dt::tuning(dt::Knob::dynamic_resident) ? 1 : 0; }
 
 extern "C" uint64_t dt_dynamic_quant_resident_launches(void) {
   return dt::resident_gate().launches.load(std::memory_order_relaxed);

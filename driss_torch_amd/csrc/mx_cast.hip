@@ -29,11 +29,11 @@ int launch_mx(const MxArgs& a) {
   // x only has to be aligned to its element: the kernels load it through element-aligned vector types
   if (a.axis == 1 && !a.transpose && aligned(a.data, 8) && nblocks < (1ll << 28)) {
     const int64_t nsuper = ceil_div(nblocks, 64);
-    int64_t waves = (int64_t)cus * tuning("mx.blocks_per_cu") * (kBlock / kWave);
+    int64_t waves = (int64_t)cus * tuning(Knob::mx_blocks_per_cu) * (kBlock / kWave);
     if (waves > nsuper) waves = nsuper;
     const unsigned grid = (unsigned)ceil_div(waves, kBlock / kWave);
     if constexpr (LAYOUT == DT_SCALE_BLOCKED) {
-      if (a.rows % 128 == 0 && a.cols % 512 == 0 && tuning("mx.row_band4")) {
+      if (a.rows % 128 == 0 && a.cols % 512 == 0 && tuning(Knob::mx_row_band4)) {
         mx_row_kernel<IN, OUT, LAYOUT, true><<<grid, kBlock, 0, a.stream>>>(a.x, (uint32_t)nblocks, (uint32_t)(a.cols / 32),
                                                                            a.data, a.scale);
         return launch_status();
@@ -48,15 +48,15 @@ int launch_mx(const MxArgs& a) {
   // mx_col_t_kernel, 16384 x 4096 36.3 vs 41.0 us.  Tile order: bands of 8 row tiles where the row count
   // allows (8192 x 8192 bf16: 36.6-37.1 us against 38.0-38.6 down the rows first), else by shape.
   if (a.axis == 0 && a.transpose && a.cols % kV == 0 && aligned(a.data, 16) && aligned(a.scale, 4) &&
-      a.rows < (1ll << 31) && a.cols < (1ll << 31) && tuning("mx.colt_via_dual")) {
+      a.rows < (1ll << 31) && a.cols < (1ll << 31) && tuning(Knob::mx_colt_via_dual)) {
     constexpr int kTileCols = 32 * kV;
     const int64_t tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)kTileCols);
     if (tiles <= 0x7FFFFFFFll) {
-      const int order = tuning("mx.dual_order") >= 0 ? tuning("mx.dual_order") : (a.rows % (8 * kDualRows) == 0 ? 2 : (a.cols < a.rows ? 1 : 0));
+      const int order = tuning(Knob::mx_dual_order) >= 0 ? tuning(Knob::mx_dual_order) : (a.rows % (8 * kDualRows) == 0 ? 2 : (a.cols < a.rows ? 1 : 0));
       // A grid of mx.colt_pipe workgroups per CU that walk the tiles with the next tile's loads in flight:
       // 8192 x 8192 bf16 36.4 against 37.5 us, 4096 x 16384 37.1 against 39.2 us, fp32 and 16384 x 4096 the same
       // (with the row-wise half as well it is slower: 48.3 against 47.8 us)
-      const int64_t pipe_grid = (int64_t)tuning("mx.colt_pipe") * device_facts().cu_count;
+      const int64_t pipe_grid = (int64_t)tuning(Knob::mx_colt_pipe) * device_facts().cu_count;
       if (pipe_grid > 0 && tiles > pipe_grid)
         mx_dual_kernel<IN, OUT, LAYOUT, false, true><<<(unsigned)pipe_grid, kBlock, 0, a.stream>>>(
             a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
@@ -79,7 +79,7 @@ int launch_mx(const MxArgs& a) {
       a.rows < (1ll << 31) && a.cols < (1ll << 31) && LAYOUT == DT_SCALE_PLAIN) {
     const int64_t tiles = (a.rows / 32) * ceil_div(a.cols, (int64_t)kWave * kV);
     if (tiles <= 0x7FFFFFFFll) {
-      int64_t grid = (int64_t)cus * tuning("mx.col_blocks_per_cu");
+      int64_t grid = (int64_t)cus * tuning(Knob::mx_col_blocks_per_cu);
       if (grid > tiles) grid = tiles;
       mx_col_kernel<IN, OUT><<<(unsigned)grid, kBlock, 0, a.stream>>>(a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data,
                                                                      a.scale, (uint32_t)tiles);
@@ -144,7 +144,7 @@ int launch_dual(const DualArgs& a) {
     return kNotTaken;
   const int64_t tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)kTileCols);
   if (tiles > 0x7FFFFFFFll) return kNotTaken;
-  const int order = tuning("mx.dual_order") >= 0 ? tuning("mx.dual_order")
+  const int order = tuning(Knob::mx_dual_order) >= 0 ? tuning(Knob::mx_dual_order)
                     : a.cols > 2 * a.rows                ? 0
                     : a.rows % (8 * kDualRows) == 0      ? 2
                                                          : 1;
@@ -200,7 +200,7 @@ extern "C" int dt_mx_fp8_quantize_dual(const void* x, int in_dtype, int64_t rows
   if (!dt::aligned(x, in_dtype == DT_F32 ? 4 : 2)) return DT_ERR_MISALIGNED;
   hipStream_t s = dt::as_hip(stream);
   DualArgs a{x, rows, cols, static_cast<uint8_t*>(data_rows), scale_rows, static_cast<uint8_t*>(data_cols_t), scale_cols_t, s};
-  const bool fast_ok = dt::tuning("mx.dual") != 0;
+  const bool fast_ok = dt::tuning(dt::Knob::mx_dual) != 0;
   if (fast_ok) {
     int st;
     switch (in_dtype) {
@@ -221,11 +221,11 @@ template <int IN, int LAYOUT>
 int launch_mx_fp4(const MxArgs& a) {
   const int64_t nblocks = a.rows * a.cols / 32;
   const int64_t nsuper = ceil_div(nblocks, (int64_t)64);
-  int64_t waves = (int64_t)device_facts().cu_count * tuning("mx.blocks_per_cu") * (kBlock / kWave);
+  int64_t waves = (int64_t)device_facts().cu_count * tuning(Knob::mx_blocks_per_cu) * (kBlock / kWave);
   if (waves > nsuper) waves = nsuper;
   const unsigned grid = (unsigned)ceil_div(waves, (int64_t)(kBlock / kWave));
   if constexpr (LAYOUT == DT_SCALE_BLOCKED) {
-    if (a.rows % 128 == 0 && a.cols % 512 == 0 && tuning("mx.row_band4")) {
+    if (a.rows % 128 == 0 && a.cols % 512 == 0 && tuning(Knob::mx_row_band4)) {
       mx_row_kernel<IN, DT_E2M1, LAYOUT, true><<<grid, kBlock, 0, a.stream>>>(a.x, (uint32_t)nblocks, (uint32_t)(a.cols / 32),
                                                                              a.data, a.scale);
       return launch_status();
@@ -244,10 +244,10 @@ int launch_mx_fp4_cols(const MxArgs& a) {
   // tensors, 2048 x 4096 6.6 / 5.9)
   constexpr int kV = InTraits<IN>::kVec;
   if constexpr (IN != DT_F32) {
-    const int64_t pipe_grid = (int64_t)tuning("mx.colt_pipe") * device_facts().cu_count;
+    const int64_t pipe_grid = (int64_t)tuning(Knob::mx_colt_pipe) * device_facts().cu_count;
     const int64_t dual_tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)(32 * kV));
-    if (a.cols % kV == 0 && tuning("mx.colt_via_dual") && pipe_grid > 0 && dual_tiles > pipe_grid && dual_tiles <= 0x7FFFFFFFll) {
-      const int order = tuning("mx.dual_order") >= 0 ? tuning("mx.dual_order") : (a.rows % (8 * kDualRows) == 0 ? 2 : (a.cols < a.rows ? 1 : 0));
+    if (a.cols % kV == 0 && tuning(Knob::mx_colt_via_dual) && pipe_grid > 0 && dual_tiles > pipe_grid && dual_tiles <= 0x7FFFFFFFll) {
+      const int order = tuning(Knob::mx_dual_order) >= 0 ? tuning(Knob::mx_dual_order) : (a.rows % (8 * kDualRows) == 0 ? 2 : (a.cols < a.rows ? 1 : 0));
       mx_dual_kernel<IN, DT_E2M1, LAYOUT, false, true><<<(unsigned)pipe_grid, kBlock, 0, a.stream>>>(
           a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
       return launch_status();
@@ -304,7 +304,7 @@ int launch_dual_fp4(const DualArgs& a) {
     return kNotTaken;
   const int64_t tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)kTileCols);
   if (tiles > 0x7FFFFFFFll) return kNotTaken;
-  const int order = tuning("mx.dual_order") >= 0 ? tuning("mx.dual_order")
+  const int order = tuning(Knob::mx_dual_order) >= 0 ? tuning(Knob::mx_dual_order)
                     : a.cols > 2 * a.rows                ? 0
                     : a.rows % (8 * kDualRows) == 0      ? 2
                                                          : 1;
@@ -328,7 +328,7 @@ extern "C" int dt_mx_fp4_quantize_dual(const void* x, int in_dtype, int64_t rows
   if (!dt::aligned(x, in_dtype == DT_F32 ? 4 : 2)) return DT_ERR_MISALIGNED;
   hipStream_t s = dt::as_hip(stream);
   DualArgs a{x, rows, cols, static_cast<uint8_t*>(data_rows), scale_rows, static_cast<uint8_t*>(data_cols_t), scale_cols_t, s};
-  if (dt::tuning("mx.dual") != 0) {
+  if (dt::tuning(dt::Knob::mx_dual) != 0) {
     int st;
     switch (in_dtype) {
       case DT_F32: st = launch_dual_fp4_in<DT_F32>(a, scale_layout); break;

@@ -360,14 +360,14 @@ constexpr size_t kLdsLimit = 160 * 1024;
 // still give every CU a group (8192 x 8192, us, one tile / two: e4m3 1 row 16.2 / 15.6, 8 rows 16.8 / 15.8,
 // 16 rows 18.3 / 16.5, 56 rows 28.9 / 20.9; e2m1 1 row 10.9 / 9.4, 56 rows 16.5 / 12.2).
 int tiles_per_group(int64_t N) {
-  const int tiles = tuning("gemm.few_rows_tiles");
+  const int tiles = tuning(Knob::gemm_few_rows_tiles);
   return tiles ? (tiles == 2 ? 2 : 1) : (N >= 32 * (int64_t)device_facts().cu_count ? 2 : 1);
 }
 Plan plan_for(bool fp4, int64_t M, int64_t N) {
   Plan p;
   p.nt = tiles_per_group(N);
   const int mt = (int)((M + 15) / 16);
-  int up = tuning("gemm.few_rows_steps");
+  int up = tuning(Knob::gemm_few_rows_steps);
   if (up != 1 && up != 2) up = mt == 1 ? 2 : 1;
   if (up == 2 && (mt > 2 || few_rows_lds_bytes(fp4, mt, 2) >= kLdsLimit)) up = 1;
   p.up = up;
@@ -412,11 +412,11 @@ int launch_few_rows(bool fp4, const uint8_t* a, const uint8_t* b, const uint8_t*
   const Plan p = plan_for(fp4, M, N);
   const int mh = (int)((M + 7) / 8);  // halves of 16-row tiles that hold rows of A
   const int64_t groups = ceil_div(N, (int64_t)16 * p.nt);
-  int per_cu = tuning("gemm.few_rows_per_cu");
+  int per_cu = tuning(Knob::gemm_few_rows_per_cu);
   if (per_cu < 1) per_cu = 2;
   int64_t grid = groups;
   if (grid > (int64_t)device_facts().cu_count * per_cu) grid = (int64_t)device_facts().cu_count * per_cu;
-  const int stagger = tuning("gemm.few_rows_stagger");
+  const int stagger = tuning(Knob::gemm_few_rows_stagger);
 #define DT_FEW(FP4, MH, NT, UP) return launch_instance<FP4, MH, NT, UP>(a, b, sfa, sfb, M, N, K, lda, ldb, o, ldo, groups, grid, stagger, stream)
 #define DT_FEW_U(FP4, MH, NT)                                                      \
   do {                                                                             \

@@ -988,7 +988,7 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
   const uint8_t* A = static_cast<const uint8_t*>(a);
   const uint8_t* B = static_cast<const uint8_t*>(b);
   hipStream_t s = as_hip(stream);
-  const int variant = tuning("gemm.variant"), split_k = tuning("gemm.split_k"), cus = device_facts().cu_count;
+  const int variant = tuning(Knob::gemm_variant), split_k = tuning(Knob::gemm_split_k), cus = device_facts().cu_count;
   const size_t room = workspace ? workspace_bytes : 0;
   const bool ragged = ring_ragged(k_bytes, A, B, lda, ldb);
   const auto ring = [&](int tile_m, int tile_n, int splits) {
@@ -996,7 +996,7 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
     return FP4 ? launch_ring_e2m1(p, ragged, tile_m, tile_n, splits) : launch_ring_e4m3(p, ragged, tile_m, tile_n, splits);
   };
   const auto by_estimate = [&]() {
-    return plan_ring(FP4, M, N, K, ragged, room, cus, split_k, variant == 3 ? tuning("gemm.tile_m") : 0, variant == 3 ? tuning("gemm.tile_n") : 0);
+    return plan_ring(FP4, M, N, K, ragged, room, cus, split_k, variant == 3 ? tuning(Knob::gemm_tile_m) : 0, variant == 3 ? tuning(Knob::gemm_tile_n) : 0);
   };
   if (variant == 9 && few_rows_fits(M, K)) return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
   if (variant == 3 || (variant == 0 && few_rows_fits(M, K))) {
@@ -1005,7 +1005,7 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
       return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
     return ring(r.tile_m, r.tile_n, r.splits);
   }
-  const GemmPlan plan = plan_gemm(FP4, M, N, K, room, cus, variant, tuning("gemm.tail_quads"), split_k);
+  const GemmPlan plan = plan_gemm(FP4, M, N, K, room, cus, variant, tuning(Knob::gemm_tail_quads), split_k);
   // tiles of 256 x 256 in whole rounds of the chip, and those behind them
   const int64_t tiles256 = ceil_div(M, 256) * ceil_div(N, 256), whole = tiles256 / cus * cus, left = tiles256 - whole;
   // <tile M, tile N, waves M, waves N, LDS ring slots, e2m1 operands>

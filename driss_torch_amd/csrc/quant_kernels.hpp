@@ -202,7 +202,7 @@ __global__ __launch_bounds__(BLOCK) void amax_kernel(const void* __restrict__ x,
   }
 }
 
-inline int reduction_grid(int64_t nvec, int block, int unroll, const char* knob) {
+inline int reduction_grid(int64_t nvec, int block, int unroll, Knob knob) {
   int64_t want = ceil_div(nvec, (int64_t)block * unroll);
   int64_t cap = (int64_t)device_facts().cu_count * tuning(knob);
   if (cap > kMaxPartials) cap = kMaxPartials;
@@ -245,12 +245,12 @@ inline int launch_amax(const void* x, int64_t numel, void* ws, float* amax_out, 
   // 95 MiB 40.3 -> 38.9; both outputs 47.8 -> 46.9, at 128 MiB 61.4 -> 61.7).
   const int64_t small_blocks = ceil_div(sp.nvec, (int64_t)kBlock * kUnroll);  // of 32 KiB
   const int block = small_blocks <= 64 || small_blocks > (nscales ? 3072 : 2048) ? 256 : small_blocks <= 128 ? 512 : 1024;
-  int grid = reduction_grid(sp.nvec, block, kUnroll, "amax.blocks_per_cu");
+  int grid = reduction_grid(sp.nvec, block, kUnroll, Knob::amax_blocks_per_cu);
   if (block == 1024) grid = std::min(grid, std::max(8, device_facts().cu_count * 5 / 64 * 8));
   uint8_t* w = static_cast<uint8_t*>(ws);
   const int64_t bytes = numel * InTraits<IN>::kBytes;
   const bool nt = nscales == 0 ? bytes > kAmaxCacheableBytes || (bytes >= kAmaxStreamedFrom && bytes <= kAmaxStreamedTo)
-                               : tuning("amax.stream_before_cast") != 0;
+                               : tuning(Knob::amax_stream_before_cast) != 0;
   uint64_t* const log = phase_log((size_t)grid * 32);
 #define DT_AMAX_B(NS, NT, B) amax_kernel<IN, B, kUnroll, NS, NT><<<grid, B, 0, stream>>>(x, sp, w, amax_out, scale_out, fmax0, fmax1, log)
 #define DT_AMAX(NS, NT) do { if (block == 1024) DT_AMAX_B(NS, NT, 1024); else if (block == 512) DT_AMAX_B(NS, NT, 512); else DT_AMAX_B(NS, NT, 256); } while (0)
@@ -444,9 +444,9 @@ inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, vo
   if (fast) {
     const int64_t nvec = numel / InTraits<IN>::kVec, tail = numel % InTraits<IN>::kVec;
     const bool small = nvec * 16 < (int64_t)64 << 20;
-    const int unroll_knob = tuning("cast.unroll");
+    const int unroll_knob = tuning(Knob::cast_unroll);
     const int unroll = unroll_knob == 2 || unroll_knob == 4 ? unroll_knob : (small && !PAIR ? 2 : 4);
-    const char* const knob = PAIR ? "cast.pair_blocks_per_cu" : "cast.blocks_per_cu";
+    const Knob knob = PAIR ? Knob::cast_pair_blocks_per_cu : Knob::cast_blocks_per_cu;
     const int per_cu = tuning(knob) > 0 ? tuning(knob) : (small && !PAIR ? 3 : 1);
     int64_t grid = ceil_div(nvec, (int64_t)kBlock * unroll);
     if (grid > (int64_t)device_facts().cu_count * per_cu) grid = (int64_t)device_facts().cu_count * per_cu;

@@ -9,6 +9,7 @@
 // src/saturated_cast.cu:20, src/mx_cast.cu:238) every op runs on the current stream of the
 // input's device.
 #include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DispatchKey.h>
@@ -54,35 +55,48 @@ int out_code(at::ScalarType dtype) {  // src/saturated_cast.cu:155-164, src/dyna
   }
 }
 
+// An output on `like`'s device, contiguous.  What at::empty comes to behind its dispatch, which costs 0.25 us per tensor
+// (0.49 against 0.73): up to a fifth of a small op's time on the host, whose outputs are two to four.  at::empty itself where it would fill
+// the memory (torch.use_deterministic_algorithms).
+Tensor new_output(at::IntArrayRef size, at::ScalarType dtype, const Tensor& like) {
+  if (C10_UNLIKELY(at::globalContext().deterministicAlgorithms() && at::globalContext().deterministicFillUninitializedMemory()))
+    return at::empty(size, like.options().dtype(dtype));
+  return Tensor(at::detail::empty_cuda(size, dtype, like.device(), std::nullopt));
+}
+
+// The same with the strides of `like`, a matrix.
+Tensor new_output_like(const Tensor& like, at::ScalarType dtype) {
+  if (C10_LIKELY(like.stride(1) == 1 && like.stride(0) == like.size(1))) return new_output(like.sizes(), dtype, like);
+  return at::empty_like(like, like.options().dtype(dtype));
+}
+
+// A buffer per (device, stream) and KIND, zero-initialised when first asked for.  A thread finds the one it used last without the lock:
+// entries are never erased, and a map's nodes stay where they are.
+template <int KIND, typename Bytes>
+Tensor& kept_for(const Tensor& like, dt_stream_t stream, Bytes bytes) {
+  static std::mutex mu;
+  static auto* cache = new std::map<std::pair<int, void*>, Tensor>();
+  thread_local std::pair<std::pair<int, void*>, Tensor*> last{{-1, nullptr}, nullptr};
+  const auto key = std::make_pair((int)like.get_device(), (void*)stream);
+  if (last.second && last.first == key) return *last.second;
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = cache->find(key);
+  if (it == cache->end()) it = cache->emplace(key, at::zeros({bytes()}, like.options().dtype(at::kByte))).first;
+  last = {key, &it->second};
+  return it->second;
+}
+
 // One reduction workspace per (device, stream), zero-initialised once and then re-armed by
 // the kernels themselves.  Leaked on purpose: tensors must not be destroyed after the HIP
 // runtime has shut down.
 Tensor& workspace_for(const Tensor& like, dt_stream_t stream) {
-  static std::mutex mu;
-  static auto* cache = new std::map<std::pair<int, void*>, Tensor>();
-  std::lock_guard<std::mutex> lock(mu);
-  auto key = std::make_pair((int)like.get_device(), (void*)stream);
-  auto it = cache->find(key);
-  if (it == cache->end()) {
-    Tensor ws = at::zeros({(int64_t)dt_workspace_bytes()}, like.options().dtype(at::kByte));
-    it = cache->emplace(key, ws).first;
-  }
-  return it->second;
+  return kept_for<0>(like, stream, [] { return (int64_t)dt_workspace_bytes(); });
 }
 
 // The same for the GEMM's split-K workspace (ticket counters that the kernel leaves zero, and
 // parked accumulators).
 Tensor& gemm_workspace_for(const Tensor& like, dt_stream_t stream) {
-  static std::mutex mu;
-  static auto* cache = new std::map<std::pair<int, void*>, Tensor>();
-  std::lock_guard<std::mutex> lock(mu);
-  auto key = std::make_pair((int)like.get_device(), (void*)stream);
-  auto it = cache->find(key);
-  if (it == cache->end()) {
-    Tensor ws = at::zeros({(int64_t)dt_mx_gemm_workspace_bytes()}, like.options().dtype(at::kByte));
-    it = cache->emplace(key, ws).first;
-  }
-  return it->second;
+  return kept_for<1>(like, stream, [] { return (int64_t)dt_mx_gemm_workspace_bytes(); });
 }
 
 void check_hp_input(const Tensor& input) {
@@ -106,7 +120,7 @@ Tensor amax(const Tensor& input) {
   TORCH_CHECK(input.numel() > 0, "amax of an empty tensor");
   Ctx ctx(input);
   Tensor x = input.is_non_overlapping_and_dense() ? input : input.contiguous();
-  Tensor out = at::empty({1}, input.options().dtype(at::kFloat));
+  Tensor out = new_output({1}, at::kFloat, input);
   Tensor& ws = workspace_for(input, ctx.stream);
   check_status(dt_amax(x.data_ptr(), in_code(x), x.numel(), out.data_ptr<float>(), ws.data_ptr(), ws.numel(), ctx.stream),
                "amax");
@@ -132,7 +146,7 @@ Tensor saturated_cast_mode(const Tensor& input, const Tensor& scale, at::ScalarT
   const bool is_transposed = strides[0] == 1 && strides[1] == input.size(0);
   const bool allowed = (is_contiguous || is_transposed) && input.storage_offset() == 0;
   Tensor x = allowed ? input : input.contiguous();
-  Tensor out = at::empty_like(x, x.options().dtype(dtype));
+  Tensor out = new_output_like(x, dtype);
   if (x.numel() == 0) return out;
   if (mode == 0) mode = scale.dim() == 0 ? DT_ROUND_BF16_SCALE_PRODUCT : DT_ROUND_F32;
   Ctx ctx(input);
@@ -157,9 +171,9 @@ std::tuple<Tensor, Tensor, Tensor> dynamic_scaled_quant_ex(const Tensor& input, 
   TORCH_CHECK(mode >= 0 && mode <= 3, "invalid product rounding mode ", mode);
   if (mode == 0) mode = DT_ROUND_BF16_SCALE_PRODUCT;
   Ctx ctx(input);
-  Tensor out = at::empty_like(input, input.options().dtype(fp8_dtype));
-  Tensor amax_t = at::empty({1}, input.options().dtype(at::kFloat));
-  Tensor scale_t = at::empty({}, input.options().dtype(at::kFloat));
+  Tensor out = new_output_like(input, fp8_dtype);
+  Tensor amax_t = new_output({1}, at::kFloat, input);
+  Tensor scale_t = new_output({}, at::kFloat, input);
   Tensor& ws = workspace_for(input, ctx.stream);
   check_status(dt_dynamic_scaled_quant(input.data_ptr(), in_code(input), input.numel(), out_code(fp8_dtype), (int)mode,
                                        out.data_ptr(), amax_t.data_ptr<float>(), scale_t.data_ptr<float>(),
@@ -180,10 +194,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> dynamic_scaled_quant_pair(const Tenso
   TORCH_CHECK(mode >= 0 && mode <= 3, "invalid product rounding mode ", mode);
   if (mode == 0) mode = DT_ROUND_BF16_SCALE_PRODUCT;
   Ctx ctx(input);
-  Tensor o4 = at::empty_like(input, input.options().dtype(at::kFloat8_e4m3fn));
-  Tensor o5 = at::empty_like(input, input.options().dtype(at::kFloat8_e5m2));
-  Tensor amax_t = at::empty({1}, input.options().dtype(at::kFloat));
-  Tensor scale_t = at::empty({2}, input.options().dtype(at::kFloat));
+  Tensor o4 = new_output_like(input, at::kFloat8_e4m3fn);
+  Tensor o5 = new_output_like(input, at::kFloat8_e5m2);
+  Tensor amax_t = new_output({1}, at::kFloat, input);
+  Tensor scale_t = new_output({2}, at::kFloat, input);
   Tensor& ws = workspace_for(input, ctx.stream);
   check_status(dt_dynamic_scaled_quant_pair(input.data_ptr(), in_code(input), input.numel(), (int)mode, o4.data_ptr(),
                                             o5.data_ptr(), amax_t.data_ptr<float>(), scale_t.data_ptr<float>(),
@@ -200,9 +214,9 @@ std::tuple<Tensor, Tensor, Tensor> dynamic_scaled_quant_rowwise(const Tensor& in
   TORCH_CHECK(input.size(0) == 0 || input.size(1) > 0, "rowwise amax over empty rows");
   Ctx ctx(input);
   const int64_t R = input.size(0), C = input.size(1);
-  Tensor out = at::empty_like(input, input.options().dtype(fp8_dtype));
-  Tensor amax_t = at::empty({R, 1}, input.options().dtype(at::kFloat));
-  Tensor scale_t = at::empty({R, 1}, input.options().dtype(at::kFloat));
+  Tensor out = new_output_like(input, fp8_dtype);
+  Tensor amax_t = new_output({R, 1}, at::kFloat, input);
+  Tensor scale_t = new_output({R, 1}, at::kFloat, input);
   check_status(dt_dynamic_scaled_quant_rowwise(input.data_ptr(), in_code(input), R, C, out_code(fp8_dtype), out.data_ptr(),
                                                amax_t.data_ptr<float>(), scale_t.data_ptr<float>(), ctx.stream),
                "dynamic_scaled_quant_rowwise");
@@ -233,11 +247,11 @@ std::tuple<Tensor, Tensor> mx_fp8_quantize_ex(const Tensor& input, int64_t block
   TORCH_CHECK(!blocked || (ax == 1) != transpose,
               "blocked scales need the scale matrix as [outer, inner/32]: (axis 1, no transpose) or (axis 0, transpose)");
   Ctx ctx(input);
-  Tensor data = transpose ? at::empty({n, m}, input.options().dtype(fp8_type))
-                          : at::empty({m, n}, input.options().dtype(fp8_type));
+  Tensor data = transpose ? new_output({n, m}, fp8_type, input)
+                          : new_output({m, n}, fp8_type, input);
   const int64_t total_blocks = other_dim * (blocked_dim / 32);
   const int64_t scale_elems = blocked ? dt_blocked_scale_bytes(other_dim, blocked_dim / 32) : total_blocks;
-  Tensor scale = at::empty({scale_elems}, input.options().dtype(at::kFloat8_e8m0fnu));
+  Tensor scale = new_output({scale_elems}, at::kFloat8_e8m0fnu, input);
   if (input.numel() == 0) return {data, scale};
   check_status(dt_mx_fp8_quantize(input.data_ptr(), in_code(input), m, n, ax, transpose ? 1 : 0, out_code(fp8_type),
                                   blocked ? DT_SCALE_BLOCKED : DT_SCALE_PLAIN, data.data_ptr(),
@@ -261,11 +275,9 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> mx_fp8_quantize_dual(const Tensor& in
   const int64_t m = input.size(0), n = input.size(1);
   TORCH_CHECK(m % 32 == 0 && n % 32 == 0, "Need block shape to evenly divide the input tensor for now");
   Ctx ctx(input);
-  const auto fp8 = input.options().dtype(fp8_type);
-  const auto e8 = input.options().dtype(at::kFloat8_e8m0fnu);
-  Tensor data_r = at::empty({m, n}, fp8), data_c = at::empty({n, m}, fp8);
-  Tensor scale_r = at::empty({blocked ? dt_blocked_scale_bytes(m, n / 32) : m * (n / 32)}, e8);
-  Tensor scale_c = at::empty({blocked ? dt_blocked_scale_bytes(n, m / 32) : n * (m / 32)}, e8);
+  Tensor data_r = new_output({m, n}, fp8_type, input), data_c = new_output({n, m}, fp8_type, input);
+  Tensor scale_r = new_output({blocked ? dt_blocked_scale_bytes(m, n / 32) : m * (n / 32)}, at::kFloat8_e8m0fnu, input);
+  Tensor scale_c = new_output({blocked ? dt_blocked_scale_bytes(n, m / 32) : n * (m / 32)}, at::kFloat8_e8m0fnu, input);
   if (input.numel() == 0) return {data_r, scale_r, data_c, scale_c};
   check_status(dt_mx_fp8_quantize_dual(input.data_ptr(), in_code(input), m, n, out_code(fp8_type),
                                        blocked ? DT_SCALE_BLOCKED : DT_SCALE_PLAIN, data_r.data_ptr(),
@@ -288,7 +300,7 @@ Tensor to_blocked(const Tensor& scale) {
   Tensor s = scale.contiguous();
   Ctx ctx(scale);
   const int64_t R = s.size(0), C = s.size(1);
-  Tensor out = at::empty({dt_blocked_scale_bytes(R, C)}, s.options());
+  Tensor out = new_output({dt_blocked_scale_bytes(R, C)}, s.scalar_type(), s);
   check_status(dt_to_blocked(static_cast<const uint8_t*>(s.data_ptr()), R, C, static_cast<uint8_t*>(out.data_ptr()),
                              ctx.stream),
                "to_blocked");
@@ -314,9 +326,8 @@ std::tuple<Tensor, Tensor> mx_fp4_quantize(const Tensor& input, bool blocked, in
   TORCH_CHECK(inner % 32 == 0, "Need block shape to evenly divide the input tensor for now");
   TORCH_CHECK(ax == 1 || n % 4 == 0, "The column-wise cast needs a multiple of 4 columns");
   Ctx ctx(input);
-  Tensor data = at::empty({outer, inner / 2}, input.options().dtype(at::kByte));
-  Tensor scale = at::empty({blocked ? dt_blocked_scale_bytes(outer, inner / 32) : outer * (inner / 32)},
-                           input.options().dtype(at::kFloat8_e8m0fnu));
+  Tensor data = new_output({outer, inner / 2}, at::kByte, input);
+  Tensor scale = new_output({blocked ? dt_blocked_scale_bytes(outer, inner / 32) : outer * (inner / 32)}, at::kFloat8_e8m0fnu, input);
   if (input.numel() == 0) return {data, scale};
   TORCH_CHECK(reinterpret_cast<std::uintptr_t>(input.data_ptr()) % 16 == 0, "Input tensor must be 16-byte aligned");
   check_status(dt_mx_fp4_quantize(input.data_ptr(), in_code(input), m, n, ax, blocked ? DT_SCALE_BLOCKED : DT_SCALE_PLAIN,
@@ -337,11 +348,9 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> mx_fp4_quantize_dual(const Tensor& in
   const int64_t m = input.size(0), n = input.size(1);
   TORCH_CHECK(m % 32 == 0 && n % 32 == 0, "Need block shape to evenly divide the input tensor for now");
   Ctx ctx(input);
-  const auto u8 = input.options().dtype(at::kByte);
-  const auto e8 = input.options().dtype(at::kFloat8_e8m0fnu);
-  Tensor data_r = at::empty({m, n / 2}, u8), data_c = at::empty({n, m / 2}, u8);
-  Tensor scale_r = at::empty({blocked ? dt_blocked_scale_bytes(m, n / 32) : m * (n / 32)}, e8);
-  Tensor scale_c = at::empty({blocked ? dt_blocked_scale_bytes(n, m / 32) : n * (m / 32)}, e8);
+  Tensor data_r = new_output({m, n / 2}, at::kByte, input), data_c = new_output({n, m / 2}, at::kByte, input);
+  Tensor scale_r = new_output({blocked ? dt_blocked_scale_bytes(m, n / 32) : m * (n / 32)}, at::kFloat8_e8m0fnu, input);
+  Tensor scale_c = new_output({blocked ? dt_blocked_scale_bytes(n, m / 32) : n * (m / 32)}, at::kFloat8_e8m0fnu, input);
   if (input.numel() == 0) return {data_r, scale_r, data_c, scale_c};
   TORCH_CHECK(reinterpret_cast<std::uintptr_t>(input.data_ptr()) % 16 == 0, "Input tensor must be 16-byte aligned");
   check_status(dt_mx_fp4_quantize_dual(input.data_ptr(), in_code(input), m, n, blocked ? DT_SCALE_BLOCKED : DT_SCALE_PLAIN,
@@ -379,7 +388,7 @@ Tensor mx_fp8_bf16(Tensor a, Tensor b, Tensor a_scale, Tensor b_scale) {
   TORCH_CHECK(b.stride(0) == 1, "Input tensor 'b' must be contiguous in the K dimension (column-major)");
   TORCH_CHECK(a_scale.is_contiguous() && b_scale.is_contiguous(), "scales must be contiguous");
   Ctx ctx(a);
-  Tensor out = at::empty({M, N}, a.options().dtype(at::kBFloat16));
+  Tensor out = new_output({M, N}, at::kBFloat16, a);
   if (M == 0 || N == 0) return out;
   const int64_t lda = M > 1 ? a.stride(0) : K, ldb = N > 1 ? b.stride(1) : K;
   Tensor& ws = gemm_workspace_for(a, ctx.stream);
@@ -423,7 +432,7 @@ Tensor mx_fp4_bf16(Tensor a, Tensor b, Tensor a_scale, Tensor b_scale) {
   TORCH_CHECK(b.stride(0) == 1, "Input tensor 'b' must be contiguous in the K dimension (column-major)");
   TORCH_CHECK(a_scale.is_contiguous() && b_scale.is_contiguous(), "scales must be contiguous");
   Ctx ctx(a);
-  Tensor out = at::empty({M, N}, a.options().dtype(at::kBFloat16));
+  Tensor out = new_output({M, N}, at::kBFloat16, a);
   if (M == 0 || N == 0) return out;
   const int64_t lda = M > 1 ? a.stride(0) : Kp, ldb = N > 1 ? b.stride(1) : Kp;
   Tensor& ws = gemm_workspace_for(a, ctx.stream);

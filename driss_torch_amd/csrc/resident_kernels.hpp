@@ -494,7 +494,7 @@ inline int launch_resident_impl(const void* x, int64_t numel, void* ws, void* ou
   int tail = (int)(numel % kV);
   const int64_t capacity = (int64_t)cus * kBlock * kResVecs;
   if constexpr (!OVERFLOW) {
-    if (nvec > capacity && nvec <= capacity * kResMaxOver && tuning("dynamic.resident_overflow"))
+    if (nvec > capacity && nvec <= capacity * kResMaxOver && tuning(Knob::dynamic_resident_overflow))
       return launch_resident_impl<IN, OUT, ROUND_BF16, ROUND_SCALE, PAIR, true>(x, numel, ws, out, out2, amax_out, scale_out,
                                                                                 fmax0, fmax1, stream);
   }
@@ -520,7 +520,7 @@ inline int launch_resident_impl(const void* x, int64_t numel, void* ws, void* ou
   uint8_t* w = static_cast<uint8_t*>(ws);
   uint8_t* o = static_cast<uint8_t*>(out);
   uint8_t* o2 = static_cast<uint8_t*>(out2);
-  const uint32_t spin_limit = (uint32_t)tuning("dynamic.resident_spin_limit");
+  const uint32_t spin_limit = (uint32_t)tuning(Knob::dynamic_resident_spin_limit);
   // Two grids of this kernel in flight at once (two streams) could each hold part of the chip
   // and wait for the rest for ever: resident launches of a device are chained: one that arrives
   // on another stream than the previous one first waits for that stream's tail.  A stream under graph capture cannot take such a dependency.
@@ -578,8 +578,8 @@ inline int launch_resident(const void* x, int in_dtype, int64_t numel, int out_d
     (void)dt_set_tuning("dynamic.resident", 0);
     return DT_ERR_RESIDENT_GAVE_UP;
   }
-  if (!tuning("dynamic.resident") || bytes < (int64_t)tuning("dynamic.resident_min_kib") * 1024) return kResidentNotTaken;
-  if (bytes >= (int64_t)tuning("dynamic.resident_gap_lo_kib") * 1024 && bytes < (int64_t)tuning("dynamic.resident_gap_hi_kib") * 1024)
+  if (!tuning(Knob::dynamic_resident) || bytes < (int64_t)tuning(Knob::dynamic_resident_min_kib) * 1024) return kResidentNotTaken;
+  if (bytes >= (int64_t)tuning(Knob::dynamic_resident_gap_lo_kib) * 1024 && bytes < (int64_t)tuning(Knob::dynamic_resident_gap_hi_kib) * 1024)
     return kResidentNotTaken;
 #define DT_RES(IN, OUT, RB, RS) \
   return launch_resident_impl<IN, OUT, RB, RS, PAIR>(x, numel, ws, out, out2, amax_out, scale_out, fmax0, fmax1, stream)

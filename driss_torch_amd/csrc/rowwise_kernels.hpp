@@ -266,7 +266,7 @@ inline int launch_rowwise_impl(const void* x, int64_t rows, int64_t cols, void* 
   uint8_t* o = static_cast<uint8_t*>(out);
   const bool base_ok = aligned(x, 16) && aligned(out, kStoreAlign), vec_ok = base_ok && cols % kV == 0;
   const int64_t row_vecs = cols / kV;
-  const int64_t block_from = tuning("rowwise.block_from_vecs");  // rows at least this long take a workgroup each
+  const int64_t block_from = tuning(Knob::rowwise_block_from_vecs);  // rows at least this long take a workgroup each
   const bool held = row_vecs >= 1 && row_vecs <= 64 * kBlock && rows <= 0x7FFFFFFFll;  // a workgroup can hold a row
   const bool edges_cached = rows * cols < kStreamEdgesFrom;
 #define DT_ROWB(NV, ACCESS) \

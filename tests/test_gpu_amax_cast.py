@@ -416,3 +416,25 @@ def test_rowwise_config3_full_size(d, in_dtype):
     # and the eager formulation on the device
     eq, eamax, escale = eager.dynamic_scaled_quant_rowwise(ag, torch.float8_e4m3fn)
     assert torch.equal(util.codes(out), util.codes(eq)) and torch.equal(scale, escale)
+
+
+@pytest.mark.parametrize("deterministic", [False, True])
+def test_outputs_have_the_strides_that_empty_like_gives(d, deterministic):
+    """matrices with one row or column and free strides there, column-major ones, and the mode in which torch fills new
+    memory: shape, strides and values of every output that follows its input's layout"""
+    wide = util.normal((3, 24, 64), 71).cuda()
+    scale = torch.tensor(1.5, device="cuda")
+    torch.use_deterministic_algorithms(deterministic)
+    try:
+        for x in (wide[0, :1], wide[:, 2][:1], wide[0, :, :1].t(), wide[1].contiguous(), wide[2].t().contiguous().t()):
+            flat = x.contiguous()
+            for got, want in ((d.saturated_cast(x, scale, torch.float8_e4m3fn), d.saturated_cast(flat.clone(), scale, torch.float8_e4m3fn)),
+                              *([(d.dynamic_scaled_quant(x, torch.float8_e5m2), d.dynamic_scaled_quant(flat.clone(), torch.float8_e5m2)),
+                                 (d.dynamic_scaled_quant_rowwise(x, torch.float8_e4m3fn)[0],
+                                  d.dynamic_scaled_quant_rowwise(flat.clone(), torch.float8_e4m3fn)[0])] if x.is_contiguous() else [])):
+                as_is = x.is_contiguous() or (x.stride(0) == 1 and x.stride(1) == x.shape[0] and x.storage_offset() == 0)
+                like = x if as_is else flat
+                assert got.stride() == torch.empty_like(like, dtype=got.dtype).stride() and got.shape == x.shape
+                assert torch.equal(util.codes(got), util.codes(want))
+    finally:
+        torch.use_deterministic_algorithms(False)
