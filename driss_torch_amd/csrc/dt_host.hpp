@@ -40,7 +40,8 @@ const DeviceFacts& device_facts();  // of the current device, cached per device
 //   mx.dual:      1 = dt_mx_fp8_quantize_dual reads x once (0: two single casts)
 //   mx.colt_via_dual: 1 = the transposed column cast runs as the one-read kernel without its row half
 //   mx.dual_order: tile order of the one-read kernel: -1 = chosen by shape, 0 = down the rows first, 1 = along
-//                 the columns first, 2 = bands of 8 row tiles
+//                 the columns first, 2 = bands of 8 row tiles (by shape only without the row-wise half)
+//   mx.dual_narrow: its tiles of 16-bit matrices: -1 = chosen by shape, 0 = 256 columns, 1 = 128
 //   mx.colt_pipe: the transposed column cast as a grid of this many workgroups per CU that walk the tiles
 //                 with the next tile's loads in flight (0 = one workgroup per tile)
 //   mx.row_band4: 1 = row-wise MX cast with blocked scales walks 4 rows x 512 elements per wave pass
@@ -69,6 +70,7 @@ const DeviceFacts& device_facts();  // of the current device, cached per device
   X(mx, col_blocks_per_cu, 32)             \
   X(mx, dual, 1)                           \
   X(mx, dual_order, -1)                    \
+  X(mx, dual_narrow, -1)                   \
   X(mx, colt_pipe, 2)                      \
   X(mx, colt_via_dual, 1)                  \
   X(mx, row_band4, 1)                      \

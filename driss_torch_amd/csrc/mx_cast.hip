@@ -134,23 +134,43 @@ struct DualArgs {
   hipStream_t stream;
 };
 
-// DT_OK when the one-read kernel was launched, kNotTaken when the shape or an alignment rules it out
 constexpr int kNotTaken = -1;
+
+// The one-read kernel on `tiles` of 128 rows x 256 (fp32: 128) columns, or, for 16-bit inputs, on tiles half as wide: where the tiles
+// are few the narrow ones halve what each lane does and fill the chip (us, wide -> narrow, MXFP8 / MXFP4, bf16: 512 x 512 5.8 -> 4.3 /
+// 5.3 -> 4.0, 1024 x 1664 7.2 -> 5.4 / 6.6 -> 5.1, 2048 x 1888 8.3 -> 7.0 / 7.7 -> 6.6, 2752 x 4096, 352 tiles, 11.7 -> 11.0 / 10.3 -> 9.6), and
+// where an MXFP8 pair's are four per CU or more and the rows begin on cache lines (8192 x 4096 29.3 -> 27.6, 8192 x 8192 50.7 -> 46.6, 14336 x 4096
+// 45.6 -> 42.0, 6240 x 11968 58.6 -> 56.2).  In between, for MXFP4 and for rows off the lines the wide ones win (4096 x 3488, 448 tiles, 14.1
+// and 16.5; 6144 x 4096, 768 tiles, 21.5 and 22.3; 8960 x 7520 56.0 and 59.7; MXFP4 8192 x 4096 22.4 and 23.5).
 template <int IN, int OUT, int LAYOUT>
-int launch_dual(const DualArgs& a) {
-  constexpr int kTileCols = 32 * InTraits<IN>::kVec;
-  if (!aligned(a.data_r, 8) || !aligned(a.data_c, 16) || !aligned(a.scale_r, 4) ||
-      !aligned(a.scale_c, 4) || a.rows >= (1ll << 31) || a.cols >= (1ll << 31))
-    return kNotTaken;
-  const int64_t tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)kTileCols);
+int launch_dual_tiles(const DualArgs& a) {
+  const int64_t bands = ceil_div(a.rows, (int64_t)kDualRows), tiles = bands * ceil_div(a.cols, (int64_t)32 * InTraits<IN>::kVec);
+  // Tile order: along the columns first, down the rows first for matrices four times as wide as tall (narrow tiles, 4096 x 14336 43.6 and
+  // 44.7 us, 2976 x 11968 32.0 and 30.8; wide ones, 8192 x 14336 93.7 and 98.1).
+  const int order = tuning(Knob::mx_dual_order) >= 0 ? tuning(Knob::mx_dual_order) : a.cols > 4 * a.rows ? 0 : 1;
+  if constexpr (IN != DT_F32) {
+    const int64_t cus = device_facts().cu_count, narrow_tiles = bands * ceil_div(a.cols, (int64_t)16 * InTraits<IN>::kVec);
+    const int knob = tuning(Knob::mx_dual_narrow);
+    const bool narrow = knob >= 0 ? knob != 0 : tiles * 8 <= cus * 11 || (OUT != DT_E2M1 && tiles >= 4 * cus && a.cols % 64 == 0);
+    if (narrow && narrow_tiles <= 0x7FFFFFFFll) {
+      mx_dual_kernel<IN, OUT, LAYOUT, true, false, 8><<<(unsigned)narrow_tiles, kBlock, 0, a.stream>>>(
+          a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data_r, a.scale_r, a.data_c, a.scale_c, order);
+      return launch_status();
+    }
+  }
   if (tiles > 0x7FFFFFFFll) return kNotTaken;
-  const int order = tuning(Knob::mx_dual_order) >= 0 ? tuning(Knob::mx_dual_order)
-                    : a.cols > 2 * a.rows                ? 0
-                    : a.rows % (8 * kDualRows) == 0      ? 2
-                                                         : 1;
   mx_dual_kernel<IN, OUT, LAYOUT><<<(unsigned)tiles, kBlock, 0, a.stream>>>(a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data_r,
                                                                            a.scale_r, a.data_c, a.scale_c, order);
   return launch_status();
+}
+
+// DT_OK when the one-read kernel was launched, kNotTaken when the shape or an alignment rules it out
+template <int IN, int OUT, int LAYOUT>
+int launch_dual(const DualArgs& a) {
+  if (!aligned(a.data_r, 8) || !aligned(a.data_c, 16) || !aligned(a.scale_r, 4) ||
+      !aligned(a.scale_c, 4) || a.rows >= (1ll << 31) || a.cols >= (1ll << 31))
+    return kNotTaken;
+  return launch_dual_tiles<IN, OUT, LAYOUT>(a);
 }
 template <int IN>
 int launch_dual_in(const DualArgs& a, int out_dtype, int layout) {
@@ -298,19 +318,10 @@ namespace {
 // both MXFP4 operands of one tensor from a single read: mx_dual_kernel with the e2m1 output code
 template <int IN, int LAYOUT>
 int launch_dual_fp4(const DualArgs& a) {
-  constexpr int kTileCols = 32 * InTraits<IN>::kVec;
   if (!aligned(a.data_r, 4) || !aligned(a.data_c, 16) || !aligned(a.scale_r, 4) || !aligned(a.scale_c, 4) ||
       a.rows >= (1ll << 31) || a.cols >= (1ll << 31))
     return kNotTaken;
-  const int64_t tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)kTileCols);
-  if (tiles > 0x7FFFFFFFll) return kNotTaken;
-  const int order = tuning(Knob::mx_dual_order) >= 0 ? tuning(Knob::mx_dual_order)
-                    : a.cols > 2 * a.rows                ? 0
-                    : a.rows % (8 * kDualRows) == 0      ? 2
-                                                         : 1;
-  mx_dual_kernel<IN, DT_E2M1, LAYOUT><<<(unsigned)tiles, kBlock, 0, a.stream>>>(a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data_r,
-                                                                               a.scale_r, a.data_c, a.scale_c, order);
-  return launch_status();
+  return launch_dual_tiles<IN, DT_E2M1, LAYOUT>(a);
 }
 template <int IN>
 int launch_dual_fp4_in(const DualArgs& a, int layout) {

@@ -570,36 +570,57 @@ __device__ __forceinline__ uint32_t other_half_max_pk16(uint32_t v) {  // v: two
   return pk_absmax16(r[0], r[1]);
 }
 
+// The same over the lanes that hold the other rows of a block of 32: two halves of a wave with 16 rows per lane, its four quarters
+// with 8.
+template <int LR>
+__device__ __forceinline__ uint32_t other_rows_max_u32(uint32_t v) {
+  if constexpr (LR == 8) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = umax(r[0], r[1]);
+  }
+  return other_half_max_u32(v);
+}
+template <int LR>
+__device__ __forceinline__ uint32_t other_rows_max_pk16(uint32_t v) {
+  if constexpr (LR == 8) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = pk_absmax16(r[0], r[1]);
+  }
+  return other_half_max_pk16(v);
+}
+
 // WITH_ROWS = false leaves out the row-wise half (data_r / scale_r unused): the transposed column
 // cast on its own.  cols then only has to be a multiple of a lane's kV columns.
+// LR: rows per lane.  8 (16-bit inputs): tiles of 128 columns, the wave's four quarters of 16 lanes hold 8 rows each; half the work per
+// lane and twice the workgroups, for matrices whose tiles of 256 columns are few (see the launch).
 // PIPE: a grid smaller than the tile count; a workgroup walks tiles blockIdx.x, blockIdx.x + gridDim.x, ...
 // and has the loads of its next tile in flight while it converts and stores the one in hand.
-template <int IN, int OUT, int LAYOUT, bool WITH_ROWS = true, bool PIPE = false>
+template <int IN, int OUT, int LAYOUT, bool WITH_ROWS = true, bool PIPE = false, int LR = 16>
 __global__ __launch_bounds__(kBlock) void mx_dual_kernel(const void* __restrict__ x, uint32_t rows, uint32_t cols,
                                                          uint8_t* __restrict__ data_r, uint8_t* __restrict__ scale_r,
                                                          uint8_t* __restrict__ data_c, uint8_t* __restrict__ scale_c, int cols_first) {
   constexpr int kV = InTraits<IN>::kVec;     // columns per lane: 8 or 4
   constexpr int kB = InTraits<IN>::kBytes;
-  constexpr int kTileCols = 32 * kV;         // 256 or 128
+  constexpr int kLanes = 2 * LR;             // of a wave, side by side along a row
+  constexpr int kTileCols = kLanes * kV;     // 256 or 128
   constexpr int kRowBlocks = kTileCols / 32; // row-direction blocks per tile row: 8 or 4
+  static_assert((LR == 16 || LR == 8) && kRowBlocks % 4 == 0, "a row's scale bytes of a tile are whole words");
   constexpr int LPB = 32 / kV;               // lanes per row-direction block: 4 or 8
   __shared__ __attribute__((aligned(16))) uint8_t tile[kTileCols * kDualPitch];
   __shared__ __attribute__((aligned(16))) uint32_t ctile[kTileCols];            // [column] -> 4 bytes, one per wave
   __shared__ __attribute__((aligned(16))) uint8_t rtile[kRowBlocks * kDualRows];  // [block][row]
-  const int tid = threadIdx.x, lane = tid % kWave, w = tid / kWave, h = lane >> 5, c8 = lane & 31;
+  const int tid = threadIdx.x, lane = tid % kWave, w = tid / kWave, h = lane / kLanes, c8 = lane % kLanes;
 
   // Tile order.  Along the columns first keeps neighbouring workgroups on the same rows of the
   // input and of the row-wise payload; down the rows first (in runs of 8 tiles per XCD, as in
   // mx_col_t_kernel) keeps them on the same rows of the transposed payload.  Measured, the first
-  // is faster unless the matrix is much wider than tall (16384 x 4096 bf16: 50 vs 57 us; 4096 x
-  // 16384: 53 vs 52 us; without the row-wise half the second wins from square on), so the host
-  // picks by shape (cols_first: 1 = the first, 0 = the second, 2 = the banded order below, which is
-  // 1-2 % ahead of the first where the row count is a multiple of 8 tiles: 8192 x 8192 bf16 46.8
-  // against 47.2-47.8 us, fp32 67.1 against 67.7 us).
+  // is faster unless the matrix is much wider than tall (without the row-wise half the second wins from
+  // square on), so the host picks by shape (cols_first: 1 = the first, 0 = the second, 2 = the banded order below,
+  // for the column half alone where the row count is a multiple of 8 tiles).
   const uint32_t row_tiles = (rows + kDualRows - 1) / kDualRows;
   const uint32_t col_tiles = (cols + kTileCols - 1) / kTileCols;
   const uint32_t ntiles = row_tiles * col_tiles;
-  const uint32_t lrow0 = w * 32 + h * 16;                      // first of this lane's 16 rows inside the tile
+  const uint32_t lrow0 = w * 32 + h * LR;                      // first of this lane's rows inside the tile
   auto locate = [&](uint32_t t, uint32_t& tr, uint32_t& tc) {
     if (cols_first == 1) {
       tr = t / col_tiles;
@@ -623,22 +644,23 @@ __global__ __launch_bounds__(kBlock) void mx_dual_kernel(const void* __restrict_
       tr = t - tc * row_tiles;
     }
   };
-  auto load_tile = [&](uint32_t t, u32x4 (&dst)[16]) {
+  auto load_tile = [&](uint32_t t, u32x4 (&dst)[LR]) {
     uint32_t ltr, ltc;
     locate(t, ltr, ltc);
     const uint32_t lr0 = ltr * kDualRows + lrow0, lc0 = ltc * kTileCols + c8 * kV;
     if (t < ntiles && lr0 < rows && lc0 < cols) {
       const uint8_t* p = static_cast<const uint8_t*>(x) + ((uint64_t)lr0 * cols + lc0) * kB;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) dst[i] = ld_x16<IN>(p + (uint64_t)i * cols * kB);
+      for (int i = 0; i < LR; ++i) dst[i] = ld_x16<IN>(p + (uint64_t)i * cols * kB);
     } else {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) dst[i] = u32x4{0u, 0u, 0u, 0u};
+      for (int i = 0; i < LR; ++i) dst[i] = u32x4{0u, 0u, 0u, 0u};
     }
   };
 
   saturate_fp8_conversions();
-  u32x4 v[16], vn[PIPE ? 16 : 1];
+  u32x4 v[LR], vn[PIPE ? LR : 1];
+  static_assert(!PIPE || LR == 16, "load_tile's argument");
   if constexpr (PIPE) load_tile(blockIdx.x, vn);
   for (uint32_t tix = blockIdx.x; tix < ntiles; tix += gridDim.x) {  // tix: number of the tile in hand
   uint32_t tr, tc;
@@ -647,16 +669,16 @@ __global__ __launch_bounds__(kBlock) void mx_dual_kernel(const void* __restrict_
   const bool active = row0 < rows && col0 < cols;              // rows % 32 == 0 and cols % 32 == 0
   if constexpr (PIPE) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = vn[i];
+    for (int i = 0; i < LR; ++i) v[i] = vn[i];
     load_tile(tix + gridDim.x, vn);  // in flight under everything below
   } else {
     load_tile(tix, v);
   }
 
-  // ---- blocks down the columns: maxima over this lane's 16 rows, then over both halves
+  // ---- blocks down the columns: maxima over this lane's rows, then over the lanes that hold the block's others
   u32x4 pm = {0u, 0u, 0u, 0u};
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
+  for (int i = 0; i < LR; ++i) {
     if constexpr (IN == DT_F32) {
       pm.x = umax(pm.x, absbits_f32(v[i].x)); pm.y = umax(pm.y, absbits_f32(v[i].y));
       pm.z = umax(pm.z, absbits_f32(v[i].z)); pm.w = umax(pm.w, absbits_f32(v[i].w));
@@ -667,11 +689,11 @@ __global__ __launch_bounds__(kBlock) void mx_dual_kernel(const void* __restrict_
   }
   uint32_t cm[kV];
   if constexpr (IN == DT_F32) {
-    cm[0] = other_half_max_u32(pm.x); cm[1] = other_half_max_u32(pm.y);
-    cm[2] = other_half_max_u32(pm.z); cm[3] = other_half_max_u32(pm.w);
+    cm[0] = other_rows_max_u32<LR>(pm.x); cm[1] = other_rows_max_u32<LR>(pm.y);
+    cm[2] = other_rows_max_u32<LR>(pm.z); cm[3] = other_rows_max_u32<LR>(pm.w);
   } else {
-    pm.x = other_half_max_pk16(pm.x); pm.y = other_half_max_pk16(pm.y);
-    pm.z = other_half_max_pk16(pm.z); pm.w = other_half_max_pk16(pm.w);
+    pm.x = other_rows_max_pk16<LR>(pm.x); pm.y = other_rows_max_pk16<LR>(pm.y);
+    pm.z = other_rows_max_pk16<LR>(pm.z); pm.w = other_rows_max_pk16<LR>(pm.w);
     if constexpr (IN == DT_BF16) {
       cm[0] = pm.x << 16; cm[1] = pm.x & 0xFFFF0000u; cm[2] = pm.y << 16; cm[3] = pm.y & 0xFFFF0000u;
       cm[4] = pm.z << 16; cm[5] = pm.z & 0xFFFF0000u; cm[6] = pm.w << 16; cm[7] = pm.w & 0xFFFF0000u;
@@ -685,16 +707,16 @@ __global__ __launch_bounds__(kBlock) void mx_dual_kernel(const void* __restrict_
     const int k = IN == DT_F32 ? c : c / 2;
     return k == 0 ? v[i].x : k == 1 ? v[i].y : k == 2 ? v[i].z : v[i].w;
   };
-  const uint32_t chunk = (uint32_t)(w * 2 + h);
+  const uint32_t chunk = (uint32_t)(w * 32 + h * LR) / 16, in_chunk = (uint32_t)(h * LR) % 16;
 #pragma unroll
   for (int c = 0; c < kV; ++c) {
     const MxScale<OUT> s = mx_scale_from_absbits<OUT>(cm[c]);
     if constexpr (OUT == DT_E2M1) {
-      // two rows of x per byte: the lane's 16 rows of a column are 8 bytes, the half h of the wave's
+      // two rows of x per byte: the lane's LR rows of a column are LR / 2 bytes, part h of the wave's
       // 16-byte chunk w of that column's 64 (byte j of a word = rows 8 q + 2 j in the low nibble, + 1 in the high)
-      uint32_t r2[2];
+      uint32_t r2[LR / 8];
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
+      for (int q = 0; q < LR / 8; ++q) {
         uint32_t r = 0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -705,13 +727,15 @@ __global__ __launch_bounds__(kBlock) void mx_dual_kernel(const void* __restrict_
         r2[q] = s.nan ? 0x77777777u : r;
       }
       const uint32_t col = (uint32_t)(c8 * kV + c);
-      *reinterpret_cast<u32x2*>(tile + col * kDualPitch4 + ((((uint32_t)w) ^ ((col >> 4) & 3u)) << 4) + h * 8) = u32x2{r2[0], r2[1]};
+      uint8_t* const at = tile + col * kDualPitch4 + ((((uint32_t)w) ^ ((col >> 4) & 3u)) << 4) + h * (LR / 2);
+      if constexpr (LR == 16) *reinterpret_cast<u32x2*>(at) = u32x2{r2[0], r2[1]};
+      else *reinterpret_cast<uint32_t*>(at) = r2[0];
       if (h == 0) reinterpret_cast<uint8_t*>(ctile)[col * 4 + w] = (uint8_t)(active ? s.byte : 0u);
       continue;
     }
-    uint32_t r[4];
+    uint32_t r[LR / 4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < LR / 4; ++q) {
       if constexpr (IN == DT_F32)
         r[q] = cvt_scaled_4x32<OUT>(word(4 * q, c), word(4 * q + 1, c), word(4 * q + 2, c), word(4 * q + 3, c), s.scale);
       else
@@ -720,15 +744,17 @@ __global__ __launch_bounds__(kBlock) void mx_dual_kernel(const void* __restrict_
       if (s.nan) r[q] = 0x7F7F7F7Fu;
     }
     const uint32_t col = (uint32_t)(c8 * kV + c);
-    *reinterpret_cast<u32x4*>(tile + col * kDualPitch + ((chunk ^ ((col >> 4) & 7u)) << 4)) = u32x4{r[0], r[1], r[2], r[3]};
+    uint8_t* const at = tile + col * kDualPitch + ((chunk ^ ((col >> 4) & 7u)) << 4) + in_chunk;
+    if constexpr (LR == 16) *reinterpret_cast<u32x4*>(at) = u32x4{r[0], r[1], r[2], r[3]};
+    else *reinterpret_cast<u32x2*>(at) = u32x2{r[0], r[1]};
     if (h == 0) reinterpret_cast<uint8_t*>(ctile)[col * 4 + w] = (uint8_t)(active ? s.byte : 0u);
   }
 
   // ---- blocks along the rows: straight to memory
-  uint32_t rb[4] = {0u, 0u, 0u, 0u};  // this lane's 16 row-scale bytes, rows in byte order
+  uint32_t rb[LR / 4] = {};  // this lane's row-scale bytes, rows in byte order
   uint8_t* drow = data_r + (uint64_t)row0 * cols + col0;
 #pragma unroll
-  for (int i = 0; i < (WITH_ROWS ? 16 : 0); ++i) {
+  for (int i = 0; i < (WITH_ROWS ? LR : 0); ++i) {
     uint32_t m = quad_umax(vec_absmax_bits<IN>(v[i]));
     if constexpr (LPB == 8) m = umax(m, dpp<kDppRowHalfMirror>(m));
     const MxScale<OUT> s = mx_scale_from_absbits<OUT>(m);
@@ -757,7 +783,11 @@ __global__ __launch_bounds__(kBlock) void mx_dual_kernel(const void* __restrict_
     }
   }
   if (WITH_ROWS && (c8 % LPB) == 0)  // inactive lanes hold zero bytes: what the padding of the blocked layout must be
-    *reinterpret_cast<u32x4*>(rtile + (c8 / LPB) * kDualRows + lrow0) = u32x4{rb[0], rb[1], rb[2], rb[3]};
+  {
+    uint8_t* const at = rtile + (c8 / LPB) * kDualRows + lrow0;
+    if constexpr (LR == 16) *reinterpret_cast<u32x4*>(at) = u32x4{rb[0], rb[1], rb[2], rb[3]};
+    else *reinterpret_cast<u32x2*>(at) = u32x2{rb[0], rb[1]};
+  }
   __syncthreads();
 
   // ---- transposed payload: kTileCols output rows (columns of x) x 8 chunks of 16 bytes

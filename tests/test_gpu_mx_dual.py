@@ -244,3 +244,32 @@ def test_to_blocked_of_any_width_at_any_byte(cabi, gpu_device, shape):
         part = whole[off:off + R * C].view(R, C)
         part.copy_(plain)
         assert torch.equal(cabi.to_blocked(part).cpu(), co.to_blocked(plain)), off
+
+
+@pytest.mark.parametrize("narrow", [0, 1], ids=["tiles of 256 columns", "tiles of 128"])
+@pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(32, 32), (128, 128), (96, 160), (160, 96), (128, 256), (288, 416), (1056, 128)],
+                         ids=lambda s: f"{s[0]}x{s[1]}")
+def test_dual_tile_widths(d, in_dtype, shape, narrow):
+    """both widths of the one-read kernel's tiles forced, at the edges of either, whatever the shape would pick: every
+    output against the two single casts, with a NaN, an infinite and an all-zero block"""
+    from driss_torch_amd import cabi
+
+    x = util.student_t(shape, 900 + shape[0], in_dtype)
+    x[0, 0], x[-1, -1] = float("nan"), float("inf")
+    x[:, shape[1] // 2] = 0
+    x[shape[0] // 2] = 0
+    xg = x.cuda()
+    cabi.set_tuning("mx.dual_narrow", narrow)
+    try:
+        for blocked in (False, True):
+            for out_dtype in (torch.float8_e4m3fn, torch.float8_e5m2):
+                got = d.mx_fp8_quantize_dual(xg, out_dtype, blocked)
+                want = (d.mx_fp8_quantize_blocked(xg, 1, out_dtype) + d.mx_fp8_quantize_blocked(xg, 0, out_dtype) if blocked else
+                        d.mx_fp8_quantize(xg, 32, 1, False, out_dtype) + d.mx_fp8_quantize(xg, 32, 0, True, out_dtype))
+                assert all(torch.equal(util.codes(a), util.codes(b)) for a, b in zip(got, want))
+            got = d.mx_fp4_quantize_dual(xg, blocked)
+            want = d.mx_fp4_quantize(xg, blocked, 1) + d.mx_fp4_quantize(xg, blocked, 0)
+            assert all(torch.equal(util.codes(a), util.codes(b)) for a, b in zip(got, want))
+    finally:
+        cabi.set_tuning("mx.dual_narrow", -1)
