@@ -41,7 +41,7 @@ const DeviceFacts& device_facts();  // of the current device, cached per device
 //   mx.colt_via_dual: 1 = the transposed column cast runs as the one-read kernel without its row half
 //   mx.dual_order: tile order of the one-read kernel: -1 = chosen by shape, 0 = down the rows first, 1 = along
 //                 the columns first, 2 = bands of 8 row tiles (by shape only without the row-wise half)
-//   mx.dual_narrow: its tiles of 16-bit matrices: -1 = chosen by shape, 0 = 256 columns, 1 = 128
+//   mx.dual_narrow: its tiles: -1 = chosen by shape, 0 = wide (256 columns of 16 bits, 128 of fp32), 1 = half as wide (fp32: columns alone)
 //   mx.colt_pipe: the transposed column cast as a grid of this many workgroups per CU that walk the tiles
 //                 with the next tile's loads in flight (0 = one workgroup per tile)
 //   mx.row_band4: 1 = row-wise MX cast with blocked scales walks 4 rows x 512 elements per wave pass

@@ -21,6 +21,39 @@ struct MxArgs {
   hipStream_t stream;
 };
 
+constexpr int kNotTaken = -1;
+
+// Transposed column cast: the one-read kernel without its row-wise half (16-byte loads, half-wave row split) wherever a lane's kV
+// columns are whole; 8192 x 8192 bf16 38.3 vs 40.2 us for mx_col_t_kernel, 16384 x 4096 36.3 vs 41.0 us.
+// Wide tiles, more than mx.colt_pipe per CU: a grid of that many workgroups that walk the tiles with the next tile's loads in flight
+// (8192 x 8192 bf16 36.4 against 37.5 us, 4096 x 16384 37.1 against 39.2 us; with the row-wise half as well it is slower).
+// Tile order: bands of 8 row tiles where the row count allows (8192 x 8192 bf16, wide: 36.6-37.1 us against 38.0-38.6 down the rows
+// first), else by shape; narrow tiles, more than 8 per CU: down the rows first (8192 x 8192 38.0 against 38.9, 4096 x 14336 32.4 and 34.4;
+// at 4 per CU it loses, 4096 x 4096 11.7 and 10.9).
+template <int IN, int OUT, int LAYOUT>
+int launch_dual_cols(const MxArgs& a, bool narrow) {
+  constexpr int kV = InTraits<IN>::kVec;
+  const int64_t bands = ceil_div(a.rows, (int64_t)kDualRows), tiles = bands * ceil_div(a.cols, (int64_t)(32 * kV));
+  const int64_t narrow_tiles = bands * dual_col_tiles<16 * kV, LAYOUT>((uint32_t)a.cols), cus = device_facts().cu_count;
+  const int64_t pipe_grid = (int64_t)tuning(Knob::mx_colt_pipe) * cus;
+  if (tuning(Knob::mx_dual_narrow) >= 0) narrow = tuning(Knob::mx_dual_narrow) != 0;
+  if (narrow_tiles > 0x7FFFFFFFll) narrow = false;
+  int order = tuning(Knob::mx_dual_order);
+  if (order < 0)
+    order = narrow && narrow_tiles > 8 * cus ? 0 : a.rows % (8 * kDualRows) == 0 ? 2 : a.cols < a.rows ? 1 : 0;
+  if (tiles > 0x7FFFFFFFll) return kNotTaken;
+  if (narrow)
+    mx_dual_kernel<IN, OUT, LAYOUT, false, false, 8><<<(unsigned)narrow_tiles, kBlock, 0, a.stream>>>(
+        a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
+  else if (pipe_grid > 0 && tiles > pipe_grid)
+    mx_dual_kernel<IN, OUT, LAYOUT, false, true><<<(unsigned)pipe_grid, kBlock, 0, a.stream>>>(
+        a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
+  else
+    mx_dual_kernel<IN, OUT, LAYOUT, false><<<(unsigned)tiles, kBlock, 0, a.stream>>>(
+        a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
+  return launch_status();
+}
+
 template <int IN, int OUT, int LAYOUT>
 int launch_mx(const MxArgs& a) {
   constexpr int kV = InTraits<IN>::kVec;
@@ -43,28 +76,17 @@ int launch_mx(const MxArgs& a) {
                                                                  a.data, a.scale);
     return launch_status();
   }
-  // Transposed column cast: the one-read kernel without its row-wise half (16-byte loads, half-wave
-  // row split) wherever a lane's kV columns are whole; 8192 x 8192 bf16 38.3 vs 40.2 us for
-  // mx_col_t_kernel, 16384 x 4096 36.3 vs 41.0 us.  Tile order: bands of 8 row tiles where the row count
-  // allows (8192 x 8192 bf16: 36.6-37.1 us against 38.0-38.6 down the rows first), else by shape.
   if (a.axis == 0 && a.transpose && a.cols % kV == 0 && aligned(a.data, 16) && aligned(a.scale, 4) &&
       a.rows < (1ll << 31) && a.cols < (1ll << 31) && tuning(Knob::mx_colt_via_dual)) {
-    constexpr int kTileCols = 32 * kV;
-    const int64_t tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)kTileCols);
-    if (tiles <= 0x7FFFFFFFll) {
-      const int order = tuning(Knob::mx_dual_order) >= 0 ? tuning(Knob::mx_dual_order) : (a.rows % (8 * kDualRows) == 0 ? 2 : (a.cols < a.rows ? 1 : 0));
-      // A grid of mx.colt_pipe workgroups per CU that walk the tiles with the next tile's loads in flight:
-      // 8192 x 8192 bf16 36.4 against 37.5 us, 4096 x 16384 37.1 against 39.2 us, fp32 and 16384 x 4096 the same
-      // (with the row-wise half as well it is slower: 48.3 against 47.8 us)
-      const int64_t pipe_grid = (int64_t)tuning(Knob::mx_colt_pipe) * device_facts().cu_count;
-      if (pipe_grid > 0 && tiles > pipe_grid)
-        mx_dual_kernel<IN, OUT, LAYOUT, false, true><<<(unsigned)pipe_grid, kBlock, 0, a.stream>>>(
-            a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
-      else
-        mx_dual_kernel<IN, OUT, LAYOUT, false><<<(unsigned)tiles, kBlock, 0, a.stream>>>(
-            a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
-      return launch_status();
-    }
+    // Narrow tiles fill the chip where tiles are few, and the 16-bit ones also beat the walking grid where there are many (us, wide ->
+    // narrow, bf16: 512 x 512 4.4 -> 3.4, 1024 x 1664 5.3 -> 4.3, 2048 x 1888 6.3 -> 5.5, 2752 x 4096, 352 tiles, 9.3 -> 8.8, 3584 x 8192, 896
+    // tiles, 18.9 -> 17.8, 8192 x 8192 40.8 -> 38.1, 4096 x 14336 35.2 -> 32.4; fp32: 512 x 512 3.4 -> 3.0, 2048 x 4096, 512 tiles, 9.8 -> 9.3).
+    // In between, and for more fp32 tiles, the wide ones win (bf16 4096 x 3488, 448 tiles, 10.6 and 11.3, 6144 x 4096, 768 tiles, 15.5 and
+    // 16.4; fp32 4096 x 4096 17.1 and 18.1, 8192 x 8192 58.9 and 61.6).
+    const int64_t tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)(32 * kV));
+    const bool narrow = IN == DT_F32 ? tiles <= 2 * cus : tiles * 8 <= 11 * cus || tiles * 2 >= 7 * cus;
+    const int st = launch_dual_cols<IN, OUT, LAYOUT>(a, narrow);
+    if (st != kNotTaken) return st;
   }
   if (a.axis == 0 && a.transpose && a.cols % 4 == 0 && aligned(a.data, 16) && aligned(a.scale, 4) &&
       a.rows < (1ll << 31) && a.cols < (1ll << 31)) {
@@ -133,8 +155,6 @@ struct DualArgs {
   uint8_t *data_r, *scale_r, *data_c, *scale_c;
   hipStream_t stream;
 };
-
-constexpr int kNotTaken = -1;
 
 // The one-read kernel on `tiles` of 128 rows x 256 (fp32: 128) columns, or, for 16-bit inputs, on tiles half as wide: where the tiles
 // are few the narrow ones halve what each lane does and fill the chip (us, wide -> narrow, MXFP8 / MXFP4, bf16: 512 x 512 5.8 -> 4.3 /
@@ -258,20 +278,20 @@ int launch_mx_fp4(const MxArgs& a) {
 // blocks down the columns, payload transposed: [cols, rows/2], scales [cols, rows/32]
 template <int IN, int LAYOUT>
 int launch_mx_fp4_cols(const MxArgs& a) {
-  // As for MXFP8, the one-read kernel without its row-wise half, on its grid of walking workgroups, for
-  // 16-bit inputs with more tiles than that grid (bf16, us, this / mx_col_t_kernel: 8192 x 8192 33.1 / 33.9,
-  // 16384 x 4096 30.5 / 35.5, 4096 x 16384 31.5 / 31.7; it loses for fp32, 55.4 / 51.9, and for small
-  // tensors, 2048 x 4096 6.6 / 5.9)
+  // As for MXFP8, the one-read kernel without its row-wise half: wide tiles for 16-bit inputs with more of them than the walking grid
+  // (bf16, us, this / mx_col_t_kernel: 8192 x 8192 33.1 / 33.9, 16384 x 4096 30.5 / 35.5, 4096 x 16384 31.5 / 31.7; it loses for fp32,
+  // 55.4 / 51.9, and for small tensors, 2048 x 4096 6.6 / 5.9), narrow ones where there are few, and where the payload's rows are off the
+  // cache lines (us, mx_col_t_kernel or wide -> narrow, bf16: 512 x 512 3.9 -> 3.2, 1024 x 1664 4.5 -> 4.1, 2752 x 4096 9.5 -> 8.0, 6240 x 11968
+  // 38.1 -> 36.5; fp32: 512 x 512 4.7 -> 3.1, 2048 x 4096 9.5 -> 8.6, 2752 x 4096 13.3 -> 11.3, 6240 x 11968 71.1 -> 61.6; not bf16
+  // 2048 x 1888, 128 tiles, 4.95 and 5.1, nor fp32 4096 x 4096 15.4 and 16.0)
   constexpr int kV = InTraits<IN>::kVec;
-  if constexpr (IN != DT_F32) {
-    const int64_t pipe_grid = (int64_t)tuning(Knob::mx_colt_pipe) * device_facts().cu_count;
-    const int64_t dual_tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)(32 * kV));
-    if (a.cols % kV == 0 && tuning(Knob::mx_colt_via_dual) && pipe_grid > 0 && dual_tiles > pipe_grid && dual_tiles <= 0x7FFFFFFFll) {
-      const int order = tuning(Knob::mx_dual_order) >= 0 ? tuning(Knob::mx_dual_order) : (a.rows % (8 * kDualRows) == 0 ? 2 : (a.cols < a.rows ? 1 : 0));
-      mx_dual_kernel<IN, DT_E2M1, LAYOUT, false, true><<<(unsigned)pipe_grid, kBlock, 0, a.stream>>>(
-          a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
-      return launch_status();
-    }
+  const int64_t dual_tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)(32 * kV));
+  const int64_t cus = device_facts().cu_count, pipe_grid = (int64_t)tuning(Knob::mx_colt_pipe) * cus;
+  const int knob = tuning(Knob::mx_dual_narrow);
+  const bool narrow = knob >= 0 ? knob != 0 : a.rows % 256 != 0 || (IN == DT_F32 ? dual_tiles <= 2 * cus : dual_tiles * 4 <= cus);
+  if (a.cols % kV == 0 && tuning(Knob::mx_colt_via_dual) && (narrow || (IN != DT_F32 && pipe_grid > 0 && dual_tiles > pipe_grid))) {
+    const int st = launch_dual_cols<IN, DT_E2M1, LAYOUT>(a, narrow);
+    if (st != kNotTaken) return st;
   }
   const int64_t tiles = ceil_div(a.rows, (int64_t)kColTRows) * ceil_div(a.cols, (int64_t)kColTCols);
   if (tiles > 0x7FFFFFFFll) return DT_ERR_INVALID_SHAPE;

@@ -589,10 +589,18 @@ __device__ __forceinline__ uint32_t other_rows_max_pk16(uint32_t v) {
   return other_half_max_pk16(v);
 }
 
+// Tiles of mx_dual_kernel across a matrix.  The padding of blocked column scales, to 128 columns, lies in the footprint of the
+// last tile, or, where tiles are narrower than that, in tiles of their own.
+template <int TILE_COLS, int LAYOUT>
+__host__ __device__ inline uint32_t dual_col_tiles(uint32_t cols) {
+  constexpr uint32_t kStep = LAYOUT == DT_SCALE_BLOCKED && TILE_COLS < 128 ? 128 : TILE_COLS;
+  return (cols + kStep - 1) / kStep * (kStep / TILE_COLS);
+}
+
 // WITH_ROWS = false leaves out the row-wise half (data_r / scale_r unused): the transposed column
 // cast on its own.  cols then only has to be a multiple of a lane's kV columns.
-// LR: rows per lane.  8 (16-bit inputs): tiles of 128 columns, the wave's four quarters of 16 lanes hold 8 rows each; half the work per
-// lane and twice the workgroups, for matrices whose tiles of 256 columns are few (see the launch).
+// LR: rows per lane.  8 (16-bit inputs, and fp32 without the rows): tiles half as wide, the wave's four quarters of 16 lanes hold 8 rows
+// each; half the work per lane and twice the workgroups, for matrices whose wide tiles are few, among others (see the launches).
 // PIPE: a grid smaller than the tile count; a workgroup walks tiles blockIdx.x, blockIdx.x + gridDim.x, ...
 // and has the loads of its next tile in flight while it converts and stores the one in hand.
 template <int IN, int OUT, int LAYOUT, bool WITH_ROWS = true, bool PIPE = false, int LR = 16>
@@ -602,9 +610,9 @@ __global__ __launch_bounds__(kBlock) void mx_dual_kernel(const void* __restrict_
   constexpr int kV = InTraits<IN>::kVec;     // columns per lane: 8 or 4
   constexpr int kB = InTraits<IN>::kBytes;
   constexpr int kLanes = 2 * LR;             // of a wave, side by side along a row
-  constexpr int kTileCols = kLanes * kV;     // 256 or 128
-  constexpr int kRowBlocks = kTileCols / 32; // row-direction blocks per tile row: 8 or 4
-  static_assert((LR == 16 || LR == 8) && kRowBlocks % 4 == 0, "a row's scale bytes of a tile are whole words");
+  constexpr int kTileCols = kLanes * kV;     // 256 or 128, or 64 (fp32, LR = 8)
+  constexpr int kRowBlocks = kTileCols / 32; // row-direction blocks per tile row: 8 or 4 (2)
+  static_assert((LR == 16 || LR == 8) && (kRowBlocks % 4 == 0 || !WITH_ROWS), "a row's scale bytes of a tile are whole words");
   constexpr int LPB = 32 / kV;               // lanes per row-direction block: 4 or 8
   __shared__ __attribute__((aligned(16))) uint8_t tile[kTileCols * kDualPitch];
   __shared__ __attribute__((aligned(16))) uint32_t ctile[kTileCols];            // [column] -> 4 bytes, one per wave
@@ -618,7 +626,7 @@ __global__ __launch_bounds__(kBlock) void mx_dual_kernel(const void* __restrict_
   // square on), so the host picks by shape (cols_first: 1 = the first, 0 = the second, 2 = the banded order below,
   // for the column half alone where the row count is a multiple of 8 tiles).
   const uint32_t row_tiles = (rows + kDualRows - 1) / kDualRows;
-  const uint32_t col_tiles = (cols + kTileCols - 1) / kTileCols;
+  const uint32_t col_tiles = dual_col_tiles<kTileCols, LAYOUT>(cols);
   const uint32_t ntiles = row_tiles * col_tiles;
   const uint32_t lrow0 = w * 32 + h * LR;                      // first of this lane's rows inside the tile
   auto locate = [&](uint32_t t, uint32_t& tr, uint32_t& tc) {

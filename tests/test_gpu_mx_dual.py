@@ -273,3 +273,29 @@ def test_dual_tile_widths(d, in_dtype, shape, narrow):
             assert all(torch.equal(util.codes(a), util.codes(b)) for a, b in zip(got, want))
     finally:
         cabi.set_tuning("mx.dual_narrow", -1)
+
+
+@pytest.mark.parametrize("narrow", [0, 1], ids=["wide tiles", "narrow tiles"])
+@pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape", [(32, 8), (128, 64), (160, 72), (96, 136), (288, 264), (1056, 128)], ids=lambda s: f"{s[0]}x{s[1]}")
+def test_column_cast_tile_widths(d, in_dtype, shape, narrow):
+    """the column casts with either width of tile forced, at the edges of both (columns off a whole block of scales as
+    well), against the oracle, with a NaN, an infinite and an all-zero block"""
+    from driss_torch_amd import cabi
+
+    x = util.student_t(shape, 950 + shape[0], in_dtype)
+    x[0, 0], x[-1, -1] = float("nan"), float("inf")
+    x[:, shape[1] // 2] = 0
+    xg = x.cuda()
+    x4, s4 = co.mx_fp4_quantize(x.t().contiguous())
+    cabi.set_tuning("mx.dual_narrow", narrow)
+    try:
+        for out_dtype in (E4, E5):
+            want, scale = co.mx_quantize(x, axis=0, transpose=True, out_dtype=out_dtype)
+            for got, s in ((d.mx_fp8_quantize(xg, 32, 0, True, out_dtype), scale), (d.mx_fp8_quantize_blocked(xg, 0, out_dtype), co.to_blocked(scale))):
+                assert torch.equal(util.codes(got[0]), want) and torch.equal(util.codes(got[1]).flatten(), s.flatten())
+        for blocked, s in ((False, s4), (True, co.to_blocked(s4))):
+            got = d.mx_fp4_quantize(xg, blocked, 0)
+            assert torch.equal(util.codes(got[0]), util.codes(x4)) and torch.equal(util.codes(got[1]).flatten(), s.flatten())
+    finally:
+        cabi.set_tuning("mx.dual_narrow", -1)
