@@ -1025,12 +1025,19 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
                                                                  (int)whole);
     }
     case kTiles256Halves:
+      // Rows off the cache lines cost the halves two requests a line, the small tiles one more window (us, halves -> 128 x 128, operands from
+      // the memory-side cache / from memory: e4m3 520 x 10704 x 2016 24.1 -> 21.1 / 28.4 -> 25.7, 986 x 4808 x 2464 26.5 -> 24.2 / 31.9 -> 26.3,
+      // 726 x 9072 x 9952 105.8 -> 93.1 / 106.2 -> 94.8; e2m1 1292 x 5232 x 10304 55.7 -> 51.2 / 67.6 -> 55.2, 3291 x 1528 x 6528 34.9 -> 36.1 /
+      // 41.7 -> 37.2).  Fewer steps or rows: about even, or the halves (e4m3 1384 x 3888 x 1440 19.2 and 18.4 / 18.4 and 19.1, 352 x 16224 x 4768
+      // 44.4 and 48.8 / 55.7 and 52.8, 145 x 22288 x 2528 23.1 and 24.2 / 28.8 and 30.4).
+      if (ragged && M > 384 && k_bytes > 15 * kBK) break;
       return launch_gemm<256, 128, 2, 2, 3, FP4, false, kHalves>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, tiles256, 0);
     case kTiles256QuadrantSchedule:
       return launch_gemm<256, 256, 2, 2, 2, FP4, false>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
     case kTiles128:
       break;
   }
+  // small tiles
   if (variant == 1) return ring(128, 128, plan.splits);
   const RingPlan r = by_estimate();
   return ring(r.tile_m, r.tile_n, r.splits);

@@ -588,6 +588,26 @@ def test_mx_gemm_small_tiles(d, cabi, size, tile, fp4):
             cabi.set_tuning(k, 0)
 
 
+@pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
+@pytest.mark.parametrize("rows", [384, 400])
+@pytest.mark.parametrize("steps", [15, 16, 17])
+def test_mx_gemm_rows_off_the_lines_on_halves_or_small_tiles(d, cabi, rows, steps, fp4):
+    """either side of the lines between the two, the last step a quarter full: the same K order, so the bits of the 256 x 256 tiles"""
+    K, N = ((steps - 1) * 128 + 32) * (2 if fp4 else 1), 8200
+    x, w = _wide_operand((rows, K), 7100 + steps).cuda(), _wide_operand((N, K), 7101).cuda()
+    if fp4:
+        (a, sa), (b, sb), op = d.mx_fp4_quantize(x, True), d.mx_fp4_quantize(w, True), d.mx_fp4_bf16
+    else:
+        (a, sa), (b, sb), op = d.mx_fp8_quantize_blocked(x), d.mx_fp8_quantize_blocked(w), d.mx_fp8_bf16
+    got = op(a, b.t(), sa, sb)
+    cabi.set_tuning("gemm.variant", 2)
+    try:
+        assert torch.equal(op(a, b.t(), sa, sb), got)
+    finally:
+        cabi.set_tuning("gemm.variant", 0)
+    assert torch.isfinite(got).all() and got.abs().max() > 0
+
+
 def _abs_product(op, a, b, sa, sb):
     """sum over k of |a| |b| with the signs of the codes taken off"""
     def magnitude(t):
