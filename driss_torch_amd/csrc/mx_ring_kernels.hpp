@@ -16,7 +16,7 @@
 //    four times as many CUs.
 // us, 128 x 128 tiles with K shared (what there was) -> here, e4m3 / e2m1, B from memory: 241 x 1336 x 6016 18.7 -> 10.3 / 20.5 ->
 // 9.8, 90 x 9304 x 3616 28.3 -> 16.7 / 19.4 -> 11.4, 487 x 3728 x 3872 28.8 -> 17.4 / 18.9 -> 11.8, 256 x 1728 x 1056 9.9 -> 5.7 / 8.5 ->
-// 5.3, 512 x 4096 x 4096 22.6 -> 17.5 / 14.8 -> 11.5, 128 x 128 x 16384 23.7 -> 10.1 / 19.4 -> 9.3, 200 x 14336 x 4096 26.1 -> 24.8 /
+// 5.3, 512 x 4096 x 4096 22.6 -> 16.2 / 14.8 -> 10.8, 128 x 128 x 16384 23.7 -> 10.1 / 19.4 -> 9.3, 200 x 14336 x 4096 26.1 -> 24.8 /
 // 16.4 -> 15.5 (there every CU has a tile already, 264 lines a step: 0.58 us).
 //
 // A stage of the ring is A's rows, B's rows (128 bytes each) and the scale chunks of one K-step.  Per step one barrier, behind a
@@ -151,13 +151,13 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int r = (wave * TM + i) * 8 + lrow;
-    off_a[i] = lane_offset(r, mis_a, phase_a, lda);
+    off_a[i] = lane_offset(r, mis_a, phase_a, lda) - (RAGGED ? 0u : i * 1024u);
     end_a[i] = mis_a + (uint32_t)((int64_t)r * lda) + left - 16;
   }
 #pragma unroll
   for (int i = 0; i < TN; ++i) {
     const int r = (wave * TN + i) * 8 + lrow;
-    off_b[i] = lane_offset(r, mis_b, phase_b, ldb);
+    off_b[i] = lane_offset(r, mis_b, phase_b, ldb) - (RAGGED ? 0u : i * 1024u);
     end_b[i] = mis_b + (uint32_t)((int64_t)r * ldb) + left - 16;
   }
   // Scales: 512 KC bytes of A's chunk row and of B's per step.  e4m3: waves 0, 1 bring the halves of A's chunk, 2 and 3
@@ -197,7 +197,10 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
     }
   };
   // load number n of a step into ring slot U: A's groups of 8 rows, B's, the scales.  FIRST: window 0, whose lanes in front of the row
-  // read its first chunk.
+  // read its first chunk.  Of whole lines the groups of a panel go out as a run: the instruction's immediate offset counts in memory
+  // and in LDS, lane offsets are lowered by as much (a row is 128 bytes or more, so none goes below zero), and M0, which nothing else
+  // here uses, is set once (us, set for each -> once: e2m1 128 x 128 tiles 128 x 8192 x 8192 19.95 -> 19.6, 64 x 64 tiles 12.65 -> 12.5; e4m3 the
+  // same within 1 %).
   auto load = [&](auto u_tag, auto n_tag, auto first_tag) __attribute__((always_inline)) {
     constexpr int n = decltype(n_tag)::value, U = decltype(u_tag)::value;
     constexpr bool FIRST = decltype(first_tag)::value;
@@ -218,9 +221,11 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
         }
         asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                      : : "s"(to), "v"(off), "s"(r), "n"(kTo) : "memory", "scc");
-      } else {
+      } else if constexpr (i == 0) {
         asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                      : : "s"(to), "v"(off), "s"(r), "s"(s), "n"(kTo) : "memory", "scc");
+      } else {
+        asm volatile("buffer_load_dwordx4 %0, %1, %2 offen offset:%3 lds" : : "v"(off), "s"(r), "s"(s), "n"(i * 1024) : "memory");
       }
     } else {
       constexpr int kTo = U * kStageBytes;
