@@ -121,11 +121,13 @@ struct RingPlan {
 
 // What a CU can have under way is what this kernel's time is made of, so the tiles and shares that a product takes
 // follow from an estimate: a step costs 2 ns per line of 128 bytes that a workgroup asks for (a CU holds some 512
-// requests, which take a microsecond from memory), or what its fragment reads and MFMAs take, and a workgroup about 3 us around
+// requests, which take a microsecond from memory), or what its fragment reads and MFMAs take, and a workgroup about 2 us around
 // its steps; sharing K costs the parked sums' way through memory.  The constants are a fit to 262 problems
-// of 1 to 3712 rows, both operand types, K on and off a multiple of 128, in each of up to 25 forms, B from memory and from the
-// memory-side cache: the form that the estimate picks takes 0.4 % longer than the best one of each problem on average, 7 % at most
-// (19 % for up to 64 rows).  `ragged`: the rows are not whole lines, a step more is on its way.
+// of 1 to 3712 rows, both operand types, K on and off a multiple of 128, and to 62 of 72 to 512 rows whose sizes are round, in each of up to 25
+// forms, B from memory and from the memory-side cache: the form that the estimate picks takes 0.4 % longer than the best one of each
+// problem on average (the round ones 0.8 %), 9 % at most (15 % for up to 64 rows).  A first fit, without the round ones, let shares
+// of K cost 0.55 and 4 us where this has 0.8 and 6.7, and took 2.4 % longer on those, 41 % at most: 128 x 8192 x 8192 from the
+// memory-side cache 23.9 -> 17.0 us, 384 x 1024 x 8192 15.5 -> 13.3.  `ragged`: the rows are not whole lines, a step more is on its way.
 inline RingPlan plan_ring(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, size_t workspace_bytes, int cus, int split_k, int tile_m,
                           int tile_n) {
   const int64_t steps = ceil_div(fp4 ? K / 2 : K, (int64_t)kBK);
@@ -138,13 +140,13 @@ inline RingPlan plan_ring(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged
       const int64_t tiles = ceil_div(M, (int64_t)bm) * ceil_div(N, (int64_t)bn);
       const int area = bm * bn / 64;  // of 256
       const int lines = (int)std::min<int64_t>(M, bm) + (int)std::min<int64_t>(N, bn) + 8;
-      const int step = std::max(2 * lines, 120 + 250 * area / 256), whole = 300 + 1400 * (bm + bn) / 256;
+      const int step = std::max(2 * lines, 200 + 280 * area / 256), whole = 450 + 760 * (bm + bn) / 256;
       const auto consider = [&](int shares, int64_t ns) {
         if (best.tile_m == 0 || ns < best.ns) best = RingPlan{bm, bn, shares, ns};
       };
       const int extra = ragged ? 1 : 0;
       if (split_k <= 1 || tiles > (int64_t)(kSplitTicketBytes / 4))
-        consider(1, whole + ceil_div(tiles, (int64_t)cus) * ((steps + extra) * step + 2900));
+        consider(1, whole + ceil_div(tiles, (int64_t)cus) * ((steps + extra) * step + 2200));
       if (tiles > (int64_t)(kSplitTicketBytes / 4) || split_k == 1) continue;
       // shares of six steps or more, a CU each; as many as asked for where that is said, if the workspace holds them
       const int t = (int)tiles, n = (int)steps, room = (int)std::min<int64_t>(parked / ((int64_t)bm * bn * 4 * t), kMaxSplits);
@@ -152,8 +154,8 @@ inline RingPlan plan_ring(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged
       for (int splits = split_k > 0 ? std::max(most, 1) : 2; splits <= std::max(most, 1); ++splits) {
         const int per = (n + splits - 1) / splits, shares = (n + per - 1) / per, groups = t * shares;
         const int rounds = groups <= cus ? 1 : (groups + cus - 1) / cus;
-        int64_t ns = whole + (int64_t)rounds * ((int64_t)(per + extra) * step + 2900);
-        if (shares > 1) ns += 1200 + (550 * shares + 4000 * std::min(groups, cus) / cus) * area / 256;
+        int64_t ns = whole + (int64_t)rounds * ((int64_t)(per + extra) * step + 2200);
+        if (shares > 1) ns += 1250 + (800 * shares + 6700 * std::min(groups, cus) / cus) * area / 256;
         consider(shares, ns);
       }
     }
@@ -162,15 +164,15 @@ inline RingPlan plan_ring(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged
 }
 
 // Does the kernel for at most 64 rows (mx_few_rows.hip) take a product in less time than `ring`?  Its workgroups walk whole rows of
-// B, 16 or 32 columns each, with all of A beside them: per round of the chip 1.8 us, and per step and column 5 ns (6 off
-// whole lines) and 2.2 ns per row of A.  The other kernel reads B at no more than 4.3 TB/s.  (Fitted to 150 problems of 1 to 64 rows:
-// what the two estimates pick takes 1.2 % longer than the better kernel at its best; what was there before, few rows for K of 2048 and
-// N of 1024 on with exceptions, took 27 % longer.)  columns: of a workgroup.
+// B, 16 or 32 columns each, with all of A beside them: per round of the chip 2.3 us, and per step and column 5.5 ns (6.6 off
+// whole lines) and 1.6 ns per row of A.  The other kernel reads B at no more than 4.8 TB/s.  (Fitted to 150 problems of 1 to 64 rows:
+// what the two estimates pick takes 0.4 % longer than the better kernel at its best, 11 % at most; a rule on sizes, few rows for K of
+// 2048 and N of 1024 on with exceptions, took 27 % longer.)  columns: of a workgroup.
 inline bool few_rows_beats(const RingPlan& ring, bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, int cus, int columns) {
   const int64_t k_bytes = fp4 ? K / 2 : K, steps = ceil_div(k_bytes, (int64_t)kBK), rows = ceil_div(M, (int64_t)8) * 8;
   const int64_t rounds = ceil_div(ceil_div(N, (int64_t)columns), (int64_t)cus);
-  const int64_t few = 1300 + 1800 * rounds + rounds * steps * (10 * columns * (ragged ? 6 : 5) + 22 * rows) / 10 - 7 * rows;
-  return few < std::max(ring.ns, 3000 + N * k_bytes / 4300);
+  const int64_t few = 1000 + 2260 * rounds + rounds * steps * (columns * (ragged ? 66 : 55) + 16 * rows) / 10 - 8 * rows;
+  return few < std::max(ring.ns, 3000 + N * k_bytes / 4800);
 }
 
 }  // namespace dt

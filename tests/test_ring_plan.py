@@ -57,6 +57,7 @@ def test_picks(lib):
     assert ring(lib, 200, 14336, 4096) == (128, 128, 1)  # smaller tiles would be two rounds of the chip
     assert ring(lib, 128, 14336, 4096)[2] == 1 and ring(lib, 256, 1728, 1056) == (64, 64, 1)
     assert ring(lib, 128, 128, 16384)[2] >= 8  # four tiles: K shared as widely as it goes
+    assert ring(lib, 128, 8192, 8192) == (64, 64, 1) and ring(lib, 384, 1024, 8192) == (64, 64, 2)  # parking 128 x 128 tiles costs more
     assert ring(lib, 512, 512, 16384) == (64, 64, 4) and ring(lib, 2048, 1824, 1888) == (128, 128, 1)
     few = lambda M, N, K, fp4=0: lib.few(fp4, M, N, K, (K // 2 if fp4 else K) % 128 != 0, ALL, CUS, 32 if N >= 8192 else 16)  # noqa: E731
     assert few(16, 8192, 8192) and few(1, 1928, 1984) and few(16, 4096, 4096, 1)
