@@ -84,7 +84,10 @@ int launch_mx(const MxArgs& a) {
     // In between, and for more fp32 tiles, the wide ones win (bf16 4096 x 3488, 448 tiles, 10.6 and 11.3, 6144 x 4096, 768 tiles, 15.5 and
     // 16.4; fp32 4096 x 4096 17.1 and 18.1, 8192 x 8192 58.9 and 61.6).
     const int64_t tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)(32 * kV));
-    const bool narrow = IN == DT_F32 ? tiles <= 2 * cus : tiles * 8 <= 11 * cus || tiles * 2 >= 7 * cus;
+    // Row-major scales: the many narrow ones lose where a column's scale bytes are no whole words (6240 x 11968 50.3 and 53.7) and in matrices
+    // four times as tall as wide (16384 x 4096 39.3 and 39.9; 14336 x 4096 35.9 -> 34.5).
+    const bool many = tiles * 2 >= 7 * cus && (LAYOUT == DT_SCALE_BLOCKED || (a.rows % 128 == 0 && a.rows < 4 * a.cols));
+    const bool narrow = IN == DT_F32 ? tiles <= 2 * cus : tiles * 8 <= 11 * cus || many;
     const int st = launch_dual_cols<IN, OUT, LAYOUT>(a, narrow);
     if (st != kNotTaken) return st;
   }
