@@ -16,7 +16,7 @@
 //    four times as many CUs.
 // us, 128 x 128 tiles with K shared (what there was) -> here, e4m3 / e2m1, B from memory: 241 x 1336 x 6016 18.7 -> 10.3 / 20.5 ->
 // 9.8, 90 x 9304 x 3616 28.3 -> 16.7 / 19.4 -> 11.4, 487 x 3728 x 3872 28.8 -> 17.4 / 18.9 -> 11.8, 256 x 1728 x 1056 9.9 -> 5.7 / 8.5 ->
-// 5.3, 512 x 4096 x 4096 22.6 -> 16.2 / 14.8 -> 10.8, 128 x 128 x 16384 23.7 -> 10.1 / 19.4 -> 9.3, 200 x 14336 x 4096 26.1 -> 24.8 /
+// 5.3, 512 x 4096 x 4096 22.6 -> 17.7 / 13.6 -> 10.5, 128 x 128 x 16384 23.7 -> 10.1 / 19.4 -> 9.3, 200 x 14336 x 4096 26.1 -> 24.8 /
 // 16.4 -> 15.5 (there every CU has a tile already, 264 lines a step: 0.58 us).
 //
 // A stage of the ring is A's rows, B's rows (128 bytes each) and the scale chunks of one K-step.  Per step one barrier, behind a
@@ -173,28 +173,18 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
   const uint32_t lds_s = lds_base + (sc_b ? kOffSB : kOffSA) + (FP4 ? 0 : (wave & 1) * 256);
 
   // A window past the last one is asked for with empty descriptors: nothing is read, and the counts stay what they are.
-  // Workgroups that share a panel run in step, and in step each of them waits for memory on every line.  So K is cut into runs of
-  // kStages windows, and half of the workgroups walk each pair of runs the other way round: whoever comes second to a run finds
-  // it in the XCD's L2.  (us, in order -> this, B from memory: e4m3 512 x 4096 x 4096 17.9 -> 16.2, 1024 x 8192 x 8192 83.2 -> 76.9, 1000 x
-  // 14336 x 4096 83.9 -> 77.7, 2048 x 4096 x 4096 44.0 -> 41.2, e2m1 512 x 4096 x 4096 11.5 -> 10.8; B in the memory-side cache: the same
-  // within 1 %, or up to 5 % shorter.  Runs in fours: the same from memory, 8 % slower from the cache.  Not for two rows of tiles or one,
-  // 200 x 14336 x 4096 from the cache 18.0 and 19.5, nor RAGGED, whose windows belong together.)
+  // Every workgroup walks K front to back, so that an entry is summed in the same order wherever in the matrix it stands.  (With half of
+  // the workgroups on runs of K in another order, so that one finds in the XCD's L2 what another one fetched, whole-line products of more than two
+  // rows of tiles take 6 to 13 % less from memory and the same from the memory-side cache, us, e4m3 512 x 4096 x 4096 17.7 and 16.2, 400 x 5120 x
+  // 5120 28.6 and 25.0, e2m1 300 x 4096 x 8192 17.9 and 16.5; but equal rows of A in different tiles then differ in the last bit.)
   uint32_t at = 0, at_s = 0;
-  const int paired_runs = !RAGGED && tiles_m > 2 ? k_steps / (2 * kStages) * 2 : 0, other_way = ((int)blockIdx.x + tile_m) & 1;
-  auto aim = [&](auto u_tag, int w) __attribute__((always_inline)) {
+  auto aim = [&](int w) __attribute__((always_inline)) {
     const bool in = w < k_windows;
     op_a.rsrc.z = in ? (int)op_a.bytes : 0;
     op_b.rsrc.z = in ? (int)op_b.bytes : 0;
     rsrc_s.z = in ? (int)bytes_s : 0;  // (RAGGED: the window past the last step asks for scales that nobody reads, or for none)
-    if constexpr (decltype(u_tag)::value == 0) {  // a run begins
-      int run = w / kStages;
-      if (run < paired_runs) run ^= other_way;
-      at = (uint32_t)run * (kStages * kBK);
-      at_s = (uint32_t)(ks_begin + run * kStages) * (512u * KC);
-    } else {
-      at += kBK;
-      at_s += 512u * KC;
-    }
+    at = (uint32_t)w * kBK;
+    at_s = (uint32_t)(ks_begin + w) * (512u * KC);
   };
   // load number n of a step into ring slot U: A's groups of 8 rows, B's, the scales.  FIRST: window 0, whose lanes in front of the row
   // read its first chunk.  Of whole lines the groups of a panel go out as a run: the instruction's immediate offset counts in memory
@@ -329,7 +319,7 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
 
   auto first = [&](auto u_tag) __attribute__((always_inline)) {
     constexpr int U = decltype(u_tag)::value;
-    aim(u_tag, U);
+    aim(U);
     auto one = [&](auto n_tag) __attribute__((always_inline)) { load(u_tag, n_tag, std::integral_constant<bool, U == 0>{}); };
     each(one, std::make_integer_sequence<int, kLoads>{});
   };
@@ -365,7 +355,7 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
         wait_loads_and_lds<(kStages - 1 - kAhead) * kLoads>();
         __syncthreads();
         read_scales(kNext, 1 - P);
-        aim(u_tag, ks + kStages);
+        aim(ks + kStages);
       }
       if constexpr (z > kBar) {
         constexpr int y = z - kBar - 1, kRest = kSlots - kBar - 1;  // y: 0 .. kRest - 1

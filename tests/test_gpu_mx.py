@@ -546,9 +546,8 @@ def test_mx_gemm_one_band_of_rows(d, cabi, size, fp4):
                          ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
 def test_mx_gemm_small_tiles(d, cabi, size, tile, fp4):
     """The kernel for few tiles, every tile of it forced: the same K order per entry as the 256 x 256 tiles have, so the same
-    bits (whole lines and more than two rows of tiles: some tiles walk runs of K in another order, within fp32 rounding of the sums);
-    with rows that are whole lines and with rows off them (contiguous, and as slices that begin 16 and 48 bytes into a line,
-    their neighbours poisoned); and shares of K within the same rounding."""
+    bits; with rows that are whole lines and with rows off them (contiguous, and as slices that begin 16 and 48 bytes into a line,
+    their neighbours poisoned); and shares of K within fp32 rounding of the sums."""
     M, K, N = size
     x, w = _wide_operand((M, K), 7000 + M).cuda(), _wide_operand((N, K), 7001 + N).cuda()
     if fp4:
@@ -561,14 +560,13 @@ def test_mx_gemm_small_tiles(d, cabi, size, tile, fp4):
             cabi.set_tuning(k, v)
         want = op(a, b.t(), sa, sb)
         assert torch.isfinite(want).all() and want.abs().max() > 0
-        # another order of the sum over K: an MFMA keeps 2^-22 of its largest addend, an addition of two sums 2^-24, at most 20 of each
-        # here: 2^-17 of the sum of magnitudes; then one bf16 rounding (8 significant bits: 2^-8 at most) on either side
+        # shares of K, the sum in another order: an MFMA keeps 2^-22 of its largest addend, an addition of two sums 2^-24, at most 20 of
+        # each here: 2^-17 of the sum of magnitudes; then one bf16 rounding (8 significant bits: 2^-8 at most) on either side
         bound = 2.0 ** -7 * want.float().abs() + 2.0 ** -17 * _abs_product(op, a, b, sa, sb)
         cabi.set_tuning("gemm.variant", 3)
         kb = a.shape[1]
-        got = op(a, b.t(), sa, sb)
-        assert torch.equal(got, want) if kb % 128 or M <= 2 * tile[0] else ((got.float() - want.float()).abs() <= bound).all()
-        assert torch.equal(op(a, b.t(), sa, sb), got)
+        for _ in range(2):
+            assert torch.equal(op(a, b.t(), sa, sb), want)
 
         def inside(t, lead, pitch):  # as columns of a wider matrix of NaN codes
             wide = torch.full((t.shape[0], pitch), 0x7F, dtype=torch.uint8, device="cuda")
@@ -586,6 +584,24 @@ def test_mx_gemm_small_tiles(d, cabi, size, tile, fp4):
     finally:
         for k in knobs:
             cabi.set_tuning(k, 0)
+
+
+@pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
+@pytest.mark.parametrize("size", [(512, 4096, 4096), (487, 3840, 3728), (390, 8192, 264), (300, 7168, 1024), (1000, 2080, 2048), (64, 4096, 1024)],
+                         ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
+def test_mx_gemm_equal_rows_have_equal_results(d, cabi, size, fp4):
+    """A row's result does not depend on where in `a` it stands, on any plan: with one row for all of `a`, all rows of the product are the
+    same bits, and so are all columns with one row for all of `b`."""
+    M, K, N = size
+    quantize, op = (d.mx_fp4_quantize, d.mx_fp4_bf16) if fp4 else (d.mx_fp8_quantize_blocked, d.mx_fp8_bf16)
+    quantized = lambda x: quantize(x.cuda(), blocked=True) if fp4 else quantize(x.cuda())  # noqa: E731
+    x, w = _wide_operand((M, K), 7300 + M), _wide_operand((N, K), 7301)
+    (a, sa), (b, sb) = quantized(x), quantized(w)
+    (a1, sa1), (b1, sb1) = quantized(x[:1].expand(M, K).contiguous()), quantized(w[:1].expand(N, K).contiguous())
+    got = op(a1, b.t(), sa1, sb)
+    assert got.abs().max() > 0 and torch.equal(got, got[:1].expand(M, N))
+    got = op(a, b1.t(), sa, sb1)
+    assert got.abs().max() > 0 and torch.equal(got, got[:, :1].expand(M, N))
 
 
 @pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
