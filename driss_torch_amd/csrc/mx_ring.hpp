@@ -24,4 +24,45 @@ inline bool ring_ragged(int64_t k_bytes, const uint8_t* a, const uint8_t* b, int
 int launch_ring_e4m3(const RingArgs& p, bool ragged, int tile_m, int tile_n, int splits);
 int launch_ring_e2m1(const RingArgs& p, bool ragged, int tile_m, int tile_n, int splits);
 
+// What the kernel's loads ask for.  A load goes through a buffer descriptor (base, number of bytes) with an offset per lane, an immediate
+// and a scalar one; one past the end reads nothing.  Whether the scalar offset counts there is left open here: a load past the end is past
+// it by its lane offset alone, and an empty descriptor goes with a scalar offset of zero.
+
+// A descriptor and the scalar offset into it for one window along K; nothing past the last window.
+struct RingAsk {
+  uint32_t bytes, at;
+};
+__host__ __device__ inline RingAsk ring_ask(bool in, uint32_t bytes, uint32_t at) { return in ? RingAsk{bytes, at} : RingAsk{0u, 0u}; }
+
+// The scales of a tile, `chunks` times 512 bytes: 512 bytes a K-step (e4m3; waves of even and odd number bring half of them each) or 1024.  The
+// descriptor ends with the last step of the share, or with the last chunk where K ends in the middle of that step.
+__host__ __device__ inline uint32_t ring_scale_bytes(bool fp4, int chunks, int end_step) {
+  const int end = end_step * (fp4 ? 2 : 1);
+  return (uint32_t)(end < chunks ? end : chunks) * 512u;
+}
+__host__ __device__ inline uint32_t ring_scale_offset(bool fp4, int wave, int lane, int step) {
+  return (uint32_t)step * (fp4 ? 1024u : 512u) + (fp4 ? lane * 16u : (wave & 1) * 256u + lane * 4u);
+}
+
+// A panel of up to 128 rows, from one step along K on: `left` bytes of each row.  mis: bytes from the descriptor's base, a multiple of 128, to
+// the first of them (RAGGED; whole lines: 0).
+struct RingPanel {
+  uint32_t mis;
+  int rows, left;
+  int64_t ld;
+  __host__ __device__ uint32_t bytes() const { return (uint32_t)((rows - 1) * ld + left + mis); }
+  // offset of a lane's 16 bytes of row r in window 0: lane L brings row L / 8 of a group of eight, and its chunk L % 8 turned by the row and by how
+  // far into a line it begins.  Rows past the matrix (whole lines): further than any descriptor reaches, as 255 rows span less than 4 GiB and a
+  // panel has 128.  (A select, not a branch: around four branches the compiler loads the kernel's arguments later, 0.25 us a launch.)
+  __host__ __device__ uint32_t start(bool ragged, int r, int lane) const {
+    const int lrow = lane >> 3;
+    const uint32_t phase = ragged ? (mis + (uint32_t)lrow * (uint32_t)ld) & 127u : 0u;
+    const uint32_t chunk = ((lane & 7) - lrow + (phase >> 4)) & 7u;
+    const uint32_t here = mis + (uint32_t)r * (uint32_t)ld - phase + chunk * 16u, nowhere = 0xF0000000u + chunk * 16u;
+    return !ragged && r >= rows ? nowhere : here;
+  }
+  // RAGGED: the row's last 16 bytes; a lane never asks for anything behind them (rows past the matrix: past the descriptor's end)
+  __host__ __device__ uint32_t end(int r) const { return mis + (uint32_t)r * (uint32_t)ld + left - 16; }
+};
+
 }  // namespace dt

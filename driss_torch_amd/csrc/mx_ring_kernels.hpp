@@ -11,7 +11,7 @@
 //    it from there on would be two requests; here stage w of the ring holds line w of every row (RAGGED), a step's
 //    fragments come out of stages w and w + 1, and each lane's addresses say which: a row's phase in its lines is the same for every step.
 //    (2048 x 1824 x 1888 e4m3 17.4 -> 14.2 us; 2048 x 1824 x 2048, whole lines, 14.0.)
-//  - rows past the matrix are past the end of a buffer descriptor and cost no request;
+//  - rows past the matrix are past the end of a buffer descriptor and cost no request (what each load asks for: mx_ring.hpp);
 //  - a tile is as small, and K shared as widely, as pays (plan_ring): 64 x 64 tiles ask for half of what 128 x 128 tiles do per step, on
 //    four times as many CUs.
 // us, 128 x 128 tiles with K shared (what there was) -> here, e4m3 / e2m1, B from memory: 241 x 1336 x 6016 18.7 -> 10.3 / 20.5 ->
@@ -118,73 +118,65 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
   int k_steps = k_steps_all, ks_begin = 0;
   if constexpr (SPLIT) {
     const int per = (k_steps + splits - 1) / splits;
-    ks_begin = split * per;
-    k_steps = k_steps - ks_begin < per ? k_steps - ks_begin : per;
+    // (scalars, which the compiler cannot tell of what comes out of a division)
+    ks_begin = __builtin_amdgcn_readfirstlane(split * per);
+    k_steps = __builtin_amdgcn_readfirstlane(k_steps - ks_begin < per ? k_steps - ks_begin : per);
   }
   const int tail_step = k_steps_all - 1 - ks_begin;  // RAGGED: the step whose scales are masked, from ks_begin on
   const int k_windows = k_steps + (RAGGED ? 1 : 0);
   const int left = k_bytes - ks_begin * kBK;  // bytes of a row from ks_begin on
 
   // ---- memory -> LDS
-  const int lrow = lane >> 3;
   struct Operand {
+    RingPanel panel;
     v4i rsrc;
     uint32_t bytes;
   };
   auto operand = [&](const uint8_t* first, int rows, int64_t ld) __attribute__((always_inline)) {
     const uint64_t p = reinterpret_cast<uint64_t>(first), base = RAGGED ? p & ~(uint64_t)127 : p;
-    return Operand{v4i{(int)(uint32_t)base, (int)((uint32_t)(base >> 32) & 0xFFFFu), 0, 0x00027000},
-                   (uint32_t)((int64_t)(rows - 1) * ld + left + (int64_t)(p - base))};
+    const RingPanel panel{(uint32_t)(p - base), rows, left, ld};
+    return Operand{panel, v4i{(int)(uint32_t)base, (int)((uint32_t)(base >> 32) & 0xFFFFu), 0, 0x00027000}, panel.bytes()};
   };
   Operand op_a = operand(A + (int64_t)m0 * lda + (int64_t)ks_begin * kBK, M - m0 < BM ? M - m0 : BM, lda);
   Operand op_b = operand(B + (int64_t)n0 * ldb + (int64_t)ks_begin * kBK, N - n0 < BN ? N - n0 : BN, ldb);
-  const uint32_t mis_a = RAGGED ? (uint32_t)(reinterpret_cast<uint64_t>(A + (int64_t)m0 * lda) & 127) : 0u;
-  const uint32_t mis_b = RAGGED ? (uint32_t)(reinterpret_cast<uint64_t>(B + (int64_t)n0 * ldb) & 127) : 0u;
-  // row r of a panel starts at byte mis + r ld of the descriptor, phase bytes into a line (the same for rows 8 apart)
-  const uint32_t phase_a = RAGGED ? (mis_a + (uint32_t)lrow * (uint32_t)lda) & 127u : 0u;
-  const uint32_t phase_b = RAGGED ? (mis_b + (uint32_t)lrow * (uint32_t)ldb) & 127u : 0u;
   uint32_t off_a[TM], off_b[TN], end_a[TM], end_b[TN];
-  auto lane_offset = [&](int r, uint32_t mis, uint32_t phase, int64_t ld) __attribute__((always_inline)) {
-    const uint32_t chunk = ((lane & 7) - lrow + (phase >> 4)) & 7u;
-    return mis + (uint32_t)((int64_t)r * ld) - phase + chunk * 16u;
-  };
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    const int r = (wave * TM + i) * 8 + lrow;
-    off_a[i] = lane_offset(r, mis_a, phase_a, lda) - (RAGGED ? 0u : i * 1024u);
-    end_a[i] = mis_a + (uint32_t)((int64_t)r * lda) + left - 16;
+    const int r = (wave * TM + i) * 8 + (lane >> 3);
+    off_a[i] = op_a.panel.start(RAGGED, r, lane) - (RAGGED ? 0u : i * 1024u);
+    end_a[i] = op_a.panel.end(r);
   }
 #pragma unroll
   for (int i = 0; i < TN; ++i) {
-    const int r = (wave * TN + i) * 8 + lrow;
-    off_b[i] = lane_offset(r, mis_b, phase_b, ldb) - (RAGGED ? 0u : i * 1024u);
-    end_b[i] = mis_b + (uint32_t)((int64_t)r * ldb) + left - 16;
+    const int r = (wave * TN + i) * 8 + (lane >> 3);
+    off_b[i] = op_b.panel.start(RAGGED, r, lane) - (RAGGED ? 0u : i * 1024u);
+    end_b[i] = op_b.panel.end(r);
   }
   // Scales: 512 KC bytes of A's chunk row and of B's per step.  e4m3: waves 0, 1 bring the halves of A's chunk, 2 and 3
   // those of B's (4 bytes per lane).  e2m1: even waves bring A's two chunks, odd ones B's (16 bytes per lane,
   // twice the same bytes).
   const bool sc_b = FP4 ? (wave & 1) != 0 : wave >= 2;
   const uint64_t sc_base = reinterpret_cast<uint64_t>(sc_b ? sfb + (int64_t)(n0 >> 7) * k_chunks * 512 : sfa + (int64_t)(m0 >> 7) * k_chunks * 512);
-  const uint32_t bytes_s = (uint32_t)k_chunks * 512u;
-  v4i rsrc_s = v4i{(int)(uint32_t)sc_base, (int)((uint32_t)(sc_base >> 32) & 0xFFFFu), 0, 0x00027000};
-  const uint32_t off_s = FP4 ? lane * 16u : (wave & 1) * 256u + lane * 4u;
+  const uint32_t bytes_s = ring_scale_bytes(FP4, k_chunks, ks_begin + k_steps);
+  const v4i rsrc_s = v4i{(int)(uint32_t)sc_base, (int)((uint32_t)(sc_base >> 32) & 0xFFFFu), (int)bytes_s, 0x00027000};
+  uint32_t off_s = ring_scale_offset(FP4, wave, lane, ks_begin - 1);  // a step is added for each window
   const uint32_t lds_base = (uint32_t)(uintptr_t)(lptr_t)lds;
   const uint32_t lds_a = lds_base + wave * TM * 1024, lds_b = lds_base + kOffB + wave * TN * 1024;
   const uint32_t lds_s = lds_base + (sc_b ? kOffSB : kOffSA) + (FP4 ? 0 : (wave & 1) * 256);
 
-  // A window past the last one is asked for with empty descriptors: nothing is read, and the counts stay what they are.
+  // A window past the last one is asked for with empty descriptors (its scales are past the end): nothing is read, and the counts stay what they are.
   // Every workgroup walks K front to back, so that an entry is summed in the same order wherever in the matrix it stands.  (With half of
   // the workgroups on runs of K in another order, so that one finds in the XCD's L2 what another one fetched, whole-line products of more than two
   // rows of tiles take 6 to 13 % less from memory and the same from the memory-side cache, us, e4m3 512 x 4096 x 4096 17.7 and 16.2, 400 x 5120 x
   // 5120 28.6 and 25.0, e2m1 300 x 4096 x 8192 17.9 and 16.5; but equal rows of A in different tiles then differ in the last bit.)
-  uint32_t at = 0, at_s = 0;
+  uint32_t at = 0;
   auto aim = [&](int w) __attribute__((always_inline)) {
     const bool in = w < k_windows;
-    op_a.rsrc.z = in ? (int)op_a.bytes : 0;
-    op_b.rsrc.z = in ? (int)op_b.bytes : 0;
-    rsrc_s.z = in ? (int)bytes_s : 0;  // (RAGGED: the window past the last step asks for scales that nobody reads, or for none)
-    at = (uint32_t)w * kBK;
-    at_s = (uint32_t)(ks_begin + w) * (512u * KC);
+    const RingAsk ask_a = ring_ask(in, op_a.bytes, (uint32_t)w * kBK), ask_b = ring_ask(in, op_b.bytes, (uint32_t)w * kBK);
+    op_a.rsrc.z = (int)ask_a.bytes;
+    op_b.rsrc.z = (int)ask_b.bytes;
+    at = ask_a.at;
+    off_s += 512u * KC;
   };
   // load number n of a step into ring slot U: A's groups of 8 rows, B's, the scales.  FIRST: window 0, whose lanes in front of the row
   // read its first chunk.  Of whole lines the groups of a panel go out as a run: the instruction's immediate offset counts in memory
@@ -219,14 +211,14 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
       }
     } else {
       constexpr int kTo = U * kStageBytes;
-      const uint32_t to = lds_s, off = off_s, s = at_s;
+      const uint32_t to = lds_s, off = off_s;
       const v4i r = rsrc_s;
-      if constexpr (FP4)  // the second chunk of a half-filled last step is past the descriptor's end
-        asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                     : : "s"(to), "v"(off), "s"(r), "s"(s), "n"(kTo) : "memory", "scc");
+      if constexpr (FP4)
+        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     : : "s"(to), "v"(off), "s"(r), "n"(kTo) : "memory", "scc");
       else
-        asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-                     : : "s"(to), "v"(off), "s"(r), "s"(s), "n"(kTo) : "memory", "scc");
+        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+                     : : "s"(to), "v"(off), "s"(r), "n"(kTo) : "memory", "scc");
     }
   };
 
@@ -252,8 +244,8 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
     // row l16 of a 16-row tile: group l16 / 8, row l16 % 8; its logical chunk c lies at position (c + l16) % 8, in the step's own window
     // or, c + phase past a line's end, in the next one
     const uint32_t row = (l16 >> 3) * 1024 + (l16 & 7) * 128, lo = row + (((kq + l16) & 7) << 4), hi = lo ^ 64u;
-    const uint32_t ph_a = RAGGED ? ((mis_a + (uint32_t)(l16 & 7) * (uint32_t)lda) & 127u) >> 4 : 0u;
-    const uint32_t ph_b = RAGGED ? ((mis_b + (uint32_t)(l16 & 7) * (uint32_t)ldb) & 127u) >> 4 : 0u;
+    const uint32_t ph_a = RAGGED ? ((op_a.panel.mis + (uint32_t)(l16 & 7) * (uint32_t)lda) & 127u) >> 4 : 0u;
+    const uint32_t ph_b = RAGGED ? ((op_b.panel.mis + (uint32_t)(l16 & 7) * (uint32_t)ldb) & 127u) >> 4 : 0u;
     const uint32_t a0 = wm * TM * 2048, b0 = kOffB + wn * TN * 2048;
     const int ta = ((m0 & 127) >> 4) + wm * TM, tb = ((n0 & 127) >> 4) + wn * TN;  // even: the first tile's number in its chunk
 #pragma unroll
