@@ -53,7 +53,7 @@ const DeviceFacts& device_facts();  // of the current device, cached per device
 //   gemm.tail_quads: 1 = tiles left over after whole rounds of 256x256 tiles run as 128x128 quadrants
 //                 or 256x128 halves when those fit the chip at once, 0 = never, 2 = always as
 //                 quadrants, 3 = always as halves
-//   gemm.split_k: 0 = share K between workgroups when the small tiles leave CUs idle (needs the
+//   gemm.split_k: of the small tiles, 0 = share K between workgroups when they leave CUs idle (needs the
 //                 workspace of the _ws entry points), 1 = never, n = n workgroups per tile
 #define DT_KNOBS(X) \
   X(gemm, few_rows_tiles, 0)               \

@@ -999,10 +999,14 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
     return plan_ring(FP4, M, N, K, ragged, room, cus, split_k, variant == 3 ? tuning(Knob::gemm_tile_m) : 0, variant == 3 ? tuning(Knob::gemm_tile_n) : 0);
   };
   if (variant == 9 && few_rows_fits(M, K)) return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
+  if (variant == 0 && few_rows_fits(M, K)) {
+    // how many workgroups are to share K does not decide between the two kernels; whether any may does
+    const RingPlan r = plan_ring(FP4, M, N, K, ragged, room, cus, split_k == 1 ? 1 : 0, 0, 0);
+    if (few_rows_beats(r, FP4, M, N, K, ragged, cus, few_rows_columns(N)))
+      return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
+  }
   if (variant == 3 || (variant == 0 && few_rows_fits(M, K))) {
     const RingPlan r = by_estimate();
-    if (variant == 0 && split_k == 0 && few_rows_beats(r, FP4, M, N, K, ragged, cus, few_rows_columns(N)))
-      return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
     return ring(r.tile_m, r.tile_n, r.splits);
   }
   const GemmPlan plan = plan_gemm(FP4, M, N, K, room, cus, variant, tuning(Knob::gemm_tail_quads), split_k);

@@ -348,6 +348,31 @@ def test_mx_gemm_few_rows_kernel_is_the_default_and_respects_strides(d, cabi):
         cabi.set_tuning("gemm.variant", 0)
 
 
+@pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
+@pytest.mark.parametrize("size", [(24, 2048, 8192), (16, 4096, 4096), (40, 4096, 4096)], ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
+def test_mx_gemm_split_k_leaves_the_few_rows_kernel_alone(d, cabi, size, fp4):
+    """gemm.split_k says how the small tiles share K: a product that takes the kernel for few rows takes it under any factor (the order of
+    its sums is its own, so the bits tell)"""
+    M, K, N = size
+    x, w = _wide_operand((M, K), 2700 + M).cuda(), _wide_operand((N, K), 2701).cuda()
+    if fp4:
+        (a, sa), (b, sb), op = d.mx_fp4_quantize(x, True), d.mx_fp4_quantize(w, True), d.mx_fp4_bf16
+    else:
+        (a, sa), (b, sb), op = d.mx_fp8_quantize_blocked(x), d.mx_fp8_quantize_blocked(w), d.mx_fp8_bf16
+    outs = {}
+    for variant, split_k in ((9, 0), (0, 0), (0, 1), (0, 3), (3, 1)):
+        cabi.set_tuning("gemm.variant", variant)
+        cabi.set_tuning("gemm.split_k", split_k)
+        try:
+            outs[variant, split_k] = op(a, b.t(), sa, sb)
+        finally:
+            cabi.set_tuning("gemm.variant", 0)
+            cabi.set_tuning("gemm.split_k", 0)
+    assert not torch.equal(outs[3, 1], outs[9, 0])
+    for split_k in (0, 1, 3):
+        assert torch.equal(outs[0, split_k], outs[9, 0]), split_k
+
+
 def _random_gemm_sizes(seed, n):
     import random
 
