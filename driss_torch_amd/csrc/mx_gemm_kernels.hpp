@@ -988,28 +988,11 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
   const uint8_t* A = static_cast<const uint8_t*>(a);
   const uint8_t* B = static_cast<const uint8_t*>(b);
   hipStream_t s = as_hip(stream);
-  const int variant = tuning(Knob::gemm_variant), split_k = tuning(Knob::gemm_split_k), cus = device_facts().cu_count;
-  const size_t room = workspace ? workspace_bytes : 0;
+  const int cus = device_facts().cu_count;
   const bool ragged = ring_ragged(k_bytes, A, B, lda, ldb);
-  const auto ring = [&](int tile_m, int tile_n, int splits) {
-    const RingArgs p{A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, workspace, s};
-    return FP4 ? launch_ring_e2m1(p, ragged, tile_m, tile_n, splits) : launch_ring_e4m3(p, ragged, tile_m, tile_n, splits);
-  };
-  const auto by_estimate = [&]() {
-    return plan_ring(FP4, M, N, K, ragged, room, cus, split_k, variant == 3 ? tuning(Knob::gemm_tile_m) : 0, variant == 3 ? tuning(Knob::gemm_tile_n) : 0);
-  };
-  if (variant == 9 && few_rows_fits(M, K)) return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
-  if (variant == 0 && few_rows_fits(M, K)) {
-    // how many workgroups are to share K does not decide between the two kernels; whether any may does
-    const RingPlan r = plan_ring(FP4, M, N, K, ragged, room, cus, split_k == 1 ? 1 : 0, 0, 0);
-    if (few_rows_beats(r, FP4, M, N, K, ragged, cus, few_rows_columns(N)))
-      return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
-  }
-  if (variant == 3 || (variant == 0 && few_rows_fits(M, K))) {
-    const RingPlan r = by_estimate();
-    return ring(r.tile_m, r.tile_n, r.splits);
-  }
-  const GemmPlan plan = plan_gemm(FP4, M, N, K, room, cus, variant, tuning(Knob::gemm_tail_quads), split_k);
+  const GemmPlan plan = plan_gemm(FP4, M, N, K, ragged, workspace ? workspace_bytes : 0, cus, few_rows_fits(M, K) ? few_rows_columns(N) : 0,
+                                  {tuning(Knob::gemm_variant), tuning(Knob::gemm_tail_quads), tuning(Knob::gemm_split_k),
+                                   tuning(Knob::gemm_tile_m), tuning(Knob::gemm_tile_n)});
   // tiles of 256 x 256 in whole rounds of the chip, and those behind them
   const int64_t tiles256 = ceil_div(M, 256) * ceil_div(N, 256), whole = tiles256 / cus * cus, left = tiles256 - whole;
   // <tile M, tile N, waves M, waves N, LDS ring slots, e2m1 operands>
@@ -1029,22 +1012,17 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
                                                                  (int)whole);
     }
     case kTiles256Halves:
-      // Rows off the cache lines cost the halves two requests a line, the small tiles one more window (us, halves -> 128 x 128, operands from
-      // the memory-side cache / from memory: e4m3 520 x 10704 x 2016 24.1 -> 21.1 / 28.4 -> 25.7, 986 x 4808 x 2464 26.5 -> 24.2 / 31.9 -> 26.3,
-      // 726 x 9072 x 9952 105.8 -> 93.1 / 106.2 -> 94.8; e2m1 1292 x 5232 x 10304 55.7 -> 51.2 / 67.6 -> 55.2, 3291 x 1528 x 6528 34.9 -> 36.1 /
-      // 41.7 -> 37.2).  Fewer steps or rows: about even, or the halves (e4m3 1384 x 3888 x 1440 19.2 and 18.4 / 18.4 and 19.1, 352 x 16224 x 4768
-      // 44.4 and 48.8 / 55.7 and 52.8, 145 x 22288 x 2528 23.1 and 24.2 / 28.8 and 30.4).
-      if (ragged && M > 384 && k_bytes > 15 * kBK) break;
       return launch_gemm<256, 128, 2, 2, 3, FP4, false, kHalves>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s, tiles256, 0);
     case kTiles256QuadrantSchedule:
       return launch_gemm<256, 256, 2, 2, 2, FP4, false>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
-    case kTiles128:
+    case kFewRows:
+      return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
+    case kSmallTiles:
       break;
   }
-  // small tiles
-  if (variant == 1) return ring(128, 128, plan.splits);
-  const RingPlan r = by_estimate();
-  return ring(r.tile_m, r.tile_n, r.splits);
+  const RingArgs p{A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, workspace, s};
+  const RingPlan& r = plan.small;
+  return FP4 ? launch_ring_e2m1(p, ragged, r.tile_m, r.tile_n, r.splits) : launch_ring_e4m3(p, ragged, r.tile_m, r.tile_n, r.splits);
 }
 
 }  // namespace dt

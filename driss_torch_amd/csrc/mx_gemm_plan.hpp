@@ -1,5 +1,5 @@
-// Which kernel a block-scaled product of more rows than the few-rows kernel takes runs on, and how many
-// workgroups share a tile's K: plain arithmetic on sizes, without the device.
+// Which kernel and tiles a block-scaled product runs on, and how many workgroups share a tile's K: plain arithmetic on sizes, without the
+// device.
 #pragma once
 
 #include <stddef.h>
@@ -12,68 +12,24 @@
 namespace dt {
 
 constexpr int kBK = 128;             // K bytes per step = one 16x16x128 MFMA
-constexpr size_t kSplitTicketBytes = 1024;        // head of the split-K workspace: one counter per 128 x 128 tile
-constexpr size_t kSplitTileBytes = 128 * 128 * 4;  // parked fp32 accumulators of one tile and split
+constexpr size_t kSplitTicketBytes = 1024;        // head of the split-K workspace: one counter per tile, 256 at most
+constexpr size_t kSplitTileBytes = 128 * 128 * 4;  // the rest: parked fp32 accumulators, room for one 128 x 128 tile per CU
 constexpr int kMaxSplits = 16;      // what gemm.split_k may force
 constexpr int kAutoMaxSplits = 12;  // what the library picks by itself
 
-// Split-K factor for the 128 x 128 tiling on request (gemm.variant 1; plan_ring below is the library's own choice, and the figures
-// here are those of the kernel before that one).  A grid of half a workgroup per CU or less leaves most of the chip idle while each workgroup walks the whole K, one K-step per memory latency / 3:
-// share K between as many workgroups per tile as fill the chip once.  What it costs is the last
-// workgroup of a tile reading every share through one CU (about 1 us per share of a full tile),
-// so shares are 16 K-steps on average or more, or 10 while there are at most four shares of a K of 5120 elements
-// or more (the last one is what is left: 41 steps are shared 11 + 11 + 11 + 8;
-// measured on MI355X, e4m3, B rotated through memory, us without -> with: 16 x 8192 x 8192 31 -> 19,
-// 128 x 8192 x 8192 42 -> 24, 1024 x 1024 x 16384 58 -> 34, 512 x 512 x 65536 219 -> 50, 128 x 128 x 16384
-// 56 -> 25, 128 x 5120 x 5120 with four shares of 10 steps 19.9 -> 17.5, with six 19.4, 256 x 5120 x 5120 with
-// three 22.7 -> 19.9, 256 x 4096 x 4096 with three 15.7 -> 16.4; e2m1 128 x 8192 x 8192 with three 24.5 -> 18.2).
-// Two shares pay where they fill four fifths of the chip or more and save more steps than the 8 us that
-// parking and adding a whole chip's tiles takes: from 56 steps on, or 32 when B comes from memory and each
-// step takes longer (256 x 8192 x 8192 41 -> 33, 512 x 4096 x 14336 69 -> 46, 128 x 14336 x 4096 24.8 -> 22.6;
-// not 1000 x 2048 x 6144 23.0 -> 25.4, 128 x 5120 x 5120 19.9 -> 22.1, nor e2m1 96 x 14336 x 4096 14.7 -> 16.0). The knob
-// gemm.split_k forces a factor (1 = never split); whatever is asked for, every split owns a step
-// and the workspace holds all shares.
-inline int plan_splits(bool fp4, int64_t M, int64_t N, int64_t k_steps, size_t workspace_bytes, int cus, int forced) {
-  const int64_t tiles = ceil_div(M, 128) * ceil_div(N, 128);
-  if (workspace_bytes <= kSplitTicketBytes || tiles > (int64_t)(kSplitTicketBytes / 4)) return 1;
-  const int64_t room = (int64_t)((workspace_bytes - kSplitTicketBytes) / kSplitTileBytes) / tiles;
-  int64_t want;
-  if (forced > 0) {
-    want = forced;
-  } else {
-    const int64_t shares = std::max(k_steps * (fp4 ? 2 : 1) >= 40 ? std::min<int64_t>(k_steps / 10, 4) : 0, k_steps / 16);
-    want = cus / tiles;
-    if (want > shares) want = shares;
-    if (want > kAutoMaxSplits) want = kAutoMaxSplits;
-    const bool two_pay = tiles * 5 >= cus * 2 && (k_steps >= 56 || (k_steps >= 32 && N * k_steps * kBK >= ((int64_t)32 << 20)));
-    if (want < 2 || (want == 2 && !two_pay)) return 1;
-  }
-  if (want > kMaxSplits) want = kMaxSplits;
-  if (want > room) want = room;
-  if (want > k_steps) want = k_steps;
-  if (want < 2) return 1;
-  const int64_t per = ceil_div(k_steps, want);
-  return (int)ceil_div(k_steps, per);
-}
-
 enum GemmTiles {
-  kTiles128,                 // small tiles, see plan_ring; on request 128 x 128 with K shared where splits > 1
+  kSmallTiles,               // the kernel for few tiles, in the form that plan_ring gives
   kTiles256Halves,           // 256 x 128 halves of 256 x 256 tiles
   kTiles256x192,
   kTiles256,
   kTiles256ThenQuads,        // whole rounds of 256 x 256, the tiles left over as 128 x 128 quadrants
   kTiles256ThenHalves,       // or as halves
-  kTiles256QuadrantSchedule  // 256 x 256 on the other tiles' main loop (on request only)
-};
-struct GemmPlan {
-  GemmTiles tiles;
-  int splits;  // workgroups that share K per tile (kTiles128)
+  kTiles256QuadrantSchedule,  // 256 x 256 on the other tiles' main loop (on request only)
+  kFewRows                   // the kernel for at most 64 rows (mx_few_rows.hip)
 };
 
-// K counts elements; workspace_bytes 0: none.  variant, tail, split_k: the knobs gemm.variant, gemm.tail_quads
-// and gemm.split_k.
-inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, size_t workspace_bytes, int cus, int variant, int tail,
-                          int split_k) {
+// The tiles of a product by its size, without the kernel for few rows.  variant, tail: the knobs gemm.variant and gemm.tail_quads.
+inline GemmTiles plan_tiles(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, int cus, int variant, int tail) {
   const int64_t tiles256 = ceil_div(M, 256) * ceil_div(N, 256);
   // 256 x 192 tiles where they fill the chip's one round better than 256 x 256 tiles do (which leave a
   // quarter of it idle or more).  At the chip's power limit a round of them takes 0.78 of a round of the
@@ -82,9 +38,9 @@ inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, size_t work
   // 48.3 -> 45.3 and 30.9 -> 29.3; 2000 x 6144 x 8192, 192 -> 256, 80.0 -> 77.7 and 50.9 -> 49.2; two rounds
   // against one and a half: 4096 x 5632 x 4096 77.9 and 77.9, 4096 x 9216 x 4096 120.9 -> 123.5).
   const int64_t tiles192 = ceil_div(M, 256) * ceil_div(N, 192);
-  if (variant == 5 || (variant == 0 && 2 * tiles256 > cus && tiles192 > tiles256 && tiles192 <= cus)) return {kTiles256x192, 1};
-  if (variant == 2) return {kTiles256, 1};
-  if (variant == 7) return {kTiles256QuadrantSchedule, 1};
+  if (variant == 5 || (variant == 0 && 2 * tiles256 > cus && tiles192 > tiles256 && tiles192 <= cus)) return kTiles256x192;
+  if (variant == 2) return kTiles256;
+  if (variant == 7) return kTiles256QuadrantSchedule;
   // One round of 128 x 128 tiles is taken before anything larger.  Between a quarter and half a round of
   // 256 x 256 tiles: as 256 x 128 halves they fill the chip once (0.8 of a round of tiles), as 128 x 128 tiles
   // two rounds (2 x 0.55) unless rows or columns past the matrix leave much of the large tiles idle.  With at
@@ -93,7 +49,13 @@ inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, size_t work
   // 34.6 -> 30.6 and 21.4 -> 16.9, 128 x 32768 x 4096 39.5 -> 35.7 and 24.9 -> 19.3 where 256 x 256 tiles take 53.1
   // and 32.3, 1152 x 3584 x 4096 26.4 -> 22.7 and 19.3 -> 15.9).
   if (variant == 0 && ceil_div(M, 128) * ceil_div(N, 128) > cus) {
-    if (tail != 0 && 4 * tiles256 > cus && 2 * tiles256 <= cus) return {kTiles256Halves, 1};
+    // Rows off the cache lines cost the halves two requests a line, the small tiles one more window (us, halves -> 128 x 128, operands from
+    // the memory-side cache / from memory: e4m3 520 x 10704 x 2016 24.1 -> 21.1 / 28.4 -> 25.7, 986 x 4808 x 2464 26.5 -> 24.2 / 31.9 -> 26.3,
+    // 726 x 9072 x 9952 105.8 -> 93.1 / 106.2 -> 94.8; e2m1 1292 x 5232 x 10304 55.7 -> 51.2 / 67.6 -> 55.2, 3291 x 1528 x 6528 34.9 -> 36.1 /
+    // 41.7 -> 37.2).  Fewer steps or rows: about even, or the halves (e4m3 1384 x 3888 x 1440 19.2 and 18.4 / 18.4 and 19.1, 352 x 16224 x 4768
+    // 44.4 and 48.8 / 55.7 and 52.8, 145 x 22288 x 2528 23.1 and 24.2 / 28.8 and 30.4).
+    if (tail != 0 && 4 * tiles256 > cus && 2 * tiles256 <= cus)
+      return ragged && M > 384 && (fp4 ? K / 2 : K) > 15 * kBK ? kSmallTiles : kTiles256Halves;
     if (tiles256 >= cus / 2) {
       // Whole rounds of the chip on 256 x 256 tiles; what is left over would keep the chip for another
       // full round however few tiles it is.  When its quadrants fit the chip at once it runs as
@@ -106,11 +68,11 @@ inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, size_t work
       // 273 -> 258).  The results are the same bits either way.
       const int64_t left = tiles256 % cus;
       if (tail != 0 && tiles256 >= cus && left > 0 && cus % 8 == 0 && (tail >= 2 || 2 * left <= cus))
-        return {tail == 2 || (tail == 1 && 4 * left <= cus) ? kTiles256ThenQuads : kTiles256ThenHalves, 1};
-      return {kTiles256, 1};
+        return tail == 2 || (tail == 1 && 4 * left <= cus) ? kTiles256ThenQuads : kTiles256ThenHalves;
+      return kTiles256;
     }
   }
-  return {kTiles128, plan_splits(fp4, M, N, ceil_div(fp4 ? K / 2 : K, (int64_t)kBK), workspace_bytes, cus, split_k)};
+  return kSmallTiles;
 }
 
 // The kernel for few tiles (mx_ring_kernels.hpp): tiles of 64 or 128 rows and columns, K shared between `splits` workgroups.
@@ -134,9 +96,9 @@ inline RingPlan plan_ring(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged
   const int64_t parked = workspace_bytes > kSplitTicketBytes ? (int64_t)(workspace_bytes - kSplitTicketBytes) : 0;
   RingPlan best{0, 0, 1, 0};
   for (int bm = 64; bm <= 128; bm += 64) {
-    if (tile_m && bm != tile_m) continue;
+    if (tile_m ? bm != tile_m : bm > 64 && M <= 64 && split_k <= 1) continue;  // (half a tile of rows that are not there is never the shorter one)
     for (int bn = 64; bn <= 128; bn += 64) {
-      if (tile_n && bn != tile_n) continue;
+      if (tile_n ? bn != tile_n : bn > 64 && N <= 64 && split_k <= 1) continue;
       const int64_t tiles = ceil_div(M, (int64_t)bm) * ceil_div(N, (int64_t)bn);
       const int area = bm * bn / 64;  // of 256
       const int lines = (int)std::min<int64_t>(M, bm) + (int)std::min<int64_t>(N, bn) + 8;
@@ -163,16 +125,45 @@ inline RingPlan plan_ring(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged
   return best;
 }
 
-// Does the kernel for at most 64 rows (mx_few_rows.hip) take a product in less time than `ring`?  Its workgroups walk whole rows of
+// What the kernel for at most 64 rows (mx_few_rows.hip) takes, in nanoseconds.  Its workgroups walk whole rows of
 // B, 16 or 32 columns each, with all of A beside them: per round of the chip 2.3 us, and per step and column 5.5 ns (6.6 off
-// whole lines) and 1.6 ns per row of A.  The other kernel reads B at no more than 4.8 TB/s.  (Fitted to 150 problems of 1 to 64 rows:
-// what the two estimates pick takes 0.4 % longer than the better kernel at its best, 11 % at most; a rule on sizes, few rows for K of
-// 2048 and N of 1024 on with exceptions, took 27 % longer.)  columns: of a workgroup.
-inline bool few_rows_beats(const RingPlan& ring, bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, int cus, int columns) {
-  const int64_t k_bytes = fp4 ? K / 2 : K, steps = ceil_div(k_bytes, (int64_t)kBK), rows = ceil_div(M, (int64_t)8) * 8;
+// whole lines) and 1.6 ns per row of A.  columns: of a workgroup.
+inline int64_t few_rows_ns(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, int cus, int columns) {
+  const int64_t steps = ceil_div(fp4 ? K / 2 : K, (int64_t)kBK), rows = ceil_div(M, (int64_t)8) * 8;
   const int64_t rounds = ceil_div(ceil_div(N, (int64_t)columns), (int64_t)cus);
-  const int64_t few = 1000 + 2260 * rounds + rounds * steps * (columns * (ragged ? 66 : 55) + 16 * rows) / 10 - 8 * rows;
-  return few < std::max(ring.ns, 3000 + N * k_bytes / 4800);
+  return 1000 + 2260 * rounds + rounds * steps * (columns * (ragged ? 66 : 55) + 16 * rows) / 10 - 8 * rows;
+}
+
+struct GemmKnobs {  // gemm.variant, gemm.tail_quads, gemm.split_k, gemm.tile_m, gemm.tile_n
+  int variant, tail, split_k, tile_m, tile_n;
+};
+struct GemmPlan {
+  GemmTiles tiles;
+  RingPlan small;  // of kSmallTiles
+};
+
+// K counts elements; ragged: see ring_ragged; workspace_bytes 0: none; few_columns: columns of B that a workgroup of the kernel for few rows
+// takes, 0 where it cannot take the product.
+// The kernel for few rows is taken where it needs less time than the small tiles, or than reading B at 4.8 TB/s, which those never exceed.
+// (Fitted to 150 problems of 1 to 64 rows: what the two estimates pick takes 0.4 % longer than the better kernel at its best, 11 % at most; a
+// rule on sizes, few rows for K of 2048 and N of 1024 on with exceptions, took 27 % longer.)  How many workgroups are to share K
+// does not decide between the two; whether any may does.
+inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, size_t workspace_bytes, int cus, int few_columns, GemmKnobs knobs) {
+  const auto small = [&](int split_k, int tile_m, int tile_n) {
+    return GemmPlan{kSmallTiles, plan_ring(fp4, M, N, K, ragged, workspace_bytes, cus, split_k, tile_m, tile_n)};
+  };
+  if (knobs.variant == 1) return small(knobs.split_k, 128, 128);
+  if (knobs.variant == 3) return small(knobs.split_k, knobs.tile_m, knobs.tile_n);
+  if (few_columns && knobs.variant == 9) return {kFewRows, {}};
+  if (few_columns && knobs.variant == 0) {
+    const int64_t few = few_rows_ns(fp4, M, N, K, ragged, cus, few_columns);
+    if (few < 3000 + N * (fp4 ? K / 2 : K) / 4800) return {kFewRows, {}};
+    const GemmPlan tiles = small(knobs.split_k == 1 ? 1 : 0, 0, 0);
+    if (few < tiles.small.ns) return {kFewRows, {}};
+    return knobs.split_k > 1 ? small(knobs.split_k, 0, 0) : tiles;
+  }
+  const GemmTiles tiles = plan_tiles(fp4, M, N, K, ragged, cus, knobs.variant, knobs.tail);
+  return tiles == kSmallTiles ? small(knobs.split_k, 0, 0) : GemmPlan{tiles, {}};
 }
 
 }  // namespace dt

@@ -1,5 +1,5 @@
-"""The rule that picks the tiles of a block-scaled product and the workgroups that share K, compiled on its own
-for the host: which launch each size takes, at the sizes where the rule turns."""
+"""The rule that picks the kernel and the tiles of a block-scaled product, compiled on its own for the host: which launch each size
+takes, at the sizes where the rule turns."""
 import ctypes as C
 import subprocess
 from pathlib import Path
@@ -7,19 +7,9 @@ from pathlib import Path
 import pytest
 
 ROOT = Path(__file__).resolve().parent.parent
-T128, HALVES, T192, T256, THEN_QUADS, THEN_HALVES, QUADRANT_SCHEDULE = range(7)
+SMALL, HALVES, T192, T256, THEN_QUADS, THEN_HALVES, QUADRANT_SCHEDULE, FEW_ROWS = range(8)
 CUS = 256
 ALL = 1024 + CUS * 128 * 128 * 4  # a workspace with room for a tile per CU
-
-# (M, K, N): workgroups that share K per 128 x 128 tile, e4m3 and e2m1; the GPU tests compute the same products
-SHARES = {(256, 8192, 8192): (2, 2), (250, 7200, 8184): (2, 1),  # two shares of a tile, even and not
-          (256, 16384, 8192): (2, 2),
-          (100, 4128, 14336): (2, 1),  # 33 steps: shares of 17 and 16
-          (128, 5120, 5120): (4, 1), (65, 5152, 5000): (4, 1),  # 40 steps, and 41 as 11 + 11 + 11 + 8
-          (200, 5120, 5120): (3, 1),
-          (128, 8192, 8192): (4, 3), (120, 8064, 8184): (4, 3), (128, 8096, 8000): (4, 3),  # e2m1: 11 + 11 + 10, last step whole, half, in part
-          (128, 16416, 4096): (8, 4),
-          (256, 4096, 4096): (1, 1), (1000, 2048, 2048): (1, 1)}  # too few steps for any
 
 
 @pytest.fixture(scope="module")
@@ -27,17 +17,17 @@ def plan(tmp_path_factory):
     where = tmp_path_factory.mktemp("plan")
     (where / "plan.cpp").write_text(
         '#include "mx_gemm_plan.hpp"\n'
-        'extern "C" int plan(int fp4, long M, long N, long K, long ws, int cus, int variant, int tail, int split_k) {\n'
-        "  const dt::GemmPlan p = dt::plan_gemm(fp4 != 0, M, N, K, (size_t)ws, cus, variant, tail, split_k);\n"
-        "  return p.tiles * 100 + p.splits;\n}\n")
+        'extern "C" int plan(int fp4, long M, long N, long K, int ragged, long ws, int cus, int few, int variant, int tail, int split_k) {\n'
+        "  const dt::GemmPlan p = dt::plan_gemm(fp4 != 0, M, N, K, ragged != 0, (size_t)ws, cus, few, {variant, tail, split_k, 0, 0});\n"
+        "  return p.tiles * 100 + p.small.splits;\n}\n")
     subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-I/opt/rocm/include",
                     f"-I{ROOT / 'include'}", f"-I{ROOT / 'driss_torch_amd' / 'csrc'}", str(where / "plan.cpp"), "-o",
                     str(where / "plan.so")], check=True)
     f = C.CDLL(str(where / "plan.so")).plan
-    f.argtypes = [C.c_int] + [C.c_long] * 4 + [C.c_int] * 4
+    f.argtypes = [C.c_int] + [C.c_long] * 3 + [C.c_int, C.c_long] + [C.c_int] * 5
 
-    def call(fp4, M, N, K, ws=ALL, cus=CUS, variant=0, tail=1, split_k=0):
-        return divmod(f(int(fp4), M, N, K, ws, cus, variant, tail, split_k), 100)
+    def call(fp4, M, N, K, ws=ALL, cus=CUS, variant=0, tail=1, split_k=0, few=0):
+        return divmod(f(int(fp4), M, N, K, (K // 2 if fp4 else K) % 128 != 0, ws, cus, few, variant, tail, split_k), 100)
 
     return call
 
@@ -45,13 +35,13 @@ def plan(tmp_path_factory):
 @pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
 @pytest.mark.parametrize("size,tiles", [
     # a quarter to half a round of 256 x 256 tiles: one round of 128 x 128 tiles where that is enough ...
-    ((65, 16648), T128), ((96, 28672), T128), ((128, 32512), T128), ((300, 10000), T128), ((1152, 3584), T128),
+    ((65, 16648), SMALL), ((96, 28672), SMALL), ((128, 32512), SMALL), ((300, 10000), SMALL), ((1152, 3584), SMALL),
     # ... also at exactly half a round of the large tiles, with half of each outside the matrix, and mirrored
-    ((65, 32520), T128), ((128, 32768), T128), ((32768, 128), T128), ((32700, 65), T128),
+    ((65, 32520), SMALL), ((128, 32768), SMALL), ((32768, 128), SMALL), ((32700, 65), SMALL),
     # one column more is two rounds of them, but one of 256 x 192 tiles
     ((128, 32776), T192), ((128, 49152), T192), ((128, 49160), T256),
     # halves where 128 x 128 tiles do not fit
-    ((129, 16648), HALVES), ((256, 32768), HALVES), ((2048, 4096), HALVES), ((300, 14336), HALVES), ((2048, 2048), T128),
+    ((129, 16648), HALVES), ((256, 32768), HALVES), ((2048, 4096), HALVES), ((300, 14336), HALVES), ((2048, 2048), SMALL),
     ((2304, 2304), HALVES),
     # more than half a round
     ((2048, 4352), T192), ((2000, 6144), T192), ((2048, 6400), T256), ((4096, 4096), T256),
@@ -68,11 +58,11 @@ def test_one_round_of_small_tiles_is_never_given_to_fewer_large_ones(plan):
             for m, n_ in ((rows, n), (n, rows)):
                 up = lambda a, b: -(-a // b)  # noqa: E731
                 if up(m, 128) * up(n_, 128) <= CUS:
-                    assert plan(False, m, n_, 1024)[0] == T128, (m, n_)
+                    assert plan(False, m, n_, 1024)[0] == SMALL, (m, n_)
 
 
 def test_knobs(plan):
-    assert plan(False, 2048, 6144, 1024, variant=1) == (T128, 1)
+    assert plan(False, 2048, 6144, 1024, variant=1) == (SMALL, 1) and plan(False, 128, 128, 16384, variant=1)[1] > 1
     assert plan(False, 16, 64, 1024, variant=2)[0] == T256
     assert plan(False, 16, 64, 1024, variant=5)[0] == T192
     assert plan(False, 16, 64, 1024, variant=7)[0] == QUADRANT_SCHEDULE
@@ -80,12 +70,22 @@ def test_knobs(plan):
     assert plan(False, 4096, 5120, 1024, tail=3)[0] == THEN_HALVES and plan(False, 4096, 6400, 1024, tail=2)[0] == THEN_QUADS
 
 
-@pytest.mark.parametrize("size", SHARES, ids=lambda s: "x".join(map(str, s)))
-def test_shares_of_k(plan, size):
-    M, K, N = size
-    for fp4 in (False, True):
-        assert plan(fp4, M, N, K) == (T128, SHARES[size][fp4])
-        assert plan(fp4, M, N, K, ws=0) == (T128, 1) and plan(fp4, M, N, K, split_k=1) == (T128, 1)
+@pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
+def test_rows_off_the_lines_take_small_tiles_instead_of_halves(plan, fp4):
+    """from 385 rows and 16 steps on, the last of them partly filled"""
+    step = 256 if fp4 else 128
+    for M, N in ((384, 12008), (385, 12008), (400, 8200), (726, 9072), (2048, 4096)):
+        for steps in (2, 15, 16, 17, 64):
+            K = (steps - 1) * step + 32
+            assert plan(fp4, M, N, K)[0] == (SMALL if M > 384 and steps > 15 else HALVES), (M, N, steps)
+            assert plan(fp4, M, N, steps * step)[0] == HALVES
+
+
+def test_few_rows(plan):
+    assert plan(False, 16, 8192, 8192, few=32)[0] == FEW_ROWS and plan(False, 16, 8192, 8192)[0] == SMALL
+    assert plan(False, 16, 64, 64, few=16, variant=9)[0] == FEW_ROWS and plan(False, 100, 64, 64, variant=9)[0] == SMALL
+    for variant, tiles in ((1, SMALL), (2, T256), (3, SMALL), (5, T192), (7, QUADRANT_SCHEDULE)):
+        assert plan(False, 16, 8192, 8192, few=32, variant=variant)[0] == tiles
 
 
 def test_shares_own_a_step_and_fit_the_workspace(plan):
@@ -96,6 +96,6 @@ def test_shares_own_a_step_and_fit_the_workspace(plan):
                 tiles = -(-M // 128) * -(-N // 128)
                 for split_k in (0, 2, 3, 5, 16, 99):
                     for room in (1, tiles, 2 * tiles + 1, 256):
-                        n = plan(fp4, M, N, K, ws=1024 + room * 128 * 128 * 4, split_k=split_k)[1]
+                        n = plan(fp4, M, N, K, ws=1024 + room * 128 * 128 * 4, split_k=split_k, variant=1)[1]
                         assert 1 <= n <= 16 and (n == 1 or n * tiles <= room)
                         assert (n - 1) * -(-steps // n) < steps  # the last share owns a step

@@ -7,7 +7,7 @@ import torch
 from oracle import c_oracle as co
 from oracle import eager
 from tests import util
-from tests.test_gemm_plan import SHARES
+from tests.test_ring_plan import SHARES
 
 pytestmark = pytest.mark.gpu
 
@@ -479,8 +479,8 @@ def test_mx_gemm_split_k(d, cabi, splits, size):
 @pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
 @pytest.mark.parametrize("size", SHARES, ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
 def test_mx_gemm_few_shares_by_rule(d, cabi, size, fp4):
-    """The sizes around which the library's own rule shares K or does not (how many shares each has is checked where
-    the rule is): integers of at most 4 times a power of two of each block's own, up to 2^3 in one operand and 2^2 in
+    """Products whose K the library's own rule shares, evenly and not, and some that it does not (how many shares each has is checked
+    where the rule is): integers of at most 4 times a power of two of each block's own, up to 2^3 in one operand and 2^2 in
     the other, so that a share that took its scales elsewhere along K would show, and every partial sum
     (at most 2^9 K < 2^24) is exact in fp32 whatever the order: the result is one bit pattern."""
     M, K, N = size
