@@ -418,7 +418,7 @@ def test_mx_gemm_schedules_agree(d, cabi, fp4, K):
 @pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
 @pytest.mark.parametrize("K", [96, 160, 256, 384, 672, 768, 1120, 1280, 1312])
 def test_mx_gemm_schedules_agree_on_every_form_of_operand(d, cabi, fp4, K):
-    """The same comparison on what a caller may pass beside library-made contiguous operands: padding of the scales
+    """The same comparison, and the small tiles beside it, on what a caller may pass beside library-made contiguous operands: padding of the scales
     full of NaN codes, row strides above K, an output inside a wider one that begins 8 bytes off a 16-byte boundary,
     a row count and a column count that are no multiples of 8 -- for every number of steps, odd and even, whole and
     partly filled last ones."""
@@ -437,8 +437,12 @@ def test_mx_gemm_schedules_agree_on_every_form_of_operand(d, cabi, fp4, K):
 
     a_view, b_view = strided(a, 16, 48 - kb % 16), strided(b, 64, 16 - kb % 16)
     outs = {}
-    for variant in (7, 2, 5):
-        cabi.set_tuning("gemm.variant", variant)
+    small = [(3, tm, tn) for tm in (64, 128) for tn in (64, 128)]
+    for variant in [7, 2, 5] + small:
+        number, tm, tn = variant if variant in small else (variant, 0, 0)
+        knobs = {"gemm.variant": number, "gemm.tile_m": tm, "gemm.tile_n": tn, "gemm.split_k": 1 if tm else 0}
+        for k, v in knobs.items():
+            cabi.set_tuning(k, v)
         try:
             outs[variant] = product(a.view(dtype), b.view(dtype), d.to_blocked(sa), d.to_blocked(sb))
             for lead, pitch in ((4, N + 24), (8, N + 28)):  # 8 bytes off a boundary; on it, with a pitch of whole vectors
@@ -447,9 +451,10 @@ def test_mx_gemm_schedules_agree_on_every_form_of_operand(d, cabi, fp4, K):
                 assert torch.equal(out[:, lead:lead + N], outs[variant]), (variant, lead)
                 assert (out[:, :lead] == 7.0).all() and (out[:, lead + N:] == 7.0).all(), (variant, lead)
         finally:
-            cabi.set_tuning("gemm.variant", 0)
+            for k in knobs:
+                cabi.set_tuning(k, 0)
     assert torch.isfinite(outs[7]).all() and outs[7].abs().max() > 0
-    assert torch.equal(outs[2], outs[7]) and torch.equal(outs[5], outs[7])
+    assert all(torch.equal(out, outs[7]) for out in outs.values())
 
 
 def _wide_operand(shape, seed):
@@ -630,11 +635,12 @@ def test_mx_gemm_equal_rows_have_equal_results(d, cabi, size, fp4):
 
 
 @pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
-@pytest.mark.parametrize("rows", [384, 400])
+@pytest.mark.parametrize("rows", [384, 385])
 @pytest.mark.parametrize("steps", [15, 16, 17])
 def test_mx_gemm_rows_off_the_lines_on_halves_or_small_tiles(d, cabi, rows, steps, fp4):
-    """either side of the lines between the two, the last step a quarter full: the same K order, so the bits of the 256 x 256 tiles"""
-    K, N = ((steps - 1) * 128 + 32) * (2 if fp4 else 1), 8200
+    """either side of the lines between the two (which size takes which is checked where the rule is), the last step a quarter full: the
+    same K order, so the bits of the 256 x 256 tiles"""
+    K, N = ((steps - 1) * 128 + 32) * (2 if fp4 else 1), 12008
     x, w = _wide_operand((rows, K), 7100 + steps).cuda(), _wide_operand((N, K), 7101).cuda()
     if fp4:
         (a, sa), (b, sb), op = d.mx_fp4_quantize(x, True), d.mx_fp4_quantize(w, True), d.mx_fp4_bf16
