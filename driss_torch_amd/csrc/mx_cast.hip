@@ -1,4 +1,5 @@
 // dt_mx_fp8_quantize / dt_to_blocked: MXFP8 cast with E8M0 block-32 scales (C ABI).
+#include "mx_cast_plan.hpp"
 #include "mx_kernels.hpp"
 
 namespace {
@@ -281,19 +282,13 @@ int launch_mx_fp4(const MxArgs& a) {
 // blocks down the columns, payload transposed: [cols, rows/2], scales [cols, rows/32]
 template <int IN, int LAYOUT>
 int launch_mx_fp4_cols(const MxArgs& a) {
-  // As for MXFP8, the one-read kernel without its row-wise half: wide tiles for 16-bit inputs with more of them than the walking grid
-  // (bf16, us, this / mx_col_t_kernel: 8192 x 8192 33.1 / 33.9, 16384 x 4096 30.5 / 35.5, 4096 x 16384 31.5 / 31.7; it loses for fp32,
-  // 55.4 / 51.9, and for small tensors, 2048 x 4096 6.6 / 5.9), narrow ones where there are few, and where the payload's rows are off the
-  // cache lines (us, mx_col_t_kernel or wide -> narrow, bf16: 512 x 512 3.9 -> 3.2, 1024 x 1664 4.5 -> 4.1, 2752 x 4096 9.5 -> 8.0, 6240 x 11968
-  // 38.1 -> 36.5; fp32: 512 x 512 4.7 -> 3.1, 2048 x 4096 9.5 -> 8.6, 2752 x 4096 13.3 -> 11.3, 6240 x 11968 71.1 -> 61.6; not bf16
-  // 2048 x 1888, 128 tiles, 4.95 and 5.1, nor fp32 4096 x 4096 15.4 and 16.0)
+  // As for MXFP8, the one-read kernel without its row-wise half, where plan_fp4_cols prefers it
   constexpr int kV = InTraits<IN>::kVec;
-  const int64_t dual_tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)(32 * kV));
-  const int64_t cus = device_facts().cu_count, pipe_grid = (int64_t)tuning(Knob::mx_colt_pipe) * cus;
-  const int knob = tuning(Knob::mx_dual_narrow);
-  const bool narrow = knob >= 0 ? knob != 0 : a.rows % 256 != 0 || (IN == DT_F32 ? dual_tiles <= 2 * cus : dual_tiles * 4 <= cus);
-  if (a.cols % kV == 0 && tuning(Knob::mx_colt_via_dual) && (narrow || (IN != DT_F32 && pipe_grid > 0 && dual_tiles > pipe_grid))) {
-    const int st = launch_dual_cols<IN, DT_E2M1, LAYOUT>(a, narrow);
+  const int64_t cus = device_facts().cu_count;
+  const Fp4Cols plan = plan_fp4_cols(IN == DT_F32, LAYOUT == DT_SCALE_BLOCKED, a.rows, a.cols, cus, (int64_t)tuning(Knob::mx_colt_pipe) * cus,
+                                     tuning(Knob::mx_dual_narrow));
+  if (a.cols % kV == 0 && tuning(Knob::mx_colt_via_dual) && plan != kFp4ColT) {
+    const int st = launch_dual_cols<IN, DT_E2M1, LAYOUT>(a, plan == kFp4Narrow);
     if (st != kNotTaken) return st;
   }
   const int64_t tiles = ceil_div(a.rows, (int64_t)kColTRows) * ceil_div(a.cols, (int64_t)kColTCols);

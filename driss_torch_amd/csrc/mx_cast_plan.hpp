@@ -1,0 +1,43 @@
+// Which kernel the MXFP4 cast down the columns takes: plain arithmetic on sizes, without the device.
+#pragma once
+
+#include <stdint.h>
+
+#include "dt_host.hpp"
+
+namespace dt {
+
+constexpr int kDualRows = 128;
+
+// mx_col_t_kernel; or mx_dual_kernel without its row-wise half, on tiles of 128 rows x 256 columns by a grid of walking workgroups, where 16-bit
+// tiles are more than that grid (us, it / mx_col_t_kernel, bf16: 8192 x 8192 33.1 / 33.9, 16384 x 4096 30.5 / 35.5; fp32 55.4 / 51.9); or the same on
+// tiles half as wide (256 -> 128 columns, fp32 128 -> 64), one workgroup each:
+//  - where tiles are few, the narrow ones fill the chip (us, before -> narrow, bf16 512 x 512 3.9 -> 3.2, 1024 x 1664 4.5 -> 4.1; not of 32 rows, 32 x
+//    15840 3.4 and 3.7, nor 2432 x 3104, 247 tiles, 6.1 and 7.0; fp32 512 x 512 4.7 -> 3.1, 2048 x 2048 6.5 -> 5.9; not 2560 x 3072, 480 tiles, 7.9 and 8.7);
+//  - fp32, just past two tiles per CU, where the others begin another round (2560 x 3584, 560 tiles, 11.5 -> 9.6), and where there are more and the
+//    transposed rows are off the cache lines (12320 x 2368 30.0 -> 26.7, 7328 x 8288 69.3 -> 56.5; 8192 x 8192 54.6 and 60.0);
+//  - 16 bits, more than one and up to one and a half per CU, of a matrix that is not four times as tall as wide (3104 x 3264 9.4 -> 7.9, 672 x 14304
+//    9.9 -> 8.3; 14592 x 672 8.0 and 8.2), and more than four per CU of one sixteen times as tall (54944 x 736 29.3 -> 24.7, 85792 x 864 48.9 -> 43.6);
+//  - 16 bits, more than one per CU, where the rows of x begin on lines (6240 x 11968 38.1 -> 36.5, 3072 x 4096 9.0 -> 7.9; 12320 x 4064 31.4 and 36.3,
+//    4960 x 16416 51.3 and 60.4), the transposed payload goes out in whole pieces of 64 bytes (row-major scales 16608 x 704 10.0 and 13.5,
+//    5056 x 21056 60.8 and 66.6), and the walking grid, if it is one, does not go in bands of row tiles (12288 x 6144 38.1 and 43.2).
+// Picked from all three at 751 sizes of 0.25 to 130 million elements, half of them round, bf16 and fp32, both layouts of the scales: 0.95 / 0.91
+// (bf16 / fp32) of the time that the first two alone take, at no size more than 1.1; at 126 others, 0.92 and 1.08.
+// pipe_grid: workgroups of the walking grid; forced: the knob mx.dual_narrow.
+enum Fp4Cols { kFp4ColT, kFp4Wide, kFp4Narrow };
+inline Fp4Cols plan_fp4_cols(bool f32, bool blocked, int64_t rows, int64_t cols, int64_t cus, int64_t pipe_grid, int forced) {
+  const int64_t tiles = ceil_div(rows, (int64_t)kDualRows) * ceil_div(cols, (int64_t)(f32 ? 128 : 256));
+  bool narrow;
+  if (forced >= 0)
+    narrow = forced != 0;
+  else if (f32)
+    narrow = tiles <= cus || (tiles > 2 * cus && (2 * tiles <= 5 * cus || rows % 128 != 0));
+  else
+    narrow = (2 * tiles <= cus && rows > 32) || (tiles > cus && 2 * tiles <= 3 * cus && rows < 4 * cols) ||
+             (tiles > 4 * cus && rows > 16 * cols) ||
+             (tiles > cus && cols % 64 == 0 && (rows % 128 == 0 || (blocked && tiles > 4 * cus)) &&
+              (tiles <= 2 * cus || rows % (8 * kDualRows) != 0));
+  return narrow ? kFp4Narrow : !f32 && pipe_grid > 0 && tiles > pipe_grid ? kFp4Wide : kFp4ColT;
+}
+
+}  // namespace dt

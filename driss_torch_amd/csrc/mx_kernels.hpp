@@ -19,6 +19,7 @@
 
 #include "dt_device.hpp"
 #include "dt_host.hpp"
+#include "mx_cast_plan.hpp"
 #include "quant_kernels.hpp"
 
 namespace dt {
@@ -557,7 +558,7 @@ __global__ __launch_bounds__(kBlock) void mx_col_t_kernel(const void* __restrict
 // LDS tile: [column][128 rows] with a pitch of 144 bytes; the 16-byte chunk index is XORed
 // with bits 4..6 of the column so that the 16 lanes of one write phase (columns kV apart) fall
 // on 16 different bank groups.
-constexpr int kDualRows = 128, kDualPitch = 144;
+constexpr int kDualPitch = 144;  // (kDualRows, the tile's 128 rows, is in mx_cast_plan.hpp)
 // (e2m1 output: a column's 128 rows are 64 bytes; pitch 80, the chunk index XORed with bits 4..5 of the column)
 constexpr int kDualPitch4 = 80;
 
