@@ -46,6 +46,8 @@ int launch_dual_cols(const MxArgs& a, bool narrow) {
   if (narrow)
     mx_dual_kernel<IN, OUT, LAYOUT, false, false, 8><<<(unsigned)narrow_tiles, kBlock, 0, a.stream>>>(
         a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
+  else if constexpr (IN == DT_F32 && OUT == DT_E2M1)
+    return kNotTaken;  // mx_col_t_kernel is the better one, see plan_fp4_cols
   else if (pipe_grid > 0 && tiles > pipe_grid)
     mx_dual_kernel<IN, OUT, LAYOUT, false, true><<<(unsigned)pipe_grid, kBlock, 0, a.stream>>>(
         a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
