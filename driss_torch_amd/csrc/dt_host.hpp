@@ -40,7 +40,7 @@ const DeviceFacts& device_facts();  // of the current device, cached per device
 //   mx.dual:      1 = dt_mx_fp8_quantize_dual reads x once (0: two single casts)
 //   mx.colt_via_dual: 1 = the transposed column cast runs as the one-read kernel without its row half
 //   mx.dual_order: tile order of the one-read kernel: -1 = chosen by shape, 0 = down the rows first, 1 = along
-//                 the columns first, 2 = bands of 8 row tiles (by shape only without the row-wise half)
+//                 the columns first, 2 = bands of 8 row tiles
 //   mx.dual_narrow: its tiles: -1 = chosen by shape, 0 = wide (256 columns of 16 bits, 128 of fp32), 1 = half as wide (fp32: columns alone)
 //   mx.colt_pipe: the transposed column cast as a grid of this many workgroups per CU that walk the tiles
 //                 with the next tile's loads in flight (0 = one workgroup per tile)

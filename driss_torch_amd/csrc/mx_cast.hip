@@ -171,14 +171,13 @@ struct DualArgs {
 template <int IN, int OUT, int LAYOUT>
 int launch_dual_tiles(const DualArgs& a) {
   const int64_t bands = ceil_div(a.rows, (int64_t)kDualRows), tiles = bands * ceil_div(a.cols, (int64_t)32 * InTraits<IN>::kVec);
-  // Tile order: along the columns first, down the rows first for matrices four times as wide as tall (narrow tiles, 4096 x 14336 43.6 and
-  // 44.7 us, 2976 x 11968 32.0 and 30.8; wide ones, 8192 x 14336 93.7 and 98.1).
-  const int order = tuning(Knob::mx_dual_order) >= 0 ? tuning(Knob::mx_dual_order) : a.cols > 4 * a.rows ? 0 : 1;
+  const int64_t cus = device_facts().cu_count, narrow_tiles = bands * ceil_div(a.cols, (int64_t)16 * InTraits<IN>::kVec);
+  const int knob = tuning(Knob::mx_dual_narrow);
+  const bool narrow = IN != DT_F32 && (knob >= 0 ? knob != 0 : tiles * 8 <= cus * 11 || (OUT != DT_E2M1 && tiles >= 4 * cus && a.cols % 64 == 0)) &&
+                      narrow_tiles <= 0x7FFFFFFFll;
+  const int order = tuning(Knob::mx_dual_order) >= 0 ? tuning(Knob::mx_dual_order) : pair_order(IN == DT_F32, OUT == DT_E2M1, narrow, a.rows, a.cols, cus);
   if constexpr (IN != DT_F32) {
-    const int64_t cus = device_facts().cu_count, narrow_tiles = bands * ceil_div(a.cols, (int64_t)16 * InTraits<IN>::kVec);
-    const int knob = tuning(Knob::mx_dual_narrow);
-    const bool narrow = knob >= 0 ? knob != 0 : tiles * 8 <= cus * 11 || (OUT != DT_E2M1 && tiles >= 4 * cus && a.cols % 64 == 0);
-    if (narrow && narrow_tiles <= 0x7FFFFFFFll) {
+    if (narrow) {
       mx_dual_kernel<IN, OUT, LAYOUT, true, false, 8><<<(unsigned)narrow_tiles, kBlock, 0, a.stream>>>(
           a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data_r, a.scale_r, a.data_c, a.scale_c, order);
       return launch_status();

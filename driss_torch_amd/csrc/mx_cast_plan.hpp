@@ -1,4 +1,5 @@
-// Which kernel the MXFP4 cast down the columns takes: plain arithmetic on sizes, without the device.
+// Which kernel the MXFP4 cast down the columns takes, and the order in which the one-read casts go over their tiles: plain arithmetic on
+// sizes, without the device.
 #pragma once
 
 #include <stdint.h>
@@ -38,6 +39,18 @@ inline Fp4Cols plan_fp4_cols(bool f32, bool blocked, int64_t rows, int64_t cols,
              (tiles > cus && cols % 64 == 0 && (rows % 128 == 0 || (blocked && tiles > 4 * cus)) &&
               (tiles <= 2 * cus || rows % (8 * kDualRows) != 0));
   return narrow ? kFp4Narrow : !f32 && pipe_grid > 0 && tiles > pipe_grid ? kFp4Wide : kFp4ColT;
+}
+
+// Tile order of the casts along both axes from one read: 0 = down the rows first, 1 = along the columns first, 2 = bands of 8 row tiles.  Along the
+// columns first (us, against down the rows: bf16 wide tiles 16384 x 4096 51.6 and 58.7, narrow ones 48.5 and 58.6, fp32 3840 x 10784 50.7 and 66.9);
+// down the rows first for matrices four times as wide as tall (narrow tiles, 2976 x 11968 30.8 and 32.0), and for fp32 ones of rows that
+// lie multiples of 32 KiB apart already from twice, while the tiles are not many (3584 x 8192 MXFP8 36.1 against 37.3, MXFP4 31.5 against 33.6; 5120
+// x 16384, 5120 tiles, 94.4 and 87.4); wide tiles of MXFP4 in bands where the row count allows and there are three per CU or more (against along
+// the columns, bf16 16384 x 2560 28.3 and 30.2, fp32 8192 x 2560 22.9 and 24.0; 14336 x 1024, 448 tiles, 12.0 and 11.4).
+inline int pair_order(bool f32, bool fp4, bool narrow, int64_t rows, int64_t cols, int64_t cus) {
+  const int64_t tiles = ceil_div(rows, (int64_t)kDualRows) * ceil_div(cols, (int64_t)(f32 ? 128 : 256));  // wide ones
+  if (cols > 4 * rows || (f32 && cols > 2 * rows && cols % 8192 == 0 && tiles <= 8 * cus)) return 0;
+  return fp4 && !narrow && rows % (8 * kDualRows) == 0 && cols <= 2 * rows && tiles >= 3 * cus ? 2 : 1;
 }
 
 }  // namespace dt

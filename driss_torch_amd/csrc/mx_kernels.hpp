@@ -625,7 +625,7 @@ __global__ __launch_bounds__(kBlock) void mx_dual_kernel(const void* __restrict_
   // mx_col_t_kernel) keeps them on the same rows of the transposed payload.  Measured, the first
   // is faster unless the matrix is much wider than tall (without the row-wise half the second wins from
   // square on), so the host picks by shape (cols_first: 1 = the first, 0 = the second, 2 = the banded order below,
-  // for the column half alone where the row count is a multiple of 8 tiles).
+  // for row counts that are multiples of 8 tiles; see the launches).
   const uint32_t row_tiles = (rows + kDualRows - 1) / kDualRows;
   const uint32_t col_tiles = dual_col_tiles<kTileCols, LAYOUT>(cols);
   const uint32_t ntiles = row_tiles * col_tiles;

@@ -1,4 +1,5 @@
-"""The rule that picks the kernel of the MXFP4 cast down the columns, compiled on its own for the host."""
+"""The rules that pick the kernel of the MXFP4 cast down the columns and the tile order of the casts along both axes, compiled on their own
+for the host."""
 import ctypes as C
 import subprocess
 from pathlib import Path
@@ -11,18 +12,26 @@ CUS = 256
 
 
 @pytest.fixture(scope="module")
-def plan(tmp_path_factory):
+def lib(tmp_path_factory):
     where = tmp_path_factory.mktemp("cast_plan")
     (where / "plan.cpp").write_text(
         '#include "mx_cast_plan.hpp"\n'
         'extern "C" int plan(int f32, int blocked, long rows, long cols, long cus, long pipe_grid, int forced) {\n'
-        "  return dt::plan_fp4_cols(f32 != 0, blocked != 0, rows, cols, cus, pipe_grid, forced);\n}\n")
+        "  return dt::plan_fp4_cols(f32 != 0, blocked != 0, rows, cols, cus, pipe_grid, forced);\n}\n"
+        'extern "C" int order(int f32, int fp4, int narrow, long rows, long cols, long cus) {\n'
+        "  return dt::pair_order(f32 != 0, fp4 != 0, narrow != 0, rows, cols, cus);\n}\n")
     subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-I/opt/rocm/include",
                     f"-I{ROOT / 'include'}", f"-I{ROOT / 'driss_torch_amd' / 'csrc'}", str(where / "plan.cpp"), "-o",
                     str(where / "plan.so")], check=True)
-    f = C.CDLL(str(where / "plan.so")).plan
-    f.argtypes = [C.c_int] * 2 + [C.c_long] * 4 + [C.c_int]
-    return lambda rows, cols, f32=False, blocked=True, forced=-1: f(f32, blocked, rows, cols, CUS, 2 * CUS, forced)
+    so = C.CDLL(str(where / "plan.so"))
+    so.plan.argtypes = [C.c_int] * 2 + [C.c_long] * 4 + [C.c_int]
+    so.order.argtypes = [C.c_int] * 3 + [C.c_long] * 3
+    return so
+
+
+@pytest.fixture(scope="module")
+def plan(lib):
+    return lambda rows, cols, f32=False, blocked=True, forced=-1: lib.plan(f32, blocked, rows, cols, CUS, 2 * CUS, forced)
 
 
 # (rows, cols): the kernel that measured best, or within 4 % of it, for (bf16 blocked, bf16 row-major, fp32)
@@ -46,3 +55,11 @@ def test_picks(plan, size):
 def test_forced(plan):
     assert plan(8192, 8192, forced=1) == NARROW and plan(512, 512, forced=0) == COL_T
     assert plan(12544, 6144, forced=0) == WIDE and plan(12544, 6144, f32=True, forced=0) == COL_T
+
+
+@pytest.mark.parametrize("f32,fp4,narrow,size,order", [
+    (0, 0, 0, (16384, 4096), 1), (0, 0, 1, (8192, 8192), 1), (0, 0, 1, (4096, 14336), 1), (0, 0, 1, (2976, 11968), 0), (0, 0, 1, (3040, 11968), 1),
+    (1, 0, 0, (3840, 10784), 1), (1, 0, 0, (3584, 8192), 0), (1, 1, 0, (3584, 8192), 0), (1, 0, 0, (4096, 16384), 1), (0, 1, 0, (3584, 8192), 1),
+    (0, 1, 0, (16384, 2560), 2), (1, 1, 0, (8192, 2560), 2), (0, 0, 0, (16384, 2560), 1), (0, 1, 0, (14336, 1024), 1), (0, 1, 0, (3040, 6528), 1)])
+def test_order_of_the_casts_along_both_axes(lib, f32, fp4, narrow, size, order):
+    assert lib.order(f32, fp4, narrow, *size, CUS) == order
