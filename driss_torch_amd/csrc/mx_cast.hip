@@ -81,16 +81,7 @@ int launch_mx(const MxArgs& a) {
   }
   if (a.axis == 0 && a.transpose && a.cols % kV == 0 && aligned(a.data, 16) && aligned(a.scale, 4) &&
       a.rows < (1ll << 31) && a.cols < (1ll << 31) && tuning(Knob::mx_colt_via_dual)) {
-    // Narrow tiles fill the chip where tiles are few, and the 16-bit ones also beat the walking grid where there are many (us, wide ->
-    // narrow, bf16: 512 x 512 4.4 -> 3.4, 1024 x 1664 5.3 -> 4.3, 2048 x 1888 6.3 -> 5.5, 2752 x 4096, 352 tiles, 9.3 -> 8.8, 3584 x 8192, 896
-    // tiles, 18.9 -> 17.8, 8192 x 8192 40.8 -> 38.1, 4096 x 14336 35.2 -> 32.4; fp32: 512 x 512 3.4 -> 3.0, 2048 x 4096, 512 tiles, 9.8 -> 9.3).
-    // In between, and for more fp32 tiles, the wide ones win (bf16 4096 x 3488, 448 tiles, 10.6 and 11.3, 6144 x 4096, 768 tiles, 15.5 and
-    // 16.4; fp32 4096 x 4096 17.1 and 18.1, 8192 x 8192 58.9 and 61.6).
-    const int64_t tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)(32 * kV));
-    // Row-major scales: the many narrow ones lose where a column's scale bytes are no whole words (6240 x 11968 50.3 and 53.7) and in matrices
-    // four times as tall as wide (16384 x 4096 39.3 and 39.9; 14336 x 4096 35.9 -> 34.5).
-    const bool many = tiles * 2 >= 7 * cus && (LAYOUT == DT_SCALE_BLOCKED || (a.rows % 128 == 0 && a.rows < 4 * a.cols));
-    const bool narrow = IN == DT_F32 ? tiles <= 2 * cus : tiles * 8 <= 11 * cus || many;
+    const bool narrow = narrow_cols(IN == DT_F32, LAYOUT == DT_SCALE_BLOCKED, a.rows, a.cols, cus);
     const int st = launch_dual_cols<IN, OUT, LAYOUT>(a, narrow);
     if (st != kNotTaken) return st;
   }

@@ -1,4 +1,4 @@
-// Which kernel the MXFP4 cast down the columns takes, and the order in which the one-read casts go over their tiles: plain arithmetic on
+// Which tiles or kernel the casts down the columns take, and the order in which the one-read casts go over their tiles: plain arithmetic on
 // sizes, without the device.
 #pragma once
 
@@ -9,6 +9,23 @@
 namespace dt {
 
 constexpr int kDualRows = 128;
+
+// MXFP8 down the columns (mx_dual_kernel without its row-wise half): tiles of 128 rows x 128 columns (fp32: 64), or twice as wide.
+// Narrow tiles fill the chip where tiles are few, and the 16-bit ones also beat the walking grid where there are many (us, wide ->
+// narrow, bf16: 512 x 512 4.4 -> 3.4, 1024 x 1664 5.3 -> 4.3, 2048 x 1888 6.3 -> 5.5, 2752 x 4096, 352 tiles, 9.3 -> 8.8, 3584 x 8192, 896
+// tiles, 18.9 -> 17.8, 8192 x 8192 40.8 -> 38.1, 4096 x 14336 35.2 -> 32.4; fp32: 512 x 512 3.4 -> 3.0, 2048 x 4096, 512 tiles, 9.8 -> 9.3).
+// In between, and for more fp32 tiles, the wide ones win (bf16 4096 x 3488, 448 tiles, 10.6 and 11.3, 6144 x 4096, 768 tiles, 15.5 and
+// 16.4; fp32 4096 x 4096 17.1 and 18.1, 8192 x 8192 58.9 and 61.6).
+// Row-major scales: the many narrow ones lose where a column's scale bytes are no whole words (6240 x 11968 50.3 and 53.7) and in matrices
+// four times as tall as wide (16384 x 4096 39.3 and 39.9; 14336 x 4096 35.9 -> 34.5).
+// fp32, blocked scales: of up to 64 columns every other narrow tile holds nothing but the padding of the scales to 128 columns, which
+// loses once they are more than one per CU (8192 x 64 4.1 -> 3.8, 16384 x 64 4.3 and 4.3, 20480 x 64 4.5 and 5.0, 65536 x 64 6.6 and 8.1; three
+// tiles of four, 20480 x 192 7.2 -> 6.8).
+inline bool narrow_cols(bool f32, bool blocked, int64_t rows, int64_t cols, int64_t cus) {
+  const int64_t tiles = ceil_div(rows, (int64_t)kDualRows) * ceil_div(cols, (int64_t)(f32 ? 128 : 256));  // wide ones
+  if (f32) return tiles <= (blocked && cols <= 64 ? cus / 2 : 2 * cus);
+  return tiles * 8 <= 11 * cus || (tiles * 2 >= 7 * cus && (blocked || (rows % 128 == 0 && rows < 4 * cols)));
+}
 
 // mx_col_t_kernel; or mx_dual_kernel without its row-wise half, on tiles of 128 rows x 256 columns by a grid of walking workgroups, where 16-bit
 // tiles are more than that grid (us, it / mx_col_t_kernel, bf16: 8192 x 8192 33.1 / 33.9, 16384 x 4096 30.5 / 35.5; fp32 55.4 / 51.9); or the same on

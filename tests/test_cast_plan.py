@@ -1,5 +1,5 @@
-"""The rules that pick the kernel of the MXFP4 cast down the columns and the tile order of the casts along both axes, compiled on their own
-for the host."""
+"""The rules that pick the tiles of the MXFP8 cast and the kernel of the MXFP4 cast down the columns and the tile order of the casts along both
+axes, compiled on their own for the host."""
 import ctypes as C
 import subprocess
 from pathlib import Path
@@ -18,6 +18,8 @@ def lib(tmp_path_factory):
         '#include "mx_cast_plan.hpp"\n'
         'extern "C" int plan(int f32, int blocked, long rows, long cols, long cus, long pipe_grid, int forced) {\n'
         "  return dt::plan_fp4_cols(f32 != 0, blocked != 0, rows, cols, cus, pipe_grid, forced);\n}\n"
+        'extern "C" int narrow_cols(int f32, int blocked, long rows, long cols, long cus) {\n'
+        "  return dt::narrow_cols(f32 != 0, blocked != 0, rows, cols, cus);\n}\n"
         'extern "C" int order(int f32, int fp4, int narrow, long rows, long cols, long cus) {\n'
         "  return dt::pair_order(f32 != 0, fp4 != 0, narrow != 0, rows, cols, cus);\n}\n")
     subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-I/opt/rocm/include",
@@ -25,6 +27,7 @@ def lib(tmp_path_factory):
                     str(where / "plan.so")], check=True)
     so = C.CDLL(str(where / "plan.so"))
     so.plan.argtypes = [C.c_int] * 2 + [C.c_long] * 4 + [C.c_int]
+    so.narrow_cols.argtypes = [C.c_int] * 2 + [C.c_long] * 3
     so.order.argtypes = [C.c_int] * 3 + [C.c_long] * 3
     return so
 
@@ -63,3 +66,12 @@ def test_forced(plan):
     (0, 1, 0, (16384, 2560), 2), (1, 1, 0, (8192, 2560), 2), (0, 0, 0, (16384, 2560), 1), (0, 1, 0, (14336, 1024), 1), (0, 1, 0, (3040, 6528), 1)])
 def test_order_of_the_casts_along_both_axes(lib, f32, fp4, narrow, size, order):
     assert lib.order(f32, fp4, narrow, *size, CUS) == order
+
+
+@pytest.mark.parametrize("f32,blocked,size,narrow", [
+    (0, 1, (512, 512), 1), (0, 0, (2752, 4096), 1), (0, 1, (4096, 3488), 0), (0, 0, (6144, 4096), 0), (0, 1, (3584, 8192), 1), (0, 1, (8192, 8192), 1),
+    (0, 1, (6240, 11968), 1), (0, 0, (6240, 11968), 0), (0, 1, (16384, 4096), 1), (0, 0, (16384, 4096), 0), (0, 0, (14336, 4096), 1),
+    (1, 1, (512, 512), 1), (1, 0, (2048, 4096), 1), (1, 1, (4096, 4096), 0), (1, 1, (8192, 8192), 0),
+    (1, 1, (16384, 64), 1), (1, 1, (20480, 64), 0), (1, 0, (20480, 64), 1), (1, 1, (65536, 32), 0), (1, 1, (20480, 192), 1), (0, 1, (20480, 64), 1)])
+def test_tiles_of_the_mxfp8_column_cast(lib, f32, blocked, size, narrow):
+    assert lib.narrow_cols(f32, blocked, *size, CUS) == narrow
