@@ -128,12 +128,12 @@ inline RingPlan plan_ring(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged
 }
 
 // What the kernel for at most 64 rows (mx_few_rows.hip) takes, in nanoseconds.  Its workgroups walk whole rows of
-// B, 16 or 32 columns each, with all of A beside them: per round of the chip 2.3 us, and per step and column 5.5 ns (6.6 off
-// whole lines) and 1.6 ns per row of A.  columns: of a workgroup.
+// B, 16 or 32 columns each, with all of A beside them: per round of the chip 2.3 us, and per step and column 5.5 ns (5.2 off
+// whole lines, where the rows do not begin on the same channels) and 1.6 ns per row of A.  columns: of a workgroup.
 inline int64_t few_rows_ns(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, int cus, int columns) {
   const int64_t steps = ceil_div(fp4 ? K / 2 : K, (int64_t)kBK), rows = ceil_div(M, (int64_t)8) * 8;
   const int64_t rounds = ceil_div(ceil_div(N, (int64_t)columns), (int64_t)cus);
-  return 1000 + 2260 * rounds + rounds * steps * (columns * (ragged ? 66 : 55) + 16 * rows) / 10 - 8 * rows;
+  return 1000 + 2260 * rounds + rounds * steps * (columns * (ragged ? 52 : 55) + 16 * rows) / 10 - 8 * rows;
 }
 
 struct GemmKnobs {  // gemm.variant, gemm.tail_quads, gemm.split_k, gemm.tile_m, gemm.tile_n
@@ -147,9 +147,12 @@ struct GemmPlan {
 // K counts elements; ragged: see ring_ragged; workspace_bytes 0: none; few_columns: columns of B that a workgroup of the kernel for few rows
 // takes, 0 where it cannot take the product.
 // The kernel for few rows is taken where it needs less time than the small tiles, or than reading B at 4.8 TB/s, which those never exceed.
-// (Fitted to 150 problems of 1 to 64 rows: what the two estimates pick takes 0.4 % longer than the better kernel at its best, 11 % at most; a
-// rule on sizes, few rows for K of 2048 and N of 1024 on with exceptions, took 27 % longer.)  How many workgroups are to share K
-// does not decide between the two; whether any may does.
+// (Fitted to 150 problems of 1 to 64 rows, and off whole lines to 340: at 350 others of 128 to 12000 columns drawn at random, half of them of
+// few columns and a long K, where the choice is close, what the two estimates pick takes 0.2 % longer than the better kernel with B from memory,
+// 13 % at most, and 1.0 % from the memory-side cache, 25 % at most, where few rows gain more.  With 6.6 ns off whole lines these were 0.25 %
+// and 1.7 %, 50 % at most: e2m1 12 x 1488 x 12064 from the cache 8.9 and 6.9 us, 1 x 168 x 10048 7.6 and 5.1, from memory 7.9 and 6.4.
+// A rule on sizes, few rows for K of 2048 and N of 1024 on with exceptions, took 27 % longer on the 150.)  How many workgroups are to
+// share K does not decide between the two; whether any may does.
 inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, size_t workspace_bytes, int cus, int few_columns, GemmKnobs knobs) {
   const auto small = [&](int split_k, int tile_m, int tile_n) {
     return GemmPlan{kSmallTiles, plan_ring(fp4, M, N, K, ragged, workspace_bytes, cus, split_k, tile_m, tile_n)};

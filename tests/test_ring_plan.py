@@ -100,6 +100,7 @@ def test_picks(lib):
         return lib.few(fp4, M, N, K, (K // 2 if fp4 else K) % 128 != 0, ALL, CUS, 32 if N >= 8192 else 16, split_k)
 
     assert few(16, 8192, 8192) and few(1, 1928, 1984) and few(16, 4096, 4096, 1)
+    assert few(1, 168, 10048, 1) and few(12, 1488, 12064, 1) and few(2, 464, 5152) and not few(64, 424, 8224)
     for split_k in (1, 2, 7):  # how many workgroups share K says nothing about the kernel for few rows; that none may can only speak for it
         assert few(16, 8192, 8192, split_k=split_k) and few(16, 4096, 4096, 1, split_k)
     assert few(16, 1024, 8192, split_k=1) and not few(16, 1024, 8192, split_k=2) and not few(16, 1024, 8192)
