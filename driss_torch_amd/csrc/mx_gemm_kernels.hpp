@@ -28,6 +28,7 @@
 
 #include "dt_device.hpp"
 #include "dt_host.hpp"
+#include "mx_few_lines.hpp"
 #include "mx_few_rows.hpp"
 #include "mx_gemm_plan.hpp"
 #include "mx_ring.hpp"
@@ -992,7 +993,8 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
   const bool ragged = ring_ragged(k_bytes, A, B, lda, ldb);
   const GemmPlan plan = plan_gemm(FP4, M, N, K, ragged, workspace ? workspace_bytes : 0, cus, few_rows_fits(M, K) ? few_rows_columns(N) : 0,
                                   {tuning(Knob::gemm_variant), tuning(Knob::gemm_tail_quads), tuning(Knob::gemm_split_k),
-                                   tuning(Knob::gemm_tile_m), tuning(Knob::gemm_tile_n)});
+                                   tuning(Knob::gemm_tile_m), tuning(Knob::gemm_tile_n), few_lines_forced_octets()},
+                                  few_lines_fits(M, K));
   // tiles of 256 x 256 in whole rounds of the chip, and those behind them
   const int64_t tiles256 = ceil_div(M, 256) * ceil_div(N, 256), whole = tiles256 / cus * cus, left = tiles256 - whole;
   // <tile M, tile N, waves M, waves N, LDS ring slots, e2m1 operands>
@@ -1017,6 +1019,10 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
       return launch_gemm<256, 256, 2, 2, 2, FP4, false>(A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
     case kFewRows:
       return launch_few_rows(FP4, A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s);
+    case kFewLines: {
+      const FewLinesArgs p{A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, s};
+      return FP4 ? launch_few_lines_e2m1(p, ragged, plan.lines.octets) : launch_few_lines_e4m3(p, ragged, plan.lines.octets);
+    }
     case kSmallTiles:
       break;
   }

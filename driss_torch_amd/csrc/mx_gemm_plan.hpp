@@ -8,6 +8,7 @@
 #include <algorithm>
 
 #include "dt_host.hpp"
+#include "mx_few_lines.hpp"
 
 namespace dt {
 
@@ -25,7 +26,8 @@ enum GemmTiles {
   kTiles256ThenQuads,        // whole rounds of 256 x 256, the tiles left over as 128 x 128 quadrants
   kTiles256ThenHalves,       // or as halves
   kTiles256QuadrantSchedule,  // 256 x 256 on the other tiles' main loop (on request only)
-  kFewRows                   // the kernel for at most 64 rows (mx_few_rows.hip)
+  kFewRows,                  // the kernel for 33 to 64 rows (mx_few_rows.hip)
+  kFewLines                  // the one for at most 32 rows by whole lines, in the form that plan_few_lines gives
 };
 
 // The tiles of a product by its size, without the kernel for few rows.  variant, tail: the knobs gemm.variant and gemm.tail_quads.
@@ -127,7 +129,7 @@ inline RingPlan plan_ring(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged
   return best;
 }
 
-// What the kernel for at most 64 rows (mx_few_rows.hip) takes, in nanoseconds.  Its workgroups walk whole rows of
+// What the kernel for 33 to 64 rows (mx_few_rows.hip) takes, in nanoseconds.  Its workgroups walk whole rows of
 // B, 16 or 32 columns each, with all of A beside them: per round of the chip 2.3 us, and per step and column 5.5 ns (5.2 off
 // whole lines, where the rows do not begin on the same channels) and 1.6 ns per row of A.  columns: of a workgroup.
 inline int64_t few_rows_ns(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, int cus, int columns) {
@@ -136,35 +138,73 @@ inline int64_t few_rows_ns(bool fp4, int64_t M, int64_t N, int64_t K, bool ragge
   return 1000 + 2260 * rounds + rounds * steps * (columns * (ragged ? 52 : 55) + 16 * rows) / 10 - 8 * rows;
 }
 
-struct GemmKnobs {  // gemm.variant, gemm.tail_quads, gemm.split_k, gemm.tile_m, gemm.tile_n
-  int variant, tail, split_k, tile_m, tile_n;
+// The kernel for at most 32 rows by whole lines (mx_few_lines_kernels.hpp): octets of columns per group, and what the estimate gives in nanoseconds.
+struct FewLinesPlan {
+  int octets;
+  int64_t ns;
+};
+
+// Per round of the chip a workgroup's turns along K take what its waves take for one, or 2.3 ns per line that they ask for, and all
+// rounds together no less than B at 5.7 TB/s; per group the sums' way through LDS.  The constants are a fit to 161 problems of 1 to 32 rows, 512 to 28672
+// columns and K of 512 to 16384, both operand types, on and off whole lines, in all eight forms each, to the geometric mean of the time with B from memory and from
+// the memory-side cache: the form that it picks takes 0.3 % longer than the best one of each problem from memory and 0.7 % from the cache.
+inline FewLinesPlan plan_few_lines(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, int cus, int octets) {
+  const int64_t k_bytes = fp4 ? K / 2 : K, steps = ceil_div(k_bytes, (int64_t)kBK);
+  const int mh = (int)((M + 7) / 8), rows_tiles = (mh + 1) / 2;
+  FewLinesPlan best{0, 0};
+  for (int nh = octets ? octets : 1; nh <= (octets ? octets : 8); ++nh) {
+    const int waves = few_lines_waves(fp4, mh, nh, ragged), tiles = rows_tiles * ((nh + 1) / 2);
+    const int64_t rounds = ceil_div(few_lines_groups(N, nh), (int64_t)cus), turns = ceil_div(steps, (int64_t)waves) + (ragged ? 1 : 0);
+    const int64_t turn = std::max<int64_t>(386 + 11 * tiles * (fp4 ? 2 : 1), waves * (8 * nh + M + 4) * 227 / 100);
+    const int64_t ns = 1770 + rounds * (125 + 190 * tiles) + std::max(rounds * turns * turn, N * k_bytes * 10 / 57000);
+    if (!best.octets || ns < best.ns) best = FewLinesPlan{nh, ns};
+  }
+  return best;
+}
+
+struct GemmKnobs {  // gemm.variant, gemm.tail_quads, gemm.split_k, gemm.tile_m, gemm.tile_n, gemm.few_rows_octets
+  int variant, tail, split_k, tile_m, tile_n, octets = 0;
 };
 struct GemmPlan {
   GemmTiles tiles;
   RingPlan small;  // of kSmallTiles
+  FewLinesPlan lines = {};  // of kFewLines
 };
 
-// K counts elements; ragged: see ring_ragged; workspace_bytes 0: none; few_columns: columns of B that a workgroup of the kernel for few rows
-// takes, 0 where it cannot take the product.
-// The kernel for few rows is taken where it needs less time than the small tiles, or than reading B at 4.8 TB/s, which those never exceed.
-// (Fitted to 150 problems of 1 to 64 rows, and off whole lines to 340: at 350 others of 128 to 12000 columns drawn at random, half of them of
+// K counts elements; ragged: see ring_ragged; workspace_bytes 0: none; few_columns: columns of B that a workgroup of the kernel for at most 64 rows
+// takes, 0 where it cannot take the product; few_lines: whether the one for at most 32 can, which then stands in its place.
+// Either is taken where it needs less time than the small tiles.  Those read B at 4.8 TB/s from memory at most, and at 6.5 to 7.3 from the memory-side cache: the
+// first is also taken where it needs less than reading B at 4.8 TB/s, the second than at 5.5, which is in between (us, small tiles and by
+// whole lines, 16 x 28672 x 4096 28.0 / 19.5 and 22.8 / 19.5; with 4.8 here 18 x 21728 x 8992 is lost, 38.4 / 30.1 and 40.2 / 36.7).
+// (33 to 64 rows: fitted to 150 problems of 1 to 64 rows, and off whole lines to 340: at 350 others of 128 to 12000 columns drawn at random, half of them of
 // few columns and a long K, where the choice is close, what the two estimates pick takes 0.2 % longer than the better kernel with B from memory,
 // 13 % at most, and 1.0 % from the memory-side cache, 25 % at most, where few rows gain more.  With 6.6 ns off whole lines these were 0.25 %
 // and 1.7 %, 50 % at most: e2m1 12 x 1488 x 12064 from the cache 8.9 and 6.9 us, 1 x 168 x 10048 7.6 and 5.1, from memory 7.9 and 6.4.
-// A rule on sizes, few rows for K of 2048 and N of 1024 on with exceptions, took 27 % longer on the 150.)  How many workgroups are to
-// share K does not decide between the two; whether any may does.
-inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, size_t workspace_bytes, int cus, int few_columns, GemmKnobs knobs) {
+// A rule on sizes, few rows for K of 2048 and N of 1024 on with exceptions, took 27 % longer on the 150.
+// Up to 32 rows: of the 161 problems that plan_few_lines is fitted to, what the estimates pick takes 1.2 / 2.2 % longer than the best of the three kernels
+// (from memory / from the cache), and 0.91 / 0.91 of what it took without the kernel by whole lines.  What that one loses to the other one for few rows
+// are products of 3 to 4 us, 17 % at most from memory: e2m1 4 x 3872 x 2720 3.9 and 4.1, 15 x 2576 x 1312 3.4 and 3.7.)
+// How many workgroups are to share K does not decide between the two; whether any may does.
+inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, size_t workspace_bytes, int cus, int few_columns, GemmKnobs knobs,
+                          bool few_lines = false) {
   const auto small = [&](int split_k, int tile_m, int tile_n) {
     return GemmPlan{kSmallTiles, plan_ring(fp4, M, N, K, ragged, workspace_bytes, cus, split_k, tile_m, tile_n)};
   };
   if (knobs.variant == 1) return small(knobs.split_k, 128, 128);
   if (knobs.variant == 3) return small(knobs.split_k, knobs.tile_m, knobs.tile_n);
-  if (few_columns && knobs.variant == 9) return {kFewRows, {}};
-  if (few_columns && knobs.variant == 0) {
-    const int64_t few = few_rows_ns(fp4, M, N, K, ragged, cus, few_columns);
-    if (few < 3000 + N * (fp4 ? K / 2 : K) / 4800) return {kFewRows, {}};
+  if (few_columns && (knobs.variant == 9 || knobs.variant == 0)) {
+    GemmPlan few{kFewRows, {}};
+    int64_t few_ns = 0;
+    if (few_lines) {
+      few = {kFewLines, {}, plan_few_lines(fp4, M, N, K, ragged, cus, knobs.octets)};
+      few_ns = few.lines.ns;
+    } else {
+      few_ns = few_rows_ns(fp4, M, N, K, ragged, cus, few_columns);
+      if (few_ns < 3000 + N * (fp4 ? K / 2 : K) / 4800) return few;
+    }
+    if (knobs.variant == 9) return few;
     const GemmPlan tiles = small(knobs.split_k == 1 ? 1 : 0, 0, 0);
-    if (few < tiles.small.ns) return {kFewRows, {}};
+    if (few_ns < std::max(tiles.small.ns, few_lines ? 3000 + N * (fp4 ? K / 2 : K) / 5500 : 0)) return few;
     return knobs.split_k > 1 ? small(knobs.split_k, 0, 0) : tiles;
   }
   const GemmTiles tiles = plan_tiles(fp4, M, N, K, ragged, cus, knobs.variant, knobs.tail);

@@ -871,3 +871,32 @@ def test_mx_gemm_config5_full_size(d):
     bound = da.abs().double() @ db.abs().double().T
     assert ((got - ref).abs() <= bound * 2**-8).all()
     assert eager.compute_error(ref, got).item() > 50
+
+
+@pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
+@pytest.mark.parametrize("octets", range(1, 9))
+def test_mx_gemm_few_lines_kernel(d, cabi, octets, fp4):
+    """the kernel for at most 32 rows by whole lines, with every number of column octets per group: one step and fewer steps than waves, rows on
+    and off the lines, every count of row octets, columns that end inside an octet's chunk, several groups per workgroup; against the float64 product of the
+    dequantized operands (bound per entry: bf16's rounding, 2^-8 of sum |a||b|), equal rows of A equal, and the same bits on a second call"""
+    cabi.set_tuning("gemm.variant", 9)
+    cabi.set_tuning("gemm.few_rows_octets", octets)
+    try:
+        for M, K, N in ((1, 32, 8), (8, 128, 8 * octets), (9, 1024, 136), (16, 2048, 264), (17, 1056, 1000), (25, 4160, 72), (32, 8192, 512),
+                        (31, 96, 128 * octets + 8), (32, 256, 2048 * octets + 136), (3, 288, 4096 * octets + 40)):
+            x, w = _wide_operand((M, K), 5000 + M + octets).cuda(), _wide_operand((N, K), 5001 + K).cuda()
+            x[M - 1] = x[0]
+            if fp4:
+                (a, ba), (b, bb), op = d.mx_fp4_quantize(x, True), d.mx_fp4_quantize(w, True), d.mx_fp4_bf16
+                a_val, b_val = (co.fp4_unpack(v).double() * torch.exp2(s.double() - 127).repeat_interleave(32, dim=1)
+                                for v, s in (co.mx_fp4_quantize(t.cpu()) for t in (x, w)))
+            else:
+                (a, ba), (b, bb), op = d.mx_fp8_quantize_blocked(x), d.mx_fp8_quantize_blocked(w), d.mx_fp8_bf16
+                a_val, b_val = (co.mx_dequant(*co.mx_quantize(t.cpu())).double() for t in (x, w))
+            y = op(a, b.t(), ba, bb)
+            exact, bound = a_val @ b_val.T, a_val.abs() @ b_val.abs().T
+            assert ((y.cpu().double() - exact).abs() <= bound * 2**-8).all(), (M, K, N)
+            assert torch.equal(y[M - 1], y[0]) and torch.equal(op(a, b.t(), ba, bb), y), (M, K, N)
+    finally:
+        cabi.set_tuning("gemm.variant", 0)
+        cabi.set_tuning("gemm.few_rows_octets", 0)
