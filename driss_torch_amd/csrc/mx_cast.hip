@@ -57,6 +57,30 @@ int launch_dual_cols(const MxArgs& a, bool narrow) {
   return launch_status();
 }
 
+// Row-wise casts.  Up to 8 MiB of x in passes of one chunk (us, passes of 64 blocks -> of a chunk, blocked scales: bf16 512 x 8192 [8 MiB]
+// 3.98 -> 3.83 and 256 x 8192 3.07 -> 2.83, fp32 512 x 4096 4.06 -> 3.64; 16 MiB: bf16 1024 x 8192 6.28 and 6.55, fp32 512 x 8192 5.70
+// and 5.85; MXFP4 5.43 and 6.04).  Rows that pad the blocked scales: a workgroup per 256 words, at most one per CU.
+constexpr int64_t kSmallRowBytes = (int64_t)8 << 20;
+template <int IN, int OUT, int LAYOUT, bool BAND4, bool SMALL>
+int launch_rows_as(const MxArgs& a) {
+  constexpr int64_t kPass = SMALL ? kWave * InTraits<IN>::kVec / 32 : 64;  // blocks
+  const int64_t nblocks = a.rows * a.cols / 32, cus = device_facts().cu_count;
+  const int64_t waves = std::min(ceil_div(nblocks, kPass), cus * tuning(Knob::mx_blocks_per_cu) * (kBlock / kWave));
+  const int64_t groups = ceil_div(waves, (int64_t)(kBlock / kWave));
+  const int64_t pad_words = LAYOUT == DT_SCALE_BLOCKED && a.rows % 128 != 0 ? ceil_div(a.cols, (int64_t)128) * 128 : 0;
+  const int64_t pad_groups = std::min(ceil_div(pad_words, (int64_t)kBlock), cus);
+  mx_row_kernel<IN, OUT, LAYOUT, BAND4, SMALL><<<(unsigned)(groups + pad_groups), kBlock, 0, a.stream>>>(
+      a.x, (uint32_t)nblocks, (uint32_t)(a.cols / 32), a.data, a.scale, (uint32_t)groups);
+  return launch_status();
+}
+template <int IN, int OUT, int LAYOUT>
+int launch_rows(const MxArgs& a) {
+  if (a.rows * a.cols * InTraits<IN>::kBytes <= kSmallRowBytes) return launch_rows_as<IN, OUT, LAYOUT, false, true>(a);
+  if constexpr (LAYOUT == DT_SCALE_BLOCKED)
+    if (a.rows % 128 == 0 && a.cols % 512 == 0 && tuning(Knob::mx_row_band4)) return launch_rows_as<IN, OUT, LAYOUT, true, false>(a);
+  return launch_rows_as<IN, OUT, LAYOUT, false, false>(a);
+}
+
 template <int IN, int OUT, int LAYOUT>
 int launch_mx(const MxArgs& a) {
   constexpr int kV = InTraits<IN>::kVec;
@@ -64,20 +88,7 @@ int launch_mx(const MxArgs& a) {
   const int cus = device_facts().cu_count;
   // x only has to be aligned to its element: the kernels load it through element-aligned vector types
   if (a.axis == 1 && !a.transpose && aligned(a.data, 8) && nblocks < (1ll << 28)) {
-    const int64_t nsuper = ceil_div(nblocks, 64);
-    int64_t waves = (int64_t)cus * tuning(Knob::mx_blocks_per_cu) * (kBlock / kWave);
-    if (waves > nsuper) waves = nsuper;
-    const unsigned grid = (unsigned)ceil_div(waves, kBlock / kWave);
-    if constexpr (LAYOUT == DT_SCALE_BLOCKED) {
-      if (a.rows % 128 == 0 && a.cols % 512 == 0 && tuning(Knob::mx_row_band4)) {
-        mx_row_kernel<IN, OUT, LAYOUT, true><<<grid, kBlock, 0, a.stream>>>(a.x, (uint32_t)nblocks, (uint32_t)(a.cols / 32),
-                                                                           a.data, a.scale);
-        return launch_status();
-      }
-    }
-    mx_row_kernel<IN, OUT, LAYOUT><<<grid, kBlock, 0, a.stream>>>(a.x, (uint32_t)nblocks, (uint32_t)(a.cols / 32),
-                                                                 a.data, a.scale);
-    return launch_status();
+    return launch_rows<IN, OUT, LAYOUT>(a);
   }
   if (a.axis == 0 && a.transpose && a.cols % kV == 0 && aligned(a.data, 16) && aligned(a.scale, 4) &&
       a.rows < (1ll << 31) && a.cols < (1ll << 31) && tuning(Knob::mx_colt_via_dual)) {
@@ -252,25 +263,6 @@ extern "C" int dt_mx_fp8_quantize_dual(const void* x, int in_dtype, int64_t rows
 }
 
 namespace {
-// MXFP4: the row-wise kernel with the e2m1 output code (same walk over the blocks, same scale stores)
-template <int IN, int LAYOUT>
-int launch_mx_fp4(const MxArgs& a) {
-  const int64_t nblocks = a.rows * a.cols / 32;
-  const int64_t nsuper = ceil_div(nblocks, (int64_t)64);
-  int64_t waves = (int64_t)device_facts().cu_count * tuning(Knob::mx_blocks_per_cu) * (kBlock / kWave);
-  if (waves > nsuper) waves = nsuper;
-  const unsigned grid = (unsigned)ceil_div(waves, (int64_t)(kBlock / kWave));
-  if constexpr (LAYOUT == DT_SCALE_BLOCKED) {
-    if (a.rows % 128 == 0 && a.cols % 512 == 0 && tuning(Knob::mx_row_band4)) {
-      mx_row_kernel<IN, DT_E2M1, LAYOUT, true><<<grid, kBlock, 0, a.stream>>>(a.x, (uint32_t)nblocks, (uint32_t)(a.cols / 32),
-                                                                             a.data, a.scale);
-      return launch_status();
-    }
-  }
-  mx_row_kernel<IN, DT_E2M1, LAYOUT><<<grid, kBlock, 0, a.stream>>>(a.x, (uint32_t)nblocks, (uint32_t)(a.cols / 32), a.data,
-                                                                   a.scale);
-  return launch_status();
-}
 // blocks down the columns, payload transposed: [cols, rows/2], scales [cols, rows/32]
 template <int IN, int LAYOUT>
 int launch_mx_fp4_cols(const MxArgs& a) {
@@ -318,9 +310,9 @@ extern "C" int dt_mx_fp4_quantize(const void* x, int in_dtype, int64_t rows, int
   if (!dt::aligned(x, 16) || !dt::aligned(data, 4)) return DT_ERR_MISALIGNED;
   MxArgs a{x, rows, cols, 1, 0, static_cast<uint8_t*>(data), scale, s};
   switch (in_dtype) {
-    case DT_F32: return blocked ? launch_mx_fp4<DT_F32, DT_SCALE_BLOCKED>(a) : launch_mx_fp4<DT_F32, DT_SCALE_PLAIN>(a);
-    case DT_BF16: return blocked ? launch_mx_fp4<DT_BF16, DT_SCALE_BLOCKED>(a) : launch_mx_fp4<DT_BF16, DT_SCALE_PLAIN>(a);
-    default: return blocked ? launch_mx_fp4<DT_F16, DT_SCALE_BLOCKED>(a) : launch_mx_fp4<DT_F16, DT_SCALE_PLAIN>(a);
+    case DT_F32: return blocked ? launch_rows<DT_F32, DT_E2M1, DT_SCALE_BLOCKED>(a) : launch_rows<DT_F32, DT_E2M1, DT_SCALE_PLAIN>(a);
+    case DT_BF16: return blocked ? launch_rows<DT_BF16, DT_E2M1, DT_SCALE_BLOCKED>(a) : launch_rows<DT_BF16, DT_E2M1, DT_SCALE_PLAIN>(a);
+    default: return blocked ? launch_rows<DT_F16, DT_E2M1, DT_SCALE_BLOCKED>(a) : launch_rows<DT_F16, DT_E2M1, DT_SCALE_PLAIN>(a);
   }
 }
 

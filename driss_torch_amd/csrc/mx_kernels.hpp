@@ -165,20 +165,47 @@ __device__ __forceinline__ u32x2 ld_x8_16bit(const void* p) {
 // row -- because those are the scales that sit next to each other in the blocked layout: the 64
 // bytes of a pass then fall into 4 runs of 16 bytes instead of 16 runs of 4, which costs a
 // quarter of the memory transactions (36.8 -> 33 us at 8192 x 8192 bf16).
-template <int IN, int OUT, int LAYOUT, bool BAND4 = false>
+//
+// SMALL: a pass is one chunk, so that a tensor that is latency and nothing else spreads over LPB times as many waves and
+// none of them works through several chunks behind its first wait (us, blocked scales, with the padding's workgroups below: bf16 1 x 4096
+// 2.89 -> 1.97, 16 x 8192 2.81 -> 2.21, 64 x 8192 2.89 -> 2.35, 512 x 4096 3.24 -> 3.00; fp32 16 x 8192 3.44 -> 2.23; an empty kernel takes
+// 1.65.  In workgroups of one wave: 16 x 8192 2.14, but 256 x 8192 3.28 against 2.84).
+//
+// The first cast_groups workgroups cast, those behind them zero the padding of blocked scales.
+template <int IN, int OUT, int LAYOUT, bool BAND4 = false, bool SMALL = false>
 __global__ __launch_bounds__(kBlock) void mx_row_kernel(const void* __restrict__ x, uint32_t nblocks,
                                                         uint32_t kblocks, uint8_t* __restrict__ data,
-                                                        uint8_t* __restrict__ scale) {
+                                                        uint8_t* __restrict__ scale, uint32_t cast_groups) {
+  static_assert(!(BAND4 && SMALL), "a pass of four rows or one of a chunk");
   static_assert(!BAND4 || LAYOUT == DT_SCALE_BLOCKED, "the 4-row pass exists for the blocked layout");
   constexpr int kV = InTraits<IN>::kVec;      // elements per vector
   constexpr int LPB = 32 / kV;                // lanes per block: 4 or 8
   constexpr int BPC = kWave / LPB;            // blocks per chunk: 16 or 8
+  constexpr int CHUNKS = SMALL ? 1 : LPB;
+  constexpr uint32_t PASS = CHUNKS * BPC;     // blocks of a pass
+  if constexpr (LAYOUT == DT_SCALE_BLOCKED && !BAND4) {
+    // The rows that pad the last band of 128 are zeroed by workgroups of their own, a word (row, four blocks) per lane in
+    // address order, beside the cast.  (Behind the cast's own loads and stores, by the few workgroups that a few rows are:
+    // 1 x 4096 2.89 us where this takes 2.05, 1 x 16384 3.88 and 2.10, 16 x 8192 2.81 and 2.56; from a launch of its own
+    // another 2 us.)
+    if (blockIdx.x >= cast_groups) {
+      const uint32_t rows = nblocks / kblocks, first = rows & 127u, col_tiles = (kblocks + 3u) >> 2;
+      uint8_t* const band = scale + (uint64_t)(rows >> 7) * col_tiles * 512u;
+      // (64 bits: a single row may have 2^28 blocks, and its band 2^33 words; once per launch, outside the cast's loop)
+      for (uint64_t i = (blockIdx.x - cast_groups) * kBlock + threadIdx.x; i < (uint64_t)col_tiles * 128u;
+           i += (uint64_t)(gridDim.x - cast_groups) * kBlock) {
+        const uint32_t j = (uint32_t)i & 127u, r = (j & 3u) * 32u + (j >> 2);  // row of word j of a 512-byte tile
+        if (r >= first) reinterpret_cast<u32_byte*>(band)[i] = 0u;
+      }
+      return;
+    }
+  }
   const int lane = threadIdx.x % kWave;
   const uint32_t nvec = nblocks * LPB;
   const u32x4* v = static_cast<const u32x4*>(x);
-  const uint32_t nsuper = (nblocks + 63u) / 64u;
+  const uint32_t nsuper = (nblocks + PASS - 1u) / PASS;
   const uint32_t wave_id = (blockIdx.x * kBlock + threadIdx.x) / kWave;
-  const uint32_t nwaves = gridDim.x * (kBlock / kWave);
+  const uint32_t nwaves = cast_groups * (kBlock / kWave);
   saturate_fp8_conversions();
 
   const uint32_t segs = kblocks / 16u;                 // BAND4: 512-element segments per row
@@ -193,17 +220,17 @@ __global__ __launch_bounds__(kBlock) void mx_row_kernel(const void* __restrict__
     }
     auto vec_index = [&](int c) -> uint32_t {
       if constexpr (BAND4) return (band_row + 32u * (c & 3)) * row_vecs + seg * (16u * LPB) + (uint32_t)(c >> 2) * kWave + lane;
-      else return sc * 64u * LPB + c * kWave + lane;
+      else return sc * (PASS * LPB) + c * kWave + lane;
     };
-    u32x4 w[LPB];
+    u32x4 w[CHUNKS];
 #pragma unroll
-    for (int c = 0; c < LPB; ++c) {
+    for (int c = 0; c < CHUNKS; ++c) {
       const uint32_t vi = vec_index(c);
       w[c] = vi < nvec ? ld_x16<IN>(v + vi) : u32x4{0u, 0u, 0u, 0u};
     }
     uint32_t mybyte = 0;
 #pragma unroll
-    for (int c = 0; c < LPB; ++c) {
+    for (int c = 0; c < CHUNKS; ++c) {
       const uint32_t vi = vec_index(c);
       uint32_t m = quad_umax(vec_absmax_bits<IN>(w[c]));
       if constexpr (LPB == 8) m = umax(m, dpp<kDppRowHalfMirror>(m));
@@ -237,8 +264,8 @@ __global__ __launch_bounds__(kBlock) void mx_row_kernel(const void* __restrict__
       scale[blocked_offset(band_row + 32u * (c & 3), seg * 16u + (c >> 2) * BPC + b, kblocks >> 2)] = (uint8_t)mybyte;
       continue;
     }
-    const uint32_t g = sc * 64u + (lane % LPB) * BPC + lane / LPB;  // block index of mybyte
-    if (g < nblocks) {
+    const uint32_t g = sc * PASS + (lane % LPB) * BPC + lane / LPB;  // block index of mybyte
+    if (lane % LPB < CHUNKS && g < nblocks) {
       if constexpr (LAYOUT == DT_SCALE_BLOCKED) {
         const uint32_t r = g / kblocks, c = g - r * kblocks;
         const int64_t at = blocked_offset(r, c, (kblocks + 3) >> 2);
@@ -247,23 +274,6 @@ __global__ __launch_bounds__(kBlock) void mx_row_kernel(const void* __restrict__
           for (uint32_t k = 1; (c + k) & 3u; ++k) scale[at + k] = 0;
       } else {
         scale[g] = (uint8_t)mybyte;
-      }
-    }
-  }
-  if constexpr (LAYOUT == DT_SCALE_BLOCKED && !BAND4) {
-    // The rows that pad the last band of 128 are zeroed here, a word (row, four blocks) per lane in address
-    // order, behind the cast's own loads and stores.  A fill of the whole buffer in a launch of its own, as
-    // it was before, cost every cast of a row count that is no multiple of 128 (each decoding step) 2 us on
-    // the device and 3.5 us of the host: 64 x 1024 bf16 issued every 10.7 -> 7.1 us, and 32 x 8192 with the
-    // e2m1 product behind it 17.6 -> 13.3 us.
-    const uint32_t rows = nblocks / kblocks, first = rows & 127u;
-    if (first) {
-      const uint32_t col_tiles = (kblocks + 3u) >> 2;
-      uint8_t* const band = scale + (uint64_t)(rows >> 7) * col_tiles * 512u;
-      // (64 bits: a single row may have 2^28 blocks, and its band 2^33 words; once per launch, outside the cast's loop)
-      for (uint64_t i = blockIdx.x * kBlock + threadIdx.x; i < (uint64_t)col_tiles * 128u; i += (uint64_t)gridDim.x * kBlock) {
-        const uint32_t j = (uint32_t)i & 127u, r = (j & 3u) * 32u + (j >> 2);  // row of word j of a 512-byte tile
-        if (r >= first) reinterpret_cast<u32_byte*>(band)[i] = 0u;
       }
     }
   }

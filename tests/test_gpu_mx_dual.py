@@ -186,6 +186,23 @@ def test_transposed_column_cast_both_kernels(d, cabi, shape, in_dtype):
             assert torch.equal(util.codes(data), cd) and torch.equal(util.codes(scale), co.to_blocked(cs))
 
 
+@pytest.mark.parametrize("shape,in_dtype", [((1, 16384), torch.bfloat16), ((3, 544), torch.float32), ((1023, 4096), torch.bfloat16),
+                                            ((1024, 4096), torch.bfloat16), ((1025, 4096), torch.bfloat16), ((512, 4096), torch.float32),
+                                            ((513, 4096), torch.float32), ((1016, 4128), torch.float16)], ids=str)
+def test_row_casts_on_both_sides_of_the_small_ones(cabi, gpu_device, shape, in_dtype):
+    """Row-wise casts in passes of one chunk and of 64 blocks, on both sides of 8 MiB: payload, plain scales and blocked ones with
+    their padding, in a buffer of 0xAB, bit for bit against the oracle."""
+    R, C = shape
+    x = _wide_range(shape, 79, in_dtype)
+    g = x.to(gpu_device)
+    for cast, (data, sc) in ((cabi.mx_fp8_quantize, co.mx_quantize(x)), (cabi.mx_fp4_quantize, co.mx_fp4_quantize(x))):
+        buf = torch.full((cabi.lib().dt_blocked_scale_bytes(R, C // 32),), 0xAB, dtype=torch.uint8, device=gpu_device)
+        got, _ = cast(g, layout=cabi.SCALE_BLOCKED, scale=buf)
+        assert torch.equal(util.codes(got), data) and torch.equal(buf.cpu(), co.to_blocked(sc))
+        got, plain = cast(g)
+        assert torch.equal(util.codes(got), data) and torch.equal(plain.view(torch.uint8).cpu().flatten(), sc.flatten())
+
+
 @pytest.mark.parametrize("shape", [(1, 32), (33, 96), (127, 160), (129, 64), (32, 32), (96, 416), (160, 288), (384, 512)],
                          ids=lambda s: f"{s[0]}x{s[1]}")
 @pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
