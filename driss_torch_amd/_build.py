@@ -41,11 +41,13 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]
-# The MX kernels: the first 14 words of a kernel's arguments arrive in registers with the launch; loaded by the kernel they stand
+# The kernels of PRELOADED: the first 14 words of a kernel's arguments arrive in registers with the launch; loaded by the kernel they stand
 # in front of its first memory request.  us a launch, back to back, loaded -> preloaded: row-wise cast 1024 x 8192 bf16 5.34 -> 5.18,
 # 4096 x 4096 8.91 -> 8.73, both casts from one read 7.06 -> 6.97 and 11.34 -> 11.13; a linear layer of few rows, cast and product, e4m3 16 x
-# 8192 x 8192 16.23 -> 16.10, e2m1 32 x 8192 x 8192 12.66 -> 12.31.  (The per-tensor kernels do not gain: cast 1024 x 1024 1.78 and 1.84.)
-MX_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
+# 8192 x 8192 16.23 -> 16.10, e2m1 32 x 8192 x 8192 12.66 -> 12.31.  (The per-tensor kernels do not gain: cast 1024 x 1024 1.78 and 1.84; nor do the large tiles of the products, whose e2m1
+# halves lose 1-3 %: 1024 x 8192 x 8192 44.1 and 44.7 from memory, 39.1 and 40.9 from the memory-side cache, 525 x 6536 x 2528 18.1 and 18.4.)
+PRELOAD_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
+PRELOADED = {"mx_cast.hip", "mx_few_rows.hip", "mx_few_lines_e4m3.hip", "mx_few_lines_e2m1.hip", "mx_ring_e4m3.hip", "mx_ring_e2m1.hip"}
 
 
 def _run(cmd: list[str]) -> None:
@@ -71,7 +73,7 @@ def build_hip_library(jobs: int = 6, phase_log: bool = False) -> Path:
 
     def compile_one(src: str) -> str:
         obj = obj_dir / (Path(src).stem + ".o")
-        _run([hipcc, *flags, *(MX_FLAGS if src.startswith("mx_") else []), f"-I{INCLUDE}", f"-I{CSRC}", "-c", str(CSRC / src), "-o", str(obj)])
+        _run([hipcc, *flags, *(PRELOAD_FLAGS if src in PRELOADED else []), f"-I{INCLUDE}", f"-I{CSRC}", "-c", str(CSRC / src), "-o", str(obj)])
         return str(obj)
 
     with ThreadPoolExecutor(max_workers=jobs) as pool:
