@@ -1026,8 +1026,8 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
     case kSmallTiles:
       break;
   }
-  const RingArgs p{A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, workspace, s};
   const RingPlan& r = plan.small;
+  const RingArgs p{A, B, sfa, sfb, M, N, K, lda, ldb, out, ldo, workspace, s, r.cols};
   return FP4 ? launch_ring_e2m1(p, ragged, r.tile_m, r.tile_n, r.splits) : launch_ring_e4m3(p, ragged, r.tile_m, r.tile_n, r.splits);
 }
 

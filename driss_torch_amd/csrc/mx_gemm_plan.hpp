@@ -82,6 +82,7 @@ inline GemmTiles plan_tiles(bool fp4, int64_t M, int64_t N, int64_t K, bool ragg
 struct RingPlan {
   int tile_m, tile_n, splits;
   int64_t ns;  // what the estimate below gives, in nanoseconds
+  int cols = 0;  // of the matrix that a tile covers, see ring_cols
 };
 
 // What a CU can have under way is what this kernel's time is made of, so the tiles and shares that a product takes
@@ -127,6 +128,23 @@ inline RingPlan plan_ring(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged
     }
   }
   return best;
+}
+
+// Columns of the matrix that a tile covers.  Where whole tiles are one round and leave CUs without one, e4m3 tiles cover fewer, in eights: each CU asks for
+// fewer lines, and B from memory that is what the launch's time is made of (us, whole tiles -> here: 200 x 5120 x 5120, 160 -> 256 tiles, 22.1 -> 18.0;
+// 88 x 21328 x 8064, 167 -> 223, 50.2 -> 43.7; 358 x 3656 x 5120 22.1 -> 19.4).  From the memory-side cache the L2s' rate bounds it from some 180 workgroups on,
+// and more of them ask for A more often (378 x 5840 x 10592 in 255 tiles 36.2 -> 40.2 us), so beyond those a tile stays wider than A's rows
+// in it; and finding a tile's scales costs 0.2 us, so not where B is below 8 MiB (67 x 1288 x 1280 5.4 -> 5.1 from memory, 5.1 -> 5.3 from the cache).
+// Of 130 products of 33 to 1500 rows drawn at random 25 change, to 0.94 / 1.00 of their time (geometric average, from memory / from the cache), where the others
+// are at 0.98 / 0.99.  Not where K is shared (more is parked: 0.99 / 1.00, 1.09 at most), in several rounds (1022 x 4752 x 4928 44.8 -> 47.2) or
+// for e2m1, whose scales come 16 bytes a lane (a word a lane costs 3 to 6 %, more than this gives).
+inline int ring_cols(const RingPlan& p, bool fp4, int64_t M, int64_t N, int64_t K, int cus) {
+  const int64_t tiles_m = ceil_div(M, (int64_t)p.tile_m), tiles_n = ceil_div(N, (int64_t)p.tile_n);
+  if (fp4 || p.splits > 1 || tiles_m * tiles_n > cus || K > ((int64_t)1 << 28) || N * K < ((int64_t)8 << 20)) return p.tile_n;  // (K: two chunks' scales in 32 bits)
+  const auto for_tiles = [&](int64_t n) { return ceil_div(N, std::max(n / tiles_m, (int64_t)1)); };
+  const int64_t rows = std::min(M, (int64_t)p.tile_m), cols = std::max(for_tiles(cus), std::min(for_tiles(cus * 17 / 24), rows + 8));
+  const int fit = (int)std::max(std::min(ceil_div(cols, (int64_t)8) * 8, (int64_t)p.tile_n), (int64_t)p.tile_n / 2);
+  return 8 * ceil_div(N, (int64_t)fit) >= 9 * tiles_n ? fit : p.tile_n;
 }
 
 // What the kernel for 33 to 64 rows (mx_few_rows.hip) takes, in nanoseconds.  Its workgroups walk whole rows of
@@ -188,7 +206,9 @@ struct GemmPlan {
 inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, size_t workspace_bytes, int cus, int few_columns, GemmKnobs knobs,
                           bool few_lines = false) {
   const auto small = [&](int split_k, int tile_m, int tile_n) {
-    return GemmPlan{kSmallTiles, plan_ring(fp4, M, N, K, ragged, workspace_bytes, cus, split_k, tile_m, tile_n)};
+    GemmPlan p{kSmallTiles, plan_ring(fp4, M, N, K, ragged, workspace_bytes, cus, split_k, tile_m, tile_n)};
+    p.small.cols = ring_cols(p.small, fp4, M, N, K, cus);
+    return p;
   };
   if (knobs.variant == 1) return small(knobs.split_k, 128, 128);
   if (knobs.variant == 3) return small(knobs.split_k, knobs.tile_m, knobs.tile_n);

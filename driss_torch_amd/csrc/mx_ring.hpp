@@ -13,6 +13,7 @@ struct RingArgs {  // operands as for dt_mx_fp8_bf16 / dt_mx_fp4_bf16, already c
   int64_t ldo;
   void* workspace;
   hipStream_t stream;
+  int cols;  // of the matrix that a tile covers (ring_cols)
 };
 
 // Rows that are no whole lines of 128 bytes, or do not begin on one: the kernel's form that deals with it.
@@ -42,6 +43,16 @@ __host__ __device__ inline uint32_t ring_scale_bytes(bool fp4, int chunks, int e
 }
 __host__ __device__ inline uint32_t ring_scale_offset(bool fp4, int wave, int lane, int step) {
   return (uint32_t)step * (fp4 ? 1024u : 512u) + (fp4 ? lane * 16u : (wave & 1) * 256u + lane * 4u);
+}
+// What is added to that for e4m3 where a tile begins anywhere in a chunk: word `word` of the 128 that go to LDS is that of the tile's row
+// t = word % 4 * 32 + word / 4 (rows past the tile: the last one's), which lies in the chunk of row0 or in the next one of the matrix, so the
+// descriptor spans both.
+__host__ __device__ inline uint32_t ring_scale_shift(int row0, int rows, int chunks, int word) {
+  const int t = (word & 3) * 32 + (word >> 2), r = row0 + (t < rows ? t : rows - 1);
+  return (uint32_t)((r >> 7) - (row0 >> 7)) * ((uint32_t)chunks * 512u) + (uint32_t)((r & 31) * 16 + ((r >> 5) & 3) * 4 - word * 4);
+}
+__host__ __device__ inline uint32_t ring_scale_span(int row0, int rows, int chunks) {
+  return (uint32_t)(((row0 + rows - 1) >> 7) - (row0 >> 7)) * ((uint32_t)chunks * 512u);
 }
 
 // A panel of up to 128 rows, from one step along K on: `left` bytes of each row.  mis: bytes from the descriptor's base, a multiple of 128, to

@@ -74,7 +74,9 @@ __device__ __forceinline__ void wait_loads_and_lds() {
 // of the arguments, which are in registers when the kernel begins; lda and ldb are below 2^32 / 255, as the host has checked.  us, with tile counts and
 // pitches behind them and both divisions below on every launch -> here, B from memory / from the memory-side cache: e4m3 44 x 4568 x 4672 10.5 -> 10.1 / 8.75 ->
 // 8.54, 83 x 6936 x 4384 e2m1 9.96 -> 9.44 / 8.63 -> 8.34; 90 products drawn at random 0.98 / 0.99 of their time, e2m1 0.975 / 0.985.)
-template <int TM, int TN, bool FP4, bool SPLIT, bool RAGGED>
+// FIT (K not shared): a tile covers fewer columns than it has, in eights, and begins anywhere in a chunk of B's scales; `splits` is 256 times the tiles
+// along a row plus the columns of one.
+template <int TM, int TN, bool FP4, bool SPLIT, bool RAGGED, bool FIT>
 __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, const uint8_t* __restrict__ sfa,
     const uint8_t* __restrict__ sfb, int M, int N, int K, uint32_t lda, uint32_t ldb, int splits, uint16_t* __restrict__ out,
@@ -96,7 +98,8 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
   const int wm = wave >> 1, wn = wave & 1;
 
   int bid = blockIdx.x;
-  const int tiles_m = (int)((uint32_t)(M + BM - 1) / BM), tiles_n = (int)((uint32_t)(N + BN - 1) / BN), nb = tiles_m * tiles_n;
+  const int tiles_m = (int)((uint32_t)(M + BM - 1) / BM), n_cols = FIT ? splits & 255 : BN;
+  const int tiles_n = FIT ? splits >> 8 : (int)((uint32_t)(N + BN - 1) / BN), nb = tiles_m * tiles_n;
   int split = 0;
   if constexpr (SPLIT) {
     split = (int)((uint32_t)bid / (uint32_t)nb);
@@ -119,7 +122,8 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
     tile_n = (int)((uint32_t)bid / (uint32_t)gm);
     tile_m = first_m + bid - tile_n * gm;
   }
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  const int m0 = tile_m * BM, n0 = tile_n * n_cols;
+  const int cols = N - n0 < n_cols ? N - n0 : n_cols;
 
   const int k_bytes = FP4 ? K / 2 : K;
   const int k_steps_all = (k_bytes + kBK - 1) / kBK;
@@ -147,7 +151,7 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
     return Operand{panel, v4i{(int)(uint32_t)base, (int)((uint32_t)(base >> 32) & 0xFFFFu), 0, 0x00027000}, panel.bytes()};
   };
   Operand op_a = operand(A + (uint64_t)m0 * lda + (int64_t)ks_begin * kBK, M - m0 < BM ? M - m0 : BM, lda);
-  Operand op_b = operand(B + (uint64_t)n0 * ldb + (int64_t)ks_begin * kBK, N - n0 < BN ? N - n0 : BN, ldb);
+  Operand op_b = operand(B + (uint64_t)n0 * ldb + (int64_t)ks_begin * kBK, cols, ldb);
   uint32_t off_a[TM], off_b[TN], end_a[TM], end_b[TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
@@ -166,14 +170,17 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
   // twice the same bytes).
   const bool sc_b = FP4 ? (wave & 1) != 0 : wave >= 2;
   const uint64_t sc_base = reinterpret_cast<uint64_t>(sc_b ? sfb + (int64_t)(n0 >> 7) * k_chunks * 512 : sfa + (int64_t)(m0 >> 7) * k_chunks * 512);
-  const uint32_t bytes_s = ring_scale_bytes(FP4, k_chunks, ks_begin + k_steps);
+  uint32_t bytes_s = ring_scale_bytes(FP4, k_chunks, ks_begin + k_steps);
+  if constexpr (FIT) bytes_s += ring_scale_span(n0, cols, k_chunks) * (uint32_t)(wave >> 1);
   const v4i rsrc_s = v4i{(int)(uint32_t)sc_base, (int)((uint32_t)(sc_base >> 32) & 0xFFFFu), (int)bytes_s, 0x00027000};
   uint32_t off_s = ring_scale_offset(FP4, wave, lane, ks_begin - 1);  // a step is added for each window
+  if constexpr (FIT) off_s += ring_scale_shift(n0, cols, k_chunks, (wave & 1) * 64 + lane) * (uint32_t)(wave >> 1);
   const uint32_t lds_base = (uint32_t)(uintptr_t)(lptr_t)lds;
   const uint32_t lds_a = lds_base + wave * TM * 1024, lds_b = lds_base + kOffB + wave * TN * 1024;
   const uint32_t lds_s = lds_base + (sc_b ? kOffSB : kOffSA) + (FP4 ? 0 : (wave & 1) * 256);
 
-  // A window past the last one is asked for with empty descriptors (its scales are past the end): nothing is read, and the counts stay what they are.
+  // A window past the last one is asked for with empty descriptors (its scales are past the end, or, FIT, others of the matrix that nothing uses): nothing
+  // else is read, and the counts stay what they are.
   // Every workgroup walks K front to back, so that an entry is summed in the same order wherever in the matrix it stands.  (With half of
   // the workgroups on runs of K in another order, so that one finds in the XCD's L2 what another one fetched, whole-line products of more than two
   // rows of tiles take 6 to 13 % less from memory and the same from the memory-side cache, us, e4m3 512 x 4096 x 4096 17.7 and 16.2, 400 x 5120 x
@@ -256,7 +263,8 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
     const uint32_t ph_a = RAGGED ? ((op_a.panel.mis + (uint32_t)(l16 & 7) * lda) & 127u) >> 4 : 0u;
     const uint32_t ph_b = RAGGED ? ((op_b.panel.mis + (uint32_t)(l16 & 7) * ldb) & 127u) >> 4 : 0u;
     const uint32_t a0 = wm * TM * 2048, b0 = kOffB + wn * TN * 2048;
-    const int ta = ((m0 & 127) >> 4) + wm * TM, tb = ((n0 & 127) >> 4) + wn * TN;  // even: the first tile's number in its chunk
+    // even: the first tile's number in its chunk (FIT: B's words come in the order of the tile's columns)
+    const int ta = ((m0 & 127) >> 4) + wm * TM, tb = (FIT ? 0 : (n0 & 127) >> 4) + wn * TN;
 #pragma unroll
     for (int q = 0; q < kSets; ++q) {
       const bool last = RAGGED && q == kSetOfLast;
@@ -461,7 +469,7 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
 #pragma unroll
   for (int p = 0; p < BM / kRowsPerPass; ++p) {
     const int row = p * kRowsPerPass + erow, m = m0 + row, n = n0 + echunk * 8;
-    if (m >= M || n >= N) continue;
+    if (m >= M || n >= N || (FIT && echunk * 8 >= n_cols)) continue;
     const u32x4 v = *reinterpret_cast<const u32x4*>(lds + row * kPitch + echunk * 16);
     uint16_t* dst = out + (int64_t)m * ldo + n;
     if (wide_stores && n + 8 <= N) {
@@ -474,15 +482,15 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
 #endif
 }
 
-template <int TM, int TN, bool FP4, bool SPLIT, bool RAGGED>
+template <int TM, int TN, bool FP4, bool SPLIT, bool RAGGED, bool FIT = false>
 int launch(const RingArgs& p, int splits) {
   constexpr int BM = 32 * TM, BN = 32 * TN;
   constexpr int kLds = stages(TM, TN) * stage_bytes(TM, TN, FP4);
   static_assert(kLds + 64 <= 160 * 1024 && kLds > 82 * 1024 && kLds >= BM * (BN * 2 + 16), "one workgroup per CU; the output tile fits too");
-  const int tiles_m = (int)ceil_div(p.M, (int64_t)BM), tiles_n = (int)ceil_div(p.N, (int64_t)BN);
+  const int tiles_m = (int)ceil_div(p.M, (int64_t)BM), tiles_n = (int)ceil_div(p.N, (int64_t)(FIT ? p.cols : BN));
   const int64_t grid = (int64_t)tiles_m * tiles_n * splits;
   if (grid > 0x7FFFFFFFll) return DT_ERR_INVALID_SHAPE;
-  auto kernel = mx_ring_kernel<TM, TN, FP4, SPLIT, RAGGED>;
+  auto kernel = mx_ring_kernel<TM, TN, FP4, SPLIT, RAGGED, FIT>;
   static std::atomic<bool> allowed[16];  // once per instantiation and device
   int dev = 0;
   (void)hipGetDevice(&dev);
@@ -496,7 +504,7 @@ int launch(const RingArgs& p, int splits) {
   }
   uint8_t* const ws = static_cast<uint8_t*>(p.workspace);
   kernel<<<(unsigned)grid, kRingWaves * kWave, kLds, p.stream>>>(
-      p.a, p.b, p.sfa, p.sfb, (int)p.M, (int)p.N, (int)p.K, (uint32_t)p.lda, (uint32_t)p.ldb, splits, static_cast<uint16_t*>(p.out), p.ldo,
+      p.a, p.b, p.sfa, p.sfb, (int)p.M, (int)p.N, (int)p.K, (uint32_t)p.lda, (uint32_t)p.ldb, FIT ? tiles_n * 256 + p.cols : splits, static_cast<uint16_t*>(p.out), p.ldo,
       (p.ldo % 8 == 0 && aligned(p.out, 16)) ? 1 : 0, ws ? reinterpret_cast<v4f*>(ws + kSplitTicketBytes) : nullptr,
       reinterpret_cast<uint32_t*>(ws));
   return launch_status();
@@ -505,6 +513,8 @@ int launch(const RingArgs& p, int splits) {
 template <int TM, int TN, bool FP4>
 int launch_tile(const RingArgs& p, bool ragged, int splits) {
   if (splits > 1) return ragged ? launch<TM, TN, FP4, true, true>(p, splits) : launch<TM, TN, FP4, true, false>(p, splits);
+  if constexpr (!FP4)
+    if (p.cols != 32 * TN) return ragged ? launch<TM, TN, FP4, false, true, true>(p, 1) : launch<TM, TN, FP4, false, false, true>(p, 1);
   return ragged ? launch<TM, TN, FP4, false, true>(p, 1) : launch<TM, TN, FP4, false, false>(p, 1);
 }
 

@@ -900,3 +900,30 @@ def test_mx_gemm_few_lines_kernel(d, cabi, octets, fp4):
     finally:
         cabi.set_tuning("gemm.variant", 0)
         cabi.set_tuning("gemm.few_rows_octets", 0)
+
+
+@pytest.mark.parametrize("tile", [(64, 64), (64, 128), (128, 64), (128, 128)], ids=lambda t: f"{t[0]}x{t[1]}")
+@pytest.mark.parametrize("size", [(64, 8192, 1032), (200, 5120, 5120), (97, 8288, 1020), (300, 4192, 3004), (129, 4128, 2100), (257, 8256, 2760)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_mx_gemm_small_tiles_that_cover_fewer_columns(d, cabi, size, tile):
+    """Tiles that begin anywhere in a chunk of B's scales, on and off whole lines, with columns that end inside a tile's eight: the same bits as on
+    the 256 x 256 tiles (one order of sums), every entry within bf16's rounding of the float64 product, and nothing written past a row's end"""
+    M, K, N = size
+    x, w = _wide_operand((M, K), 6100 + M).cuda(), _wide_operand((N, K), 6101 + K).cuda()
+    (a, sa), (b, sb) = ((q, _poisoned_blocked(d, s.view(torch.uint8).view(len(q), -1))) for q, s in (d.mx_fp8_quantize(x), d.mx_fp8_quantize(w)))
+    a_val, b_val = (co.mx_dequant(*co.mx_quantize(t.cpu())).cuda().double() for t in (x, w))
+    exact, bound = a_val @ b_val.T, a_val.abs() @ b_val.abs().T
+    want = torch.full((M, N + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    out = want.clone()
+    for variant, dst in ((2, want), (3, out)):
+        cabi.set_tuning("gemm.variant", variant)
+        cabi.set_tuning("gemm.split_k", 1)
+        cabi.set_tuning("gemm.tile_m", tile[0])
+        cabi.set_tuning("gemm.tile_n", tile[1])
+        try:
+            cabi.mx_fp8_bf16(a, b, sa, sb, dst[:, :N])
+        finally:
+            for knob in ("variant", "split_k", "tile_m", "tile_n"):
+                cabi.set_tuning("gemm." + knob, 0)
+    assert torch.equal(out, want) and (out[:, N:] == 7).all()
+    assert ((out[:, :N].double() - exact).abs() <= bound * 2**-8).all()
