@@ -17,6 +17,8 @@ constexpr size_t kWsTicket = 0;             // u32 arrival counter, zero between
 constexpr size_t kWsRunning = 128;          // u32 running max of |x| bits, zero between launches
 constexpr size_t kWsAmax = 64;              // f32 amax of the last reduction
 constexpr size_t kWsScale = 68;             // f32 scale[2] derived from it
+constexpr size_t kWsPartials = 3072;        // u32 maxima of a reduction's workgroups, for the cast behind it
+constexpr int kWsPartialWords = 256;
 constexpr size_t kWsBytes = 4096;
 
 struct DeviceFacts {

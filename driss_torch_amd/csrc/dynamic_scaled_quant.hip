@@ -3,8 +3,8 @@
 // For a caller that has said that its process owns the GPU (dt_set_exclusive_gpu, DRISS_TORCH_RESIDENT=1),
 // a tensor that fits the chip's registers and LDS (128 MiB on 256 CUs) goes through one kernel
 // that holds it there between the reduction and the cast (resident_kernels.hpp).  Otherwise
-// the work is two stream-ordered kernels: the amax reduction, whose last workgroup also derives
-// the scale(s) into the workspace, and the streaming cast, which reads the scale from there;
+// the work is two stream-ordered kernels: the amax reduction, whose workgroups leave their maxima in the
+// workspace, and the streaming cast, which derives the scale(s) from them (FromPartials in quant_kernels.hpp);
 // the second read of x is then served from the memory-side cache as far as it fits.
 #include "quant_kernels.hpp"
 #include "resident_kernels.hpp"
@@ -61,11 +61,7 @@ extern "C" int dt_dynamic_scaled_quant(const void* x, int in_dtype, int64_t nume
   const int res = dt::launch_resident<false>(x, in_dtype, numel, out_dtype, round_mode, workspace, out, nullptr, amax_out,
                                              scale_out, fm, 0.f, s);
   if (res == DT_OK || res == DT_ERR_RESIDENT_GAVE_UP) return res;
-  int st = in_dtype == DT_F32 ? dt::launch_amax<DT_F32>(x, numel, workspace, amax_out, scale_out, 1, fm, 0.f, s)
-                              : dt::launch_amax<DT_BF16>(x, numel, workspace, amax_out, scale_out, 1, fm, 0.f, s);
-  if (st) return st;
-  const float* scale = reinterpret_cast<const float*>(static_cast<const uint8_t*>(workspace) + dt::kWsScale);
-  return dt::launch_cast<false>(x, in_dtype, numel, scale, out_dtype, round_mode, out, nullptr, s);
+  return dt::launch_amax_cast<false>(x, in_dtype, numel, out_dtype, round_mode, workspace, out, nullptr, amax_out, scale_out, fm, 0.f, s);
 }
 
 extern "C" int dt_dynamic_scaled_quant_noalloc(const void* x, int in_dtype, int64_t numel, int out_dtype, int round_mode,
@@ -122,9 +118,10 @@ extern "C" int dt_dynamic_scaled_quant_pair(const void* x, int in_dtype, int64_t
                                               amax_out, scale_out, 448.0f, 57344.0f, dt::as_hip(stream));
     if (res == DT_OK || res == DT_ERR_RESIDENT_GAVE_UP) return res;
   }
-  if (int st = dt_amax_scales(x, in_dtype, numel, amax_out, scale_out, workspace, workspace_bytes, stream)) return st;
-  const float* scale = reinterpret_cast<const float*>(static_cast<const uint8_t*>(workspace) + dt::kWsScale);
-  return dt::launch_cast<true>(x, in_dtype, numel, scale, DT_E4M3FN, round_mode, out_e4m3fn, out_e5m2, dt::as_hip(stream));
+  if (numel == 0) return DT_ERR_EMPTY;
+  if (int st = dt::check_workspace(workspace, workspace_bytes)) return st;
+  return dt::launch_amax_cast<true>(x, in_dtype, numel, DT_E4M3FN, round_mode, workspace, out_e4m3fn, out_e5m2, amax_out, scale_out, 448.0f,
+                                    57344.0f, dt::as_hip(stream));
 }
 
 extern "C" int dt_dynamic_scaled_quant_rowwise(const void* x, int in_dtype, int64_t rows, int64_t cols, int out_dtype,

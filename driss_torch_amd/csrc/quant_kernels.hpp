@@ -55,6 +55,8 @@ __device__ __forceinline__ uint32_t absbits_of(const void* x, int64_t i) {
 // folds it into a running maximum in the workspace with one atomic and takes a ticket; the
 // workgroup that draws the last ticket writes amax (and, when NSCALES > 0, the fp8 scales
 // derived from it) and re-arms the workspace for the next launch.
+// NSCALES = kPartials: each workgroup leaves its maximum in a word of its own, and the cast behind it does the rest (FromPartials).
+constexpr int kPartials = -1;
 template <int IN, int BLOCK, int UNROLL, int NSCALES, bool NT>
 __global__ __launch_bounds__(BLOCK) void amax_kernel(const void* __restrict__ x, Split sp,
                                                       uint8_t* __restrict__ ws, float* __restrict__ amax_out,
@@ -157,6 +159,11 @@ __global__ __launch_bounds__(BLOCK) void amax_kernel(const void* __restrict__ x,
   }
   m = block_umax<BLOCK / kWave>(m, lds);
   stamp(2);
+  if constexpr (NSCALES == kPartials) {
+    if (tid == 0) reinterpret_cast<uint32_t*>(ws + kWsPartials)[blockIdx.x] = m;
+    stamp(3);
+    return;
+  }
 
   // Publishing the tensor's maximum: amax, the scales derived from it, into the workspace and to the caller
   auto publish = [&](uint32_t bits) {
@@ -211,7 +218,8 @@ inline int reduction_grid(int64_t nvec, int block, int unroll, Knob knob) {
   return want < 1 ? 1 : (int)want;
 }
 
-// Enqueue the amax reduction.  nscales: 0 = amax only, 1 = scale for fmax0, 2 = both.
+// Enqueue the amax reduction.  nscales: 0 = amax only, 1 = scale for fmax0, 2 = both.  partials (with scales): leave the workgroups' maxima for the cast,
+// whose number goes there; without the atomics, workgroups of 256 threads on every CU are the best ones at any size.
 //
 // Streaming or cacheable loads: a cast of the same tensor follows nearly every reduction (always when
 // scales are asked for), and its workgroups walk the tensor in the reduction's order, so that a run of
@@ -231,7 +239,7 @@ inline int reduction_grid(int64_t nvec, int block, int unroll, Knob knob) {
 constexpr int64_t kAmaxCacheableBytes = (int64_t)40 << 20, kAmaxStreamedFrom = (int64_t)3 << 19, kAmaxStreamedTo = (int64_t)4 << 20;
 template <int IN>
 inline int launch_amax(const void* x, int64_t numel, void* ws, float* amax_out, float* scale_out, int nscales,
-                       float fmax0, float fmax1, hipStream_t stream) {
+                       float fmax0, float fmax1, hipStream_t stream, int* partials = nullptr) {
   constexpr int kUnroll = 8;
   Split sp = split_for_vectors<IN>(x, numel);
   // Few, large workgroups for all but the smallest and the largest tensors: a workgroup ends with two
@@ -244,17 +252,19 @@ inline int launch_amax(const void* x, int64_t numel, void* ws, float* amax_out, 
   // large workgroups stay ahead up to 96 MiB (both kernels, one output: 63 MiB 27.8 -> 26.4, 80 MiB 34.3 -> 32.4,
   // 95 MiB 40.3 -> 38.9; both outputs 47.8 -> 46.9, at 128 MiB 61.4 -> 61.7).
   const int64_t small_blocks = ceil_div(sp.nvec, (int64_t)kBlock * kUnroll);  // of 32 KiB
-  const int block = small_blocks <= 64 || small_blocks > (nscales ? 3072 : 2048) ? 256 : small_blocks <= 128 ? 512 : 1024;
+  const int block = partials || small_blocks <= 64 || small_blocks > (nscales ? 3072 : 2048) ? 256 : small_blocks <= 128 ? 512 : 1024;
   int grid = reduction_grid(sp.nvec, block, kUnroll, Knob::amax_blocks_per_cu);
   if (block == 1024) grid = std::min(grid, std::max(8, device_facts().cu_count * 5 / 64 * 8));
   uint8_t* w = static_cast<uint8_t*>(ws);
   const int64_t bytes = numel * InTraits<IN>::kBytes;
+  if (partials) *partials = grid = std::min(grid, kWsPartialWords);
   const bool nt = nscales == 0 ? bytes > kAmaxCacheableBytes || (bytes >= kAmaxStreamedFrom && bytes <= kAmaxStreamedTo)
                                : tuning(Knob::amax_stream_before_cast) != 0;
   uint64_t* const log = phase_log((size_t)grid * 32);
 #define DT_AMAX_B(NS, NT, B) amax_kernel<IN, B, kUnroll, NS, NT><<<grid, B, 0, stream>>>(x, sp, w, amax_out, scale_out, fmax0, fmax1, log)
 #define DT_AMAX(NS, NT) do { if (block == 1024) DT_AMAX_B(NS, NT, 1024); else if (block == 512) DT_AMAX_B(NS, NT, 512); else DT_AMAX_B(NS, NT, 256); } while (0)
-  if (nscales == 0) { if (nt) DT_AMAX(0, true); else DT_AMAX(0, false); }
+  if (partials) { if (nt) DT_AMAX_B(kPartials, true, 256); else DT_AMAX_B(kPartials, false, 256); }
+  else if (nscales == 0) { if (nt) DT_AMAX(0, true); else DT_AMAX(0, false); }
   else if (nscales == 1) { if (nt) DT_AMAX(1, true); else DT_AMAX(1, false); }
   else { if (nt) DT_AMAX(2, true); else DT_AMAX(2, false); }
 #undef DT_AMAX
@@ -333,15 +343,25 @@ __device__ __forceinline__ uint8_t cast_one(const void* x, int64_t i, float s) {
 // Aligned streaming cast: x 16-byte aligned, out aligned to its packed store.  The tail
 // (< one vector) is done by the first workgroup.  With PAIR the same read also feeds a
 // second output of the other fp8 type with its own scale (scale[1], out2).
-template <int IN, int OUT, bool ROUND_BF16, bool ROUND_SCALE, bool PAIR, int UNROLL>
+// Where the scale comes from when the reduction in front left its workgroups' maxima in the workspace (PARTIALS; `scale` points to them): every workgroup
+// takes their maximum while its first loads of x are under way, the first one writes amax and the scales out.  The kernel boundary is all that
+// the two kernels need between them: the reduction ends without its two dependent atomics per workgroup on one address (0.65 us each, and a queue), and
+// may have all CUs read.  us, both kernels, amax and scales by the last workgroup -> here, rotated buffers: bf16 to one type 512 x 512 5.05 -> 4.30,
+// 1024 x 4096 9.06 -> 7.06, 1024 x 8192 11.4 -> 9.2, 2048 x 8192 15.3 -> 12.7, 8192 x 4096 28.6 -> 26.9, 8192 x 8192 53.1 -> 51.6, to both 63.0 -> 61.5; fp32
+// 1024 x 8192 13.5 -> 11.1, 8192 x 8192 91.1 -> 89.8.
+struct FromPartials {
+  int count = 0;
+  float fmax0 = 0.f, fmax1 = 0.f;
+  float *amax_out = nullptr, *scale_out = nullptr;
+};
+template <int IN, int OUT, bool ROUND_BF16, bool ROUND_SCALE, bool PAIR, int UNROLL, bool PARTIALS = false>
 __global__ __launch_bounds__(kBlock) void cast_kernel(const void* __restrict__ x, int64_t nvec, int64_t tail,
                                                       const float* __restrict__ scale, uint8_t* __restrict__ out,
-                                                      uint8_t* __restrict__ out2) {
+                                                      uint8_t* __restrict__ out2, FromPartials from) {
   constexpr int kV = InTraits<IN>::kVec;
   constexpr int OUT2 = OUT == DT_E4M3FN ? DT_E5M2 : DT_E4M3FN;
   saturate_fp8_conversions();
-  float s = scale[0], s2 = PAIR ? scale[1] : 0.f;
-  if constexpr (ROUND_SCALE) { s = round_to_bf16(s); s2 = round_to_bf16(s2); }
+  float s, s2 = 0.f;
   const u32x4* v = static_cast<const u32x4*>(x);
   // batches of UNROLL loads, software-pipelined over two register sets (see amax_kernel)
   constexpr int P = UNROLL;
@@ -359,9 +379,46 @@ __global__ __launch_bounds__(kBlock) void cast_kernel(const void* __restrict__ x
       if constexpr (PAIR) cast_vec<IN, OUT2, ROUND_BF16>(w[u], s2, out2, j + u * stride);
     }
   };
+  u32x4 wa[P], wb[P];
+  if constexpr (PARTIALS) {
+    static_assert(kWsPartialWords <= kBlock, "a word per thread");
+    __shared__ uint32_t lds[kBlock / kWave];
+    uint32_t m = (int)threadIdx.x < from.count ? reinterpret_cast<const uint32_t*>(scale)[threadIdx.x] : 0u;
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+      const int64_t j = i + u * stride;
+      wa[u] = ld_stream(v + (j < nvec ? j : nvec - 1));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    m = block_umax<kBlock / kWave>(m, lds);
+    const float amax = as_f32(m);
+    s = amax_to_scale(amax, from.fmax0);
+    if constexpr (PAIR) s2 = amax_to_scale(amax, from.fmax1);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      if (from.amax_out) *from.amax_out = amax;
+      if (from.scale_out) {
+        from.scale_out[0] = s;
+        if constexpr (PAIR) from.scale_out[1] = s2;
+      }
+    }
+  } else {
+    s = scale[0];
+    if constexpr (PAIR) s2 = scale[1];
+  }
+  if constexpr (ROUND_SCALE) { s = round_to_bf16(s); s2 = round_to_bf16(s2); }
+  if (PARTIALS && !whole_batch_at(i)) {
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+      const int64_t j = i + u * stride;
+      if (j < nvec) {
+        cast_vec<IN, OUT, ROUND_BF16>(wa[u], s, out, j);
+        if constexpr (PAIR) cast_vec<IN, OUT2, ROUND_BF16>(wa[u], s2, out2, j);
+      }
+    }
+    i = nvec;
+  }
   if (whole_batch_at(i)) {
-    u32x4 wa[P], wb[P];
-    load_batch(wa, i);
+    if constexpr (!PARTIALS) load_batch(wa, i);
     for (;;) {
       if (!whole_batch_at(i + step)) { cast_batch(wa, i); i += step; break; }
       load_batch(wb, i + step);
@@ -427,9 +484,15 @@ __global__ __launch_bounds__(kBlock) void cast_kernel_unaligned(const void* __re
   }
 }
 
+template <int IN>
+inline bool cast_takes_vectors(const void* x, const void* out, const void* out2) {
+  constexpr size_t kStoreAlign = IN == DT_F32 ? 4 : 8;
+  return aligned(x, 16) && aligned(out, kStoreAlign) && aligned(out2, kStoreAlign);  // (none: aligned)
+}
+
 template <int IN, int OUT, bool ROUND_BF16, bool ROUND_SCALE, bool PAIR>
 inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, void* out, void* out2,
-                            hipStream_t stream) {
+                            hipStream_t stream, const FromPartials& from) {
   // Large tensors: batches of 4 loads per lane, software-pipelined (4..8 in flight), from ONE workgroup per
   // CU: the best point of the measured grid {1, 2, 4 workgroups per CU} (8192^2 bf16 32.5 / 32.9 / 36.0 us,
   // fp32 54.2 / 60.1 / 66 us, bf16 to both fp8 types 45.1 / 45.3 / 47.8 us); more in flight is slower.
@@ -437,11 +500,9 @@ inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, vo
   // drain) weigh more: batches of 2 from three workgroups per CU, which reach their full rate sooner
   // (us, rotated buffers, batches of 4 and 1 workgroup per CU against this: bf16 4096^2 10.1 -> 9.6,
   // 2048^2 4.2 -> 3.9; no difference from 64 MiB on).  The knobs force either (0 = by size).
-  constexpr size_t kStoreAlign = IN == DT_F32 ? 4 : 8;
   uint8_t* o = static_cast<uint8_t*>(out);
   uint8_t* o2 = static_cast<uint8_t*>(out2);
-  const bool fast = aligned(x, 16) && aligned(out, kStoreAlign) && (!PAIR || aligned(out2, kStoreAlign));
-  if (fast) {
+  if (cast_takes_vectors<IN>(x, out, out2)) {
     const int64_t nvec = numel / InTraits<IN>::kVec, tail = numel % InTraits<IN>::kVec;
     const bool small = nvec * 16 < (int64_t)64 << 20;
     const int unroll_knob = tuning(Knob::cast_unroll);
@@ -455,8 +516,10 @@ inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, vo
     // with 46 and 734 workgroups, 7.9 with 48 and 736)
     if (grid > 8) grid = ceil_div(grid, (int64_t)8) * 8;
     if (grid < 1) grid = 1;
-    if (unroll == 2) cast_kernel<IN, OUT, ROUND_BF16, ROUND_SCALE, PAIR, 2><<<(unsigned)grid, kBlock, 0, stream>>>(x, nvec, tail, scale, o, o2);
-    else cast_kernel<IN, OUT, ROUND_BF16, ROUND_SCALE, PAIR, 4><<<(unsigned)grid, kBlock, 0, stream>>>(x, nvec, tail, scale, o, o2);
+#define DT_CAST_AS(U, P) cast_kernel<IN, OUT, ROUND_BF16, ROUND_SCALE, PAIR, U, P><<<(unsigned)grid, kBlock, 0, stream>>>(x, nvec, tail, scale, o, o2, from)
+    if (from.count) { if (unroll == 2) DT_CAST_AS(2, true); else DT_CAST_AS(4, true); }
+    else { if (unroll == 2) DT_CAST_AS(2, false); else DT_CAST_AS(4, false); }
+#undef DT_CAST_AS
   } else {
     int64_t grid = ceil_div(numel / InTraits<IN>::kVec, (int64_t)kBlock);
     if (grid > device_facts().cu_count) grid = device_facts().cu_count;
@@ -470,8 +533,8 @@ inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, vo
 // other fp8 type with scale[1].
 template <bool PAIR>
 inline int launch_cast(const void* x, int in_dtype, int64_t numel, const float* scale, int out_dtype,
-                       int round_mode, void* out, void* out2, hipStream_t stream) {
-#define DT_CAST(IN, OUT, RB, RS) return launch_cast_impl<IN, OUT, RB, RS, PAIR>(x, numel, scale, out, out2, stream)
+                       int round_mode, void* out, void* out2, hipStream_t stream, const FromPartials& from = {}) {
+#define DT_CAST(IN, OUT, RB, RS) return launch_cast_impl<IN, OUT, RB, RS, PAIR>(x, numel, scale, out, out2, stream, from)
   if (in_dtype == DT_F32) {
     if (out_dtype == DT_E4M3FN) DT_CAST(DT_F32, DT_E4M3FN, false, false);
     DT_CAST(DT_F32, DT_E5M2, false, false);
@@ -487,6 +550,23 @@ inline int launch_cast(const void* x, int in_dtype, int64_t numel, const float* 
   if (out_dtype == DT_E4M3FN) DT_CAST(DT_BF16, DT_E4M3FN, true, true);
   DT_CAST(DT_BF16, DT_E5M2, true, true);
 #undef DT_CAST
+}
+
+// The amax reduction and the cast with the scales derived from it.  (Not a vector long, or off the cast's alignments: the last workgroup of the reduction
+// makes the scales.)
+template <bool PAIR>
+inline int launch_amax_cast(const void* x, int in_dtype, int64_t numel, int out_dtype, int round_mode, void* ws, void* out, void* out2,
+                            float* amax_out, float* scale_out, float fmax0, float fmax1, hipStream_t stream) {
+  const bool f32 = in_dtype == DT_F32;
+  int partials = 0;
+  const bool direct = numel >= 8 && (f32 ? cast_takes_vectors<DT_F32>(x, out, out2) : cast_takes_vectors<DT_BF16>(x, out, out2));
+  const int nscales = PAIR ? 2 : 1;
+  const int st = f32 ? launch_amax<DT_F32>(x, numel, ws, amax_out, scale_out, nscales, fmax0, fmax1, stream, direct ? &partials : nullptr)
+                     : launch_amax<DT_BF16>(x, numel, ws, amax_out, scale_out, nscales, fmax0, fmax1, stream, direct ? &partials : nullptr);
+  if (st) return st;
+  const uint8_t* const w = static_cast<const uint8_t*>(ws);
+  const float* scale = reinterpret_cast<const float*>(w + (direct ? kWsPartials : kWsScale));
+  return launch_cast<PAIR>(x, in_dtype, numel, scale, out_dtype, round_mode, out, out2, stream, FromPartials{partials, fmax0, fmax1, amax_out, scale_out});
 }
 
 inline int check_cast_args(const void* x, int in_dtype, int64_t numel, int out_dtype, int round_mode, const void* out) {

@@ -284,6 +284,30 @@ def test_dynamic_quant_config2_full_size(d):
 
 
 @pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("numel", [1, 3, 4, 7, 8, 9, 15, 2047, 2051, 16384, 16391, 131080, 524288, 600007, 4194304, 4194312, 4300001], ids=str)
+def test_dynamic_quant_scale_from_workgroup_maxima(d, cabi, numel, in_dtype):
+    """the cast takes the reduction's maxima itself: the largest element in the first place, in the last and in between, a NaN in the last, a
+    larger tensor's maxima still in the workspace, an input off its vectors (the other way to the scale), and nothing written past the end"""
+    cabi.dynamic_scaled_quant(torch.full((4200000,), 1e30, dtype=in_dtype, device="cuda"), FP8[0], 3)
+    a = util.student_t((numel + 1,), 1700 + numel % 97, in_dtype)[1:].clone()
+    for at, value in ((0, 1000.0), (numel - 1, -3000.0), (numel // 2, 1e5), (numel - 1, float("nan"))):
+        a[at] = value
+        mode = 2 if in_dtype == torch.bfloat16 else 3
+        for off in (0, 1):
+            buf = torch.zeros(numel + 8, dtype=in_dtype, device="cuda")
+            x = buf[off:off + numel]
+            x.copy_(a)
+            outs = [torch.full((numel + 64,), 0xAB, dtype=torch.uint8, device="cuda") for _ in FP8]
+            o4, o5, amax, scales = cabi.dynamic_scaled_quant_pair(x, mode, outs[0][:numel].view(FP8[0]), outs[1][:numel].view(FP8[1]))
+            for i, fp8 in enumerate(FP8):
+                ref, ramax, rscale = co.dynamic_scaled_quant(a, fp8, mode)
+                out, amax1, scale1 = cabi.dynamic_scaled_quant(x, fp8, mode)
+                assert torch.equal(util.codes(out), ref) and torch.equal(outs[i][:numel].cpu(), ref) and (outs[i][numel:] == 0xAB).all()
+                for got, want in ((amax, ramax), (amax1, ramax), (scale1, rscale), (scales[i:i + 1], rscale)):
+                    assert torch.equal(got.cpu().view(torch.int32), want.view(torch.int32)) or (got.isnan().all() and want.isnan().all())
+
+
+@pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("vecs", [1, 131072, 262144, 524288, 1048576, 4194304], ids=str)
 def test_amax_between_workgroup_sizes(d, in_dtype, vecs):
     """Tensors of as many 16-byte vectors as the largest that take workgroups of 256, 512, 1024 threads (and few of them), and one
