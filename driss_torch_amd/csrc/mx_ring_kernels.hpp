@@ -238,12 +238,6 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
     }
   };
 
-  v4f acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-
   // ---- fragments and scales of the step in ring slot U
   v8i fa[TM], fb[2][TN];
   int sa[2][KC][TM], sb[2][KC][TN];
@@ -333,6 +327,16 @@ __global__ __launch_bounds__(kRingWaves* kWave) void mx_ring_kernel(
     each(one, std::make_integer_sequence<int, kLoads>{});
   };
   each(first, std::make_integer_sequence<int, kStages>{});
+  // acc becomes zero here, under the first loads.  Each tile's zeros are made values of their own: of one zero for all of them the compiler makes
+  // copies in front of the loop, the last of them in the wait states that the first MFMA, whose statement it does not look into, needs behind it.
+  v4f acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+      asm volatile("" : "+v"(acc[i][j]));
+    }
   wait_loads_and_lds<(kStages - kAhead) * kLoads>();
   __syncthreads();
   read_scales(0, 0);
