@@ -115,7 +115,7 @@ int dt_workspace_init(void* workspace, size_t workspace_bytes, dt_stream_t strea
   if (workspace_bytes < dt::kWsBytes) return DT_ERR_WORKSPACE;
   if (!dt::aligned(workspace, 256)) return DT_ERR_MISALIGNED;
   // a fill kernel rather than hipMemsetAsync, so the call is safe under graph capture
-  dt::zero_words_kernel<<<dt::kWsBytes / 4 / 256, 256, 0, dt::as_hip(stream)>>>(static_cast<uint32_t*>(workspace), dt::kWsBytes / 4);
+  dt::launcher(dt::zero_words_kernel, dt::kWsBytes / 4 / 256, 256, 0, dt::as_hip(stream))(static_cast<uint32_t*>(workspace), dt::kWsBytes / 4);
   return dt::launch_status();
 }
 

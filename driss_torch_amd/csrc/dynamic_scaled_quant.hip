@@ -75,7 +75,7 @@ extern "C" int dt_dynamic_scaled_quant_noalloc(const void* x, int in_dtype, int6
   hipStream_t s = dt::as_hip(stream);
   // The array keeps whatever the last call on this device left in it.  A completed call leaves its
   // counters at zero, but one that was cut short would not: start from zero every time.
-  clear_scratch_kernel<<<dt::kWsBytes / 4 / 256, 256, 0, s>>>(reinterpret_cast<uint32_t*>(ws));
+  dt::launcher(clear_scratch_kernel, dt::kWsBytes / 4 / 256, 256, 0, s)(reinterpret_cast<uint32_t*>(ws));
   if (int e = dt::launch_status()) return e;
   const float fm = fmax_of(out_dtype);
   st = in_dtype == DT_F32 ? dt::launch_amax<DT_F32>(x, numel, ws, amax_out, scale_out, 1, fm, 0.f, s)

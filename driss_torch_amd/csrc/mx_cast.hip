@@ -9,7 +9,7 @@ using namespace dt;
 int zero_blocked_padding(uint8_t* scale, int64_t SR, int64_t SC, hipStream_t s) {
   if (SR % 128 == 0 && SC % 4 == 0) return DT_OK;  // the cast writes every byte
   const int64_t n = dt_blocked_scale_bytes(SR, SC);
-  fill_bytes_kernel<<<(unsigned)std::min<int64_t>(ceil_div(n, 256), 4096), 256, 0, s>>>(scale, n, 0);
+  launcher(fill_bytes_kernel, (unsigned)std::min<int64_t>(ceil_div(n, 256), 4096), 256, 0, s)(scale, n, 0);
   return launch_status();
 }
 
@@ -44,15 +44,15 @@ int launch_dual_cols(const MxArgs& a, bool narrow) {
     order = narrow && narrow_tiles > 8 * cus ? 0 : a.rows % (8 * kDualRows) == 0 ? 2 : a.cols < a.rows ? 1 : 0;
   if (tiles > 0x7FFFFFFFll) return kNotTaken;
   if (narrow)
-    mx_dual_kernel<IN, OUT, LAYOUT, false, false, 8><<<(unsigned)narrow_tiles, kBlock, 0, a.stream>>>(
+    launcher(mx_dual_kernel<IN, OUT, LAYOUT, false, false, 8>, (unsigned)narrow_tiles, kBlock, 0, a.stream)(
         a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
   else if constexpr (IN == DT_F32 && OUT == DT_E2M1)
     return kNotTaken;  // mx_col_t_kernel is the better one, see plan_fp4_cols
   else if (pipe_grid > 0 && tiles > pipe_grid)
-    mx_dual_kernel<IN, OUT, LAYOUT, false, true><<<(unsigned)pipe_grid, kBlock, 0, a.stream>>>(
+    launcher(mx_dual_kernel<IN, OUT, LAYOUT, false, true>, (unsigned)pipe_grid, kBlock, 0, a.stream)(
         a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
   else
-    mx_dual_kernel<IN, OUT, LAYOUT, false><<<(unsigned)tiles, kBlock, 0, a.stream>>>(
+    launcher(mx_dual_kernel<IN, OUT, LAYOUT, false>, (unsigned)tiles, kBlock, 0, a.stream)(
         a.x, (uint32_t)a.rows, (uint32_t)a.cols, nullptr, nullptr, a.data, a.scale, order);
   return launch_status();
 }
@@ -69,7 +69,7 @@ int launch_rows_as(const MxArgs& a) {
   const int64_t groups = ceil_div(waves, (int64_t)(kBlock / kWave));
   const int64_t pad_words = LAYOUT == DT_SCALE_BLOCKED && a.rows % 128 != 0 ? ceil_div(a.cols, (int64_t)128) * 128 : 0;
   const int64_t pad_groups = std::min(ceil_div(pad_words, (int64_t)kBlock), cus);
-  mx_row_kernel<IN, OUT, LAYOUT, BAND4, SMALL><<<(unsigned)(groups + pad_groups), kBlock, 0, a.stream>>>(
+  launcher(mx_row_kernel<IN, OUT, LAYOUT, BAND4, SMALL>, (unsigned)(groups + pad_groups), kBlock, 0, a.stream)(
       a.x, (uint32_t)nblocks, (uint32_t)(a.cols / 32), a.data, a.scale, (uint32_t)groups);
   return launch_status();
 }
@@ -100,7 +100,7 @@ int launch_mx(const MxArgs& a) {
       a.rows < (1ll << 31) && a.cols < (1ll << 31)) {
     const int64_t tiles = ceil_div(a.rows, (int64_t)kColTRows) * ceil_div(a.cols, (int64_t)kColTCols);
     if (tiles <= 0x7FFFFFFFll) {
-      mx_col_t_kernel<IN, OUT, LAYOUT><<<(unsigned)tiles, kBlock, 0, a.stream>>>(a.x, (uint32_t)a.rows, (uint32_t)a.cols,
+      launcher(mx_col_t_kernel<IN, OUT, LAYOUT>, (unsigned)tiles, kBlock, 0, a.stream)(a.x, (uint32_t)a.rows, (uint32_t)a.cols,
                                                                               a.data, a.scale);
       return launch_status();
     }
@@ -111,7 +111,7 @@ int launch_mx(const MxArgs& a) {
     if (tiles <= 0x7FFFFFFFll) {
       int64_t grid = (int64_t)cus * tuning(Knob::mx_col_blocks_per_cu);
       if (grid > tiles) grid = tiles;
-      mx_col_kernel<IN, OUT><<<(unsigned)grid, kBlock, 0, a.stream>>>(a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data,
+      launcher(mx_col_kernel<IN, OUT>, (unsigned)grid, kBlock, 0, a.stream)(a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data,
                                                                      a.scale, (uint32_t)tiles);
       return launch_status();
     }
@@ -122,7 +122,7 @@ int launch_mx(const MxArgs& a) {
         a.rows < (1ll << 31) && a.cols < (1ll << 31)) {
       const int64_t tiles = ceil_div(a.rows, (int64_t)kDualRows) * ceil_div(a.cols, (int64_t)(32 * kV));
       if (tiles <= 0x7FFFFFFFll) {
-        mx_row_t_kernel<IN, OUT><<<(unsigned)tiles, kBlock, 0, a.stream>>>(a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data,
+        launcher(mx_row_t_kernel<IN, OUT>, (unsigned)tiles, kBlock, 0, a.stream)(a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data,
                                                                           a.scale);
         return launch_status();
       }
@@ -145,7 +145,7 @@ int launch_mx(const MxArgs& a) {
   if constexpr (LAYOUT == DT_SCALE_BLOCKED) {
     if (int st = zero_blocked_padding(a.scale, outer, inner_blocks, a.stream)) return st;
   }
-  mx_any_kernel<IN, OUT, LAYOUT><<<(unsigned)ceil_div(total, kBlock), kBlock, 0, a.stream>>>(
+  launcher(mx_any_kernel<IN, OUT, LAYOUT>, (unsigned)ceil_div(total, kBlock), kBlock, 0, a.stream)(
       a.x, outer, inner_blocks, xos, xes, dos, des, s_rows, s_cols, s_t, a.data, a.scale);
   return launch_status();
 }
@@ -180,13 +180,13 @@ int launch_dual_tiles(const DualArgs& a) {
   const int order = tuning(Knob::mx_dual_order) >= 0 ? tuning(Knob::mx_dual_order) : pair_order(IN == DT_F32, OUT == DT_E2M1, narrow, a.rows, a.cols, cus);
   if constexpr (IN != DT_F32) {
     if (narrow) {
-      mx_dual_kernel<IN, OUT, LAYOUT, true, false, 8><<<(unsigned)narrow_tiles, kBlock, 0, a.stream>>>(
+      launcher(mx_dual_kernel<IN, OUT, LAYOUT, true, false, 8>, (unsigned)narrow_tiles, kBlock, 0, a.stream)(
           a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data_r, a.scale_r, a.data_c, a.scale_c, order);
       return launch_status();
     }
   }
   if (tiles > 0x7FFFFFFFll) return kNotTaken;
-  mx_dual_kernel<IN, OUT, LAYOUT><<<(unsigned)tiles, kBlock, 0, a.stream>>>(a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data_r,
+  launcher(mx_dual_kernel<IN, OUT, LAYOUT>, (unsigned)tiles, kBlock, 0, a.stream)(a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data_r,
                                                                            a.scale_r, a.data_c, a.scale_c, order);
   return launch_status();
 }
@@ -277,7 +277,7 @@ int launch_mx_fp4_cols(const MxArgs& a) {
   }
   const int64_t tiles = ceil_div(a.rows, (int64_t)kColTRows) * ceil_div(a.cols, (int64_t)kColTCols);
   if (tiles > 0x7FFFFFFFll) return DT_ERR_INVALID_SHAPE;
-  mx_col_t_kernel<IN, DT_E2M1, LAYOUT><<<(unsigned)tiles, kBlock, 0, a.stream>>>(a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data,
+  launcher(mx_col_t_kernel<IN, DT_E2M1, LAYOUT>, (unsigned)tiles, kBlock, 0, a.stream)(a.x, (uint32_t)a.rows, (uint32_t)a.cols, a.data,
                                                                                 a.scale);
   return launch_status();
 }
@@ -363,8 +363,8 @@ extern "C" int dt_to_blocked(const uint8_t* scale, int64_t R, int64_t C, uint8_t
   const int64_t groups = dt_blocked_scale_bytes(R, C) / 16;
   if (dt::ceil_div(R * C, 256) > 0x7FFFFFFFll) return DT_ERR_INVALID_SHAPE;
   const unsigned grid = (unsigned)std::min<int64_t>(dt::ceil_div(groups, (int64_t)dt::kBlock), (int64_t)dt::device_facts().cu_count * 16);
-  if (R * C < 4) dt::to_blocked_kernel<true, uint32_t><<<grid, dt::kBlock, 0, s>>>(scale, R, C, groups, out);
-  else if ((groups >> 5) <= 0xFFFFFFFFll) dt::to_blocked_kernel<false, uint32_t><<<grid, dt::kBlock, 0, s>>>(scale, R, C, groups, out);
-  else dt::to_blocked_kernel<false, uint64_t><<<grid, dt::kBlock, 0, s>>>(scale, R, C, groups, out);
+  if (R * C < 4) dt::launcher(dt::to_blocked_kernel<true, uint32_t>, grid, dt::kBlock, 0, s)(scale, R, C, groups, out);
+  else if ((groups >> 5) <= 0xFFFFFFFFll) dt::launcher(dt::to_blocked_kernel<false, uint32_t>, grid, dt::kBlock, 0, s)(scale, R, C, groups, out);
+  else dt::launcher(dt::to_blocked_kernel<false, uint64_t>, grid, dt::kBlock, 0, s)(scale, R, C, groups, out);
   return dt::launch_status();
 }

@@ -317,7 +317,7 @@ int launch(const FewLinesArgs& p) {
     if (tracked) allowed[dev].store(true, std::memory_order_relaxed);
   }
   const int64_t groups = few_lines_groups(p.N, NH), cus = device_facts().cu_count;
-  kernel<<<(unsigned)(groups < cus ? groups : cus), kWaves * kWave, kLds, p.stream>>>(
+  launcher(kernel, (unsigned)(groups < cus ? groups : cus), kWaves * kWave, kLds, p.stream)(
       p.a, p.b, p.sfa, p.sfb, (int)p.M, (int)p.N, (int)p.K, (uint32_t)p.lda, (uint32_t)p.ldb, (int)groups, static_cast<uint16_t*>(p.out), p.ldo);
   return launch_status();
 }

@@ -381,7 +381,7 @@ int launch_instance(const uint8_t* a, const uint8_t* b, const uint8_t* sfa, cons
       if (tracked) allowed[dev].store(true, std::memory_order_relaxed);
     }
   }
-  kernel<<<(unsigned)grid, kFewWaves * kWave, kLds, stream>>>(a, b, sfa, sfb, (int)M, (int)N, (int)K, lda, ldb, out, ldo, (int)groups,
+  launcher(kernel, (unsigned)grid, kFewWaves * kWave, kLds, stream)(a, b, sfa, sfb, (int)M, (int)N, (int)K, lda, ldb, out, ldo, (int)groups,
                                                             stagger);
   return launch_status();
 }

@@ -19,7 +19,7 @@ extern "C" int dt_mx_gemm_workspace_init(void* workspace, size_t workspace_bytes
   if (workspace_bytes < dt::kSplitTicketBytes) return DT_ERR_WORKSPACE;
   if (!dt::aligned(workspace, 256)) return DT_ERR_MISALIGNED;
   // a fill kernel rather than hipMemsetAsync, so the call is safe under graph capture
-  dt::zero_tickets_kernel<<<1, dt::kSplitTicketBytes / 4, 0, dt::as_hip(stream)>>>(static_cast<uint32_t*>(workspace));
+  dt::launcher(dt::zero_tickets_kernel, 1, dt::kSplitTicketBytes / 4, 0, dt::as_hip(stream))(static_cast<uint32_t*>(workspace));
   return dt::launch_status();
 }
 

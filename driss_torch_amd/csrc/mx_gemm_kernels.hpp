@@ -949,7 +949,7 @@ int launch_gemm_impl(const uint8_t* a, const uint8_t* b, const uint8_t* sfa, con
   }
   int64_t grid = (int64_t)tiles_m * tiles_n;
   if (blocks > 0) grid = kParts ? (MODE == kQuads ? 32 : 16) * ceil_div(blocks, (int64_t)8) : blocks;
-  kernel<<<(unsigned)grid, WAVES_M * WAVES_N * kWave, lds_bytes, stream>>>(
+  launcher(kernel, (unsigned)grid, WAVES_M * WAVES_N * kWave, lds_bytes, stream)(
       a, b, sfa, sfb, (int)M, (int)N, (int)K, lda, ldb, static_cast<uint16_t*>(out), ldo, tiles_m, tiles_n,
       (ldo % 8 == 0 && aligned(out, 16)) ? 1 : 0, first_block, phase_log((size_t)grid * 64));
   return launch_status();

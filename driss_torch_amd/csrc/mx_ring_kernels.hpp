@@ -507,7 +507,7 @@ int launch(const RingArgs& p, int splits) {
     if (tracked) allowed[dev].store(true, std::memory_order_relaxed);
   }
   uint8_t* const ws = static_cast<uint8_t*>(p.workspace);
-  kernel<<<(unsigned)grid, kRingWaves * kWave, kLds, p.stream>>>(
+  launcher(kernel, (unsigned)grid, kRingWaves * kWave, kLds, p.stream)(
       p.a, p.b, p.sfa, p.sfb, (int)p.M, (int)p.N, (int)p.K, (uint32_t)p.lda, (uint32_t)p.ldb, FIT ? tiles_n * 256 + p.cols : splits, static_cast<uint16_t*>(p.out), p.ldo,
       (p.ldo % 8 == 0 && aligned(p.out, 16)) ? 1 : 0, ws ? reinterpret_cast<v4f*>(ws + kSplitTicketBytes) : nullptr,
       reinterpret_cast<uint32_t*>(ws));

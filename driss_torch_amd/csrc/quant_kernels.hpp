@@ -261,7 +261,7 @@ inline int launch_amax(const void* x, int64_t numel, void* ws, float* amax_out, 
   const bool nt = nscales == 0 ? bytes > kAmaxCacheableBytes || (bytes >= kAmaxStreamedFrom && bytes <= kAmaxStreamedTo)
                                : tuning(Knob::amax_stream_before_cast) != 0;
   uint64_t* const log = phase_log((size_t)grid * 32);
-#define DT_AMAX_B(NS, NT, B) amax_kernel<IN, B, kUnroll, NS, NT><<<grid, B, 0, stream>>>(x, sp, w, amax_out, scale_out, fmax0, fmax1, log)
+#define DT_AMAX_B(NS, NT, B) launcher(amax_kernel<IN, B, kUnroll, NS, NT>, grid, B, 0, stream)(x, sp, w, amax_out, scale_out, fmax0, fmax1, log)
 #define DT_AMAX(NS, NT) do { if (block == 1024) DT_AMAX_B(NS, NT, 1024); else if (block == 512) DT_AMAX_B(NS, NT, 512); else DT_AMAX_B(NS, NT, 256); } while (0)
   if (partials) { if (nt) DT_AMAX_B(kPartials, true, 256); else DT_AMAX_B(kPartials, false, 256); }
   else if (nscales == 0) { if (nt) DT_AMAX(0, true); else DT_AMAX(0, false); }
@@ -516,7 +516,7 @@ inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, vo
     // with 46 and 734 workgroups, 7.9 with 48 and 736)
     if (grid > 8) grid = ceil_div(grid, (int64_t)8) * 8;
     if (grid < 1) grid = 1;
-#define DT_CAST_AS(U, P) cast_kernel<IN, OUT, ROUND_BF16, ROUND_SCALE, PAIR, U, P><<<(unsigned)grid, kBlock, 0, stream>>>(x, nvec, tail, scale, o, o2, from)
+#define DT_CAST_AS(U, P) launcher(cast_kernel<IN, OUT, ROUND_BF16, ROUND_SCALE, PAIR, U, P>, (unsigned)grid, kBlock, 0, stream)(x, nvec, tail, scale, o, o2, from)
     if (from.count) { if (unroll == 2) DT_CAST_AS(2, true); else DT_CAST_AS(4, true); }
     else { if (unroll == 2) DT_CAST_AS(2, false); else DT_CAST_AS(4, false); }
 #undef DT_CAST_AS
@@ -524,7 +524,7 @@ inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, vo
     int64_t grid = ceil_div(numel / InTraits<IN>::kVec, (int64_t)kBlock);
     if (grid > device_facts().cu_count) grid = device_facts().cu_count;
     if (grid < 1) grid = 1;
-    cast_kernel_unaligned<IN, OUT, ROUND_BF16, ROUND_SCALE, PAIR><<<(unsigned)grid, kBlock, 0, stream>>>(x, numel, scale, o, o2);
+    launcher(cast_kernel_unaligned<IN, OUT, ROUND_BF16, ROUND_SCALE, PAIR>, (unsigned)grid, kBlock, 0, stream)(x, numel, scale, o, o2);
   }
   return launch_status();
 }

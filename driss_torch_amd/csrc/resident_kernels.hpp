@@ -551,7 +551,7 @@ inline int launch_resident_impl(const void* x, int64_t numel, void* ws, void* ou
       return kResidentNotTaken;
     }
   }
-  kernel<<<(unsigned)grid, kBlock, kResLdsBytes, stream>>>(x, nvec, tail, w, o, o2, amax_out, scale_out, fmax0, fmax1,
+  launcher(kernel, (unsigned)grid, kBlock, kResLdsBytes, stream)(x, nvec, tail, w, o, o2, amax_out, scale_out, fmax0, fmax1,
                                                          spin_limit, gate.gave_up_dev[dev], log);
   const int st = launch_status();
   if (st == DT_OK) {

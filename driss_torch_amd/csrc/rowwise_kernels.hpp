@@ -270,7 +270,7 @@ inline int launch_rowwise_impl(const void* x, int64_t rows, int64_t cols, void* 
   const bool held = row_vecs >= 1 && row_vecs <= 64 * kBlock && rows <= 0x7FFFFFFFll;  // a workgroup can hold a row
   const bool edges_cached = rows * cols < kStreamEdgesFrom;
 #define DT_ROWB(NV, ACCESS) \
-  rowwise_block_resident_kernel<IN, OUT, NV, ACCESS><<<(unsigned)rows, kBlock, 0, stream>>>(x, cols, o, amax_out, scale_out)
+  launcher(rowwise_block_resident_kernel<IN, OUT, NV, ACCESS>, (unsigned)rows, kBlock, 0, stream)(x, cols, o, amax_out, scale_out)
 #define DT_ROWB_ANY_LENGTH(ACCESS, SHORT_ACCESS)       \
   do {                                                 \
     if (row_vecs <= 1 * kBlock) DT_ROWB(1, SHORT_ACCESS);    \
@@ -282,7 +282,7 @@ inline int launch_rowwise_impl(const void* x, int64_t rows, int64_t cols, void* 
     else DT_ROWB(64, ACCESS);                          \
   } while (0)
   const unsigned wave_grid = (unsigned)ceil_div(rows, kRowsPerBlock);
-#define DT_ROW(NV, ACCESS) rowwise_wave_kernel<IN, OUT, NV, ACCESS><<<wave_grid, kBlock, 0, stream>>>(x, rows, cols, o, amax_out, scale_out)
+#define DT_ROW(NV, ACCESS) launcher(rowwise_wave_kernel<IN, OUT, NV, ACCESS>, wave_grid, kBlock, 0, stream)(x, rows, cols, o, amax_out, scale_out)
 #define DT_ROW_ANY_LENGTH(ACCESS)                      \
   do {                                                 \
     if (row_vecs <= 1 * kWave) DT_ROW(1, ACCESS);      \
@@ -313,9 +313,9 @@ inline int launch_rowwise_impl(const void* x, int64_t rows, int64_t cols, void* 
 #undef DT_ROW
 #undef DT_ROW_ANY_LENGTH
   } else if (vec_ok) {
-    rowwise_block_kernel<IN, OUT, true><<<(unsigned)rows, kBlock, 0, stream>>>(x, cols, o, amax_out, scale_out);
+    launcher(rowwise_block_kernel<IN, OUT, true>, (unsigned)rows, kBlock, 0, stream)(x, cols, o, amax_out, scale_out);
   } else {
-    rowwise_block_kernel<IN, OUT, false><<<(unsigned)rows, kBlock, 0, stream>>>(x, cols, o, amax_out, scale_out);
+    launcher(rowwise_block_kernel<IN, OUT, false>, (unsigned)rows, kBlock, 0, stream)(x, cols, o, amax_out, scale_out);
   }
   return launch_status();
 }
