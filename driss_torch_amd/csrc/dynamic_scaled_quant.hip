@@ -78,11 +78,7 @@ extern "C" int dt_dynamic_scaled_quant_noalloc(const void* x, int in_dtype, int6
   dt::launcher(clear_scratch_kernel, dt::kWsBytes / 4 / 256, 256, 0, s)(reinterpret_cast<uint32_t*>(ws));
   if (int e = dt::launch_status()) return e;
   const float fm = fmax_of(out_dtype);
-  st = in_dtype == DT_F32 ? dt::launch_amax<DT_F32>(x, numel, ws, amax_out, scale_out, 1, fm, 0.f, s)
-                          : dt::launch_amax<DT_BF16>(x, numel, ws, amax_out, scale_out, 1, fm, 0.f, s);
-  if (st) return st;
-  return dt::launch_cast<false>(x, in_dtype, numel, reinterpret_cast<const float*>(ws + dt::kWsScale), out_dtype, round_mode,
-                                out, nullptr, s);
+  return dt::launch_amax_cast<false>(x, in_dtype, numel, out_dtype, round_mode, ws, out, nullptr, amax_out, scale_out, fm, 0.f, s);
 }
 
 extern "C" int dt_amax_scales(const void* x, int in_dtype, int64_t numel, float* amax_out, float* scale_out,
