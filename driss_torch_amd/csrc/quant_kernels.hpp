@@ -500,15 +500,19 @@ inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, vo
   // drain) weigh more: batches of 2 from three workgroups per CU, which reach their full rate sooner
   // (us, rotated buffers, batches of 4 and 1 workgroup per CU against this: bf16 4096^2 10.1 -> 9.6,
   // 2048^2 4.2 -> 3.9; no difference from 64 MiB on).  The knobs force either (0 = by size).
+  // Behind a reduction of the same call (FromPartials) x comes out of the caches as far as they reach, and the small batches win up to the 256 MiB of
+  // the memory-side cache, with both outputs too (us, both kernels, 4 and 1 -> 2 and 3: bf16 one output 66 MiB 28.3 -> 26.4, 128 MiB 51.0 -> 49.7, 256 MiB
+  // 102.9 -> 100.0, both 512 x 512 5.1 -> 4.6, 16 MiB 10.8 -> 10.1, 32 MiB 16.3 -> 14.8, 66 MiB 33.3 -> 31.3, 128 MiB 61.7 -> 60.0; fp32 both 64 MiB 25.4 -> 24.5,
+  // 256 MiB 101.1 -> 99.5; beyond that they lose, 428 MiB both 212.7 and 215.5; four workgroups per CU: 32 MiB 14.3, fp32 256 MiB 102.5).
   uint8_t* o = static_cast<uint8_t*>(out);
   uint8_t* o2 = static_cast<uint8_t*>(out2);
   if (cast_takes_vectors<IN>(x, out, out2)) {
     const int64_t nvec = numel / InTraits<IN>::kVec, tail = numel % InTraits<IN>::kVec;
-    const bool small = nvec * 16 < (int64_t)64 << 20;
+    const bool small = from.count ? nvec * 16 <= (int64_t)256 << 20 : !PAIR && nvec * 16 < (int64_t)64 << 20;
     const int unroll_knob = tuning(Knob::cast_unroll);
-    const int unroll = unroll_knob == 2 || unroll_knob == 4 ? unroll_knob : (small && !PAIR ? 2 : 4);
+    const int unroll = unroll_knob == 2 || unroll_knob == 4 ? unroll_knob : (small ? 2 : 4);
     const Knob knob = PAIR ? Knob::cast_pair_blocks_per_cu : Knob::cast_blocks_per_cu;
-    const int per_cu = tuning(knob) > 0 ? tuning(knob) : (small && !PAIR ? 3 : 1);
+    const int per_cu = tuning(knob) > 0 ? tuning(knob) : (small ? 3 : 1);
     int64_t grid = ceil_div(nvec, (int64_t)kBlock * unroll);
     if (grid > (int64_t)device_facts().cu_count * per_cu) grid = (int64_t)device_facts().cu_count * per_cu;
     // whole rounds of the eight XCDs: run r of kBlock vectors is then read by XCD r % 8, as in the reduction
