@@ -19,7 +19,7 @@ for _p in (hip_lib_path, lib_path):
         raise ImportError(f"{_p} is missing: build it with `python driss_torch_amd/_build.py`")
 torch.ops.load_library(str(lib_path.resolve()))
 
-ops = torch.ops.DrissTorch  # (the wrappers call the one overload of each: 0.1 us a call less than to have it looked for)
+ops = torch.ops.DrissTorch
 Tensor = torch.Tensor
 
 # product rounding of x*scale for bf16 inputs (see include/driss_torch_hip.h: dt_round_mode)
@@ -51,44 +51,44 @@ def saturated_cast(x: Tensor, scale: Tensor, out_dtype: torch.dtype, transpose: 
     product (and the scale) in bf16, a scale of rank >= 1 promotes the product to fp32.
     """
     assert not transpose, "Transpose is not supported yet"
-    return ops.saturated_cast.default(x, scale, out_dtype, transpose)
+    return ops.saturated_cast(x, scale, out_dtype, transpose)
 
 
 def saturated_cast_mode(x: Tensor, scale: Tensor, out_dtype: torch.dtype, mode: int) -> Tensor:
     """``saturated_cast`` with the product rounding mode given explicitly (ROUND_*)."""
-    return ops.saturated_cast_mode.default(x, scale, out_dtype, False, mode)
+    return ops.saturated_cast_mode(x, scale, out_dtype, False, mode)
 
 
 def amax(x: Tensor) -> Tensor:
     """max(abs(x)) as an fp32 tensor of shape [1] (reference: driss_torch/__init__.py:41-43)."""
-    return ops.amax.default(x)
+    return ops.amax(x)
 
 
 def dynamic_scaled_quant(inpt: Tensor, dtype: torch.dtype) -> Tensor:
     """amax -> scale -> saturated cast in one call (reference: driss_torch/__init__.py:46-47)."""
-    return ops.dynamic_scaled_quant.default(inpt, dtype)
+    return ops.dynamic_scaled_quant(inpt, dtype)
 
 
 def dynamic_scaled_quant_ex(inpt: Tensor, dtype: torch.dtype, mode: int = ROUND_AUTO) -> Tuple[Tensor, Tensor, Tensor]:
     """As ``dynamic_scaled_quant`` but also returns (amax [1], scale 0-dim)."""
-    return ops.dynamic_scaled_quant_ex.default(inpt, dtype, mode)
+    return ops.dynamic_scaled_quant_ex(inpt, dtype, mode)
 
 
 def dynamic_scaled_quant_pair(inpt: Tensor, mode: int = ROUND_AUTO) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
     """e4m3fn and e5m2 casts from one amax and one read: (e4m3fn, e5m2, amax [1], scale [2])."""
-    return ops.dynamic_scaled_quant_pair.default(inpt, mode)
+    return ops.dynamic_scaled_quant_pair(inpt, mode)
 
 
 def dynamic_scaled_quant_rowwise(inpt: Tensor, dtype: torch.dtype) -> Tuple[Tensor, Tensor, Tensor]:
     """Per-row scales: (fp8 [R,C], amax [R,1], scale [R,1]); the product is taken in fp32."""
-    return ops.dynamic_scaled_quant_rowwise.default(inpt, dtype)
+    return ops.dynamic_scaled_quant_rowwise(inpt, dtype)
 
 
 def sweep_mm(x: Tensor, w: Tensor, x_scale: Tensor, w_scale: Tensor, bias: Optional[Tensor], out_dtype: torch.dtype,
              use_fast_accum: bool, cluster_shape_x: int, cluster_shape_y: int, cluster_shape_z: int, transposed: bool,
              swizzle: int) -> Tensor:
     """Schema kept from the reference (driss_torch/__init__.py:50-77); not built, raises."""
-    return ops.sweep_mm.default(x, w, x_scale, w_scale, bias, out_dtype, use_fast_accum, cluster_shape_x, cluster_shape_y,
+    return ops.sweep_mm(x, w, x_scale, w_scale, bias, out_dtype, use_fast_accum, cluster_shape_x, cluster_shape_y,
                         cluster_shape_z, transposed, swizzle)
 
 
@@ -98,7 +98,7 @@ def mx_fp8_bf16(a: Tensor, b: Tensor, a_scale: Tensor, b_scale: Tensor) -> Tenso
 
     a: [M, K] row-major; b: [K, N] with stride(0) == 1 (an [N, K] tensor transposed).
     """
-    return ops.mx_fp8_bf16.default(a, b, a_scale, b_scale)
+    return ops.mx_fp8_bf16(a, b, a_scale, b_scale)
 
 
 def mx_fp4_bf16(a: Tensor, b: Tensor, a_scale: Tensor, b_scale: Tensor) -> Tensor:
@@ -108,7 +108,7 @@ def mx_fp4_bf16(a: Tensor, b: Tensor, a_scale: Tensor, b_scale: Tensor) -> Tenso
     a: [M, K/2] row-major, b: [K/2, N] with stride(0) == 1; two e2m1 values per byte (uint8 or
     float4_e2m1fn_x2 storage), the even element in the low nibble.
     """
-    return ops.mx_fp4_bf16.default(a, b, a_scale, b_scale)
+    return ops.mx_fp4_bf16(a, b, a_scale, b_scale)
 
 
 def mx_fp8_quantize(input: Tensor, block_size: int = 32, axis: int = 1, transpose: bool = False,
@@ -119,7 +119,7 @@ def mx_fp8_quantize(input: Tensor, block_size: int = 32, axis: int = 1, transpos
     ``transpose``; the flat scale tensor is the row-major scale matrix [M, N/32] (axis 1),
     [M/32, N] (axis 0), [N/32, M] (axis 1, transpose) or [N, M/32] (axis 0, transpose).
     """
-    return ops.mx_fp8_quantize.default(input, block_size, axis, transpose, ScalarType)
+    return ops.mx_fp8_quantize(input, block_size, axis, transpose, ScalarType)
 
 
 mx_cast = mx_fp8_quantize
@@ -129,7 +129,7 @@ def mx_fp8_quantize_blocked(input: Tensor, axis: int = 1, ScalarType: torch.dtyp
                             ) -> Tuple[Tensor, Tensor]:
     """MXFP8 cast whose scales come out in the blocked layout ``mx_fp8_bf16`` reads, with K as
     the contiguous payload dimension: axis 1 -> payload [M, N]; axis 0 -> payload [N, M]."""
-    return ops.mx_fp8_quantize_ex.default(input, 32, axis, axis % 2 == 0, ScalarType, True)
+    return ops.mx_fp8_quantize_ex(input, 32, axis, axis % 2 == 0, ScalarType, True)
 
 
 def mx_fp8_quantize_dual(input: Tensor, ScalarType: torch.dtype = torch.float8_e4m3fn, blocked: bool = False
@@ -138,7 +138,7 @@ def mx_fp8_quantize_dual(input: Tensor, ScalarType: torch.dtype = torch.float8_e
     scale_t)``.  The first pair equals ``mx_fp8_quantize(input)``, the second
     ``mx_fp8_quantize(input.t().contiguous())``: the operand for a forward product and the one for the
     weight-gradient product.  ``blocked`` selects the scale layout ``mx_fp8_bf16`` reads."""
-    return ops.mx_fp8_quantize_dual.default(input, ScalarType, blocked)
+    return ops.mx_fp8_quantize_dual(input, ScalarType, blocked)
 
 
 def mx_fp4_quantize(input: Tensor, blocked: bool = False, axis: int = 1) -> Tuple[Tensor, Tensor]:
@@ -148,18 +148,18 @@ def mx_fp4_quantize(input: Tensor, blocked: bool = False, axis: int = 1) -> Tupl
     payload [M, N/2], scale matrix [M, N/32]; axis 0: blocks down the columns with the payload
     transposed, [N, M/2] and [N, M/32], which equals the axis-1 cast of ``input.t().contiguous()``.
     ``blocked`` selects the scale layout the GEMM reads; otherwise the flat scale tensor is row-major."""
-    return ops.mx_fp4_quantize.default(input, blocked, axis)
+    return ops.mx_fp4_quantize(input, blocked, axis)
 
 
 def mx_fp4_quantize_dual(input: Tensor, blocked: bool = False) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
     """Both MXFP4 operands of ``input`` [M, N] from one read: ``(data [M, N/2], scale, data_t [N, M/2],
     scale_t)``, equal to ``mx_fp4_quantize(input, blocked, 1) + mx_fp4_quantize(input, blocked, 0)``."""
-    return ops.mx_fp4_quantize_dual.default(input, blocked)
+    return ops.mx_fp4_quantize_dual(input, blocked)
 
 
 def to_blocked(scale: Tensor) -> Tensor:
     """[R, C] E8M0 scale matrix -> flat blocked 128x4 layout (zero padded)."""
-    return ops.to_blocked.default(scale)
+    return ops.to_blocked(scale)
 
 
 # The fake implementations register from the module the operator library names as their home
