@@ -45,6 +45,21 @@ constexpr int few_lines_waves(bool fp4, int mh, int nh, bool ragged) {
   return few_lines_stages_of(4, fp4, mh, nh) >= least ? 4 : 2;
 }
 
+// Whole lines of B go out in runs of four loads: load i of an octet's eight rows has i % 4 KiB as its immediate offset, which counts in memory and in LDS, so its
+// lane offsets are lowered by as much.  Octets are not in the order of their columns (load 3 may be column 8 of its chunk, and a column that is not there is the
+// last one, in front of that), so with rows of a few lines the lowered offset of a byte can lie in front of the chunk: B's descriptor begins
+// kFewLinesBias bytes in front of it, and no lane offset depends on how a sum below zero is taken.
+constexpr uint32_t kFewLinesBias = 3 * 1024;
+constexpr uint32_t few_lines_immediate(int load) { return (uint32_t)(load % 4) * 1024u; }
+__host__ __device__ inline uint32_t few_lines_lane_offset(uint32_t row, uint32_t ldb, uint32_t in_row, int load) {
+  return kFewLinesBias + row * ldb + in_row - few_lines_immediate(load);
+}
+// The row of B, from the group's first chunk on, that lane octet row lrow of load i brings: a column that is not there reads the last one's bytes
+__host__ __device__ inline uint32_t few_lines_row(uint32_t first_octet, int i, uint32_t lrow, uint32_t rows) {
+  const uint32_t r = octet_column(first_octet + i) - (first_octet >> 4) * 128u + lrow;
+  return r < rows ? r : rows - 1u;
+}
+
 // What the kernel takes: scale chunks of up to 4 K bytes in 32 bits
 inline bool few_lines_fits(int64_t M, int64_t K) { return M <= 32 && K <= ((int64_t)1 << 29); }
 

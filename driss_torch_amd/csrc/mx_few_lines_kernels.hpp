@@ -91,10 +91,11 @@ __global__ __launch_bounds__(few_lines_waves(FP4, MH, NH, RAGGED) * kWave) void 
     return ((((uint32_t)lane & 7u) - lrow + (phase >> 4)) & 7u) * 16u - phase;
   };
   const uint32_t in_a = in_octet(mis_a, lda), in_b = in_octet(mis_b, ldb);
-  // (whole lines go out in runs of four loads: the immediate offset counts in memory and in LDS, lane offsets are lowered by as much)
+  // (whole lines go out in runs of four loads, see few_lines_lane_offset; A's load i is rows 8 i and up, 128 bytes or more each)
+  constexpr uint32_t kBias = RAGGED ? 0u : kFewLinesBias;
   uint32_t off_a[MH], off_b[NH];
 #pragma unroll
-  for (int i = 0; i < MH; ++i) off_a[i] = (uint32_t)(i * 8 + lrow) * lda + in_a - (RAGGED ? 0u : (i & 3) * 1024u);
+  for (int i = 0; i < MH; ++i) off_a[i] = (uint32_t)(i * 8 + lrow) * lda + in_a - (RAGGED ? 0u : few_lines_immediate(i));
   // scale words: lanes 0 to 31 those of B, the others A's, or 64 of each
   const int arow = kOneScaleLoad ? lane & 31 : lane, arow_in = arow < M ? arow : M - 1;
   const uint64_t sa_lane = reinterpret_cast<uint64_t>(sfa) + (uint32_t)(arow_in & 31) * 16u + (uint32_t)(arow_in >> 5) * 4u;
@@ -106,16 +107,15 @@ __global__ __launch_bounds__(few_lines_waves(FP4, MH, NH, RAGGED) * kWave) void 
   uint32_t at = 0;
   auto enter = [&](int group) __attribute__((always_inline)) {
     const uint32_t first = (uint32_t)group * NH, n0 = (first >> 4) * 128u;
-    const uint64_t p = pb + (uint64_t)n0 * ldb;
+    const uint64_t p = pb + (uint64_t)n0 * ldb - kBias;
     rsrc_b.x = (int)(uint32_t)p;
     rsrc_b.y = (int)((uint32_t)(p >> 32) & 0xFFFFu);
     const int rows = N - (int)n0;
-    bytes_b = (uint32_t)((rows < 256 ? rows : 256) - 1) * ldb + left;  // a group lies in two chunks of 128 rows at most
+    bytes_b = (uint32_t)((rows < 256 ? rows : 256) - 1) * ldb + left + kBias;  // a group lies in two chunks of 128 rows at most
 #pragma unroll
     for (int i = 0; i < NH; ++i) {
-      uint32_t r = octet_column(first + i) - n0 + lrow;
-      r = r < (uint32_t)rows ? r : (uint32_t)rows - 1u;  // a column that is not there reads the last one's bytes and is never stored
-      off_b[i] = r * ldb + in_b - (RAGGED ? 0u : (i & 3) * 1024u);
+      const uint32_t r = few_lines_row(first, i, lrow, (uint32_t)rows);  // (a column that is not there is never stored)
+      off_b[i] = RAGGED ? r * ldb + in_b : few_lines_lane_offset(r, ldb, in_b, i);
     }
     const uint32_t i = (uint32_t)(kOneScaleLoad ? lane & 31 : lane) >> 3, octet = first + (i < NH ? i : NH - 1);
     const uint32_t chunks = (uint32_t)(N + 127) >> 7, chunk = (octet >> 4) < chunks ? octet >> 4 : chunks - 1;
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(few_lines_waves(FP4, MH, NH, RAGGED) * kWave) void 
       else if constexpr (i % 4 == 0)
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" : : "s"(dst), "v"(lane_off), "s"(r), "s"(k_now) : "memory");
       else
-        asm volatile("buffer_load_dwordx4 %0, %1, %2 offen offset:%3 lds" : : "v"(lane_off), "s"(r), "s"(k_now), "n"((i % 4) * 1024) : "memory");
+        asm volatile("buffer_load_dwordx4 %0, %1, %2 offen offset:%3 lds" : : "v"(lane_off), "s"(r), "s"(k_now), "n"(few_lines_immediate(i)) : "memory");
     };
     auto load_b = [&](auto i) __attribute__((always_inline)) { load(i, decltype(i)::value * 1024, off_b[decltype(i)::value], rsrc_b); };
     auto load_a = [&](auto i) __attribute__((always_inline)) { load(i, kOffA + decltype(i)::value * 1024, off_a[decltype(i)::value], rsrc_a); };
