@@ -285,15 +285,24 @@ def test_dynamic_quant_config2_full_size(d):
 
 @pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("numel", [1, 3, 4, 7, 8, 9, 15, 2047, 2051, 16384, 16391, 131080, 524288, 600007, 4194304, 4194312, 4300001], ids=str)
-def test_dynamic_quant_scale_from_workgroup_maxima(d, cabi, numel, in_dtype):
+@pytest.mark.parametrize("unroll", [0, 4])
+def test_dynamic_quant_scale_from_workgroup_maxima(d, cabi, numel, in_dtype, unroll):
     """the cast takes the reduction's maxima itself: the largest element in the first place, in the last and in between, a NaN in the last, a
-    larger tensor's maxima still in the workspace, an input off its vectors (the other way to the scale), and nothing written past the end"""
+    larger tensor's maxima still in the workspace, an input off its vectors (the other way to the scale), and nothing written past the end;
+    every rounding of the product, in the small batches of these sizes and in those that tensors beyond 256 MiB take"""
+    cabi.set_tuning("cast.unroll", unroll)
+    try:
+        _check_scale_from_workgroup_maxima(cabi, numel, in_dtype)
+    finally:
+        cabi.set_tuning("cast.unroll", 0)
+
+
+def _check_scale_from_workgroup_maxima(cabi, numel, in_dtype):
     cabi.dynamic_scaled_quant(torch.full((4200000,), 1e30, dtype=in_dtype, device="cuda"), FP8[0], 3)
     a = util.student_t((numel + 1,), 1700 + numel % 97, in_dtype)[1:].clone()
     for at, value in ((0, 1000.0), (numel - 1, -3000.0), (numel // 2, 1e5), (numel - 1, float("nan"))):
         a[at] = value
-        mode = 2 if in_dtype == torch.bfloat16 else 3
-        for off in (0, 1):
+        for off, mode in [(off, mode) for off in (0, 1) for mode in ((1, 2, 3) if in_dtype == torch.bfloat16 else (3,))]:
             buf = torch.zeros(numel + 8, dtype=in_dtype, device="cuda")
             x = buf[off:off + numel]
             x.copy_(a)

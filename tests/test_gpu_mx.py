@@ -876,14 +876,17 @@ def test_mx_gemm_config5_full_size(d):
 @pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
 @pytest.mark.parametrize("octets", range(1, 9))
 def test_mx_gemm_few_lines_kernel(d, cabi, octets, fp4):
-    """the kernel for at most 32 rows by whole lines, with every number of column octets per group: one step and fewer steps than waves, rows on
-    and off the lines, every count of row octets, columns that end inside an octet's chunk, several groups per workgroup; against the float64 product of the
-    dequantized operands (bound per entry: bf16's rounding, 2^-8 of sum |a||b|), equal rows of A equal, and the same bits on a second call"""
+    """the kernel for at most 32 rows by whole lines, every form of it: every number of column octets per group, and for every count of row octets fewer
+    steps than waves and more than the stages of all of them, rows on the lines and off them; one step, columns that end inside an octet's chunk,
+    several groups per workgroup; against the float64 product of the dequantized operands (bound per entry: bf16's rounding, 2^-8 of sum |a||b|), equal
+    rows of A equal, and the same bits on a second call"""
+    line = 256 if fp4 else 128
+    every_form = [(M, K, 8 * octets + 136) for M in (2, 12, 20, 30) for steps in (3, 41) for K in (steps * line, steps * line + 32)]
     cabi.set_tuning("gemm.variant", 9)
     cabi.set_tuning("gemm.few_rows_octets", octets)
     try:
         for M, K, N in ((1, 32, 8), (8, 128, 8 * octets), (9, 1024, 136), (16, 2048, 264), (17, 1056, 1000), (25, 4160, 72), (32, 8192, 512),
-                        (31, 96, 128 * octets + 8), (32, 256, 2048 * octets + 136), (3, 288, 4096 * octets + 40)):
+                        (31, 96, 128 * octets + 8), (32, 256, 2048 * octets + 136), (3, 288, 4096 * octets + 40), *every_form):
             x, w = _wide_operand((M, K), 5000 + M + octets).cuda(), _wide_operand((N, K), 5001 + K).cuda()
             x[M - 1] = x[0]
             if fp4:
