@@ -13,6 +13,9 @@ namespace dt {
 // of octet 4 q + b (rows 32 b + 8 q to 32 b + 8 q + 7) in word b of its lines 8 q to 8 q + 7, so that four octets in a row share 128 bytes of them.
 __host__ __device__ inline uint32_t octet_column(uint32_t octet) { return (octet >> 4) * 128u + (octet & 3u) * 32u + ((octet >> 2) & 3u) * 8u; }
 
+// The scale word of a row of an octet, in its chunk
+__host__ __device__ inline uint32_t octet_scale_word(uint32_t octet, uint32_t row) { return ((octet >> 2) & 3u) * 128u + row * 16u + (octet & 3u) * 4u; }
+
 // Groups of `octets` octets each that hold a column of the matrix.
 inline int64_t few_lines_groups(int64_t N, int octets) {
   const int64_t whole = N / 128 * 16, rest = N % 128;

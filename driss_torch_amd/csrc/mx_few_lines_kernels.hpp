@@ -119,8 +119,7 @@ __global__ __launch_bounds__(few_lines_waves(FP4, MH, NH, RAGGED) * kWave) void 
     }
     const uint32_t i = (uint32_t)(kOneScaleLoad ? lane & 31 : lane) >> 3, octet = first + (i < NH ? i : NH - 1);
     const uint32_t chunks = (uint32_t)(N + 127) >> 7, chunk = (octet >> 4) < chunks ? octet >> 4 : chunks - 1;
-    const uint64_t sb_lane = reinterpret_cast<uint64_t>(sfb) + (uint64_t)chunk * ((uint32_t)k_chunks * 512u) + ((octet >> 2) & 3u) * 128u +
-                             (lane & 7) * 16u + (octet & 3u) * 4u;
+    const uint64_t sb_lane = reinterpret_cast<uint64_t>(sfb) + (uint64_t)chunk * ((uint32_t)k_chunks * 512u) + octet_scale_word(octet, lane & 7);
     s_lane = !kOneScaleLoad || lane < 32 ? sb_lane : sa_lane;
     at = RAGGED ? 0u : (((uint32_t)group * 8u + (uint32_t)wave) * 2654435761u >> 16) * (uint32_t)n_steps >> 16;
   };

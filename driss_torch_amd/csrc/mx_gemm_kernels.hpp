@@ -992,9 +992,9 @@ int mx_gemm(const void* a, const void* b, const uint8_t* sfa, const uint8_t* sfb
   const int cus = device_facts().cu_count;
   const bool ragged = ring_ragged(k_bytes, A, B, lda, ldb);
   const GemmPlan plan = plan_gemm(FP4, M, N, K, ragged, workspace ? workspace_bytes : 0, cus, few_rows_fits(M, K) ? few_rows_columns(N) : 0,
+                                  few_lines_fits(M, K),
                                   {tuning(Knob::gemm_variant), tuning(Knob::gemm_tail_quads), tuning(Knob::gemm_split_k),
-                                   tuning(Knob::gemm_tile_m), tuning(Knob::gemm_tile_n), few_lines_forced_octets()},
-                                  few_lines_fits(M, K));
+                                   tuning(Knob::gemm_tile_m), tuning(Knob::gemm_tile_n), few_lines_forced_octets()});
   // tiles of 256 x 256 in whole rounds of the chip, and those behind them
   const int64_t tiles256 = ceil_div(M, 256) * ceil_div(N, 256), whole = tiles256 / cus * cus, left = tiles256 - whole;
   // <tile M, tile N, waves M, waves N, LDS ring slots, e2m1 operands>

@@ -203,8 +203,8 @@ struct GemmPlan {
 // (from memory / from the cache), and 0.91 / 0.91 of what it took without the kernel by whole lines.  What that one loses to the other one for few rows
 // are products of 3 to 4 us, 17 % at most from memory: e2m1 4 x 3872 x 2720 3.9 and 4.1, 15 x 2576 x 1312 3.4 and 3.7.)
 // How many workgroups are to share K does not decide between the two; whether any may does.
-inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, size_t workspace_bytes, int cus, int few_columns, GemmKnobs knobs,
-                          bool few_lines = false) {
+inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, size_t workspace_bytes, int cus, int few_columns, bool few_lines,
+                          GemmKnobs knobs) {
   const auto small = [&](int split_k, int tile_m, int tile_n) {
     GemmPlan p{kSmallTiles, plan_ring(fp4, M, N, K, ragged, workspace_bytes, cus, split_k, tile_m, tile_n)};
     p.small.cols = ring_cols(p.small, fp4, M, N, K, cus);

@@ -7,7 +7,7 @@ from pathlib import Path
 import pytest
 
 ROOT = Path(__file__).resolve().parent.parent
-SMALL, HALVES, T192, T256, THEN_QUADS, THEN_HALVES, QUADRANT_SCHEDULE, FEW_ROWS = range(8)
+SMALL, HALVES, T192, T256, THEN_QUADS, THEN_HALVES, QUADRANT_SCHEDULE, FEW_ROWS, FEW_LINES = range(9)
 CUS = 256
 ALL = 1024 + CUS * 128 * 128 * 4  # a workspace with room for a tile per CU
 
@@ -18,7 +18,7 @@ def plan(tmp_path_factory):
     (where / "plan.cpp").write_text(
         '#include "mx_gemm_plan.hpp"\n'
         'extern "C" int plan(int fp4, long M, long N, long K, int ragged, long ws, int cus, int few, int variant, int tail, int split_k) {\n'
-        "  const dt::GemmPlan p = dt::plan_gemm(fp4 != 0, M, N, K, ragged != 0, (size_t)ws, cus, few, {variant, tail, split_k, 0, 0});\n"
+        "  const dt::GemmPlan p = dt::plan_gemm(fp4 != 0, M, N, K, ragged != 0, (size_t)ws, cus, few, few && dt::few_lines_fits(M, K), {variant, tail, split_k, 0, 0});\n"
         "  return p.tiles * 100 + p.small.splits;\n}\n")
     subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-I/opt/rocm/include",
                     f"-I{ROOT / 'include'}", f"-I{ROOT / 'driss_torch_amd' / 'csrc'}", str(where / "plan.cpp"), "-o",
@@ -82,10 +82,13 @@ def test_rows_off_the_lines_take_small_tiles_instead_of_halves(plan, fp4):
 
 
 def test_few_rows(plan):
-    assert plan(False, 16, 8192, 8192, few=32)[0] == FEW_ROWS and plan(False, 16, 8192, 8192)[0] == SMALL
-    assert plan(False, 16, 64, 64, few=16, variant=9)[0] == FEW_ROWS and plan(False, 100, 64, 64, variant=9)[0] == SMALL
+    for M in (1, 16, 32, 33, 48):
+        assert plan(True, M, 2048, 4096, few=16)[0] == (FEW_LINES if M <= 32 else FEW_ROWS) and plan(True, M, 2048, 4096)[0] == SMALL
+        assert plan(False, M, 64, 64, few=16, variant=9)[0] == (FEW_LINES if M <= 32 else FEW_ROWS)
+    assert plan(False, 100, 64, 64, variant=9)[0] == SMALL
     for variant, tiles in ((1, SMALL), (2, T256), (3, SMALL), (5, T192), (7, QUADRANT_SCHEDULE)):
-        assert plan(False, 16, 8192, 8192, few=32, variant=variant)[0] == tiles
+        for M in (16, 40):
+            assert plan(False, M, 8192, 8192, few=32, variant=variant)[0] == tiles
 
 
 def test_shares_own_a_step_and_fit_the_workspace(plan):

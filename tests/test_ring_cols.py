@@ -33,7 +33,7 @@ extern "C" int words(int N, int cols, int chunks) {
   return 0;
 }
 extern "C" long plan(int fp4, long M, long N, long K, int ragged, long ws, int cus) {
-  const dt::GemmPlan p = dt::plan_gemm(fp4 != 0, M, N, K, ragged != 0, (size_t)ws, cus, 0, {3, 1, 0, 0, 0});
+  const dt::GemmPlan p = dt::plan_gemm(fp4 != 0, M, N, K, ragged != 0, (size_t)ws, cus, 0, false, {3, 1, 0, 0, 0});
   return ((p.small.tile_m * 1000L + p.small.tile_n) * 100 + p.small.splits) * 1000 + p.small.cols;
 }
 """

@@ -1,4 +1,4 @@
-"""The estimate that picks the small tiles of a block-scaled product, the workgroups that share K and the kernel for few
+"""The estimate that picks the small tiles of a block-scaled product, the workgroups that share K and the kernels for few
 rows, compiled on its own for the host."""
 import ctypes as C
 import subprocess
@@ -57,7 +57,8 @@ def lib(tmp_path_factory):
         "  const dt::RingPlan p = dt::plan_ring(fp4 != 0, M, N, K, ragged != 0, (size_t)ws, cus, split_k, tm, tn);\n"
         "  return (p.tile_m * 1000L + p.tile_n) * 100 + p.splits;\n}\n"
         'extern "C" int few(int fp4, long M, long N, long K, int ragged, long ws, int cus, int columns, int split_k) {\n'
-        "  return dt::plan_gemm(fp4 != 0, M, N, K, ragged != 0, (size_t)ws, cus, columns, {0, 1, split_k, 0, 0}).tiles == dt::kFewRows;\n}\n")
+        "  const dt::GemmTiles t = dt::plan_gemm(fp4 != 0, M, N, K, ragged != 0, (size_t)ws, cus, columns, dt::few_lines_fits(M, K), {0, 1, split_k, 0, 0}).tiles;\n"
+        "  return t == dt::kFewRows || t == dt::kFewLines;\n}\n")
     subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-I/opt/rocm/include",
                     f"-I{ROOT / 'include'}", f"-I{ROOT / 'driss_torch_amd' / 'csrc'}", str(where / "plan.cpp"), "-o",
                     str(where / "plan.so")], check=True)
@@ -101,10 +102,11 @@ def test_picks(lib):
 
     assert few(16, 8192, 8192) and few(1, 1928, 1984) and few(16, 4096, 4096, 1)
     assert few(1, 168, 10048, 1) and few(12, 1488, 12064, 1) and few(2, 464, 5152) and not few(64, 424, 8224)
-    for split_k in (1, 2, 7):  # how many workgroups share K says nothing about the kernel for few rows; that none may can only speak for it
-        assert few(16, 8192, 8192, split_k=split_k) and few(16, 4096, 4096, 1, split_k)
-    assert few(16, 1024, 8192, split_k=1) and not few(16, 1024, 8192, split_k=2) and not few(16, 1024, 8192)
-    assert not few(64, 8192, 8192) and not few(32, 28672, 10848) and not few(32, 14336, 4096, 1) and not few(16, 5120, 5120)
+    for split_k in (1, 2, 7):  # how many workgroups share K says nothing about the kernels for few rows; that none may can only speak for them
+        assert few(16, 8192, 8192, split_k=split_k) and few(16, 4096, 4096, 1, split_k) and few(40, 4096, 4096, split_k=split_k)
+    assert few(40, 1024, 8192, split_k=1) and not few(40, 1024, 8192, split_k=2) and not few(40, 1024, 8192)
+    assert few(16, 1024, 8192) and few(16, 5120, 5120)  # at most 32 rows: by whole lines
+    assert not few(64, 8192, 8192) and not few(32, 28672, 10848) and not few(32, 14336, 4096, 1)
 
 
 @pytest.mark.parametrize("size", SHARES, ids=lambda s: "x".join(map(str, s)))
