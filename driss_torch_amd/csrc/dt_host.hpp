@@ -50,10 +50,11 @@ const DeviceFacts& device_facts();  // of the current device, cached per device
 //   gemm.variant: 0 = pick the tile by problem size, 1 = 128x128 tiles, 2 = 256x256 tiles, 3 = tiles of 64 or 128 rows
 //                 and columns as gemm.tile_m and gemm.tile_n say (0 = by the estimate), 5 = 256x192 tiles,
 //                 7 = 256x256 tiles on the main loop of the smaller ones (quadrants of the wave tile, no L2 prefetch;
-//                 the same bits), 9 = the kernels for at most 64 rows whatever the other dimensions
+//                 the same bits), 9 = the kernels for at most 64 rows whatever the other dimensions, 10 = the one that loads B into registers
+//                 (mx_few_rows.hip) whichever of them the rule takes
 //   gemm.few_rows_tiles: 16-column tiles per group of columns of those kernels: 0 = by the problem's size, 1, 2
-//   gemm.few_rows_per_cu, gemm.few_rows_stagger: of the one for 33 to 64 rows, workgroups per CU (0: two) and the staggered walk along K;
-//                 gemm.few_rows_steps: taken for the sake of its callers, its batches are of one step
+//   gemm.few_rows_per_cu, gemm.few_rows_stagger, gemm.few_rows_steps: of the one that loads B into registers, workgroups per CU (0: two), the
+//                 staggered walk along K, steps per batch of loads (0: two for at most 16 rows, else one; 1, 2: up to 32 rows)
 //   gemm.few_rows_octets: columns per group of the one for at most 32 rows, in eights: 0 = by the problem's size, 1 to 8
 //   gemm.tail_quads: 1 = tiles left over after whole rounds of 256x256 tiles run as 128x128 quadrants
 //                 or 256x128 halves when those fit the chip at once, 0 = never, 2 = always as

@@ -1,11 +1,12 @@
-// The block-scaled GEMM for 33 to 64 rows: out[M,N] = (A 2^sfa)(B 2^sfb)^T with e4m3 or e2m1 operands.  (Up to 32 rows, where A's share of a stage
+// The block-scaled GEMM for few rows (M <= 64): out[M,N] = (A 2^sfa)(B 2^sfb)^T with e4m3 or e2m1 operands.  (Up to 32 rows, where A's share of a stage
 // in LDS leaves B room enough, the kernel of mx_few_lines_kernels.hpp reads B by whole lines; at 34 x 1280 x 2400 e2m1 this one takes 4.5 us and that
-// one, with room for 64 rows, 5.4, at 50 x 1504 x 3264 e4m3 6.9 and 8.1, at 64 x 8192 x 8192 21.7 and 20.1, where the small tiles take 20.0.)
+// one, with room for 64 rows, 5.4, at 50 x 1504 x 3264 e4m3 6.9 and 8.1, at 64 x 8192 x 8192 21.7 and 20.1, where the small tiles take 20.0.  Of at most 32 rows this
+// one keeps the short rows of few columns that are no whole lines, see few_rows_instead_of_lines.)
 //
 // Such a problem is one pass over B, and a tile with a 128- or 256-row A panel would idle most of its
 // MFMAs and leave the chip to a handful of workgroups.  Here a workgroup of 8 waves owns a group of
 // 16 NT rows of B (= output columns) at a time and every row of A; its waves share K between them in
-// turns of one panel step of 128 bytes, so the workgroup as a whole walks 16 NT whole rows of B.
+// turns of UP panel steps of 128 bytes, so the workgroup as a whole walks 16 NT whole rows of B.
 //
 // B goes straight from memory into the registers the MFMA takes: a lane's part of an operand is two
 // 16-byte pieces of one row, 64 bytes apart, and the four lanes that share a row read 64 contiguous bytes
@@ -24,7 +25,7 @@
 // its fragments from there (16-byte chunks XOR-swizzled inside each group of 8 rows: conflict-free),
 // and A's blocked scale chunks travel the same way.  No other wave reads that region: no barrier.
 //
-// A batch (one step) is in registers / LDS while the next one's loads are in flight.  All of a batch's
+// A batch (UP steps) is in registers / LDS while the next one's loads are in flight.  All of a batch's
 // memory instructions are written as assembly and counted by hand (one s_waitcnt per batch): the
 // compiler does not see the LDS-DMA loads, and its own counts would make a batch wait for part of the
 // next one.  The waves' partial sums meet in LDS and are added in wave order; one wave per 16 x 16
@@ -78,15 +79,15 @@ __device__ __forceinline__ void wait_loads() {
 
 // MH: A's rows in halves of a 16-row tile (8 rows, one LDS-DMA instruction per step); the second half of
 // the last tile is not fetched when no row of A lies in it (its sums are never stored)
-template <bool FP4, int MH, int NT>
+template <bool FP4, int MH, int NT, int UP>
 __global__ __launch_bounds__(kFewWaves* kWave) void mx_few_rows_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                                                                      const uint8_t* __restrict__ sfa, const uint8_t* __restrict__ sfb,
                                                                      int M, int N, int K, int64_t lda, int64_t ldb,
                                                                      uint16_t* __restrict__ out, int64_t ldo, int groups, int stagger) {
-  constexpr int WAVES = kFewWaves, UP = 1;  // UP: panel steps per batch
+  constexpr int WAVES = kFewWaves;
   constexpr int MT = (MH + 1) / 2;
   constexpr int KC = FP4 ? 2 : 1;  // MFMAs, and blocked scale chunks, per panel step of 128 bytes of a row
-  static_assert(MH >= 5 && MH <= 8 && NT >= 1 && NT <= 2, "33 to 64 rows of A, 16 or 32 columns per group");
+  static_assert(MH >= 1 && MH <= 8 && NT >= 1 && NT <= 2 && UP >= 1, "at most 64 rows of A, 32 columns per group");
   // LDS of a wave: two sets of [A rows of a batch: step, tile, half of 8 rows, 8 rows x 128 B][A scale chunks of the batch]
   constexpr int kPanel = UP * MT * 2048;
   constexpr int kScaleLoads = (UP * KC + 1) / 2;  // of 1 KiB = two scale chunks
@@ -348,8 +349,13 @@ __global__ __launch_bounds__(kFewWaves* kWave) void mx_few_rows_kernel(const uin
   }
 }
 
-constexpr size_t few_rows_lds_bytes(bool fp4, int mt) {
-  return (size_t)kFewWaves * 2 * ((size_t)mt * 2048 + (size_t)(((fp4 ? 2 : 1) + 1) / 2) * 1024);
+// Shape of the launch for a problem: 16-column tiles per group (NT), panel steps per batch (UP)
+struct Plan {
+  int nt, up;
+};
+
+constexpr size_t few_rows_lds_bytes(bool fp4, int mt, int up) {
+  return (size_t)kFewWaves * 2 * ((size_t)up * mt * 2048 + (size_t)((up * (fp4 ? 2 : 1) + 1) / 2) * 1024);
 }
 constexpr size_t kLdsLimit = 160 * 1024;
 
@@ -360,14 +366,24 @@ int tiles_per_group(int64_t N) {
   const int tiles = tuning(Knob::gemm_few_rows_tiles);
   return tiles ? (tiles == 2 ? 2 : 1) : (N >= 32 * (int64_t)device_facts().cu_count ? 2 : 1);
 }
+Plan plan_for(bool fp4, int64_t M, int64_t N) {
+  Plan p;
+  p.nt = tiles_per_group(N);
+  const int mt = (int)((M + 15) / 16);
+  int up = tuning(Knob::gemm_few_rows_steps);
+  if (up != 1 && up != 2) up = mt == 1 ? 2 : 1;
+  if (up == 2 && (mt > 2 || few_rows_lds_bytes(fp4, mt, 2) >= kLdsLimit)) up = 1;
+  p.up = up;
+  return p;
+}
 
-template <bool FP4, int MH, int NT>
+template <bool FP4, int MH, int NT, int UP>
 int launch_instance(const uint8_t* a, const uint8_t* b, const uint8_t* sfa, const uint8_t* sfb, int64_t M, int64_t N, int64_t K,
                     int64_t lda, int64_t ldb, uint16_t* out, int64_t ldo, int64_t groups, int64_t grid, int stagger,
                     hipStream_t stream) {
-  constexpr size_t kLds = few_rows_lds_bytes(FP4, (MH + 1) / 2);
+  constexpr size_t kLds = few_rows_lds_bytes(FP4, (MH + 1) / 2, UP);
   static_assert(kLds <= kLdsLimit, "two sets per wave fit the CU's LDS");
-  auto kernel = mx_few_rows_kernel<FP4, MH, NT>;
+  auto kernel = mx_few_rows_kernel<FP4, MH, NT, UP>;
   if (kLds > 64 * 1024) {  // once per instantiation and device
     static std::atomic<bool> allowed[16];
     int dev = 0;
@@ -382,7 +398,7 @@ int launch_instance(const uint8_t* a, const uint8_t* b, const uint8_t* sfa, cons
     }
   }
   launcher(kernel, (unsigned)grid, kFewWaves * kWave, kLds, stream)(a, b, sfa, sfb, (int)M, (int)N, (int)K, lda, ldb, out, ldo, (int)groups,
-                                                            stagger);
+                                                                    stagger);
   return launch_status();
 }
 
@@ -396,19 +412,28 @@ int few_rows_columns(int64_t N) { return 16 * tiles_per_group(N); }
 int launch_few_rows(bool fp4, const uint8_t* a, const uint8_t* b, const uint8_t* sfa, const uint8_t* sfb, int64_t M, int64_t N,
                     int64_t K, int64_t lda, int64_t ldb, void* out, int64_t ldo, hipStream_t stream) {
   uint16_t* o = static_cast<uint16_t*>(out);
-  const int nt = tiles_per_group(N);
+  const Plan p = plan_for(fp4, M, N);
   const int mh = (int)((M + 7) / 8);  // halves of 16-row tiles that hold rows of A
-  const int64_t groups = ceil_div(N, (int64_t)16 * nt);
+  const int64_t groups = ceil_div(N, (int64_t)16 * p.nt);
   int per_cu = tuning(Knob::gemm_few_rows_per_cu);
   if (per_cu < 1) per_cu = 2;
   int64_t grid = groups;
   if (grid > (int64_t)device_facts().cu_count * per_cu) grid = (int64_t)device_facts().cu_count * per_cu;
   const int stagger = tuning(Knob::gemm_few_rows_stagger);
-#define DT_FEW(FP4, MH, NT) return launch_instance<FP4, MH, NT>(a, b, sfa, sfb, M, N, K, lda, ldb, o, ldo, groups, grid, stagger, stream)
-#define DT_FEW_N(FP4, MH) do { if (nt == 2) DT_FEW(FP4, MH, 2); else DT_FEW(FP4, MH, 1); } while (0)
+#define DT_FEW(FP4, MH, NT, UP) return launch_instance<FP4, MH, NT, UP>(a, b, sfa, sfb, M, N, K, lda, ldb, o, ldo, groups, grid, stagger, stream)
+#define DT_FEW_U(FP4, MH, NT)                                                      \
+  do {                                                                             \
+    if constexpr (MH <= 4 && few_rows_lds_bytes(FP4, (MH + 1) / 2, 2) < kLdsLimit) { if (p.up == 2) DT_FEW(FP4, MH, NT, 2); } \
+    DT_FEW(FP4, MH, NT, 1);                                                        \
+  } while (0)
+#define DT_FEW_N(FP4, MH) do { if (p.nt == 2) DT_FEW_U(FP4, MH, 2); else DT_FEW_U(FP4, MH, 1); } while (0)
 #define DT_FEW_M(FP4)                         \
   do {                                        \
     switch (mh) {                             \
+      case 1: DT_FEW_N(FP4, 1);               \
+      case 2: DT_FEW_N(FP4, 2);               \
+      case 3: DT_FEW_N(FP4, 3);               \
+      case 4: DT_FEW_N(FP4, 4);               \
       case 5: DT_FEW_N(FP4, 5);               \
       case 6: DT_FEW_N(FP4, 6);               \
       case 7: DT_FEW_N(FP4, 7);               \
@@ -419,6 +444,7 @@ int launch_few_rows(bool fp4, const uint8_t* a, const uint8_t* b, const uint8_t*
   else DT_FEW_M(false);
 #undef DT_FEW_M
 #undef DT_FEW_N
+#undef DT_FEW_U
 #undef DT_FEW
   return DT_ERR_LAUNCH;  // not reached
 }

@@ -26,7 +26,7 @@ enum GemmTiles {
   kTiles256ThenQuads,        // whole rounds of 256 x 256, the tiles left over as 128 x 128 quadrants
   kTiles256ThenHalves,       // or as halves
   kTiles256QuadrantSchedule,  // 256 x 256 on the other tiles' main loop (on request only)
-  kFewRows,                  // the kernel for 33 to 64 rows (mx_few_rows.hip)
+  kFewRows,                  // the kernel for at most 64 rows that loads B into registers (mx_few_rows.hip)
   kFewLines                  // the one for at most 32 rows by whole lines, in the form that plan_few_lines gives
 };
 
@@ -147,7 +147,7 @@ inline int ring_cols(const RingPlan& p, bool fp4, int64_t M, int64_t N, int64_t 
   return 8 * ceil_div(N, (int64_t)fit) >= 9 * tiles_n ? fit : p.tile_n;
 }
 
-// What the kernel for 33 to 64 rows (mx_few_rows.hip) takes, in nanoseconds.  Its workgroups walk whole rows of
+// What the kernel of mx_few_rows.hip takes for a product of at most 64 rows, in nanoseconds.  Its workgroups walk whole rows of
 // B, 16 or 32 columns each, with all of A beside them: per round of the chip 2.3 us, and per step and column 5.5 ns (5.2 off
 // whole lines, where the rows do not begin on the same channels) and 1.6 ns per row of A.  columns: of a workgroup.
 inline int64_t few_rows_ns(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, int cus, int columns) {
@@ -180,6 +180,19 @@ inline FewLinesPlan plan_few_lines(bool fp4, int64_t M, int64_t N, int64_t K, bo
   return best;
 }
 
+// Which of the two kernels a product of at most 32 rows is for: the one of mx_few_rows.hip keeps the short rows of few columns that are no whole lines,
+// a workgroup of 16 columns per CU at most.  A wave by whole lines asks for a window more than it has steps there, and reads a step's fragments out of two;
+// the other one has 16 steps of at most 16 rows in its waves' first turn (us, by whole lines and there, from memory / from the
+// memory-side cache: e2m1 32 x 280 x 544 3.42 / 3.67 and 2.77 / 3.00, 19 x 2520 x 1344 3.90 / 3.72 and 3.47 / 3.12, 30 x 2368 x 4576 7.05 / 5.97 and 6.64 / 4.65,
+// 4 x 3872 x 2720 4.78 / 3.88 and 4.71 / 3.28, e4m3 25 x 400 x 320 3.16 / 3.33 and 2.81 / 2.95, 1 x 3168 x 1120 4.19 / 3.61 and 4.08 / 3.23).  Of 519 problems
+// of 1 to 32 rows drawn at random, half of them on whole lines, none of these is faster there by more than 3 %, and beyond these limits none
+// by more than 7 %.
+inline bool few_rows_instead_of_lines(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, int cus) {
+  const int64_t steps = ceil_div(fp4 ? K / 2 : K, (int64_t)kBK);
+  if (!ragged || N > 16 * (int64_t)cus) return false;
+  return steps <= (fp4 && M > 16 ? 24 : 16) && (fp4 || M > 16 || steps > 8);
+}
+
 struct GemmKnobs {  // gemm.variant, gemm.tail_quads, gemm.split_k, gemm.tile_m, gemm.tile_n, gemm.few_rows_octets
   int variant, tail, split_k, tile_m, tile_n, octets = 0;
 };
@@ -190,7 +203,8 @@ struct GemmPlan {
 };
 
 // K counts elements; ragged: see ring_ragged; workspace_bytes 0: none; few_columns: columns of B that a workgroup of the kernel for at most 64 rows
-// takes, 0 where it cannot take the product; few_lines: whether the one for at most 32 can, which then stands in its place.
+// takes, 0 where it cannot take the product; few_lines: whether the one for at most 32 can, which then stands in its place unless
+// few_rows_instead_of_lines.
 // Either is taken where it needs less time than the small tiles.  Those read B at 4.8 TB/s from memory at most, and at 6.5 to 7.3 from the memory-side cache: the
 // first is also taken where it needs less than reading B at 4.8 TB/s, the second than at 5.5, which is in between (us, small tiles and by
 // whole lines, 16 x 28672 x 4096 28.0 / 19.5 and 22.8 / 19.5; with 4.8 here 18 x 21728 x 8992 is lost, 38.4 / 30.1 and 40.2 / 36.7).
@@ -200,8 +214,8 @@ struct GemmPlan {
 // and 1.7 %, 50 % at most: e2m1 12 x 1488 x 12064 from the cache 8.9 and 6.9 us, 1 x 168 x 10048 7.6 and 5.1, from memory 7.9 and 6.4.
 // A rule on sizes, few rows for K of 2048 and N of 1024 on with exceptions, took 27 % longer on the 150.
 // Up to 32 rows: of the 161 problems that plan_few_lines is fitted to, what the estimates pick takes 1.2 / 2.2 % longer than the best of the three kernels
-// (from memory / from the cache), and 0.91 / 0.91 of what it took without the kernel by whole lines.  What that one loses to the other one for few rows
-// are products of 3 to 4 us, 17 % at most from memory: e2m1 4 x 3872 x 2720 3.9 and 4.1, 15 x 2576 x 1312 3.4 and 3.7.)
+// (from memory / from the cache), and 0.91 / 0.91 of what it took without the kernel by whole lines.  What that one lost to the other one for few
+// rows stays with it.)
 // How many workgroups are to share K does not decide between the two; whether any may does.
 inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, size_t workspace_bytes, int cus, int few_columns, bool few_lines,
                           GemmKnobs knobs) {
@@ -212,10 +226,12 @@ inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged
   };
   if (knobs.variant == 1) return small(knobs.split_k, 128, 128);
   if (knobs.variant == 3) return small(knobs.split_k, knobs.tile_m, knobs.tile_n);
+  if (few_columns && knobs.variant == 10) return {kFewRows, {}};
   if (few_columns && (knobs.variant == 9 || knobs.variant == 0)) {
     GemmPlan few{kFewRows, {}};
     int64_t few_ns = 0;
-    if (few_lines) {
+    const bool by_lines = few_lines && (knobs.octets || !few_rows_instead_of_lines(fp4, M, N, K, ragged, cus));
+    if (by_lines) {
       few = {kFewLines, {}, plan_few_lines(fp4, M, N, K, ragged, cus, knobs.octets)};
       few_ns = few.lines.ns;
     } else {
@@ -224,7 +240,7 @@ inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged
     }
     if (knobs.variant == 9) return few;
     const GemmPlan tiles = small(knobs.split_k == 1 ? 1 : 0, 0, 0);
-    if (few_ns < std::max(tiles.small.ns, few_lines ? 3000 + N * (fp4 ? K / 2 : K) / 5500 : 0)) return few;
+    if (few_ns < std::max(tiles.small.ns, by_lines ? 3000 + N * (fp4 ? K / 2 : K) / 5500 : 0)) return few;
     return knobs.split_k > 1 ? small(knobs.split_k, 0, 0) : tiles;
   }
   const GemmTiles tiles = plan_tiles(fp4, M, N, K, ragged, cus, knobs.variant, knobs.tail);

@@ -84,11 +84,25 @@ def test_rows_off_the_lines_take_small_tiles_instead_of_halves(plan, fp4):
 def test_few_rows(plan):
     for M in (1, 16, 32, 33, 48):
         assert plan(True, M, 2048, 4096, few=16)[0] == (FEW_LINES if M <= 32 else FEW_ROWS) and plan(True, M, 2048, 4096)[0] == SMALL
-        assert plan(False, M, 64, 64, few=16, variant=9)[0] == (FEW_LINES if M <= 32 else FEW_ROWS)
+        assert plan(False, M, 64, 128, few=16, variant=9)[0] == (FEW_LINES if M <= 32 else FEW_ROWS)
     assert plan(False, 100, 64, 64, variant=9)[0] == SMALL
     for variant, tiles in ((1, SMALL), (2, T256), (3, SMALL), (5, T192), (7, QUADRANT_SCHEDULE)):
         for M in (16, 40):
             assert plan(False, M, 8192, 8192, few=32, variant=variant)[0] == tiles
+
+
+def test_short_rows_off_the_lines_keep_the_kernel_that_loads_b_into_registers(plan):
+    """of at most 32 rows, those of up to 16 columns per CU and of few steps"""
+    for fp4, M, steps in ((True, 1, 16), (True, 16, 16), (True, 17, 24), (True, 32, 24), (False, 16, 16), (False, 17, 16), (False, 32, 16)):
+        step = 256 if fp4 else 128
+        for N in (8, 1024, 4096):
+            for n, off in ((steps, 32), (steps + 1, 32), (steps, step)):
+                few = plan(fp4, M, N, (n - 1) * step + off, few=16)[0]
+                assert few == (FEW_ROWS if n == steps and off == 32 else FEW_LINES), (fp4, M, N, n, off)
+        assert plan(fp4, M, 4104, (steps - 1) * step + 32, few=16, variant=9)[0] == FEW_LINES
+        assert plan(fp4, M, 4104, steps * step, few=16, variant=10)[0] == FEW_ROWS
+    assert plan(False, 16, 1024, 9 * 128 - 96, few=16)[0] == FEW_ROWS and plan(False, 16, 1024, 8 * 128 - 96, few=16)[0] == FEW_LINES
+    assert plan(False, 17, 1024, 32, few=16)[0] == FEW_ROWS and plan(True, 1, 1024, 32, few=16)[0] == FEW_ROWS
 
 
 def test_shares_own_a_step_and_fit_the_workspace(plan):

@@ -293,11 +293,12 @@ def test_mx_gemm_ignores_the_padding_of_the_scale_buffers(d, cabi, variant, size
 @pytest.mark.parametrize("size", [(1, 640, 8), (16, 2048, 256), (17, 96, 2056), (33, 1120, 264), (48, 416, 136), (64, 8192, 512),
                                   (5, 32, 24), (64, 160, 16), (8, 416, 264), (9, 288, 40), (24, 1120, 136), (28, 416, 264),
                                   (40, 2048, 64), (52, 160, 520), (56, 2080, 72)], ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
-def test_mx_gemm_few_rows_kernel(d, cabi, size):
-    """the kernel for problems of at most 64 rows (16 columns per workgroup, K shared between its eight
-    waves, operands straight from memory): every count of 8-row halves of A's tiles, ragged M and N, K with a partly
+@pytest.mark.parametrize("variant", [9, 10])
+def test_mx_gemm_few_rows_kernel(d, cabi, size, variant):
+    """the kernels for problems of at most 64 rows, the one that the rule takes (9) and the one with 16 columns per workgroup, K shared between its
+    eight waves, B straight from memory (10): every count of 8-row halves of A's tiles, ragged M and N, K with a partly
     filled last 128-element step; forced here for every N, and checked against the exact product"""
-    cabi.set_tuning("gemm.variant", 9)
+    cabi.set_tuning("gemm.variant", variant)
     try:
         _check_gemm(d, *size, 2100 + size[0], "randn")
     finally:
@@ -313,7 +314,7 @@ def test_mx_gemm_few_rows_kernel_walks_many_column_groups(d, cabi, size, knobs):
     the first batch of the next one already on its way while it adds up and stores the one in hand (the sums
     are parked in the LDS set that has just been used up); every launch shape, with and without the staggered
     walk along K; the exact product, and the same bits on a second call"""
-    cabi.set_tuning("gemm.variant", 9)
+    cabi.set_tuning("gemm.variant", 10)
     for k, v in knobs.items():
         cabi.set_tuning("gemm.few_rows_" + k, v)
     try:
@@ -349,7 +350,7 @@ def test_mx_gemm_few_rows_kernel_is_the_default_and_respects_strides(d, cabi):
 
 
 @pytest.mark.parametrize("fp4", [False, True], ids=["e4m3", "e2m1"])
-@pytest.mark.parametrize("size", [(24, 2048, 8192), (16, 4096, 4096), (40, 4096, 4096)], ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
+@pytest.mark.parametrize("size", [(24, 2048, 8192), (16, 4096, 4096), (40, 4096, 4096), (24, 1312, 2048)], ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
 def test_mx_gemm_split_k_leaves_the_few_rows_kernel_alone(d, cabi, size, fp4):
     """gemm.split_k says how the small tiles share K: a product that takes the kernel for few rows takes it under any factor (the order of
     its sums is its own, so the bits tell)"""
@@ -767,8 +768,9 @@ def test_mx_gemm_small_vs_c_oracle_exact_products(d):
 
 @pytest.mark.parametrize("size", [(16, 256, 136), (40, 352, 264), (64, 1152, 48)], ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
 @pytest.mark.parametrize("tiles", [1, 2])
-def test_mx_gemm_few_rows_kernel_vs_c_oracle_exact_products(d, cabi, size, tiles):
-    """the kernel for few rows on operands whose products and partial sums are exact (see the test above):
+@pytest.mark.parametrize("variant", [9, 10])
+def test_mx_gemm_few_rows_kernel_vs_c_oracle_exact_products(d, cabi, size, tiles, variant):
+    """the kernels for few rows on operands whose products and partial sums are exact (see the test above):
     bit for bit the C oracle's float64 reference rounded to bf16, for one and two 16-column tiles per
     wave and a K with a partly filled last step"""
     M, K, N = size
@@ -779,7 +781,7 @@ def test_mx_gemm_few_rows_kernel_vs_c_oracle_exact_products(d, cabi, size, tiles
     b = b * (torch.rand(N, K, generator=g) < 0.5)
     ad, asc = d.mx_fp8_quantize(a.bfloat16().cuda())
     bd, bsc = d.mx_fp8_quantize(b.bfloat16().cuda())
-    cabi.set_tuning("gemm.variant", 9)
+    cabi.set_tuning("gemm.variant", variant)
     cabi.set_tuning("gemm.few_rows_tiles", tiles)
     try:
         out = d.mx_fp8_bf16(ad, bd.t(), d.to_blocked(asc.view(M, K // 32)), d.to_blocked(bsc.view(N, K // 32)))

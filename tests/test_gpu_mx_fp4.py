@@ -91,15 +91,16 @@ def test_mx_fp4_gemm_k_of_any_whole_number_of_blocks(d, cabi, variant, K):
 @pytest.mark.parametrize("size", [(1, 640, 8), (16, 2048, 256), (17, 96, 2056), (33, 1312, 264), (48, 480, 136), (64, 8192, 512),
                                   (5, 32, 24), (24, 4128, 4104), (8, 480, 264), (28, 416, 264), (40, 2048, 64), (52, 160, 520),
                                   (56, 2080, 72)], ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
-def test_mx_fp4_gemm_few_rows_kernel(d, cabi, size):
-    """the kernel for problems of at most 64 rows, forced for every N (the last size takes it by default
-    too): every count of 16-row tiles, ragged M and N, K with a partly filled last 128-element step"""
-    cabi.set_tuning("gemm.variant", 9)
+@pytest.mark.parametrize("variant", [9, 10])
+def test_mx_fp4_gemm_few_rows_kernel(d, cabi, size, variant):
+    """the kernels for problems of at most 64 rows, the rule's (9; one size takes it by default too) and the one that loads B into registers (10), forced for
+    every N: every count of 16-row tiles, ragged M and N, K with a partly filled last 128-element step"""
+    cabi.set_tuning("gemm.variant", variant)
     try:
         out = _check(d, *size, 2300 + size[0], "randn")
     finally:
         cabi.set_tuning("gemm.variant", 0)
-    if size[2] >= 4096:
+    if size[2] >= 4096 and variant == 9:
         assert torch.equal(_check(d, *size, 2300 + size[0], "randn"), out)
 
 
@@ -149,12 +150,13 @@ def test_mx_fp4_gemm_bit_exact_when_sums_fit_fp32(d):
 
 
 @pytest.mark.parametrize("tiles", [1, 2])
-def test_mx_fp4_gemm_few_rows_kernel_bit_exact_when_sums_fit_fp32(d, cabi, tiles):
-    """the kernel for few rows on the operands of the test above (exact in fp32 in any order): bit for bit
+@pytest.mark.parametrize("variant", [9, 10])
+def test_mx_fp4_gemm_few_rows_kernel_bit_exact_when_sums_fit_fp32(d, cabi, tiles, variant):
+    """the kernels for few rows on the operands of the test above (exact in fp32 in any order): bit for bit
     the C oracle's reference, for one and two 16-column tiles per wave, every count of 16-row tiles and a K
     with a partly filled last 128-element step"""
     g = util.gen(92)
-    cabi.set_tuning("gemm.variant", 9)
+    cabi.set_tuning("gemm.variant", variant)
     cabi.set_tuning("gemm.few_rows_tiles", tiles)
     try:
         for (M, K, N) in ((16, 384, 136), (33, 480, 264), (64, 1312, 48), (50, 512, 40)):
