@@ -165,7 +165,10 @@ struct FewLinesPlan {
 // Per round of the chip a workgroup's turns along K take what its waves take for one, or 2.3 ns per line that they ask for, and all
 // rounds together no less than B at 5.7 TB/s; per group the sums' way through LDS.  The constants are a fit to 161 problems of 1 to 32 rows, 512 to 28672
 // columns and K of 512 to 16384, both operand types, on and off whole lines, in all eight forms each, to the geometric mean of the time with B from memory and from
-// the memory-side cache: the form that it picks takes 0.3 % longer than the best one of each problem from memory and 0.7 % from the cache.
+// the memory-side cache: the form that it picks takes 0.3 % longer than the best one of each problem from memory and 0.7 % from the cache.  What it is held against is
+// 2 % more, 10 % for e4m3 off whole lines: of 799 problems of 1 to 32 rows, most of them where small tiles are close, the choice between the two then takes 0.18 % longer
+// than the shorter one (geometric mean of both; 0.51 % without it, with 22 problems more than 8 % longer instead of 6), e4m3 2 x 16904 x 1120 by lines 9.9 / 7.0 and
+// small tiles 8.2 / 5.9 us, 18 x 1480 x 15328 15.9 / 11.4 and 12.2 / 10.6.
 inline FewLinesPlan plan_few_lines(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged, int cus, int octets) {
   const int64_t k_bytes = fp4 ? K / 2 : K, steps = ceil_div(k_bytes, (int64_t)kBK);
   const int mh = (int)((M + 7) / 8), rows_tiles = (mh + 1) / 2;
@@ -177,6 +180,7 @@ inline FewLinesPlan plan_few_lines(bool fp4, int64_t M, int64_t N, int64_t K, bo
     const int64_t ns = 1770 + rounds * (125 + 190 * tiles) + std::max(rounds * turns * turn, N * k_bytes * 10 / 57000);
     if (!best.octets || ns < best.ns) best = FewLinesPlan{nh, ns};
   }
+  best.ns = best.ns * (ragged && !fp4 ? 110 : 102) / 100;
   return best;
 }
 
@@ -206,7 +210,7 @@ struct GemmPlan {
 // takes, 0 where it cannot take the product; few_lines: whether the one for at most 32 can, which then stands in its place unless
 // few_rows_instead_of_lines.
 // Either is taken where it needs less time than the small tiles.  Those read B at 4.8 TB/s from memory at most, and at 6.5 to 7.3 from the memory-side cache: the
-// first is also taken where it needs less than reading B at 4.8 TB/s, the second than at 5.5, which is in between (us, small tiles and by
+// first is also taken where it needs less than reading B at 4.8 TB/s, the second than at 5.2, which is in between (us, small tiles and by
 // whole lines, 16 x 28672 x 4096 28.0 / 19.5 and 22.8 / 19.5; with 4.8 here 18 x 21728 x 8992 is lost, 38.4 / 30.1 and 40.2 / 36.7).
 // (33 to 64 rows: fitted to 150 problems of 1 to 64 rows, and off whole lines to 340: at 350 others of 128 to 12000 columns drawn at random, half of them of
 // few columns and a long K, where the choice is close, what the two estimates pick takes 0.2 % longer than the better kernel with B from memory,
@@ -240,7 +244,7 @@ inline GemmPlan plan_gemm(bool fp4, int64_t M, int64_t N, int64_t K, bool ragged
     }
     if (knobs.variant == 9) return few;
     const GemmPlan tiles = small(knobs.split_k == 1 ? 1 : 0, 0, 0);
-    if (few_ns < std::max(tiles.small.ns, by_lines ? 3000 + N * (fp4 ? K / 2 : K) / 5500 : 0)) return few;
+    if (few_ns < std::max(tiles.small.ns, by_lines ? 2700 + N * (fp4 ? K / 2 : K) / 5200 : 0)) return few;
     return knobs.split_k > 1 ? small(knobs.split_k, 0, 0) : tiles;
   }
   const GemmTiles tiles = plan_tiles(fp4, M, N, K, ragged, cus, knobs.variant, knobs.tail);
