@@ -32,7 +32,7 @@ const DeviceFacts& device_facts();  // of the current device, cached per device
 //                 workgroups and so assumes that this process has the GPU to itself: 0 unless the caller
 //                 opts in (dt_set_exclusive_gpu, or DRISS_TORCH_RESIDENT=1 in the environment when the
 //                 library is loaded); dynamic.resident_min_kib = smallest such
-//                 tensor; sizes in [resident_gap_lo_kib, resident_gap_hi_kib) take the two kernels
+//                 tensor (-1: as measured, 58 MiB, of 16-bit tensors to both types 52); sizes in [resident_gap_lo_kib, resident_gap_hi_kib) take the two kernels
 //                 dynamic.resident_overflow: 1 = tensors of up to 4 x the chip's capacity keep what fits
 //                 and read only the rest twice
 //   amax.blocks_per_cu: most workgroups per CU of a reduction in workgroups of 256 or 512 threads (those of 1024 are at
@@ -87,7 +87,7 @@ const DeviceFacts& device_facts();  // of the current device, cached per device
   X(gemm, split_k, 0)                      \
   X(gemm, tail_quads, 1)                   \
   X(dynamic, resident, 0)                  \
-  X(dynamic, resident_min_kib, 32768)      \
+  X(dynamic, resident_min_kib, -1)         \
   X(dynamic, resident_gap_lo_kib, 0)       \
   X(dynamic, resident_gap_hi_kib, 0)       \
   X(dynamic, resident_overflow, 1)         \

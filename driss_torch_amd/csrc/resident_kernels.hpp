@@ -563,14 +563,19 @@ inline int launch_resident_impl(const void* x, int64_t numel, void* ws, void* ou
   }
 }
 
+// The smallest tensor that takes the kernel.  Below, the two kernels win: the cast's second read of x comes out of the caches faster than this kernel's barrier
+// and its launch with 144 KB of LDS cost, the more so since the cast takes the maxima of the reduction's workgroups itself.  us, this kernel and the two, buffers
+// rotated through memory: bf16 to one type 32 MiB 17.2 and 12.5, 48 MiB 20.5 and 18.9, 56 MiB 22.6 and 22.0, 58 MiB 22.9 and 23.0, 60 MiB 23.2 and
+// 23.4, 64 MiB 23.4 and 24.7, 96 MiB 31.2 and 36.7; to both 32 MiB 19.6 and 14.7, 48 MiB 23.3 and 22.9, 52 MiB 24.7 and 24.8, 56 MiB 24.9 and 26.5, 64 MiB
+// 27.2 and 29.8; fp32 to one 56 MiB 20.3 and 19.5, 58 MiB 20.5 and 20.4, 62 MiB 20.9 and 21.6, to both 56 MiB 21.8 and 21.4, 58 MiB 22.0 and 22.2.
+inline int64_t resident_min_bytes(int in_dtype, bool pair) {
+  const int64_t kib = tuning(Knob::dynamic_resident_min_kib);
+  return kib >= 0 ? kib * 1024 : (int64_t)(pair && in_dtype != DT_F32 ? 52 : 58) << 20;
+}
+
 template <bool PAIR>
 inline int launch_resident(const void* x, int in_dtype, int64_t numel, int out_dtype, int round_mode, void* ws, void* out,
                            void* out2, float* amax_out, float* scale_out, float fmax0, float fmax1, hipStream_t stream) {
-  // Where the two kernels win: below about 32 MiB the cast's second read of x comes out of the caches faster than this kernel's barrier
-  // and its launch with 144 KB of LDS cost.  Since the cast takes the maxima of the reduction's workgroups itself that holds up to 56 MiB with one output and
-  // 48 with both (us, this kernel against the two, both fp8 outputs / one, bf16: 32 MiB 19.5 vs 16.0 / 17.2 vs 12.6, 40 MiB 21.5 vs 21.1 / 19.3 vs 16.7, 48 MiB
-  // 22.9 vs 24.4 / 20.4 vs 18.8, 56 MiB 25.8 vs 28.0 / 22.6 vs 21.9, 64 MiB 27.4 vs 31.3 / 23.4 vs 26.4, 96 MiB 36.8 vs 45.8 / 31.0 vs 38.0, 128 MiB 43.7 vs
-  // 60.1 / 36.0 vs 50.3); the size from which a caller that has opted in gets the one kernel is part of what it was told, and the knob moves it.
   const int64_t bytes = numel * (in_dtype == DT_F32 ? 4 : 2);
   // An earlier launch of the one-kernel path on this device gave up waiting for the whole chip (its
   // outputs are NaN): say so once, and leave the path off for the rest of the process.
@@ -578,7 +583,7 @@ inline int launch_resident(const void* x, int in_dtype, int64_t numel, int out_d
     (void)dt_set_tuning("dynamic.resident", 0);
     return DT_ERR_RESIDENT_GAVE_UP;
   }
-  if (!tuning(Knob::dynamic_resident) || bytes < (int64_t)tuning(Knob::dynamic_resident_min_kib) * 1024) return kResidentNotTaken;
+  if (!tuning(Knob::dynamic_resident) || bytes < resident_min_bytes(in_dtype, PAIR)) return kResidentNotTaken;
   if (bytes >= (int64_t)tuning(Knob::dynamic_resident_gap_lo_kib) * 1024 && bytes < (int64_t)tuning(Knob::dynamic_resident_gap_hi_kib) * 1024)
     return kResidentNotTaken;
 #define DT_RES(IN, OUT, RB, RS) \

@@ -224,13 +224,13 @@ def test_resident_not_taken_on_a_stream_restricted_to_some_cus(cabi):
 def test_one_kernel_path_needs_the_opt_in(gpu_device):
     """without the opt-in (dt_set_exclusive_gpu / DRISS_TORCH_RESIDENT) the torch op and the C ABI never
     launch the kernel that waits for the whole chip, whatever the tensor's size: they run the reduction and
-    the cast, with the same bits; with it a tensor of 32 MiB and more takes the one kernel"""
+    the cast, with the same bits; with it a tensor of 58 MiB and more takes the one kernel (of 16 bits to both types: 52 MiB)"""
     import driss_torch_amd as d
     from driss_torch_amd import cabi as c
 
     L = c.lib()
     keep = L.dt_get_exclusive_gpu()
-    x = util.normal_with_outliers((4096, 4096), 5)  # 32 MiB of bf16: the smallest size of the one-kernel path
+    x = util.normal_with_outliers((7424, 4096), 5)  # 58 MiB of bf16: the smallest size of the one-kernel path
     xg = x.cuda()
     ref, ramax, _ = co.dynamic_scaled_quant(x, E4, co.ROUND_V2)
     try:
@@ -248,6 +248,13 @@ def test_one_kernel_path_needs_the_opt_in(gpu_device):
         torch.cuda.synchronize()
         assert L.dt_dynamic_quant_resident_launches() == n0 + 1
         assert torch.equal(util.codes(out), ref)
+        for bits, mib, pair in ((16, 58, False), (16, 52, True), (32, 58, False), (32, 58, True)):
+            big = torch.ones(mib << 20, dtype=torch.uint8, device=gpu_device).view(torch.bfloat16 if bits == 16 else torch.float32)
+            for t, taken in ((big, 1), (big[:-8], 0)):
+                n0 = L.dt_dynamic_quant_resident_launches()
+                d.dynamic_scaled_quant_pair(t) if pair else d.dynamic_scaled_quant(t, E4)
+                torch.cuda.synchronize()
+                assert L.dt_dynamic_quant_resident_launches() == n0 + taken, (bits, mib, pair)
     finally:
         L.dt_set_exclusive_gpu(keep)
 
