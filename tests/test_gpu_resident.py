@@ -250,7 +250,7 @@ def test_one_kernel_path_needs_the_opt_in(gpu_device):
         assert torch.equal(util.codes(out), ref)
         for bits, mib, pair in ((16, 58, False), (16, 52, True), (32, 58, False), (32, 58, True)):
             big = torch.ones(mib << 20, dtype=torch.uint8, device=gpu_device).view(torch.bfloat16 if bits == 16 else torch.float32)
-            for t, taken in ((big, 1), (big[:-8], 0)):
+            for t, taken in ((big.view(1, -1), 1), (big[:-8].view(1, -1), 0)):
                 n0 = L.dt_dynamic_quant_resident_launches()
                 d.dynamic_scaled_quant_pair(t) if pair else d.dynamic_scaled_quant(t, E4)
                 torch.cuda.synchronize()
