@@ -218,8 +218,8 @@ inline int reduction_grid(int64_t nvec, int block, int unroll, Knob knob) {
   return want < 1 ? 1 : (int)want;
 }
 
-// Enqueue the amax reduction.  nscales: 0 = amax only, 1 = scale for fmax0, 2 = both.  partials (with scales): leave the workgroups' maxima for the cast,
-// whose number goes there; without the atomics, workgroups of 256 threads on every CU are the best ones at any size.
+// Enqueue the amax reduction.  nscales: 0 = amax only, 1 = scale for fmax0, 2 = both.  PARTIALS (with scales): leave the workgroups' maxima for the cast,
+// their number in *partials; without the atomics, workgroups of 256 threads on every CU are the best ones at any size.
 //
 // Streaming or cacheable loads: a cast of the same tensor follows nearly every reduction (always when
 // scales are asked for), and its workgroups walk the tensor in the reduction's order, so that a run of
@@ -237,7 +237,7 @@ inline int reduction_grid(int64_t nvec, int block, int unroll, Knob knob) {
 // the cast 6.3 -> 6.1, 2 MiB 4.4 -> 4.1 and 6.6 -> 6.2, 4 MiB 4.8 -> 4.5 and 7.3 -> 7.0; 5 MiB 5.8 -> 5.5 and 8.4 -> 8.2,
 // but out of the caches 6.2 -> 7.1 with the cast; 1 MiB, which comes out of the caches anyway, 3.6 -> 3.8).
 constexpr int64_t kAmaxCacheableBytes = (int64_t)40 << 20, kAmaxStreamedFrom = (int64_t)3 << 19, kAmaxStreamedTo = (int64_t)4 << 20;
-template <int IN>
+template <int IN, bool PARTIALS = false>
 inline int launch_amax(const void* x, int64_t numel, void* ws, float* amax_out, float* scale_out, int nscales,
                        float fmax0, float fmax1, hipStream_t stream, int* partials = nullptr) {
   constexpr int kUnroll = 8;
@@ -252,22 +252,26 @@ inline int launch_amax(const void* x, int64_t numel, void* ws, float* amax_out, 
   // large workgroups stay ahead up to 96 MiB (both kernels, one output: 63 MiB 27.8 -> 26.4, 80 MiB 34.3 -> 32.4,
   // 95 MiB 40.3 -> 38.9; both outputs 47.8 -> 46.9, at 128 MiB 61.4 -> 61.7).
   const int64_t small_blocks = ceil_div(sp.nvec, (int64_t)kBlock * kUnroll);  // of 32 KiB
-  const int block = partials || small_blocks <= 64 || small_blocks > (nscales ? 3072 : 2048) ? 256 : small_blocks <= 128 ? 512 : 1024;
+  const int block = PARTIALS || small_blocks <= 64 || small_blocks > (nscales ? 3072 : 2048) ? 256 : small_blocks <= 128 ? 512 : 1024;
   int grid = reduction_grid(sp.nvec, block, kUnroll, Knob::amax_blocks_per_cu);
   if (block == 1024) grid = std::min(grid, std::max(8, device_facts().cu_count * 5 / 64 * 8));
   uint8_t* w = static_cast<uint8_t*>(ws);
   const int64_t bytes = numel * InTraits<IN>::kBytes;
-  if (partials) *partials = grid = std::min(grid, kWsPartialWords);
+  if constexpr (PARTIALS) *partials = grid = std::min(grid, kWsPartialWords);
   const bool nt = nscales == 0 ? bytes > kAmaxCacheableBytes || (bytes >= kAmaxStreamedFrom && bytes <= kAmaxStreamedTo)
                                : tuning(Knob::amax_stream_before_cast) != 0;
   uint64_t* const log = phase_log((size_t)grid * 32);
 #define DT_AMAX_B(NS, NT, B) launcher(amax_kernel<IN, B, kUnroll, NS, NT>, grid, B, 0, stream)(x, sp, w, amax_out, scale_out, fmax0, fmax1, log)
 #define DT_AMAX(NS, NT) do { if (block == 1024) DT_AMAX_B(NS, NT, 1024); else if (block == 512) DT_AMAX_B(NS, NT, 512); else DT_AMAX_B(NS, NT, 256); } while (0)
-  if (partials) { if (nt) DT_AMAX_B(kPartials, true, 256); else DT_AMAX_B(kPartials, false, 256); }
-  else if (nscales == 0) { if (nt) DT_AMAX(0, true); else DT_AMAX(0, false); }
-  else if (nscales == 1) { if (nt) DT_AMAX(1, true); else DT_AMAX(1, false); }
-  else { if (nt) DT_AMAX(2, true); else DT_AMAX(2, false); }
+  if constexpr (PARTIALS) {
+    if (nt) DT_AMAX_B(kPartials, true, 256); else DT_AMAX_B(kPartials, false, 256);
+  } else {
+    if (nscales == 0) { if (nt) DT_AMAX(0, true); else DT_AMAX(0, false); }
+    else if (nscales == 1) { if (nt) DT_AMAX(1, true); else DT_AMAX(1, false); }
+    else { if (nt) DT_AMAX(2, true); else DT_AMAX(2, false); }
+  }
 #undef DT_AMAX
+#undef DT_AMAX_B
   return launch_status();
 }
 
@@ -343,7 +347,7 @@ __device__ __forceinline__ uint8_t cast_one(const void* x, int64_t i, float s) {
 // Aligned streaming cast: x 16-byte aligned, out aligned to its packed store.  The tail
 // (< one vector) is done by the first workgroup.  With PAIR the same read also feeds a
 // second output of the other fp8 type with its own scale (scale[1], out2).
-// Where the scale comes from when the reduction in front left its workgroups' maxima in the workspace (PARTIALS; `scale` points to them): every workgroup
+// Where the scale comes from when the reduction in front left its workgroups' maxima in the workspace (FROM: a FromPartials; `scale` points to them): every workgroup
 // takes their maximum while its first loads of x are under way, the first one writes amax and the scales out.  The kernel boundary is all that
 // the two kernels need between them: the reduction ends without its two dependent atomics per workgroup on one address (0.65 us each, and a queue), and
 // may have all CUs read.  us, both kernels, amax and scales by the last workgroup -> here, rotated buffers: bf16 to one type 512 x 512 5.05 -> 4.30,
@@ -354,10 +358,11 @@ struct FromPartials {
   float fmax0 = 0.f, fmax1 = 0.f;
   float *amax_out = nullptr, *scale_out = nullptr;
 };
-template <int IN, int OUT, bool ROUND_BF16, bool ROUND_SCALE, bool PAIR, int UNROLL, bool PARTIALS = false>
+template <int IN, int OUT, bool ROUND_BF16, bool ROUND_SCALE, bool PAIR, int UNROLL, typename... FROM>
 __global__ __launch_bounds__(kBlock) void cast_kernel(const void* __restrict__ x, int64_t nvec, int64_t tail,
                                                       const float* __restrict__ scale, uint8_t* __restrict__ out,
-                                                      uint8_t* __restrict__ out2, FromPartials from) {
+                                                      uint8_t* __restrict__ out2, FROM... given) {
+  constexpr bool PARTIALS = sizeof...(FROM) != 0;
   constexpr int kV = InTraits<IN>::kVec;
   constexpr int OUT2 = OUT == DT_E4M3FN ? DT_E5M2 : DT_E4M3FN;
   saturate_fp8_conversions();
@@ -381,6 +386,7 @@ __global__ __launch_bounds__(kBlock) void cast_kernel(const void* __restrict__ x
   };
   u32x4 wa[P], wb[P];
   if constexpr (PARTIALS) {
+    const FromPartials from{given...};
     static_assert(kWsPartialWords <= kBlock, "a word per thread");
     __shared__ uint32_t lds[kBlock / kWave];
     uint32_t m = (int)threadIdx.x < from.count ? reinterpret_cast<const uint32_t*>(scale)[threadIdx.x] : 0u;
@@ -490,9 +496,10 @@ inline bool cast_takes_vectors(const void* x, const void* out, const void* out2)
   return aligned(x, 16) && aligned(out, kStoreAlign) && aligned(out2, kStoreAlign);  // (none: aligned)
 }
 
-template <int IN, int OUT, bool ROUND_BF16, bool ROUND_SCALE, bool PAIR>
+template <int IN, int OUT, bool ROUND_BF16, bool ROUND_SCALE, bool PAIR, typename... FROM>
 inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, void* out, void* out2,
-                            hipStream_t stream, const FromPartials& from) {
+                            hipStream_t stream, const FROM&... given) {
+  constexpr bool PARTIALS = sizeof...(FROM) != 0;  // the caller has checked the alignments then, and that there is a vector
   // Large tensors: batches of 4 loads per lane, software-pipelined (4..8 in flight), from ONE workgroup per
   // CU: the best point of the measured grid {1, 2, 4 workgroups per CU} (8192^2 bf16 32.5 / 32.9 / 36.0 us,
   // fp32 54.2 / 60.1 / 66 us, bf16 to both fp8 types 45.1 / 45.3 / 47.8 us); more in flight is slower.
@@ -506,9 +513,9 @@ inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, vo
   // 256 MiB 101.1 -> 99.5; beyond that they lose, 428 MiB both 212.7 and 215.5; four workgroups per CU: 32 MiB 14.3, fp32 256 MiB 102.5).
   uint8_t* o = static_cast<uint8_t*>(out);
   uint8_t* o2 = static_cast<uint8_t*>(out2);
-  if (cast_takes_vectors<IN>(x, out, out2)) {
+  if (PARTIALS || cast_takes_vectors<IN>(x, out, out2)) {
     const int64_t nvec = numel / InTraits<IN>::kVec, tail = numel % InTraits<IN>::kVec;
-    const bool small = from.count ? nvec * 16 <= (int64_t)256 << 20 : !PAIR && nvec * 16 < (int64_t)64 << 20;
+    const bool small = PARTIALS ? nvec * 16 <= (int64_t)256 << 20 : !PAIR && nvec * 16 < (int64_t)64 << 20;
     const int unroll_knob = tuning(Knob::cast_unroll);
     const int unroll = unroll_knob == 2 || unroll_knob == 4 ? unroll_knob : (small ? 2 : 4);
     const Knob knob = PAIR ? Knob::cast_pair_blocks_per_cu : Knob::cast_blocks_per_cu;
@@ -520,11 +527,11 @@ inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, vo
     // with 46 and 734 workgroups, 7.9 with 48 and 736)
     if (grid > 8) grid = ceil_div(grid, (int64_t)8) * 8;
     if (grid < 1) grid = 1;
-#define DT_CAST_AS(U, P) launcher(cast_kernel<IN, OUT, ROUND_BF16, ROUND_SCALE, PAIR, U, P>, (unsigned)grid, kBlock, 0, stream)(x, nvec, tail, scale, o, o2, from)
-    if (from.count) { if (unroll == 2) DT_CAST_AS(2, true); else DT_CAST_AS(4, true); }
-    else { if (unroll == 2) DT_CAST_AS(2, false); else DT_CAST_AS(4, false); }
+#define DT_CAST_AS(U) \
+  launcher(cast_kernel<IN, OUT, ROUND_BF16, ROUND_SCALE, PAIR, U, FROM...>, (unsigned)grid, kBlock, 0, stream)(x, nvec, tail, scale, o, o2, given...)
+    if (unroll == 2) DT_CAST_AS(2); else DT_CAST_AS(4);
 #undef DT_CAST_AS
-  } else {
+  } else if constexpr (!PARTIALS) {
     int64_t grid = ceil_div(numel / InTraits<IN>::kVec, (int64_t)kBlock);
     if (grid > device_facts().cu_count) grid = device_facts().cu_count;
     if (grid < 1) grid = 1;
@@ -534,11 +541,11 @@ inline int launch_cast_impl(const void* x, int64_t numel, const float* scale, vo
 }
 
 // Runtime (in_dtype, out_dtype, round_mode) -> template instance.  `pair` adds out2 of the
-// other fp8 type with scale[1].
-template <bool PAIR>
+// other fp8 type with scale[1].  given: a FromPartials, or nothing.
+template <bool PAIR, typename... FROM>
 inline int launch_cast(const void* x, int in_dtype, int64_t numel, const float* scale, int out_dtype,
-                       int round_mode, void* out, void* out2, hipStream_t stream, const FromPartials& from = {}) {
-#define DT_CAST(IN, OUT, RB, RS) return launch_cast_impl<IN, OUT, RB, RS, PAIR>(x, numel, scale, out, out2, stream, from)
+                       int round_mode, void* out, void* out2, hipStream_t stream, const FROM&... given) {
+#define DT_CAST(IN, OUT, RB, RS) return launch_cast_impl<IN, OUT, RB, RS, PAIR>(x, numel, scale, out, out2, stream, given...)
   if (in_dtype == DT_F32) {
     if (out_dtype == DT_E4M3FN) DT_CAST(DT_F32, DT_E4M3FN, false, false);
     DT_CAST(DT_F32, DT_E5M2, false, false);
@@ -562,15 +569,20 @@ template <bool PAIR>
 inline int launch_amax_cast(const void* x, int in_dtype, int64_t numel, int out_dtype, int round_mode, void* ws, void* out, void* out2,
                             float* amax_out, float* scale_out, float fmax0, float fmax1, hipStream_t stream) {
   const bool f32 = in_dtype == DT_F32;
-  int partials = 0;
-  const bool direct = numel >= 8 && (f32 ? cast_takes_vectors<DT_F32>(x, out, out2) : cast_takes_vectors<DT_BF16>(x, out, out2));
   const int nscales = PAIR ? 2 : 1;
-  const int st = f32 ? launch_amax<DT_F32>(x, numel, ws, amax_out, scale_out, nscales, fmax0, fmax1, stream, direct ? &partials : nullptr)
-                     : launch_amax<DT_BF16>(x, numel, ws, amax_out, scale_out, nscales, fmax0, fmax1, stream, direct ? &partials : nullptr);
-  if (st) return st;
   const uint8_t* const w = static_cast<const uint8_t*>(ws);
-  const float* scale = reinterpret_cast<const float*>(w + (direct ? kWsPartials : kWsScale));
-  return launch_cast<PAIR>(x, in_dtype, numel, scale, out_dtype, round_mode, out, out2, stream, FromPartials{partials, fmax0, fmax1, amax_out, scale_out});
+  if (numel >= 8 && (f32 ? cast_takes_vectors<DT_F32>(x, out, out2) : cast_takes_vectors<DT_BF16>(x, out, out2))) {
+    int partials = 0;
+    const int st = f32 ? launch_amax<DT_F32, true>(x, numel, ws, amax_out, scale_out, nscales, fmax0, fmax1, stream, &partials)
+                       : launch_amax<DT_BF16, true>(x, numel, ws, amax_out, scale_out, nscales, fmax0, fmax1, stream, &partials);
+    if (st) return st;
+    return launch_cast<PAIR>(x, in_dtype, numel, reinterpret_cast<const float*>(w + kWsPartials), out_dtype, round_mode, out, out2, stream,
+                             FromPartials{partials, fmax0, fmax1, amax_out, scale_out});
+  }
+  const int st = f32 ? launch_amax<DT_F32>(x, numel, ws, amax_out, scale_out, nscales, fmax0, fmax1, stream)
+                     : launch_amax<DT_BF16>(x, numel, ws, amax_out, scale_out, nscales, fmax0, fmax1, stream);
+  if (st) return st;
+  return launch_cast<PAIR>(x, in_dtype, numel, reinterpret_cast<const float*>(w + kWsScale), out_dtype, round_mode, out, out2, stream);
 }
 
 inline int check_cast_args(const void* x, int in_dtype, int64_t numel, int out_dtype, int round_mode, const void* out) {
